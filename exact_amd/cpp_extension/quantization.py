@@ -134,6 +134,9 @@ def tune_pack_geometry(data, bits, reps=5):
 def _pack_geometry(data, bits):
     """The split to ask for: the remembered one, after tuning when that is due."""
     key = (data.shape[1], bits)
+    octs = key[0] // 8
+    if key[0] % 8 or octs & (octs - 1):
+        return 0                     # the split is a choice only for a power of two of whole octs
     if key not in _PACK_GEOMETRY:
         if not (config.autotune_pack and data.is_cuda and data.numel() >= _TUNE_MIN_ELEMENTS
                 and len(pack_geometry_candidates(key[0])) > 1) or torch.cuda.is_current_stream_capturing():

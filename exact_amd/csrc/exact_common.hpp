@@ -21,6 +21,25 @@ __device__ __forceinline__ void nt_store4(float* p, float a, float b, float c, f
   __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
 }
 
+// The same width at any element boundary: rows whose length is no multiple of 16 bytes start anywhere.  The
+// hardware takes such accesses as one instruction (amdhsa runs with unaligned access on); what they cost is
+// the extra line where a piece straddles two, which neighbouring lanes of a contiguous run share anyway.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef half8 half8_any __attribute__((aligned(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+
+// x / d for x < 2^16 and 1 <= d < 2^16 as one multiply: m = ceil(2^32 / d).  The error x (m d - 2^32) / (d 2^32)
+// stays below 1 / d because m d - 2^32 < d and x d < 2^32.  d = 1 gives m = 2^32, which does not fit: the caller
+// passes 0 for it.
+inline uint32_t small_divisor(uint32_t d) { return d == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
+__device__ __forceinline__ uint32_t small_divide(uint32_t x, uint32_t m) {
+  return m == 0 ? x : static_cast<uint32_t>((static_cast<uint64_t>(x) * m) >> 32);
+}
+
 // ---- launch helpers --------------------------------------------------------
 inline int launch_status() {
   hipError_t e = hipGetLastError();

@@ -60,20 +60,11 @@ __device__ __forceinline__ void store_oct(float* __restrict__ p, int nv, const f
 }
 
 // fp16 activations (the reference's kernels are also instantiated for at::Half,
-// quantization_cuda_kernel.cu:132-150): one oct is 16 bytes.  VEC == 4 here
-// means "whole octs, 16-byte aligned" (G % 8 == 0).
-template <int VEC, bool FULL>
-__device__ __forceinline__ void load_oct_half(const half_t* __restrict__ p, int nv, float (&v)[8]) {
-  if constexpr (VEC == 4) {
-    typedef half_t half8 __attribute__((ext_vector_type(8)));
-    half8 q = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (FULL || nv > 0) q = __builtin_nontemporal_load(reinterpret_cast<const half8*>(p));
+// quantization_cuda_kernel.cu:132-150): one oct is 16 bytes, here a whole and aligned one.
+__device__ __forceinline__ void load_oct_half(const half_t* __restrict__ p, float (&v)[8]) {
+  const half8 q = __builtin_nontemporal_load(reinterpret_cast<const half8*>(p));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = static_cast<float>(q[i]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (i < nv) ? static_cast<float>(__builtin_nontemporal_load(p + i)) : 0.f;
-  }
+  for (int i = 0; i < 8; ++i) v[i] = static_cast<float>(q[i]);
 }
 
 // 8 consecutive floats that every workgroup reads again (per-column
@@ -246,7 +237,7 @@ __global__ __launch_bounds__(kBlock) void pack_kernel(const PackArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[k][i] = 0.f;
     } else {
-      if constexpr (HALF) load_oct_half<VEC, FULL>(hw + (row_off + static_cast<off_t>(d0)), nv[k], v[k]);
+      if constexpr (HALF) load_oct_half(hw + (row_off + static_cast<off_t>(d0)), v[k]);
       else load_oct<VEC, FULL>(xw + (row_off + static_cast<off_t>(d0)), nv[k], v[k]);
     }
     if constexpr (ACT) {
@@ -451,7 +442,6 @@ __global__ __launch_bounds__(kBlock) void pack_kernel(const PackArgs a) {
       if (a.out_vec == 8) {
         // one 8-byte store: written as two struct members, the compiler hoists the
         // first word's store out of this branch and issues two 4-byte stores
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
         const u32x2 both = {w0, w1};
         *reinterpret_cast<u32x2*>(dst) = both;
       } else if (a.out_vec == 4) {
@@ -468,6 +458,234 @@ __global__ __launch_bounds__(kBlock) void pack_kernel(const PackArgs a) {
     a.packed[a.pad_index] = 0;
     if constexpr (ACT)
       for (int64_t i = a.mask_tail_begin; i < a.mask_tail_end; ++i) a.mask_bytes[i] = 0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// pack, rows of any length up to 1024: statistics + quantise + pack in one pass
+// ---------------------------------------------------------------------------
+// The form for rows that are not a power-of-two number of whole, aligned octs
+// (those keep pack_kernel: no workgroup barrier ahead of the quantiser).  A row
+// of 301 columns has 38 octs: on a power of two of lanes 64 slots are spent on
+// them and each lane of a row starts at another alignment, which left that form
+// with element-wise loads -- 98 us for [100003, 301] fp16, 0.8 TB/s.  Here a
+// workgroup's rows lie one after the other in memory and its octs are dealt to
+// the threads in that order: thread t takes octs t, t + T, ..., whatever row they
+// are in.  What that costs is that a row's statistics meet in LDS (8 bytes per
+// oct, then 8 lanes per row) instead of in registers; what it gives is
+//   * 16-byte loads at any element boundary, neighbouring lanes on neighbouring
+//     bytes (the last oct of a row reads on into the next row and drops that);
+//   * no idle slots but those of the last round: the host picks the rows and
+//     threads per workgroup that fill it best (plan_flat);
+//   * packed bytes in runs across the rows' ends, 8 at a time.
+// Random numbers and arithmetic are those of pack_kernel, bit for bit.
+struct PackFlatArgs {
+  const void* x;          // fp32, or fp16 (HALF)
+  const float* noise;     // nullable
+  uint32_t seed_lo, seed_hi, off_lo, off_hi;
+  int64_t N, total;       // rows, N * G
+  int G, opr, rows;       // columns, octs per row, rows per workgroup (a multiple of 8)
+  uint32_t opr_div;       // small_divisor(opr)
+  uint8_t* packed;
+  int64_t pad_index;
+  float* scale_f32;       // outputs, each nullable
+  float* min_f32;
+  uint16_t* scale_16;     // bf16, or fp16 (HALF)
+  uint16_t* min_16;
+};
+
+constexpr int kFlatThreads = 512;  // at most
+
+// 8 elements from flat index `at`, of which the caller uses those inside the tensor: the window moves back where it
+// would pass the tensor's end (only the last row's last oct, and idle lanes), and the elements wanted are then read
+// again one by one.
+template <bool HALF>
+__device__ __forceinline__ void load_window8(const void* base, int64_t at, int64_t total, float (&v)[8]) {
+  const int64_t last = total - 8;
+  const int64_t from = at < last ? at : (last > 0 ? last : 0);
+  if (total >= 8) {  // the same for the whole launch
+    if constexpr (HALF) {
+      const half8 q = __builtin_nontemporal_load(reinterpret_cast<const half8_any*>(static_cast<const half_t*>(base) + from));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = static_cast<float>(q[i]);
+    } else {
+      const float* p = static_cast<const float*>(base) + from;
+      const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p));
+      const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(p + 4));
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    }
+  }
+}
+template <bool HALF>
+__device__ __forceinline__ void mend_window8(const void* base, int64_t at, int64_t total, float (&v)[8]) {
+  if (__builtin_expect(at + 8 > total, 0)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = 0.f;
+      if (at + i < total)
+        v[i] = HALF ? static_cast<float>(static_cast<const half_t*>(base)[at + i]) : static_cast<const float*>(base)[at + i];
+    }
+  }
+}
+
+// the first nv (1 .. 8) of eight bytes, at any address: one store, or up to three for the last oct of a row
+__device__ __forceinline__ void store_bytes8(uint8_t* dst, int nv, uint32_t w0, uint32_t w1) {
+  if (nv == 8) {
+    const u32x2 both = {w0, w1};
+    *reinterpret_cast<u32x2_any*>(dst) = both;
+    return;
+  }
+  if (nv & 4) {
+    *reinterpret_cast<u32_any*>(dst) = w0;
+    dst += 4;
+    w0 = w1;
+  }
+  if (nv & 2) {
+    *reinterpret_cast<u16_any*>(dst) = static_cast<uint16_t>(w0);
+    dst += 2;
+    w0 >>= 16;
+  }
+  if (nv & 1) *dst = static_cast<uint8_t>(w0);
+}
+
+template <int BITS, int OPT, bool NOISE_IN, bool HALF>
+__global__ __launch_bounds__(kFlatThreads) void pack_flat_kernel(const PackFlatArgs a) {
+  constexpr int WPT = 8 / BITS;
+  constexpr float B = static_cast<float>((1 << BITS) - 1);
+  // per oct of the workgroup: first its (min, max) as order keys, later its eight codes; then (min, scale) per row
+  HIP_DYNAMIC_SHARED(uint2, oct_lds)
+  const int t = threadIdx.x;
+  const int T = blockDim.x;
+  float2* row_lds = reinterpret_cast<float2*>(oct_lds + OPT * T);
+  const int64_t row_base = static_cast<int64_t>(blockIdx.x) * a.rows;
+  const int rows_here = a.N - row_base < a.rows ? static_cast<int>(a.N - row_base) : a.rows;
+  const int octs_here = rows_here * a.opr;
+  const int64_t flat_base = row_base * a.G;
+
+  float v[OPT][8];
+  float un[NOISE_IN ? OPT : 1][8];
+  int row_of[OPT], oct_of[OPT];
+#pragma unroll
+  for (int k = 0; k < OPT; ++k) {
+    const int local = k * T + t;
+    row_of[k] = static_cast<int>(small_divide(static_cast<uint32_t>(local), a.opr_div));
+    oct_of[k] = local - row_of[k] * a.opr;
+    // lanes past the workgroup's octs re-read its first and are not used
+    const int64_t at = flat_base + (local < octs_here ? row_of[k] * a.G + 8 * oct_of[k] : 0);
+    load_window8<HALF>(a.x, at, a.total, v[k]);
+    if constexpr (NOISE_IN) load_window8<false>(a.noise, at, a.total, un[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < OPT; ++k) {
+    const int local = k * T + t;
+    if (local < octs_here) {
+      const int64_t at = flat_base + row_of[k] * a.G + 8 * oct_of[k];
+      mend_window8<HALF>(a.x, at, a.total, v[k]);
+      if constexpr (NOISE_IN) mend_window8<false>(a.noise, at, a.total, un[k]);
+      const int nv = min(8, a.G - 8 * oct_of[k]);
+      if (nv < 8) {
+#pragma unroll
+        for (int i = 1; i < 8; ++i) v[k][i] = i < nv ? v[k][i] : v[k][0];  // neutral in the statistics; never stored
+      }
+      float lo = v[k][0], hi = v[k][0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) {
+        lo = fminf(lo, v[k][i]);
+        hi = fmaxf(hi, v[k][i]);
+      }
+      // fminf / fmaxf pass over a NaN unless every element is one, as the sequence from +-infinity does
+      oct_lds[local] = make_uint2(static_cast<uint32_t>(order_key(fminf(lo, __builtin_inff()))),
+                                  static_cast<uint32_t>(order_key(fmaxf(hi, -__builtin_inff()))));
+    }
+  }
+  __syncthreads();
+  for (int first = 0; first < rows_here; first += T >> 3) {
+    const int r = first + (t >> 3);
+    const bool ok = r < rows_here;
+    int lo = 0x7FFFFFFF, hi = static_cast<int>(0x80000000u);
+    for (int c = t & 7; c < a.opr; c += 8) {
+      const uint2 m = oct_lds[(ok ? r : 0) * a.opr + c];
+      lo = min(lo, static_cast<int>(m.x));
+      hi = max(hi, static_cast<int>(m.y));
+    }
+    lo = min(lo, dpp_lanes<0xB1>(lo));
+    hi = max(hi, dpp_lanes<0xB1>(hi));
+    lo = min(lo, dpp_lanes<0x4E>(lo));
+    hi = max(hi, dpp_lanes<0x4E>(hi));
+    lo = min(lo, dpp_lanes<0x141>(lo));
+    hi = max(hi, dpp_lanes<0x141>(hi));
+    if (ok && (t & 7) == 0) {
+      const float mnv = key_value(lo);
+      float sc;
+      // ops.py:39, two roundings (see pack_kernel)
+      if constexpr (HALF) {
+        const float recip = round_to_half(1.0f / round_to_half(key_value(hi) - mnv));
+        sc = round_to_half(recip * B);
+      } else {
+        const float recip = 1.0f / (key_value(hi) - mnv);
+        sc = recip * B;
+      }
+      row_lds[r] = make_float2(mnv, sc);
+      if (a.scale_f32) (a.scale_f32 + row_base)[r] = sc;
+      if (a.min_f32) (a.min_f32 + row_base)[r] = mnv;
+      if (a.scale_16) (a.scale_16 + row_base)[r] = HALF ? half_bits(sc) : f32_to_bf16_rne(sc);
+      if (a.min_16) (a.min_16 + row_base)[r] = HALF ? half_bits(mnv) : f32_to_bf16_rne(mnv);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < OPT; ++k) {
+    const int local = k * T + t;
+    if (local < octs_here) {
+      const float2 par = row_lds[row_of[k]];
+      float u[8];
+      if constexpr (NOISE_IN) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) u[i] = un[k][i];
+      } else {
+        const Philox4 r = philox4x32_10(static_cast<uint32_t>(oct_of[k]), static_cast<uint32_t>(row_base) + static_cast<uint32_t>(row_of[k]),
+                                        a.off_lo, a.off_hi, a.seed_lo, a.seed_hi);
+        philox_uniform8(r, u);
+      }
+      uint32_t q[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float tq = v[k][i] - par.x;
+        if constexpr (HALF) tq = round_to_half(tq);
+        tq = tq * par.y;
+        if constexpr (HALF) tq = round_to_half(tq);
+        q[i] = code_in_low_byte(tq + u[i]);
+      }
+      const uint2 codes = make_uint2(low_bytes4(q[0], q[1], q[2], q[3]), low_bytes4(q[4], q[5], q[6], q[7]));
+      if constexpr (WPT == 1)  // one row per byte: nothing to combine
+        store_bytes8(a.packed + row_base * a.G + (row_of[k] * a.G + 8 * oct_of[k]), min(8, a.G - 8 * oct_of[k]), codes.x, codes.y);
+      else
+        oct_lds[local] = codes;
+    } else if (local < a.rows * a.opr) {
+      oct_lds[local] = make_uint2(0u, 0u);  // rows past the end of the tensor in its last group of rows
+    }
+  }
+  if (blockIdx.x == 0 && t == 0) a.packed[a.pad_index] = 0;
+  if constexpr (WPT == 1) return;
+  __syncthreads();
+  // one packed oct = the same oct of the 8 / BITS rows of a group
+  const int groups = (rows_here + WPT - 1) / WPT;
+  uint8_t* const out = a.packed + (row_base / WPT) * a.G;
+  for (int item = t; item < groups * a.opr; item += T) {
+    const int g = static_cast<int>(small_divide(static_cast<uint32_t>(item), a.opr_div));
+    const int j = item - g * a.opr;
+    uint32_t w0 = 0, w1 = 0;
+#pragma unroll
+    for (int i = 0; i < WPT; ++i) {
+      // uint8 accumulator of the reference: bits shifted past bit 7 vanish
+      constexpr uint32_t kByte = 0x01010101u;
+      const uint32_t keep = (0xFFu >> (i * BITS)) * kByte;
+      const uint2 c = oct_lds[(g * WPT + i) * a.opr + j];
+      w0 |= (c.x & keep) << (i * BITS);
+      w1 |= (c.y & keep) << (i * BITS);
+    }
+    store_bytes8(out + (g * a.G + 8 * j), min(8, a.G - 8 * j), w0, w1);
   }
 }
 
@@ -555,14 +773,89 @@ __global__ void zero_byte_kernel(uint8_t* p) { *p = 0; }
 
 static bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
+// How pack_flat_kernel deals rows of `opr` octs to a workgroup: rows (a multiple of 8, so that every workgroup owns
+// whole groups of rows at every bit width), threads and octs per thread.
+struct FlatGeometry {
+  int rows, threads, opt;
+};
+
+// Measured over widths of 25 to 1000 columns: 256 threads of four octs are the fastest or within 3 % of it (320 and
+// 384 threads fill better on paper and are 10 - 20 % slower: the compute unit's wavefront slots), except where eight
+// rows leave too many of the 1024 slots empty (65 .. 80 octs per row): 512 threads of four, 39.7 against 40.2 us at
+// [72012, 602] fp32 and 39.6 against 42.8 us in fp16.  A short tensor is spread over the chip before its workgroups
+// are filled, with as few octs per thread as its rows then need.
+static FlatGeometry plan_flat(int opr, int64_t N) {
+  FlatGeometry g{1024 / opr / 8 * 8, kBlock, 4};
+  if (g.rows * opr < 645) {
+    g.threads = 2 * kBlock;
+    g.rows = 2048 / opr / 8 * 8;
+  }
+  while (g.rows > 8 && (N + g.rows - 1) / g.rows < 1024) g.rows = (g.rows / 2 + 7) / 8 * 8;
+  if (g.rows * opr <= 4 * kBlock) g.threads = kBlock;
+  while (g.opt > 1 && g.rows * opr <= g.opt / 2 * g.threads) g.opt /= 2;
+  return g;
+}
+
+template <int BITS, bool NOISE_IN, bool HALF>
+static void launch_flat_opt(const PackFlatArgs& a, int opt, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
+  if (opt == 4) hipLaunchKernelGGL((pack_flat_kernel<BITS, 4, NOISE_IN, HALF>), grid, block, lds, s, a);
+  else if (opt == 2) hipLaunchKernelGGL((pack_flat_kernel<BITS, 2, NOISE_IN, HALF>), grid, block, lds, s, a);
+  else hipLaunchKernelGGL((pack_flat_kernel<BITS, 1, NOISE_IN, HALF>), grid, block, lds, s, a);
+}
+
+template <bool NOISE_IN, bool HALF>
+static void launch_flat_bits(const PackFlatArgs& a, int bits, int opt, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
+  switch (bits) {
+    case 1: return launch_flat_opt<1, NOISE_IN, HALF>(a, opt, grid, block, lds, s);
+    case 2: return launch_flat_opt<2, NOISE_IN, HALF>(a, opt, grid, block, lds, s);
+    case 4: return launch_flat_opt<4, NOISE_IN, HALF>(a, opt, grid, block, lds, s);
+    default: return launch_flat_opt<8, NOISE_IN, HALF>(a, opt, grid, block, lds, s);
+  }
+}
+
+// x [N, G], G <= 1024, at any element alignment
+template <bool HALF>
+static void launch_flat(const void* x, const float* noise, uint64_t seed, uint64_t offset, int64_t N, int64_t G, int bits,
+                        uint8_t* packed, int64_t pad_index, float* scale_f32, float* min_f32, uint16_t* scale_16,
+                        uint16_t* min_16, hipStream_t s) {
+  PackFlatArgs a{};
+  a.x = x;
+  a.noise = noise;
+  a.seed_lo = static_cast<uint32_t>(seed);
+  a.seed_hi = static_cast<uint32_t>(seed >> 32);
+  a.off_lo = static_cast<uint32_t>(offset);
+  a.off_hi = static_cast<uint32_t>(offset >> 32);
+  a.N = N;
+  a.total = N * G;
+  a.G = static_cast<int>(G);
+  a.opr = static_cast<int>((G + 7) / 8);
+  a.opr_div = small_divisor(static_cast<uint32_t>(a.opr));
+  a.packed = packed;
+  a.pad_index = pad_index;
+  a.scale_f32 = scale_f32;
+  a.min_f32 = min_f32;
+  a.scale_16 = scale_16;
+  a.min_16 = min_16;
+  const FlatGeometry g = plan_flat(a.opr, N);
+  a.rows = g.rows;
+  const dim3 grid(static_cast<unsigned>((N + g.rows - 1) / g.rows)), block(static_cast<unsigned>(g.threads));
+  const size_t lds = sizeof(uint2) * static_cast<size_t>(g.opt * g.threads + g.rows);  // at most 16 KB + 16 KB
+  if (noise) launch_flat_bits<true, HALF>(a, bits, g.opt, grid, block, lds, s);
+  else launch_flat_bits<false, HALF>(a, bits, g.opt, grid, block, lds, s);
+}
+
 template <int BITS, int OPT, bool NOISE_IN, bool FUSED>
 static void launch_pack_variant(const PackArgs& a, bool vec4, bool full, dim3 grid, hipStream_t s) {
-  if (vec4 && full)
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, true, NOISE_IN, FUSED>), grid, dim3(kBlock), 0, s, a);
-  else if (vec4)
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, false, NOISE_IN, FUSED>), grid, dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 1, false, NOISE_IN, FUSED>), grid, dim3(kBlock), 0, s, a);
+  if constexpr (FUSED) {  // whole rows only: everything else goes to pack_flat_kernel
+    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, true, NOISE_IN, true>), grid, dim3(kBlock), 0, s, a);
+  } else {
+    if (vec4 && full)
+      hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, true, NOISE_IN, false>), grid, dim3(kBlock), 0, s, a);
+    else if (vec4)
+      hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, false, NOISE_IN, false>), grid, dim3(kBlock), 0, s, a);
+    else
+      hipLaunchKernelGGL((pack_kernel<BITS, OPT, 1, false, NOISE_IN, false>), grid, dim3(kBlock), 0, s, a);
+  }
 }
 
 template <int BITS, bool NOISE_IN, bool FUSED>
@@ -624,6 +917,12 @@ static int pack_common(const float* x, const float* mn, const float* scale, cons
   }
 
   const Geometry g = plan_rows(G, do_fused ? 4 : 1, opt_hint);
+  const bool vec4 = (G % 4 == 0) && aligned(x, 16) && (!noise || aligned(noise, 16));
+  const bool full = g.full && vec4;
+  if (do_fused && !full) {
+    launch_flat<false>(x, noise, seed, offset, N, G, bits, packed, pad_index, scale_f32, min_f32, scale_bf16, min_bf16, s);
+    return launch_status();
+  }
   PackArgs a{};
   a.x = x;
   a.noise = noise;
@@ -644,10 +943,8 @@ static int pack_common(const float* x, const float* mn, const float* scale, cons
   a.scale_bf16 = do_fused ? scale_bf16 : nullptr;
   a.min_bf16 = do_fused ? min_bf16 : nullptr;
   a.out_vec = (G % 8 == 0 && aligned(packed, 8)) ? 8 : (G % 4 == 0 && aligned(packed, 4)) ? 4 : 1;
-  const bool vec4 = (G % 4 == 0) && aligned(x, 16) && (!noise || aligned(noise, 16));
   const int rows_per_wg = kBlock >> g.lpr_log2;
   const dim3 grid(static_cast<unsigned>((N + rows_per_wg - 1) / rows_per_wg), static_cast<unsigned>(g.grid_y));
-  const bool full = g.full && vec4;
   if (do_fused) {
     if (noise) launch_pack_bits<true, true>(a, bits, g.opt, vec4, full, grid, s);
     else launch_pack_bits<false, true>(a, bits, g.opt, vec4, full, grid, s);
@@ -685,31 +982,21 @@ static void launch_act_bits(const PackArgs& a, int bits, int opt, bool full, dim
   }
 }
 
-// ---- fp16 activations (HALF form): statistics + pack in one launch, G <= 1024 --
-template <int BITS, int OPT, bool NOISE_IN>
-static void launch_half_variant(const PackArgs& a, bool whole, bool full, dim3 grid, hipStream_t s) {
-  if (whole && full)
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, true, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
-  else if (whole)
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 4, false, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((pack_kernel<BITS, OPT, 1, false, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
-}
-
+// ---- fp16 activations (HALF form), rows of whole octs on whole lanes: statistics + pack in one launch, G <= 1024 --
 template <int BITS, bool NOISE_IN>
-static void launch_half_opt(const PackArgs& a, int opt, bool whole, bool full, dim3 grid, hipStream_t s) {
-  if (opt == 4) return launch_half_variant<BITS, 4, NOISE_IN>(a, whole, full, grid, s);
-  if (opt == 2) return launch_half_variant<BITS, 2, NOISE_IN>(a, whole, full, grid, s);
-  launch_half_variant<BITS, 1, NOISE_IN>(a, whole, full, grid, s);
+static void launch_half_opt(const PackArgs& a, int opt, dim3 grid, hipStream_t s) {
+  if (opt == 4) hipLaunchKernelGGL((pack_kernel<BITS, 4, 4, true, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
+  else if (opt == 2) hipLaunchKernelGGL((pack_kernel<BITS, 2, 4, true, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
+  else hipLaunchKernelGGL((pack_kernel<BITS, 1, 4, true, NOISE_IN, true, false, true>), grid, dim3(kBlock), 0, s, a);
 }
 
 template <bool NOISE_IN>
-static void launch_half_bits(const PackArgs& a, int bits, int opt, bool whole, bool full, dim3 grid, hipStream_t s) {
+static void launch_half_bits(const PackArgs& a, int bits, int opt, dim3 grid, hipStream_t s) {
   switch (bits) {
-    case 1: return launch_half_opt<1, NOISE_IN>(a, opt, whole, full, grid, s);
-    case 2: return launch_half_opt<2, NOISE_IN>(a, opt, whole, full, grid, s);
-    case 4: return launch_half_opt<4, NOISE_IN>(a, opt, whole, full, grid, s);
-    default: return launch_half_opt<8, NOISE_IN>(a, opt, whole, full, grid, s);
+    case 1: return launch_half_opt<1, NOISE_IN>(a, opt, grid, s);
+    case 2: return launch_half_opt<2, NOISE_IN>(a, opt, grid, s);
+    case 4: return launch_half_opt<4, NOISE_IN>(a, opt, grid, s);
+    default: return launch_half_opt<8, NOISE_IN>(a, opt, grid, s);
   }
 }
 
@@ -867,6 +1154,11 @@ int exact_minmax_pack_f16(const uint16_t* x, const float* noise, uint64_t seed, 
   if (!x) return EXACT_E_NULL;
   if (!aligned(x, 2)) return EXACT_E_ALIGN;
   const Geometry g = plan_rows(G, 4);
+  // whole octs: 16-byte loads of x (and of supplied fp32 noise)
+  if (!g.full || !aligned(x, 16) || (noise && !aligned(noise, 16))) {
+    launch_flat<true>(x, noise, seed, offset, N, G, bits, packed, pad_index, nullptr, nullptr, scale_f16, min_f16, s);
+    return launch_status();
+  }
   PackArgs a{};
   a.x = reinterpret_cast<const float*>(x);  // the HALF form reads it as fp16
   a.noise = noise;
@@ -883,12 +1175,10 @@ int exact_minmax_pack_f16(const uint16_t* x, const float* noise, uint64_t seed, 
   a.scale_bf16 = scale_f16;
   a.min_bf16 = min_f16;
   a.out_vec = (G % 8 == 0 && aligned(packed, 8)) ? 8 : (G % 4 == 0 && aligned(packed, 4)) ? 4 : 1;
-  // whole octs: 16-byte loads of x (and of supplied fp32 noise)
-  const bool whole = (G % 8 == 0) && aligned(x, 16) && (!noise || aligned(noise, 16));
   const int rows_per_wg = kBlock >> g.lpr_log2;
   const dim3 grid(static_cast<unsigned>((N + rows_per_wg - 1) / rows_per_wg), 1u);
-  if (noise) launch_half_bits<true>(a, bits, g.opt, whole, g.full && whole, grid, s);
-  else launch_half_bits<false>(a, bits, g.opt, whole, g.full && whole, grid, s);
+  if (noise) launch_half_bits<true>(a, bits, g.opt, grid, s);
+  else launch_half_bits<false>(a, bits, g.opt, grid, s);
   return launch_status();
 }
 
