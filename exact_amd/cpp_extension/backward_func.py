@@ -212,6 +212,76 @@ def native_batch_norm_backward(grad_out, input, weight, running_mean, running_va
     return grad_input, grad_weight, grad_bias
 
 
+def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, eps):
+    """The statistics half of native_batch_norm in training mode -> (mean,
+    1 / sqrt(var + eps), weight * that), with running_mean / running_var updated
+    in place; None where the library's kernels do not apply (the caller then
+    takes the framework's routines).  From 1024 rows on: below, the framework's
+    reduction is no slower."""
+    def vector_ok(t):
+        return (t is None or (t.dtype == torch.float32 and t.device == matrix.device and t.is_contiguous()
+                              and t.numel() == matrix.shape[1]))
+
+    usable = (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
+              and 0 < matrix.shape[1] <= 8192 and 1024 <= matrix.shape[0] < 2 ** 31
+              and vector_ok(weight) and vector_ok(running_mean) and vector_ok(running_var)
+              and (running_mean is None) == (running_var is None) and momentum is not None and _atomics_allowed())
+    if not usable:
+        return None
+    N, K = matrix.shape
+    buffer = torch.empty((6, K), dtype=torch.float32, device=matrix.device)      # sums [2, K], centre, mean, invstd, mult
+    rc = _lib.lib().exact_bn_stats_f32(_checks.ptr(matrix), N, K, float(eps), float(momentum), _checks.ptr(weight),
+                                       _checks.ptr(running_mean), _checks.ptr(running_var), _checks.ptr(buffer),
+                                       _checks.ptr(buffer[3]), _checks.ptr(buffer[4]), _checks.ptr(buffer[5]),
+                                       _checks.stream_ptr(matrix))
+    _lib.check(rc, "batch_norm_statistics")
+    if running_mean is not None:
+        torch.autograd.graph.increment_version((running_mean, running_var))
+    return buffer[3], buffer[4], buffer[5]
+
+
+def batch_norm_apply(matrix, mean, mult, bias):
+    """(matrix - mean) * mult + bias per column, for the statistics above."""
+    out = torch.empty_like(matrix)
+    if bias is not None:
+        bias = bias.detach().to(torch.float32).contiguous()
+    rc = _lib.lib().exact_bn_apply_f32(_checks.ptr(matrix), _checks.ptr(mean), _checks.ptr(mult), _checks.ptr(bias), *matrix.shape,
+                                       _checks.ptr(out), _checks.stream_ptr(matrix))
+    _lib.check(rc, "batch_norm_apply")
+    return out
+
+
+def batch_norm_backward_packed(grad_out, mask, p, quantized, weight, mean, invstd, output_mask):
+    """native_batch_norm_backward on an input that is still packed, behind a joint
+    ReLU / dropout mask where `mask` is given (dropout_bwd): -> (grad_input,
+    grad_weight, grad_bias), or None where the kernels do not apply (the caller
+    then dequantises and takes the separate routines)."""
+    packed, bits, scale, mn = quantized
+    vectors = [t for t in (mean, invstd, weight) if t is not None]
+    usable = (bits in (1, 2, 4, 8) and grad_out.dim() == 2 and grad_out.dtype == torch.float32 and _checks.on_device(grad_out)
+              and grad_out.is_contiguous() and grad_out.data_ptr() % 16 == 0
+              and 1024 <= grad_out.shape[0] < 2 ** 31 and 0 < grad_out.shape[1] <= 8192 and grad_out.shape[1] % 4 == 0
+              and packed.dtype == torch.int8 and packed.is_contiguous() and packed.data_ptr() % 4 == 0
+              and packed.numel() * (8 // bits) >= grad_out.numel()
+              and scale.dtype == torch.bfloat16 and mn.dtype == torch.bfloat16
+              and scale.numel() == mn.numel() == grad_out.shape[0] and scale.is_contiguous() and mn.is_contiguous()
+              and all(t.device == grad_out.device for t in (packed, scale, mn, *vectors))
+              and all(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == grad_out.shape[1] for t in vectors)
+              and _atomics_allowed())
+    if not usable:
+        return None
+    N, K = grad_out.shape
+    sums = torch.empty((2, K), dtype=torch.float32, device=grad_out.device)
+    grad_input = torch.empty_like(grad_out) if output_mask[0] else None
+    grad_weight = torch.empty(K, dtype=torch.float32, device=grad_out.device) if output_mask[1] else None
+    rc = _lib.lib().exact_bn_backward_packed_f32(_checks.ptr(grad_out), _checks.ptr(mask), float(p), _checks.ptr(packed), bits,
+                                                 _checks.ptr(scale), _checks.ptr(mn), _checks.ptr(mean), _checks.ptr(invstd),
+                                                 _checks.ptr(weight), N, K, _checks.ptr(sums), _checks.ptr(grad_input),
+                                                 _checks.ptr(grad_weight), _checks.stream_ptr(grad_out))
+    _lib.check(rc, "batch_norm_backward_packed")
+    return grad_input, grad_weight, sums[0] if output_mask[2] else None
+
+
 def _elu_backward_cuda(grad_output, data, alpha):
     """backward_func_cuda_kernel.cu:6-36: x >= 0 ? grad : alpha * grad * exp(x)."""
     grad_output, data = grad_output.contiguous(), data.contiguous()

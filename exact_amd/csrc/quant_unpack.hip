@@ -43,16 +43,6 @@ struct UnpackArgs {
   float* out;
 };
 
-// RN(q / s) from r = RN(1 / s): y = RN(q r), e = q - y s (exact, one FMA),
-// result = RN(y + e r).  Markstein's correction step; for 0 <= q <= 255 and
-// every fp32 significand of s it equals the IEEE quotient bit for bit (checked
-// exhaustively on the CPU: 2^23 significands x 256 values of q).
-__device__ __forceinline__ float exact_quotient(float q, float s, float r) {
-  const float y = q * r;
-  const float e = __fmaf_rn(-y, s, q);
-  return __fmaf_rn(e, r, y);
-}
-
 // How scale / min (and, for fp16, the output) are stored.
 enum ParamKind { kParamF32 = 0, kParamBF16 = 1, kParamF16 = 2 };
 

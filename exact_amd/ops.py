@@ -299,6 +299,19 @@ class qlinear(Function):
         return (*grads, None, None, None, None)
 
 
+def _batch_norm_backward_packed(grad_output, mask, p, kept, weight, mean, invstd, wanted):
+    """The batch norm's backward straight from the compressed copy of its input,
+    or None where that needs the dequantised one (no compression, plain-tensor
+    quantiser, an unusual layout).  A copy that was swapped out comes back to the
+    device first."""
+    if not config.compress_activation or config.simulate or kept.randmat is not None:
+        return None
+    packed, bits, scale, mn = kept.quantized
+    if packed.device != scale.device:
+        packed = packed.to(scale.device, non_blocking=True)
+    return ext_backward_func.batch_norm_backward_packed(grad_output, mask, p, (packed, bits, scale, mn), weight, mean, invstd, wanted)
+
+
 class qbatch_norm(Function):
     """Training-mode batch norm that keeps its input compressed (reference ops.py:206-254)."""
 
@@ -306,8 +319,14 @@ class qbatch_norm(Function):
     def forward(ctx, input, running_mean, running_var, weight, bias,  # noqa: A002
                 training, exponential_average_factor, eps, scheme):
         kept = CompressedActivation.compress(input, scheme, project=False)
-        output, save_mean, save_invstd = ext_backward_func.native_batch_norm(
-            input, weight, bias, running_mean, running_var, training, exponential_average_factor, eps)
+        stats = (ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps)
+                 if training else None)
+        if stats is not None:
+            save_mean, save_invstd, mult = stats
+            output = ext_backward_func.batch_norm_apply(input, save_mean, mult, bias)
+        else:
+            output, save_mean, save_invstd = ext_backward_func.native_batch_norm(
+                input, weight, bias, running_mean, running_var, training, exponential_average_factor, eps)
         ctx.kept = kept
         ctx.stats = (weight, running_mean, running_var, save_mean, save_invstd, training, eps)
         return output
@@ -315,12 +334,19 @@ class qbatch_norm(Function):
     @staticmethod
     def backward(ctx, grad_output):
         weight, running_mean, running_var, save_mean, save_invstd, training, eps = ctx.stats
-        x_hat = ctx.kept.restore()
-        ctx.kept = None
-        empty_cache(config.empty_cache_threshold)
         wanted = [ctx.needs_input_grad[0], ctx.needs_input_grad[3], ctx.needs_input_grad[4]]
+        kept, ctx.kept = ctx.kept, None
+        grad_output = grad_output.contiguous()
+        grads = _batch_norm_backward_packed(grad_output, None, 0.0, kept, weight, save_mean, save_invstd, wanted) if training else None
+        if grads is not None:
+            empty_cache(config.empty_cache_threshold)
+            g_in, g_w, g_b = grads
+            return g_in, None, None, g_w, g_b, None, None, None, None
+        x_hat = kept.restore()
+        del kept
+        empty_cache(config.empty_cache_threshold)
         g_in, g_w, g_b = ext_backward_func.native_batch_norm_backward(
-            grad_output.contiguous(), x_hat, weight, running_mean, running_var, save_mean, save_invstd, training, eps,
+            grad_output, x_hat, weight, running_mean, running_var, save_mean, save_invstd, training, eps,
             wanted)
         # the device routine returns tensors for masked-out outputs too (e.g. without affine parameters)
         g_in, g_w, g_b = (g if w else None for g, w in zip((g_in, g_w, g_b), wanted))
@@ -692,14 +718,18 @@ class qbn_relu_dropout(Function):
     def forward(ctx, input, running_mean, running_var, weight, bias,  # noqa: A002
                 exponential_average_factor, eps, p, bits, scheme):
         kept = CompressedActivation.compress(input, scheme, project=False)
-        rows = input.shape[0]
-        var, mean = ext_backward_func.batch_statistics(input)
-        invstd = torch.rsqrt(var + eps)
-        if running_mean is not None:                       # the bookkeeping of native_batch_norm
-            running_mean.mul_(1 - exponential_average_factor).add_(mean, alpha=exponential_average_factor)
-            running_var.mul_(1 - exponential_average_factor).add_(var * (rows / max(rows - 1, 1)),
-                                                                   alpha=exponential_average_factor)
-        mult = invstd if weight is None else weight * invstd
+        stats = ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps)
+        if stats is not None:
+            mean, invstd, mult = stats
+        else:
+            rows = input.shape[0]
+            var, mean = ext_backward_func.batch_statistics(input)
+            invstd = torch.rsqrt(var + eps)
+            if running_mean is not None:                   # the bookkeeping of native_batch_norm
+                running_mean.mul_(1 - exponential_average_factor).add_(mean, alpha=exponential_average_factor)
+                running_var.mul_(1 - exponential_average_factor).add_(var * (rows / max(rows - 1, 1)),
+                                                                       alpha=exponential_average_factor)
+            mult = invstd if weight is None else weight * invstd
         shift = torch.zeros_like(mean) if bias is None else bias.detach()
         out, mask, packed, scale, mn = ext_quantization.bn_relu_dropout_minmax_pack(
             input, mean, mult.contiguous(), shift.contiguous(), p, bits)
@@ -714,11 +744,18 @@ class qbn_relu_dropout(Function):
     def backward(ctx, grad_output, *unused):
         (mask,) = ctx.saved_tensors
         weight, running_mean, running_var, save_mean, save_invstd, eps = ctx.stats
-        grad_normalised = ext_quantization.dropout_bwd(grad_output, mask, ctx.p)
-        x_hat = ctx.kept.restore()
-        ctx.kept = None
-        empty_cache(config.empty_cache_threshold)
         wanted = [ctx.needs_input_grad[0], ctx.needs_input_grad[3], ctx.needs_input_grad[4]]
+        kept, ctx.kept = ctx.kept, None
+        grad_output = grad_output.contiguous()
+        grads = _batch_norm_backward_packed(grad_output, mask, ctx.p, kept, weight, save_mean, save_invstd, wanted)
+        if grads is not None:
+            empty_cache(config.empty_cache_threshold)
+            g_in, g_w, g_b = grads
+            return g_in, None, None, g_w, g_b, None, None, None, None, None
+        grad_normalised = ext_quantization.dropout_bwd(grad_output, mask, ctx.p)
+        x_hat = kept.restore()
+        del kept
+        empty_cache(config.empty_cache_threshold)
         g_in, g_w, g_b = ext_backward_func.native_batch_norm_backward(
             grad_normalised, x_hat, weight, running_mean, running_var, save_mean, save_invstd, True, eps, wanted)
         g_in, g_w, g_b = (g if w else None for g, w in zip((g_in, g_w, g_b), wanted))

@@ -1,0 +1,72 @@
+"""The batch norm on wide matrices and on the packed copy of its input
+(exact_bn_stats_f32, exact_bn_apply_f32, exact_bn_backward_packed_f32) against
+the same formulas in float64 on the dequantised input."""
+import pytest
+import torch
+
+from exact_amd import ops
+from exact_amd.conf import config
+from exact_amd.cpp_extension import backward_func as bf
+from exact_amd.cpp_extension import quantization as extq
+
+
+# a width below, at and above one column block (1024 columns in fours, 256 otherwise); rows that end inside a pass
+@pytest.mark.parametrize("N,K", [(1024, 1), (1027, 100), (1500, 257), (2049, 512), (1025, 1028), (1030, 1100)])
+def test_statistics_and_normalisation(backend, N, K):
+    g = torch.Generator().manual_seed(N + K)
+    x = torch.randn(N, K, generator=g) * 1.5 + 40.0          # mean 27 deviations from zero
+    w, b = torch.rand(K, generator=g) + 0.5, torch.randn(K, generator=g)
+    rm, rv = torch.randn(K, generator=g).to(backend), torch.rand(K, generator=g).to(backend)
+    rm0, rv0, versions = rm.cpu().double(), rv.cpu().double(), (rm._version, rv._version)
+    mean, invstd, mult = bf.batch_norm_statistics(x.to(backend), w.to(backend), rm, rv, 0.3, 1e-5)
+    var64, mean64 = torch.var_mean(x.double(), dim=0, unbiased=False)
+    inv64 = torch.rsqrt(var64 + 1e-5)
+    # the mean rounds at 40: 2^-24 * 40, a few times; the moments of about one unit carry 1e-6 relative
+    assert (mean.cpu() - mean64).abs().max() < 2e-5
+    assert ((invstd.cpu() - inv64) / inv64).abs().max() < 1e-5 and ((mult.cpu() - w * inv64) / (w * inv64)).abs().max() < 1e-5
+    assert (rm.cpu() - (0.7 * rm0 + 0.3 * mean64)).abs().max() < 1e-5
+    assert (rv.cpu() - (0.7 * rv0 + 0.3 * var64 * N / (N - 1))).abs().max() < 1e-4
+    assert rm._version > versions[0] and rv._version > versions[1]
+    y = bf.batch_norm_apply(x.to(backend), mean, mult, b.to(backend))
+    assert (y.cpu() - ((x - mean64) * inv64 * w + b)).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("N,K,masked", [(1024, 4, True), (1031, 100, True), (1029, 256, False), (1026, 1028, True)])
+def test_backward_from_the_packed_input(backend, bits, N, K, masked):
+    g = torch.Generator().manual_seed(N + K + bits)
+    x = torch.randn(N, K, generator=g).to(backend)
+    dy = torch.randn(N, K, generator=g).to(backend)
+    w = (torch.rand(K, generator=g) + 0.5).to(backend)
+    p = 0.3 if masked else 0.0
+    mask = extq.relu_dropout_fwd(torch.randn(N, K, generator=g).to(backend), p)[1] if masked else None
+    packed, scale, mn = extq.minmax_pack(x, bits)
+    mean, invstd, _ = bf.batch_norm_statistics(x, w, None, None, 0.1, 1e-5)
+    dx, dw, db = bf.batch_norm_backward_packed(dy, mask, p, (packed, bits, scale, mn), w, mean, invstd, [True, True, True])
+    x_hat = extq.unpack_bf16param(packed, bits, scale, mn, N, K).double()
+    gr = (extq.dropout_bwd(dy, mask, p) if masked else dy).double()
+    xmu, inv = x_hat - mean.double(), invstd.double()
+    s0, s1 = gr.sum(0), (gr * xmu).sum(0)
+    want = (gr - s0 / N - xmu * inv * inv * s1 / N) * inv * w.double()
+    assert (dx - want).abs().max() < 1e-5 * want.abs().max()
+    assert (db - s0).abs().max() < 1e-6 * gr.abs().sum(0).max()
+    assert (dw - s1 * inv).abs().max() < 2e-6 * (gr * xmu).abs().sum(0).max()
+    only = bf.batch_norm_backward_packed(dy, mask, p, (packed, bits, scale, mn), None, mean, invstd, [False, False, True])
+    assert only[0] is None and only[1] is None and (only[2] - s0).abs().max() < 1e-6 * gr.abs().sum(0).max()
+
+
+def test_what_the_kernels_do_not_take_goes_to_the_separate_routines(backend):
+    x, dy = torch.randn(1100, 10).to(backend), torch.randn(1100, 10).to(backend)
+    packed, scale, mn = extq.minmax_pack(x, 2)
+    mean, invstd, _ = bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5)
+    copy = (packed, 2, scale, mn)
+    want = [True, True, True]
+    assert bf.batch_norm_backward_packed(dy, None, 0.0, copy, None, mean, invstd, want) is None            # 10 % 4
+    assert bf.batch_norm_statistics(x[:, :9], None, None, None, 0.1, 1e-5) is None                         # strided
+    assert bf.batch_norm_statistics(x[:1000], None, None, None, 0.1, 1e-5) is None                         # short
+    assert bf.batch_norm_statistics(x, None, torch.zeros(9).to(backend), torch.zeros(9).to(backend), 0.1, 1e-5) is None
+    config.deterministic_reductions = True
+    assert bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5) is None
+    kept = ops.CompressedActivation(copy, None, x.shape, x.shape)
+    config.simulate = True
+    assert ops._batch_norm_backward_packed(dy, None, 0.0, kept, None, mean, invstd, want) is None
