@@ -99,13 +99,12 @@ _EXTRA_FIELDS = {
     # matrix-core kernel (config.matrix_cores == "bf16") from this many rows on;
     # shorter operands keep the framework's GEMM, which is as fast there.
     "tall_gemm_min_rows": 16384,
-    # ... when the result has at most 64 columns (20 - 35 % faster than the
-    # framework's fp32 GEMM there) or the reduction runs over at least this many
-    # features (10 - 20 % faster at 256 and 604; slower at 100 - 128).
-    "tall_gemm_min_depth": 192,
-    # ... and, for such wide results, at most this many rows: at 2.4 M rows the
-    # framework's GEMM reaches 127 TFLOP/s and the two are equal.
-    "tall_gemm_max_rows_wide": 1000000,
+    # ... and, for results of more than 64 columns, a reduction over at least this
+    # many features and at most this many rows: no limit by default (82 against
+    # 129 us at [169343, 128] x [128, 256], 2.0 against 2.5 ms at [2449029, 256] x
+    # [256, 256], 0.67 against 0.86 at [2449029, 46] x [46, 256]).
+    "tall_gemm_min_depth": 1,
+    "tall_gemm_max_rows_wide": 2 ** 31 - 1,
 }
 
 

@@ -109,13 +109,11 @@ def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     """x[N, D] . M (+ bias[K]) (+ addend[N, K]) -> [N, K], where M = `matrix`
     ([D, K]) or, with transposed=True, the transpose of `matrix` ([K, D]: a weight
     as F.linear holds it).  `into` names the result tensor; it may be `addend`
-    itself (accumulate in place).  Tall fp32 device operands with a narrow result
-    (config.tall_gemm_min_rows; a result of at most 64 columns or a reduction over
-    at least config.tall_gemm_min_depth features of at most
-    config.tall_gemm_max_rows_wide rows) take the library's
-    kernel (six bf16 matrix-core products per fp32 product, fp32 accuracy,
-    reproducible; config.matrix_cores == "bf16"); everything else the
-    framework's GEMM."""
+    itself (accumulate in place).  Tall fp32 device operands with an even number of
+    features (config.tall_gemm_min_rows, tall_gemm_min_depth and
+    tall_gemm_max_rows_wide) take the library's kernel (six bf16 matrix-core
+    products per fp32 product, fp32 accuracy, reproducible; config.matrix_cores ==
+    "bf16"); everything else the framework's GEMM."""
     M = matrix.t() if transposed else matrix
     usable = (config.matrix_cores == "bf16" and x.dim() == 2 and matrix.dim() == 2 and x.dtype == torch.float32
               and matrix.dtype == torch.float32 and _checks.on_device(x) and _checks.on_device(matrix)

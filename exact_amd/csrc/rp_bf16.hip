@@ -42,6 +42,7 @@
 namespace exact {
 
 constexpr int kStepFeatures = 16;  // K of one MFMA
+constexpr int kRpXcds = 8;         // accelerator complex dies of an MI355X, each with its own L2
 
 // Eight consecutive floats of a row starting at column `col`, zeros from column
 // `limit` on; VEC = the widest aligned access (limit % VEC == 0, col % VEC == 0).
@@ -63,6 +64,18 @@ __device__ __forceinline__ void load8(const float* __restrict__ row, int col, in
       const float q = *src;
       v[p] = ok ? q : 0.f;
     }
+  }
+}
+
+// The same eight floats where they lie inside the row: two 16-byte loads at any element boundary.  Rows whose length
+// is no multiple of four took 8- or 4-byte loads here, two to four times as many of the same lines.
+__device__ __forceinline__ void load8_inside(const float* __restrict__ src, float (&v)[8]) {
+  const f32x4_any* q = reinterpret_cast<const f32x4_any*>(src);
+  const f32x4 lo = q[0], hi = q[1];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = lo[i];
+    v[4 + i] = hi[i];
   }
 }
 
@@ -145,7 +158,7 @@ __device__ __forceinline__ void rp_fwd_rows(const float* __restrict__ X, const u
     float a[KS][8];
     if ((s0 + KS) * kStepFeatures <= D) {  // wave-uniform: the KS steps lie inside the row, nothing to mask
 #pragma unroll
-      for (int sb = 0; sb < KS; ++sb) load8<VEC>(xrow, (s0 + sb) * kStepFeatures + 8 * half, 0x7FFFFFFF, a[sb]);
+      for (int sb = 0; sb < KS; ++sb) load8_inside(xrow + (s0 + sb) * kStepFeatures + 8 * half, a[sb]);
     } else {
 #pragma unroll
       for (int sb = 0; sb < KS; ++sb) load8<VEC>(xrow, (s0 + sb) * kStepFeatures + 8 * half, D, a[sb]);  // zeros past the row
@@ -348,12 +361,7 @@ __global__ __launch_bounds__(kWave) void rp_fwd_pack_bf16_kernel(const RpPackArg
 // exact_tall_gemm_prepare_bf16, which also takes M transposed (a weight as
 // F.linear holds it).  No atomics: the result does not depend on the launch.
 constexpr int kGemmXcds = 8;       // accelerator complex dies of an MI355X, each with its own L2
-constexpr int kGemmSlabTiles = 4;  // column tiles (of 32) one launch covers
-constexpr int kGemmRowTiles = 1;   // row tiles (of 32) per wavefront in the form without LDS
-constexpr int kGemmSteps = 4;      // k-steps whose loads are issued together there
-// Slabs that fill their launch share the fragments through LDS (tall_gemm_lds_bf16_kernel): results of up to two
-// column tiles as one slab with four k-steps per chunk, wider ones in slabs of four tiles with two steps per chunk
-// (measured: 64 against 77 us at 256 -> 40, 200 against 230 at 256 -> 256; the other splits tried were slower).
+constexpr int kGemmSlabTiles = 4;  // column tiles (of 32) per wavefront at most
 
 __global__ __launch_bounds__(kBlock) void gemm_prepare_kernel(const float* __restrict__ M, int64_t ld, int transposed,
                                                               int D, int K, u32x4* __restrict__ table) {
@@ -381,95 +389,18 @@ __global__ __launch_bounds__(kBlock) void gemm_prepare_kernel(const float* __res
   dst[2 * kWave] = s.lo;
 }
 
-// A wavefront owns RT row tiles (32 RT rows) and NT column tiles, with the loads of KS k-steps of X in flight.
-// Measured on [169343 .. 2449029, 100 .. 604] x [.., 40 .. 352]: one row tile, four column tiles and four steps
-// is the fastest split (two or three row tiles per wavefront -- every fragment of M then serves several
-// products -- cost more in occupancy than they save in fragment loads: 330 against 236 us at 256 x 256).  The
-// kernel then equals the framework's fp32 GEMM at 256 output columns and beats it by 20 - 25 % at 40 - 47.
-template <int VEC, int RT, int NT, int KS>
-__global__ __launch_bounds__(kWave) void tall_gemm_bf16_kernel(const float* __restrict__ X,
-                                                               const u32x4* __restrict__ table, int64_t N, int D, int K,
-                                                               int tiles, int tile0, const float* __restrict__ bias,
-                                                               const float* addend, int64_t ldc, float* out,
-                                                               int64_t ldo) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int half = lane >> 5, l32 = lane & 31;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * (kTile * RT);
-  const u32x4* frags = table + 1;
-  const float* xrow[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int64_t r = row0 + rt * kTile + l32;
-    xrow[rt] = X + (r < N ? r : N - 1) * D;
-  }
-  const int total = (D + kStepFeatures - 1) / kStepFeatures;
-  floatx16 acc[RT][NT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[rt][nt][v] = 0.f;
-
-  for (int s0 = 0; s0 < total; s0 += KS) {
-    float a[KS][RT][8];
-    if ((s0 + KS) * kStepFeatures <= D) {  // wave-uniform: the KS steps lie inside the row, nothing to mask
-#pragma unroll
-      for (int sb = 0; sb < KS; ++sb)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) load8<VEC>(xrow[rt], (s0 + sb) * kStepFeatures + 8 * half, 0x7FFFFFFF, a[sb][rt]);
-    } else {
-#pragma unroll
-      for (int sb = 0; sb < KS; ++sb)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) load8<VEC>(xrow[rt], (s0 + sb) * kStepFeatures + 8 * half, D, a[sb][rt]);
-    }
-#pragma unroll
-    for (int sb = 0; sb < KS; ++sb) {
-      const int st = (s0 + sb < total) ? s0 + sb : s0;  // a step past the row meets zeros: any valid fragment will do
-      Split8 pieces[RT];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) pieces[rt] = split3x8(a[sb][rt]);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const u32x4* src = frags + (static_cast<int64_t>(st) * tiles + tile0 + nt) * 3 * kWave + lane;
-        u32x4 b[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p) b[p] = src[p * kWave];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) acc[rt][nt] = step_product<3>(pieces[rt], b, acc[rt][nt]);
-      }
-    }
-  }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int col = (tile0 + nt) * kTile + l32;
-    const float b = (bias != nullptr && col < K) ? bias[col] : 0.f;
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t n = row0 + rt * kTile + 8 * (v / 4) + 4 * half + (v % 4);
-        if (n < N && col < K) {
-          float val = acc[rt][nt][v];
-          if (bias != nullptr) val = val + b;
-          if (addend != nullptr) val = val + addend[n * ldc + col];
-          __builtin_nontemporal_store(val, out + n * ldo + col);
-        }
-      }
-  }
-}
-
-// The same product with the fragments of M shared by a workgroup: four wavefronts (128 rows) copy the fragments
-// of KS k-steps x NT column tiles into LDS once and all read them from there, so the L2 sees a quarter of the
-// fragment traffic and the wavefronts' fragment loads become LDS reads.  For results wider than a few tiles, where
-// every wavefront of the form above streams the whole slab of M through the vector memory pipeline.
-template <int VEC, int RT, int NT, int KS>
-__global__ __launch_bounds__(kBlock) void tall_gemm_lds_bf16_kernel(const float* __restrict__ X,
-                                                                    const u32x4* __restrict__ table, int64_t N, int D,
-                                                                    int K, int tiles, int slabs,
-                                                                    const float* __restrict__ bias, const float* addend,
-                                                                    int64_t ldc, float* out, int64_t ldo) {
+// A workgroup of four wavefronts (128 rows) copies the fragments of KS k-steps x NT column tiles into LDS once and all
+// read them from there; each wavefront owns 32 rows and a slab of NT column tiles.  What bounds it at [169343, 256] x
+// [256, 256]: six matrix-core products per fp32 product (67 us at the 1.9 GHz the chip holds under this load), the
+// vector instructions that split X, and HBM (58 us) -- overlapped only by other wavefronts, so their number is what
+// counts: four tiles with one k-step per chunk at four wavefronts per SIMD 144 us, two steps at three 151, the next
+// chunk fetched ahead into a second buffer at two 204, two row tiles per wavefront 287.  Narrower slabs take longer
+// chunks (two steps for three tiles, four for one and two: 45 against 57 us at 256 -> 40 with four wavefronts forced).
+template <int NT, int KS>
+__global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(const float* __restrict__ X, const u32x4* __restrict__ table,
+                                                              int64_t N, int D, int K, int tiles, int slabs,
+                                                              const float* __restrict__ bias, const float* addend,
+                                                              int64_t ldc, float* out, int64_t ldo) {
   HIP_DYNAMIC_SHARED(u32x4, shared_frags)  // [KS][NT][3][64]
   // One launch covers `slabs` column slabs of NT tiles each.  Workgroups are handed to the 8 XCDs (each with its own
   // L2) round-robin by index, so the workgroups of one row block -- one per slab -- take indices 8 apart: they run on
@@ -478,60 +409,46 @@ __global__ __launch_bounds__(kBlock) void tall_gemm_lds_bf16_kernel(const float*
   const int64_t in_group = blockIdx.x % (kGemmXcds * slabs);
   const int64_t row_block = blockIdx.x / (kGemmXcds * slabs) * kGemmXcds + in_group % kGemmXcds;
   const int tile0 = static_cast<int>(in_group / kGemmXcds) * NT;
-  if (row_block * (kBlock / kWave) * (kTile * RT) >= N) return;
-  constexpr int kUnits = KS * NT * 3 * kWave;             // 16-byte units per chunk
-  constexpr int kPerThread = kUnits / kBlock;             // KS * NT * 3 / 4
-  static_assert(kUnits % kBlock == 0, "whole units per thread");
-  constexpr int kStepUnits = NT * 3 * kWave;              // contiguous in the table for one k-step
+  if (row_block * (kBlock / kWave) * kTile >= N) return;
+  constexpr int kUnits = KS * NT * 3 * kWave;  // 16-byte units per chunk
+  constexpr int kPerThread = (kUnits + kBlock - 1) / kBlock;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
   const int half = lane >> 5, l32 = lane & 31;
-  // a wavefront owns RT row tiles, so that a fragment read from LDS could serve RT products.  Measured at
-  // [169343, 256] x [256, 256]: 201 us with one row tile, 287 with two, 280 with three -- the kernel lives on
-  // the number of wavefronts in flight (registers per wavefront), not on fragment reads; RT = 1 is what is launched
-  const int64_t row0 = (row_block * (kBlock / kWave) + wave) * (kTile * RT);
+  const int64_t row0 = (row_block * (kBlock / kWave) + wave) * kTile;
   const u32x4* frags = table + 1;
-  const float* xrow[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int64_t r = row0 + rt * kTile + l32;
-    xrow[rt] = X + (r < N ? r : N - 1) * D;
-  }
+  const float* xrow = X + (row0 + l32 < N ? row0 + l32 : N - 1) * D;
   const int total = (D + kStepFeatures - 1) / kStepFeatures;
-  floatx16 acc[RT][NT];
+  floatx16 acc[NT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[rt][nt][v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[nt][v] = 0.f;
 
-  for (int s0 = 0; s0 < total; s0 += KS) {
-    float a[KS][RT][8];
-    if ((s0 + KS) * kStepFeatures <= D) {  // wave-uniform: the KS steps lie inside the row, nothing to mask
-#pragma unroll
-      for (int sb = 0; sb < KS; ++sb)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) load8<VEC>(xrow[rt], (s0 + sb) * kStepFeatures + 8 * half, 0x7FFFFFFF, a[sb][rt]);
-    } else {
-#pragma unroll
-      for (int sb = 0; sb < KS; ++sb)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) load8<VEC>(xrow[rt], (s0 + sb) * kStepFeatures + 8 * half, D, a[sb][rt]);
-    }
-    // this thread's share of the chunk's fragments: global -> registers -> LDS
-    u32x4 mine[kPerThread];
+  // This thread's share of a chunk's fragments.  A step past the row meets zeros of X and a tile past the last column
+  // feeds accumulators that are never stored: any valid fragment will do for either.
+  const int step_units = tiles * 3 * kWave;  // of the table: at most 4096 / 32 tiles and 4096 / 16 steps, 32-bit offsets
+  auto fetch_frags = [&](int s0, u32x4 (&mine)[kPerThread]) {
 #pragma unroll
     for (int u = 0; u < kPerThread; ++u) {
-      const int c = u * kBlock + static_cast<int>(threadIdx.x);  // unit of the chunk
-      const int sb = c / kStepUnits, within = c - sb * kStepUnits;
-      const int st = (s0 + sb < total) ? s0 + sb : s0;            // a step past the row meets zeros of X
-      mine[u] = frags[(static_cast<int64_t>(st) * tiles + tile0) * 3 * kWave + within];
+      int c = u * kBlock + static_cast<int>(threadIdx.x);  // unit of the chunk: [step][tile][piece][lane]
+      if (c >= kUnits) c = 0;                              // not parked
+      const int sb = c / (NT * 3 * kWave), tp = c / kWave % (NT * 3);
+      const int st = s0 + sb < total ? s0 + sb : s0;
+      const int tile = tile0 + tp / 3 < tiles ? tile0 + tp / 3 : tiles - 1;
+      mine[u] = frags[static_cast<uint32_t>(st * step_units + (tile * 3 + tp % 3) * kWave + (c & (kWave - 1)))];
     }
-    __syncthreads();  // the previous chunk has been read by every wavefront
+  };
+  auto fetch_rows = [&](int s0, float (&a)[KS][8]) {
+    if ((s0 + KS) * kStepFeatures <= D) {  // wave-uniform: the KS steps lie inside the row, nothing to mask
 #pragma unroll
-    for (int u = 0; u < kPerThread; ++u) shared_frags[u * kBlock + threadIdx.x] = mine[u];
-    __syncthreads();
+      for (int sb = 0; sb < KS; ++sb) load8_inside(xrow + (s0 + sb) * kStepFeatures + 8 * half, a[sb]);
+    } else {
+#pragma unroll
+      for (int sb = 0; sb < KS; ++sb) load8<2>(xrow, (s0 + sb) * kStepFeatures + 8 * half, D, a[sb]);
+    }
+  };
+  auto multiply = [&](const float (&a)[KS][8]) {
 #pragma unroll
     for (int sb = 0; sb < KS; ++sb) {
       u32x4 b[NT][3];
@@ -539,82 +456,133 @@ __global__ __launch_bounds__(kBlock) void tall_gemm_lds_bf16_kernel(const float*
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int p = 0; p < 3; ++p) b[nt][p] = shared_frags[((sb * NT + nt) * 3 + p) * kWave + lane];
+      const Split8 pieces = split3x8(a[sb]);
+      // the six products of step_product<3>, in its order for every tile, issued tile after tile: consecutive
+      // matrix-core instructions write different accumulators and none waits for its predecessor
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const Split8 pieces = split3x8(a[sb][rt]);
-        // the six products of step_product<3>, in its order for every tile, issued tile after tile: consecutive
-        // matrix-core instructions write different accumulators and none waits for its predecessor
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.mid, b[nt][1], acc[nt]);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.mid, b[nt][1], acc[rt][nt]);
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.lo, b[nt][0], acc[nt]);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.lo, b[nt][0], acc[rt][nt]);
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.hi, b[nt][2], acc[nt]);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.hi, b[nt][2], acc[rt][nt]);
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.mid, b[nt][0], acc[nt]);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.mid, b[nt][0], acc[rt][nt]);
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.hi, b[nt][1], acc[nt]);
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.hi, b[nt][1], acc[rt][nt]);
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma_bf16(pieces.hi, b[nt][0], acc[nt]);
+    }
+  };
+
+  for (int s0 = 0; s0 < total; s0 += KS) {
+    float a[KS][8];
+    fetch_rows(s0, a);
+    u32x4 mine[kPerThread];
+    fetch_frags(s0, mine);
+    __syncthreads();  // the previous chunk has been read by every wavefront
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = mfma_bf16(pieces.hi, b[nt][0], acc[rt][nt]);
+    for (int u = 0; u < kPerThread; ++u) {
+      const int c = u * kBlock + static_cast<int>(threadIdx.x);
+      if (kUnits % kBlock == 0 || c < kUnits) shared_frags[c] = mine[u];
+    }
+    __syncthreads();
+    multiply(a);
+  }
+  // Accumulator register v is row 8 (v / 4) + 4 half + v % 4 of the wavefront's 32.
+  float* first = out + (row0 + 4 * half) * ldo + tile0 * kTile + l32;
+  // Rows all inside (all but the last wavefront of the matrix): the addresses advance by additions.  A bounds test
+  // and a 64-bit product per element were a third of the kernel's vector instructions (183 against 144 us).
+  if (row0 + kTile <= N) {
+    const float* add = addend == nullptr ? nullptr : addend + (row0 + 4 * half) * ldc + tile0 * kTile + l32;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int col = (tile0 + nt) * kTile + l32;
+      if (col >= K) continue;
+      const float b = bias != nullptr ? bias[col] : 0.f;
+      float* dst = first + nt * kTile;
+      if (addend == nullptr) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          __builtin_nontemporal_store(bias != nullptr ? acc[nt][v] + b : acc[nt][v], dst);
+          dst += v % 4 == 3 ? 5 * ldo : ldo;
+        }
+      } else {
+        const float* src = add + nt * kTile;
+        float more[16];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          more[v] = *src;
+          src += v % 4 == 3 ? 5 * ldc : ldc;
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          __builtin_nontemporal_store((bias != nullptr ? acc[nt][v] + b : acc[nt][v]) + more[v], dst);
+          dst += v % 4 == 3 ? 5 * ldo : ldo;
+        }
       }
     }
+    return;
   }
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int col = (tile0 + nt) * kTile + l32;
     const float b = (bias != nullptr && col < K) ? bias[col] : 0.f;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t n = row0 + rt * kTile + 8 * (v / 4) + 4 * half + (v % 4);
-        if (n < N && col < K) {
-          float val = acc[rt][nt][v];
-          if (bias != nullptr) val = val + b;
-          if (addend != nullptr) val = val + addend[n * ldc + col];
-          __builtin_nontemporal_store(val, out + n * ldo + col);
-        }
+    for (int v = 0; v < 16; ++v) {
+      const int64_t n = row0 + 8 * (v / 4) + 4 * half + (v % 4);
+      if (n < N && col < K) {
+        float val = acc[nt][v];
+        if (bias != nullptr) val = val + b;
+        if (addend != nullptr) val = val + addend[n * ldc + col];
+        __builtin_nontemporal_store(val, out + n * ldo + col);
       }
+    }
   }
 }
 
 // ---- backward ----------------------------------------------------------------
 // out[N, D] = Xr[N, k] . R^T: the reduction runs over the k kept columns (at most
 // 128: 8 k-steps); a wavefront owns 32 rows and a slab of NT * 32 output columns
-// (grid.y tiles D), the four wavefronts of a workgroup four consecutive row
+// of the result, the four wavefronts of a workgroup four consecutive row
 // tiles.  They share the slab's fragments, copied from the table into LDS; the
 // [N, D] result leaves through a per-wavefront LDS tile of 8 rows as 16-byte
-// streaming stores over whole rows of the slab (D % 4 == 0, `out` 16-byte
-// aligned), else as 4-byte stores from the accumulator layout.  The tile is
-// private to its wavefront, whose LDS accesses complete in order, so the
-// hand-over inside it needs no workgroup barrier.
+// stores at any element boundary.  The tile is private to its wavefront, whose
+// LDS accesses complete in order, so the hand-over inside it needs no workgroup
+// barrier.  Bound by writing [N, D]: with D no multiple of 32 neighbouring slabs
+// share lines, so the slabs of one row block take workgroup indices 8 apart (one
+// XCD, about the same time: 446 -> 175 us at
+// [232965, 76] x [602, 76]^T, where the stores were 4 bytes wide and the slabs apart).
 template <int NT>
 constexpr int bwd_tile_pitch() { return NT * kTile + 8; }  // 4 * pitch = 32 (mod 64): the two half-waves hit different banks
 
-template <int VEC, int NT, int BP, int KS, bool STAGED>  // KS: k-steps whose loads are issued (2, 4 or 8 >= the steps of k)
+template <int VEC, int NT, int BP, int KS>  // KS: k-steps whose loads are issued (2, 4 or 8 >= the steps of k)
 __global__ __launch_bounds__(kBlock) void rp_bwd_bf16_kernel(const float* __restrict__ Xr,
                                                              const u32x4* __restrict__ table, int64_t N, int D,
-                                                             int k, float* __restrict__ out) {
-  HIP_DYNAMIC_SHARED(u32x4, frag)  // the slab's fragments [step][NT][piece][lane], then (STAGED) the four output tiles
+                                                             int k, int slabs, float* __restrict__ out) {
+  HIP_DYNAMIC_SHARED(u32x4, frag)  // the slab's fragments [step][NT][piece][lane], then the four output tiles
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
   const int half = lane >> 5;
   const int l32 = lane & 31;
-  const int dbase = blockIdx.y * (NT * kTile);
-  const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave) * kTile;
+  const int64_t in_group = blockIdx.x % (kRpXcds * slabs);
+  const int slab = static_cast<int>(in_group / kRpXcds);
+  const int64_t row_block = blockIdx.x / (kRpXcds * slabs) * kRpXcds + in_group % kRpXcds;
+  if (row_block * (kBlock / kWave) * kTile >= N) return;  // whole workgroup, before any barrier
+  const int dbase = slab * (NT * kTile);
+  const int64_t row0 = (row_block * (kBlock / kWave) + wave) * kTile;
   const int64_t my_row = (row0 + l32 < N) ? row0 + l32 : N - 1;
   const float* xrow = Xr + my_row * k;
   const TableShape ts = table_shape(D, k, BP);
   const int steps = ts.steps_k;  // <= KS
   const u32x4* bwd = table + 1 + ts.fwd_units();
 
-  // my loads first, then the fragments of this slab: tiles blockIdx.y * NT .. + NT - 1 (past the last tile: zeros)
+  // my loads first, then the fragments of this slab: tiles slab * NT .. + NT - 1 (past the last tile: zeros)
   float a[KS][8];
 #pragma unroll
   for (int sb = 0; sb < KS; ++sb) load8<VEC>(xrow, sb * kStepFeatures + 8 * half, k, a[sb]);
   for (int idx = threadIdx.x; idx < steps * NT * BP * kWave; idx += kBlock) {
     const int l = idx & (kWave - 1), p = (idx / kWave) % BP, nt = (idx / (kWave * BP)) % NT, st = idx / (kWave * BP * NT);
-    const int tile = blockIdx.y * NT + nt;
+    const int tile = slab * NT + nt;
     u32x4 w = {0u, 0u, 0u, 0u};
     if (tile < ts.tiles_d) w = bwd[((static_cast<int64_t>(st) * ts.tiles_d + tile) * BP + p) * kWave + l];
     frag[idx] = w;
@@ -648,36 +616,30 @@ __global__ __launch_bounds__(kBlock) void rp_bwd_bf16_kernel(const float* __rest
       for (int v = 0; v < 16; ++v) acc[nt][v] = acc[nt][v] * c;
   }
 
-  if constexpr (STAGED) {
-    constexpr int PC = bwd_tile_pitch<NT>();
-    constexpr int kQuadsPerRow = NT * kTile / 4;
-    float* Ct = reinterpret_cast<float*>(frag + steps * NT * BP * kWave) + wave * (8 * PC);  // [8][PC], this wavefront's own
+  constexpr int PC = bwd_tile_pitch<NT>();
+  constexpr int kQuadsPerRow = NT * kTile / 4;
+  float* Ct = reinterpret_cast<float*>(frag + steps * NT * BP * kWave) + wave * (8 * PC);  // [8][PC], this wavefront's own
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {  // rows 8 g .. 8 g + 7 of the wavefront's 32
-      wave_sync_lds();             // the tile's previous contents have been read
+  for (int g = 0; g < 4; ++g) {  // rows 8 g .. 8 g + 7 of the wavefront's 32
+    wave_sync_lds();             // the tile's previous contents have been read
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) Ct[(4 * half + r) * PC + nt * kTile + l32] = acc[nt][4 * g + r];
-      wave_sync_lds();
+      for (int r = 0; r < 4; ++r) Ct[(4 * half + r) * PC + nt * kTile + l32] = acc[nt][4 * g + r];
+    wave_sync_lds();
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const int f = j * kWave + lane;
-        const int tr = f / kQuadsPerRow, tq = f - tr * kQuadsPerRow;
-        const int64_t rr = row0 + 8 * g + tr;
-        const int cj = dbase + 4 * tq;
-        const f32x4 q = *reinterpret_cast<const f32x4*>(Ct + tr * PC + 4 * tq);
-        if (rr < N && cj < D) __builtin_nontemporal_store(q, reinterpret_cast<f32x4*>(out + rr * D + cj));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int cj = dbase + nt * kTile + l32;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t rr = row0 + 8 * (v / 4) + 4 * half + (v % 4);
-        if (rr < N && cj < D) __builtin_nontemporal_store(acc[nt][v], out + rr * D + cj);
+    for (int j = 0; j < NT; ++j) {
+      const int f = j * kWave + lane;
+      const int tr = f / kQuadsPerRow, tq = f - tr * kQuadsPerRow;
+      const int64_t rr = row0 + 8 * g + tr;
+      const int cj = dbase + 4 * tq;
+      const f32x4 q = *reinterpret_cast<const f32x4*>(Ct + tr * PC + 4 * tq);
+      if (rr >= N || cj >= D) continue;
+      float* dst = out + rr * D + cj;
+      if (cj + 4 <= D) {
+        *reinterpret_cast<f32x4_any*>(dst) = q;
+      } else {
+        for (int i = 0; i < D - cj; ++i) dst[i] = q[i];
       }
     }
   }
@@ -716,22 +678,17 @@ static int rp_fwd_pack_bf16_launch(const RpPackArgs& a, const u32x4* table, hipS
 template <int VEC, int BP, int KS>
 static int rp_bwd_bf16_launch(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
   const int steps = (k + kStepFeatures - 1) / kStepFeatures;
-  const bool staged = D % 4 == 0 && al16(out);
-  // output slab per workgroup: 128 columns; 64 when the fragments of a 128-column slab (and the tiles) pass 64 KB
+  // output slab per workgroup: 128 columns; 64 when the fragments of a 128-column slab and the tiles pass 64 KB
   const size_t frag4 = static_cast<size_t>(steps) * 4 * BP * kWave * 16;
-  const size_t tiles4 = staged ? sizeof(float) * (kBlock / kWave) * 8 * bwd_tile_pitch<4>() : 0;
-  const int nt = (frag4 + tiles4 <= 64 * 1024) ? 4 : 2;
-  const dim3 grid(static_cast<unsigned>((N + 127) / 128), static_cast<unsigned>((D + nt * kTile - 1) / (nt * kTile)));
-  const dim3 block(kBlock);
-  if (nt == 4) {
-    const size_t lds = frag4 + tiles4;
-    if (staged) hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 4, BP, KS, true>), grid, block, lds, s, Xr, table, N, D, k, out);
-    else hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 4, BP, KS, false>), grid, block, lds, s, Xr, table, N, D, k, out);
-  } else {
-    const size_t lds = frag4 / 2 + (staged ? sizeof(float) * (kBlock / kWave) * 8 * bwd_tile_pitch<2>() : 0);
-    if (staged) hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 2, BP, KS, true>), grid, block, lds, s, Xr, table, N, D, k, out);
-    else hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 2, BP, KS, false>), grid, block, lds, s, Xr, table, N, D, k, out);
-  }
+  const size_t lds4 = frag4 + sizeof(float) * (kBlock / kWave) * 8 * bwd_tile_pitch<4>();
+  const size_t lds2 = frag4 / 2 + sizeof(float) * (kBlock / kWave) * 8 * bwd_tile_pitch<2>();
+  const int nt = lds4 <= 64 * 1024 ? 4 : 2;
+  const int slabs = (D + nt * kTile - 1) / (nt * kTile);
+  const int64_t groups = ((N + 127) / 128 + kRpXcds - 1) / kRpXcds * kRpXcds * slabs;
+  if (groups > 0x7FFFFFFF) return EXACT_E_SHAPE;
+  const dim3 grid(static_cast<unsigned>(groups)), block(kBlock);
+  if (nt == 4) hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 4, BP, KS>), grid, block, lds4, s, Xr, table, N, D, k, slabs, out);
+  else hipLaunchKernelGGL((rp_bwd_bf16_kernel<VEC, 2, BP, KS>), grid, block, lds2, s, Xr, table, N, D, k, slabs, out);
   return launch_status();
 }
 
@@ -882,61 +839,25 @@ int exact_tall_gemm_bf16_f32(const float* X, const void* table, int64_t N, int64
   if (N == 0) return EXACT_OK;
   if (!X || !table || !out) return EXACT_E_NULL;
   if (!al16(table) || !al8(X)) return EXACT_E_ALIGN;
-  const bool quads = D % 4 == 0 && al16(X);  // 16-byte loads of X, else 8-byte ones
   hipStream_t s = static_cast<hipStream_t>(stream);
   const u32x4* t = static_cast<const u32x4*>(table);
   const int d = static_cast<int>(D), kk = static_cast<int>(K);
   const int tiles = (kk + kTile - 1) / kTile;
-  const int64_t rows_per_wave = static_cast<int64_t>(kTile) * kGemmRowTiles;
-  const dim3 grid(static_cast<unsigned>((N + rows_per_wave - 1) / rows_per_wave)), block(kWave);
-#ifndef EXACT_GEMM_LDS_ROW_TILES
-#define EXACT_GEMM_LDS_ROW_TILES 1
-#endif
-  constexpr int kLdsRowTiles = EXACT_GEMM_LDS_ROW_TILES;  // row tiles per wavefront in the LDS form
-  const int64_t lrows = static_cast<int64_t>(4) * kTile * kLdsRowTiles;  // four wavefronts
-  const int64_t lgroups = ((N + lrows - 1) / lrows + kGemmXcds - 1) / kGemmXcds;  // groups of 8 row blocks
-  if (lgroups * kGemmXcds * (tiles / kGemmSlabTiles + 1) > 0x7FFFFFFF) return EXACT_E_SHAPE;
-  const dim3 lblock(kBlock);
-#define EXACT_GEMM_LDS(NTV, KSV)                                                                                    \
-  do {                                                                                                              \
-    if (quads)                                                                                                      \
-      hipLaunchKernelGGL((tall_gemm_lds_bf16_kernel<4, kLdsRowTiles, NTV, KSV>), lgrid, lblock,                     \
-                         sizeof(u32x4) * KSV * NTV * 3 * kWave, s, X, t, N, d, kk, tiles, slabs, bias, addend, ldc, out, ldo); \
-    else                                                                                                            \
-      hipLaunchKernelGGL((tall_gemm_lds_bf16_kernel<2, kLdsRowTiles, NTV, KSV>), lgrid, lblock,                     \
-                         sizeof(u32x4) * KSV * NTV * 3 * kWave, s, X, t, N, d, kk, tiles, slabs, bias, addend, ldc, out, ldo); \
-  } while (0)
-#define EXACT_GEMM_GO(NTV)                                                                                          \
-  do {                                                                                                              \
-    if (quads)                                                                                                      \
-      hipLaunchKernelGGL((tall_gemm_bf16_kernel<4, kGemmRowTiles, NTV, kGemmSteps>), grid, block, 0, s, X, t, N, d, kk, tiles, \
-                         tile0, bias, addend, ldc, out, ldo);                                                      \
-    else                                                                                                            \
-      hipLaunchKernelGGL((tall_gemm_bf16_kernel<2, kGemmRowTiles, NTV, kGemmSteps>), grid, block, 0, s, X, t, N, d, kk, tiles, \
-                         tile0, bias, addend, ldc, out, ldo);                                                      \
-  } while (0)
-  if (tiles == 2) {
-    const int slabs = 1;
-    const dim3 lgrid(static_cast<unsigned>(lgroups * kGemmXcds));
-    EXACT_GEMM_LDS(2, 4);
-    return launch_status();
+  // slabs of equal width, at most four tiles: every slab in one launch, less than one tile per slab for padding
+  const int slabs = (tiles + kGemmSlabTiles - 1) / kGemmSlabTiles;
+  const int64_t rows = static_cast<int64_t>(kBlock / kWave) * kTile;
+  const int64_t groups = ((N + rows - 1) / rows + kGemmXcds - 1) / kGemmXcds;  // groups of 8 row blocks
+  if (groups * kGemmXcds * slabs > 0x7FFFFFFF) return EXACT_E_SHAPE;
+  const dim3 grid(static_cast<unsigned>(groups * kGemmXcds * slabs)), block(kBlock);
+#define EXACT_GEMM_GO(NT, KS)                                                                                          \
+  hipLaunchKernelGGL((tall_gemm_kernel<NT, KS>), grid, block, sizeof(u32x4) * KS * NT * 3 * kWave, s, X, t, N, d, kk, \
+                     tiles, slabs, bias, addend, ldc, out, ldo)
+  switch ((tiles + slabs - 1) / slabs) {
+    case 1: EXACT_GEMM_GO(1, 4); break;
+    case 2: EXACT_GEMM_GO(2, 4); break;
+    case 3: EXACT_GEMM_GO(3, 2); break;
+    default: EXACT_GEMM_GO(4, 1); break;
   }
-  // every full slab of four tiles in one launch (slabs of two tiles, twice as many sharing an L2 and four
-  // wavefronts per SIMD instead of three, measured 5 - 8 % slower: each slab splits X into bf16 pieces again)
-  if (const int slabs = tiles / kGemmSlabTiles) {
-    const dim3 lgrid(static_cast<unsigned>(lgroups * kGemmXcds * slabs));
-    EXACT_GEMM_LDS(4, 2);
-  }
-  if (const int tile0 = tiles / kGemmSlabTiles * kGemmSlabTiles; tile0 < tiles) {  // a last, narrower slab
-    const int nt = tiles - tile0;
-    switch (nt) {
-      case 1: EXACT_GEMM_GO(1); break;
-      case 2: EXACT_GEMM_GO(2); break;
-      case 3: EXACT_GEMM_GO(3); break;
-      default: EXACT_GEMM_GO(4); break;
-    }
-  }
-#undef EXACT_GEMM_LDS
 #undef EXACT_GEMM_GO
   return launch_status();
 }
