@@ -30,8 +30,10 @@ def spmm_csr(rowptr, col, value, mat, reduce):
     {sum, mean} (spmm_cuda.cu:106-170)."""
     if reduce not in REDUCE:
         raise NotImplementedError(f"reduce='{reduce}': use spmm_max_fw / spmm_min_fw for max and min")
-    if isinstance(mat, torch.Tensor) and mat.dtype == torch.float16:
-        # fp16 activations (autocast): gather and accumulate in fp32, round the result once
+    reproducible = config.deterministic_spmm or torch.are_deterministic_algorithms_enabled()
+    half = isinstance(mat, torch.Tensor) and mat.dtype == torch.float16
+    if half and (reproducible or not _checks.on_device(mat)):
+        # fp16 activations (autocast): accumulate in fp32, round the result once
         return spmm_csr(rowptr, col, value, mat.float(), reduce).to(torch.float16)
     _check_index(rowptr, "rowptr")
     _check_index(col, "col")
@@ -39,7 +41,7 @@ def spmm_csr(rowptr, col, value, mat, reduce):
         raise RuntimeError("mat must be CUDA tensor")
     if mat.dim() != 2:
         raise RuntimeError("Input mismatch: mat must be 2-D [N, K]")
-    if mat.dtype != torch.float32:
+    if mat.dtype != torch.float32 and not half:
         raise RuntimeError("The type of mat is not correct!")
     if value is not None:
         if not _checks.on_device(value):
@@ -55,8 +57,7 @@ def spmm_csr(rowptr, col, value, mat, reduce):
     rowptr, col = rowptr.contiguous(), col.contiguous()
     M = rowptr.numel() - 1
     n_cols, K = mat.shape
-    out = torch.empty((M, K), dtype=mat.dtype, device=mat.device)
-    reproducible = config.deterministic_spmm or torch.are_deterministic_algorithms_enabled()
+    out = torch.empty((M, K), dtype=torch.float32, device=mat.device)
     if reproducible:
         mat = mat.contiguous()
         rc = _lib.lib().exact_spmm_csr_rowwise_f32(ptr(rowptr), ptr(col), ptr(value), rowptr.element_size(), ptr(mat),
@@ -64,11 +65,11 @@ def spmm_csr(rowptr, col, value, mat, reduce):
                                                    _checks.stream_ptr(mat))
     else:
         mat = _aligned_rows(mat, col.numel())
-        rc = _lib.lib().exact_spmm_csr_strided_f32(ptr(rowptr), ptr(col), ptr(value), rowptr.element_size(), ptr(mat),
-                                                   mat.stride(0), M, n_cols, K, col.numel(), REDUCE[reduce], ptr(out), K,
-                                                   _checks.stream_ptr(mat))
+        kernel = _lib.lib().exact_spmm_csr_strided_f16 if half else _lib.lib().exact_spmm_csr_strided_f32
+        rc = kernel(ptr(rowptr), ptr(col), ptr(value), rowptr.element_size(), ptr(mat), mat.stride(0), M, n_cols, K,
+                    col.numel(), REDUCE[reduce], ptr(out), K, _checks.stream_ptr(mat))
     _lib.check(rc, f"spmm_{reduce}")
-    return out
+    return out.to(torch.float16) if half else out          # one rounding of the fp32 sum
 
 
 def _aligned_rows(mat, nnz):
@@ -81,8 +82,9 @@ def _aligned_rows(mat, nnz):
     if mat.stride(1) != 1 or mat.stride(0) < mat.shape[1]:
         mat = mat.contiguous()
     n_cols, K = mat.shape
-    if K > 128 and K % 32 != 0 and mat.stride(0) == K and n_cols > 0 and nnz >= 16 * n_cols:
-        padded = torch.empty((n_cols, (K + 31) // 32 * 32), dtype=mat.dtype, device=mat.device)
+    line = 128 // mat.element_size()
+    if K > 128 and K % line != 0 and mat.stride(0) == K and n_cols > 0 and nnz >= 16 * n_cols:
+        padded = torch.empty((n_cols, (K + line - 1) // line * line), dtype=mat.dtype, device=mat.device)
         padded[:, :K].copy_(mat)
         return padded[:, :K]
     return mat

@@ -141,6 +141,12 @@ int exact_spmm_csr_strided_f32(const void *rowptr, const void *col, const float 
                                int64_t n_cols, int64_t K, int64_t nnz, int reduce,
                                float *out, int64_t ldo, void *stream);
 
+/* The same for fp16 X: gathered as it is, accumulated and returned in fp32. */
+int exact_spmm_csr_strided_f16(const void *rowptr, const void *col, const float *val,
+                               int idx_bytes, const uint16_t *X, int64_t ldx, int64_t M,
+                               int64_t n_cols, int64_t K, int64_t nnz, int reduce,
+                               float *out, int64_t ldo, void *stream);
+
 /* The same product with a reproducible result: one wavefront per row, entries
  * added in CSR order with one multiply and one add each (the order of the
  * reference kernel, spmm_cuda.cu:85-90), no atomics.  Slower on hub rows. */
