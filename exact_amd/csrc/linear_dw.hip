@@ -251,8 +251,147 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_bf16_kernel(const float* 
     }
 }
 
-template <int MK, int MD, int WK, bool BF16>
-static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int Kout, int D, float* out,
+// The same with the fragments shared.  Above, every wavefront splits the fragments of its own rows and columns, and the
+// split (44 vector instructions per fragment) competes with the matrix cores.  Here the four wavefronts divide the
+// fragments of a step between them, split each once and hand the pieces round through LDS, in two buffers so that one
+// barrier per step suffices; the rows of the step after next are on their way while a step is multiplied.
+// [169343, 256]^T x [169343, 256]: 247 -> 161 us, [169343, 256]^T x [.., 128] 140 -> 95, [232965, 47]^T x [.., 300]
+// 166 -> 134.  Where a workgroup's block is one tile or fewer wavefronts share a fragment the barrier costs more than
+// the split ([20000, 40]^T x [.., 128] 25 -> 33, [2449029, 47]^T x [.., 64] 306 -> 359, [2449029, 256]^T x [.., 25]
+// 560 -> 620): those keep the form above.
+//
+// fp16 operands (autocast) are widened as they are loaded: exact, and exact again as bf16 pieces ([40000, 256]^T x
+// [.., 256]: 59 us; the framework's fp16 product takes 123 and rounds its partial sums' result once, as the caller does).
+template <int MK, int MD, int WK, typename T>
+__global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __restrict__ dY, int64_t ldy,
+                                                                const T* __restrict__ X, int64_t ldx, int64_t N,
+                                                                int Kout, int D, int64_t rows_per_slab, int blocks_d, int blocks, int64_t slabs,
+                                                                float* __restrict__ out) {
+  constexpr int WD = 4 / WK;
+  constexpr int KT = MK * WK, DT = MD * WD, F = KT + DT;  // fragments of a step: KT of dY, then DT of X
+  constexpr int FPW = (F + 3) / 4;                        // of them, per wavefront: wave, wave + 4, ..
+  constexpr int64_t kRows = 16;                           // rows per step
+  HIP_DYNAMIC_SHARED(u32x4, shared)                       // [2][F][piece][lane]
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int half = lane >> 5;
+  const int l32 = lane & 31;
+  int block;
+  int64_t slab;
+  if (!dw_block_and_slab(blocks, slabs, block, slab)) return;  // whole workgroup, before any barrier
+  const int bk = block / blocks_d, bd = block % blocks_d;
+  const int wk = wave / WD, wd = wave % WD;
+  const int k0 = (bk * WK + wk) * (32 * MK);
+  const int d0 = (bd * WD + wd) * (32 * MD);
+  const bool active = k0 < Kout && d0 < D;  // wave-uniform; an inactive wavefront still brings its fragments
+  const int64_t n_begin = slab * rows_per_slab;
+  const int64_t n_end = (n_begin + rows_per_slab < N) ? n_begin + rows_per_slab : N;
+
+  // my fragments' columns; past the last column: clamped, they only feed accumulators that are never stored
+  const T* src[FPW];
+  int64_t ld[FPW];
+#pragma unroll
+  for (int j = 0; j < FPW; ++j) {
+    const int f = wave + 4 * j < F ? wave + 4 * j : F - 1;
+    const bool is_y = f < KT;
+    const int c = is_y ? (bk * KT + f) * 32 + l32 : (bd * DT + f - KT) * 32 + l32;
+    src[j] = is_y ? dY + min(c, Kout - 1) : X + min(c, D - 1);
+    ld[j] = is_y ? ldy : ldx;
+  }
+  floatx16 acc[MK][MD];
+#pragma unroll
+  for (int i = 0; i < MK; ++i)
+#pragma unroll
+    for (int j = 0; j < MD; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  T raw[FPW][8];
+  auto load_step = [&](int64_t n0) {
+    if (n0 + kRows <= n_end) {  // the same in the whole workgroup: the step lies inside the slab, nothing to clamp
+#pragma unroll
+      for (int j = 0; j < FPW; ++j) {
+        const T* p = src[j] + (n0 + 8 * half) * ld[j];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          raw[j][e] = *p;
+          p += ld[j];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < FPW; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int64_t row = n0 + 8 * half + e;
+          const T v = src[j][(row < N ? row : N - 1) * ld[j]];
+          raw[j][e] = row < n_end ? v : static_cast<T>(0.f);
+        }
+    }
+  };
+  auto park_step = [&](int buffer) {
+#pragma unroll
+    for (int j = 0; j < FPW; ++j) {
+      const int f = wave + 4 * j;
+      if (f >= F) continue;  // wave-uniform
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(raw[j][e]);
+      const Split8 s = split3x8(v);
+      u32x4* dst = shared + (buffer * F + f) * 3 * kWave + lane;
+      dst[0] = s.hi;
+      dst[kWave] = s.mid;
+      dst[2 * kWave] = s.lo;
+    }
+  };
+  auto multiply = [&](int buffer) {
+    const u32x4* base = shared + buffer * F * 3 * kWave + lane;
+    u32x4 b[MD][3];
+#pragma unroll
+    for (int j = 0; j < MD; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) b[j][p] = base[((KT + wd * MD + j) * 3 + p) * kWave];
+#pragma unroll
+    for (int i = 0; i < MK; ++i) {
+      const u32x4* fa = base + (wk * MK + i) * 3 * kWave;
+      const Split8 a = {fa[0], fa[kWave], fa[2 * kWave]};
+#pragma unroll
+      for (int j = 0; j < MD; ++j) acc[i][j] = step_product<3>(a, b[j], acc[i][j]);
+    }
+  };
+
+  if (n_begin >= n_end) return;  // an empty slab: whole workgroup
+  load_step(n_begin);
+  park_step(0);
+  load_step(n_begin + kRows);  // past the slab: clamped addresses, zeroed values
+  __syncthreads();
+  int buffer = 0;
+  for (int64_t n0 = n_begin; n0 < n_end; n0 += kRows) {
+    if (active) multiply(buffer);
+    buffer ^= 1;
+    if (n0 + kRows < n_end) {   // the same in the whole workgroup
+      park_step(buffer);        // last read before the barrier that ended the previous step
+      load_step(n0 + 2 * kRows);
+      __syncthreads();
+    }
+  }
+  if (!active) return;
+
+#pragma unroll
+  for (int i = 0; i < MK; ++i)
+#pragma unroll
+    for (int j = 0; j < MD; ++j) {
+      const int cj = d0 + 32 * j + l32;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ri = k0 + 32 * i + 8 * (v / 4) + 4 * half + (v % 4);
+        if (ri < Kout && cj < D) unsafeAtomicAdd(out + static_cast<int64_t>(ri) * D + cj, acc[i][j][v]);
+      }
+    }
+}
+
+template <int MK, int MD, int WK, bool BF16, typename T>
+static void launch_dw(const T* dY, int64_t ldy, const T* X, int64_t ldx, int64_t N, int Kout, int D, float* out,
                       hipStream_t s) {
   constexpr int WD = 4 / WK;
   const int blocks_k = (Kout + 32 * MK * WK - 1) / (32 * MK * WK);
@@ -265,12 +404,15 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   rows = (rows + 15) / 16 * 16;  // whole batches (8 rows) resp. steps (16 rows)
   slabs = (N + rows - 1) / rows;
   const dim3 grid(static_cast<unsigned>((slabs + kDwXcds - 1) / kDwXcds * kDwXcds * blocks));
-  if (BF16) hipLaunchKernelGGL((linear_dw_bf16_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  constexpr size_t lds = sizeof(u32x4) * 2 * (MK * WK + MD * WD) * 3 * kWave;
+  constexpr bool shared = sizeof(T) == 2 || (MK == 2 && MD == 2 && WK < 4) || MK == 1;  // measured, see the kernel
+  if constexpr (BF16 && shared) hipLaunchKernelGGL((linear_dw_shared_kernel<MK, MD, WK, T>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  else if constexpr (BF16) hipLaunchKernelGGL((linear_dw_bf16_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
   else hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
 }
 
-template <bool BF16>
-static int linear_dw_any(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
+template <bool BF16, typename T>
+static int linear_dw_any(const T* dY, int64_t ldy, const T* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                          float* out, hipStream_t s) {
   if (N < 0 || Kout < 0 || D < 0 || Kout > 65536 || D > 65536 || N > (int64_t{1} << 40)) return EXACT_E_SHAPE;
   if (ldy < Kout || ldx < D) return EXACT_E_SHAPE;
@@ -283,15 +425,15 @@ static int linear_dw_any(const float* dY, int64_t ldy, const float* X, int64_t l
     // wavefront block: up to 64 x 64 of dW (wider blocks need more accumulator registers than two wavefronts
     // per SIMD leave); the four wavefronts side by side along the longer extent when the other fits one wavefront
     if (K <= 32) {
-      if (Dd <= 128) launch_dw<1, 1, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<1, 2, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 128) launch_dw<1, 1, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<1, 2, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
     } else if (K <= 64) {
-      if (Dd <= 128) launch_dw<2, 1, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<2, 2, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 128) launch_dw<2, 1, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<2, 2, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
     } else {
-      if (Dd <= 32) launch_dw<2, 1, 4, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else if (Dd <= 64) launch_dw<2, 2, 4, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<2, 2, 2, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 32) launch_dw<2, 1, 4, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else if (Dd <= 64) launch_dw<2, 2, 4, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<2, 2, 2, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
     }
   }
   return launch_status();
@@ -305,12 +447,18 @@ extern "C" {
 
 int exact_linear_dw_f32(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                         float* out, void* stream) {
-  return linear_dw_any<false>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
+  return linear_dw_any<false, float>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
 }
 
 int exact_linear_dw_bf16_f32(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                              float* out, void* stream) {
-  return linear_dw_any<true>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
+  return linear_dw_any<true, float>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
+}
+
+int exact_linear_dw_f16(const uint16_t* dY, int64_t ldy, const uint16_t* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
+                        float* out, void* stream) {
+  return linear_dw_any<true, half_t>(reinterpret_cast<const half_t*>(dY), ldy, reinterpret_cast<const half_t*>(X), ldx, N, Kout, D,
+                                     out, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"
