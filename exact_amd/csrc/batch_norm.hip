@@ -91,8 +91,8 @@ __device__ __forceinline__ void bn_meet(const BnBlock& b, int K, const float (&s
   }
 }
 
-// sums[k] = sum_n (x - center), sums[K + k] = sum_n (x - center)^2.  [50000, 512]: 22 us (4.6 TB/s); the framework's
-// one-call routine took 504 us there, with two workgroups.
+// sums[k] = sum_n (x - center), sums[K + k] = sum_n (x - center)^2.  [50000, 512]: 36 us (2.8 TB/s); the framework's
+// statistics took 504 us there, with two workgroups; [169343, 256]: 42 us.
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restrict__ x, const float* __restrict__ center,
                                                             int64_t N, int K, int64_t rows_per_wg, float* __restrict__ sums) {
@@ -205,7 +205,8 @@ __global__ __launch_bounds__(kBlock) void bn_apply_kernel(const float* __restric
 // each read dy, one mask bit and `bits` code bits per element: neither the masked gradient nor the dequantised
 // input is ever written to memory.  A thread takes four consecutive rows of its four columns per step: with 1 and 2
 // bits their codes are one 32-bit word, and four 16-byte loads of dy are in flight.  At [169343, 256] INT2 with a
-// mask the two passes replace mask 58 + dequantise 36 + reduce 68 + apply 100 us.
+// mask the two passes take 76 + 90 us where mask 58 + dequantise 36 + reduce 68 + apply 100 were; at [50000, 512]
+// without one 44 + 56 for dequantise 22 + reduce 699 + apply 59.
 struct BnBackward {
   const float* dy;
   const uint32_t* mask;  // null: g = dy
