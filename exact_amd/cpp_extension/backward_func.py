@@ -88,21 +88,18 @@ def weight_gradient(grad_output, input):  # noqa: A002
 
 # ---- the dense products of a layer on the bf16 matrix cores ---------------------
 def _gemm_table(matrix, transposed, D, K):
-    """Operand fragments of `matrix` for exact_tall_gemm_bf16_f32, remembered on the
-    tensor until it changes (a weight is prepared once per optimiser step)."""
-    key = (bool(transposed), matrix._version, matrix.data_ptr(), tuple(matrix.shape), matrix.stride(0))
-    cached = getattr(matrix, "_exact_gemm_table", None)
-    if cached is not None and cached[0] == key:
-        return cached[1]
+    """Operand fragments of `matrix` for exact_tall_gemm_bf16_f32, made anew for every
+    product on the stream it runs on (one launch of 4 us).  None is remembered: a
+    weight changes through `.data` without raising its version, a captured graph has
+    to read the weight of its replay, and another stream would have to wait for the
+    one that made the copy."""
     L = _lib.lib()
     table = torch.empty(int(L.exact_tall_gemm_table_nbytes(D, K)), dtype=torch.uint8, device=matrix.device)
     rc = L.exact_tall_gemm_prepare_bf16(_checks.ptr(matrix), matrix.stride(0), int(bool(transposed)), D, K, _checks.ptr(table),
                                         _checks.stream_ptr(matrix))
     _lib.check(rc, "tall_matmul (prepare)")
-    try:
-        matrix._exact_gemm_table = (key, table)
-    except AttributeError:
-        pass
+    # a mark for tests and profiles that the library's kernel took this operand; nothing reads it here
+    matrix._exact_gemm_table = (D, K)
     return table
 
 

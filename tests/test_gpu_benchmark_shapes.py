@@ -132,7 +132,7 @@ def test_tall_gemm_takes_rows_aligned_to_eight_bytes(cuda):
 
 
 def test_tall_gemm_reprepares_a_changed_matrix(cuda):
-    """The fragment table is remembered on the matrix and rebuilt when it changes in place (an optimiser step)."""
+    """The product follows a matrix that changes in place (an optimiser step)."""
     config.matrix_cores = "bf16"
     x = _ints((20000, 64), cuda, 1)
     w = torch.nn.Parameter(_ints((48, 64), cuda, 2))
