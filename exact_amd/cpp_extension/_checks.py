@@ -15,6 +15,16 @@ def on_device(t):
     return t.is_cuda
 
 
+def plain_values(*tensors):
+    """True where a kernel may stand in for differentiable operations on these
+    tensors (None is skipped) without anyone missing them: no tensor subclass, no
+    forward-mode tangent, no trace being recorded, no dispatch mode listening."""
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    unpack = torch.autograd.forward_ad.unpack_dual
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and unpack(t).tangent is None for t in tensors if t is not None)
+
+
 def check_device_tensor(t, name, dim=None, dtypes=(torch.float32,)):
     if not isinstance(t, torch.Tensor):
         _fail(f"{name} must be a tensor!")
