@@ -87,22 +87,6 @@ def weight_gradient(grad_output, input):  # noqa: A002
 
 
 # ---- the dense products of a layer on the bf16 matrix cores ---------------------
-def _gemm_table(matrix, transposed, D, K):
-    """Operand fragments of `matrix` for exact_tall_gemm_bf16_f32, made anew for every
-    product on the stream it runs on (one launch of 4 us).  None is remembered: a
-    weight changes through `.data` without raising its version, a captured graph has
-    to read the weight of its replay, and another stream would have to wait for the
-    one that made the copy."""
-    L = _lib.lib()
-    table = torch.empty(int(L.exact_tall_gemm_table_nbytes(D, K)), dtype=torch.uint8, device=matrix.device)
-    rc = L.exact_tall_gemm_prepare_bf16(_checks.ptr(matrix), matrix.stride(0), int(bool(transposed)), D, K, _checks.ptr(table),
-                                        _checks.stream_ptr(matrix))
-    _lib.check(rc, "tall_matmul (prepare)")
-    # a mark for tests and profiles that the library's kernel took this operand; nothing reads it here
-    matrix._exact_gemm_table = (D, K)
-    return table
-
-
 def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     """x[N, D] . M (+ bias[K]) (+ addend[N, K]) -> [N, K], where M = `matrix`
     ([D, K]) or, with transposed=True, the transpose of `matrix` ([K, D]: a weight
@@ -110,8 +94,9 @@ def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     itself (accumulate in place).  Tall fp32 device operands with an even number of
     features (config.tall_gemm_min_rows, tall_gemm_min_depth and
     tall_gemm_max_rows_wide) take the library's kernel (six bf16 matrix-core
-    products per fp32 product, fp32 accuracy, reproducible; config.matrix_cores ==
-    "bf16"); everything else the framework's GEMM."""
+    products per fp32 product, fp32 accuracy, reproducible, infinities and the ends
+    of the range as in fp32; config.matrix_cores == "bf16"); everything else the
+    framework's GEMM."""
     M = matrix.t() if transposed else matrix
     usable = (config.matrix_cores == "bf16" and x.dim() == 2 and matrix.dim() == 2 and x.dtype == torch.float32
               and matrix.dtype == torch.float32 and _checks.on_device(x) and _checks.on_device(matrix)
@@ -143,13 +128,18 @@ def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     N, D = x.shape
     K = M.shape[1]
     out = into if into is not None else torch.empty((N, K), dtype=torch.float32, device=x.device)
-    table = _gemm_table(matrix, transposed, D, K)
-    rc = _lib.lib().exact_tall_gemm_bf16_f32(_checks.ptr(x), _checks.ptr(table), N, D, K,
-                                             _checks.ptr(bias) if bias is not None else None,
-                                             _checks.ptr(addend) if addend is not None else None,
-                                             addend.stride(0) if addend is not None else K, _checks.ptr(out), out.stride(0),
-                                             _checks.stream_ptr(x))
+    # The weight's fragments are made by every call, on its stream and in scratch of its own (one launch of 5 us), and
+    # not remembered: a weight changes through `.data` without raising its version, a captured graph has to read the
+    # weight of its replay, and another stream would have to wait for the one that made the copy.
+    L = _lib.lib()
+    work = torch.empty(int(L.exact_tall_product_work_nbytes(D, K)), dtype=torch.uint8, device=x.device)
+    rc = L.exact_tall_product_f32(_checks.ptr(x), _checks.ptr(matrix), matrix.stride(0), int(bool(transposed)), N, D, K,
+                                  _checks.ptr(bias) if bias is not None else None,
+                                  _checks.ptr(addend) if addend is not None else None,
+                                  addend.stride(0) if addend is not None else K, _checks.ptr(out), out.stride(0),
+                                  _checks.ptr(work), _checks.stream_ptr(x))
     _lib.check(rc, "tall_matmul")
+    matrix._exact_gemm_table = (D, K)     # a mark for tests and profiles that the kernel took this operand; nothing reads it here
     return out
 
 

@@ -363,44 +363,218 @@ __global__ __launch_bounds__(kWave) void rp_fwd_pack_bf16_kernel(const RpPackArg
 constexpr int kGemmXcds = 8;       // accelerator complex dies of an MI355X, each with its own L2
 constexpr int kGemmSlabTiles = 4;  // column tiles (of 32) per wavefront at most
 
+// The ranges in which the pieces carry a row of X and a column of M (by its largest magnitude), see below.
+constexpr float kSmallRow = 0x1p-72f, kLargeRow = 0x1p+100f;
+constexpr float kSmallColumn = 0x1p-28f, kLargeColumn = 0x1p+10f;
+
+// the larger magnitude, NaN if either is one
+__device__ __forceinline__ float magnitude_or(float largest, float v) {
+  return __builtin_elementwise_maximum(largest, __builtin_elementwise_abs(v));
+}
+// The binary exponent that brings a largest magnitude into [1, 2); 0 for a column or row of zeros.
+__device__ __forceinline__ int unit_exponent(float largest) {
+  int e = 1;
+  if (largest > 0.f) frexpf(largest, &e);
+  return e - 1;
+}
+__device__ __forceinline__ float finite_magnitude(float v) {
+  const float m = fabsf(v);
+  return m <= 0x1.fffffep+127f ? m : 0.f;  // infinities and NaN set no scale
+}
+
+// Eight entries of M as pieces whose sum is the entry whatever it is: an infinity or a NaN stands in `hi` alone, a
+// finite value beyond bf16's largest takes the largest below it.
+__device__ __forceinline__ Split8 split3x8_any(const float (&v)[8]) {
+  Split8 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float rest[2];
+    uint32_t hi = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float x = v[2 * i + j];
+      const uint32_t magnitude = __float_as_uint(x) & 0x7FFFFFFFu;
+      const uint32_t shift = 16 * j;
+      if (magnitude < 0x7F800000u && ((hi >> shift) & 0x7F80u) == 0x7F80u)
+        hi = (hi & ~(0xFFFFu << shift)) | ((__float_as_uint(x) >> 16) << shift);
+      rest[j] = magnitude < 0x7F800000u ? x - (j ? high_bf16(hi) : low_bf16(hi)) : 0.f;
+    }
+    const uint32_t mid = pack_bf16x2(rest[0], rest[1]);
+    s.hi[i] = hi;
+    s.mid[i] = mid;
+    s.lo[i] = pack_bf16x2(rest[0] - low_bf16(mid), rest[1] - high_bf16(mid));
+  }
+  return s;
+}
+
+// A workgroup makes `steps_per_wg` k-steps of one column tile.  With `exps` a column whose largest magnitude is not
+// between kSmallColumn and kLargeColumn is brought into [1, 2) by a power of two (exact), so that its pieces add up to
+// it whatever it is.  The workgroups of a tile each find the 32 exponents (0: as it is) for themselves; behind the
+// exponents of all columns one word per tile says whether any is not 0 or any column holds an infinity or a NaN.
 __global__ __launch_bounds__(kBlock) void gemm_prepare_kernel(const float* __restrict__ M, int64_t ld, int transposed,
-                                                              int D, int K, u32x4* __restrict__ table) {
+                                                              int D, int K, int steps_per_wg, u32x4* __restrict__ table,
+                                                              int32_t* __restrict__ exps) {
+  __shared__ float part[2][kBlock];
+  __shared__ int column_exp[kTile], flags[kTile];
   const TableShape ts = table_shape(D, K, 3);
-  const int64_t frags = static_cast<int64_t>(ts.steps_d) * ts.tiles_k * kWave;
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (idx == 0) {
-    u32x4 head = {0u, 0u, 0u, 0u};
+  const int t = threadIdx.x, tile = blockIdx.x;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) {
+    const u32x4 head = {0u, 0u, 0u, 0u};
     table[0] = head;
   }
-  if (idx >= frags) return;
-  const int l = static_cast<int>(idx & (kWave - 1));
-  const int tile = static_cast<int>((idx / kWave) % ts.tiles_k), step = static_cast<int>(idx / (static_cast<int64_t>(kWave) * ts.tiles_k));
-  float r[8];
+  if (exps) {
+    // 8 threads a column; neighbouring lanes on neighbouring addresses either way M lies
+    const int cl = transposed ? t >> 3 : t & 31, g = transposed ? t & 7 : t >> 5;
+    const int c = tile * kTile + cl;
+    const float* src = M + (transposed ? static_cast<int64_t>(c < K ? c : K - 1) * ld : static_cast<int64_t>(c < K ? c : K - 1));
+    const int64_t stride = transposed ? 1 : ld;
+    float m = 0.f, all = 0.f;  // of the finite entries, of all
+    constexpr int kFlight = 32;  // loads in flight per thread: 256 rows in one latency
+    for (int d = g; d < D; d += 8 * kFlight) {
+      float v[kFlight];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int d = step * kStepFeatures + 8 * (l >> 5) + i, c = tile * kTile + (l & 31);
-    const bool inside = d < D && c < K;
-    r[i] = inside ? (transposed ? M[static_cast<int64_t>(c) * ld + d] : M[static_cast<int64_t>(d) * ld + c]) : 0.f;
+      for (int i = 0; i < kFlight; ++i) v[i] = src[(d + 8 * i < D ? d + 8 * i : d) * stride];
+#pragma unroll
+      for (int i = 0; i < kFlight; ++i) {
+        m = fmaxf(m, finite_magnitude(v[i]));
+        all = magnitude_or(all, v[i]);
+      }
+    }
+    part[0][cl * 8 + g] = m;
+    part[1][cl * 8 + g] = all;
+    __syncthreads();
+    if (t < kTile) {
+      m = all = 0.f;
+      for (int i = 0; i < 8; ++i) {
+        m = fmaxf(m, part[0][t * 8 + i]);
+        all = magnitude_or(all, part[1][t * 8 + i]);
+      }
+      const bool inside = tile * kTile + t < K;
+      const int e = !inside || (m >= kSmallColumn && m < kLargeColumn) ? 0 : unit_exponent(m);
+      column_exp[t] = e;
+      if (blockIdx.y == 0) exps[tile * kTile + t] = e;
+      flags[t] = e != 0 || (inside && !(all <= 0x1.fffffep+127f));
+    }
+    __syncthreads();
+    if (blockIdx.y == 0 && t == 0) {
+      int32_t f = 0;
+      for (int i = 0; i < kTile; ++i) f |= flags[i];
+      exps[ts.tiles_k * kTile + tile] = f;
+    }
   }
-  u32x4* dst = table + 1 + (static_cast<int64_t>(step) * ts.tiles_k + tile) * 3 * kWave + l;
-  const Split8 s = split3x8(r);
-  dst[0] = s.hi;
-  dst[kWave] = s.mid;
-  dst[2 * kWave] = s.lo;
+  const int l = t & (kWave - 1), c = tile * kTile + (l & 31);
+  const int first = static_cast<int>(blockIdx.y) * steps_per_wg;
+  const int end = first + steps_per_wg < ts.steps_d ? first + steps_per_wg : ts.steps_d;
+  for (int step = first + (t >> 6); step < end; step += kBlock / kWave) {
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int d = step * kStepFeatures + 8 * (l >> 5) + i;
+      const bool inside = d < D && c < K;
+      r[i] = inside ? (transposed ? M[static_cast<int64_t>(c) * ld + d] : M[static_cast<int64_t>(d) * ld + c]) : 0.f;
+      if (exps) r[i] = ldexpf(r[i], -column_exp[l & 31]);
+    }
+    u32x4* dst = table + 1 + (static_cast<int64_t>(step) * ts.tiles_k + tile) * 3 * kWave + l;
+    const Split8 s = split3x8_any(r);
+    dst[0] = s.hi;
+    dst[kWave] = s.mid;
+    dst[2 * kWave] = s.lo;
+  }
+}
+
+static void gemm_prepare(const float* M, int64_t ld, int transposed, int D, int K, u32x4* table, int32_t* exps, hipStream_t s) {
+  const TableShape ts = table_shape(D, K, 3);
+  // four steps a workgroup, one per wavefront, while that makes at most 512 workgroups: each reads its tile's columns whole
+  const int wanted = ts.tiles_k < 512 ? 512 / ts.tiles_k : 1;
+  const int groups = (ts.steps_d + 3) / 4 < wanted ? (ts.steps_d + 3) / 4 : wanted;
+  const int per_wg = (ts.steps_d + groups - 1) / groups;
+  hipLaunchKernelGGL(gemm_prepare_kernel, dim3(static_cast<unsigned>(ts.tiles_k), static_cast<unsigned>((ts.steps_d + per_wg - 1) / per_wg)),
+                     dim3(kBlock), 0, s, M, ld, transposed, D, K, per_wg, table, exps);
+}
+
+// ---- values that the three pieces do not carry --------------------------------
+// The pieces of an element of X reach from 2^-133 to bf16's largest number: an infinite or larger element turns into
+// infinity minus infinity, and one near the smallest normal number keeps its leading digits only.  A wavefront
+// therefore keeps the largest magnitude of each of its rows (four instructions a k-step).  Where that is within
+// kSmallRow .. kLargeRow, what the pieces of a smaller element lack is below 2^-61 of it, and with the columns of M
+// between kSmallColumn and kLargeColumn no product of pieces that counts leaves the normal range either way.  A
+// wavefront with a row outside (or a NaN in one), and every wavefront at a tile with such a column, forms the tile on
+// the fp32 matrix instruction instead, from the row and the columns scaled by powers of two, in which infinities and
+// NaN go through as in any fp32 product.
+__device__ __forceinline__ bool row_needs_fp32(float largest) {
+  return largest != 0.f && !(largest >= kSmallRow && largest < kLargeRow);
+}
+
+__device__ __forceinline__ void tall_gemm_fp32_tiles(const float* xrow, const u32x4* frags, const int32_t* exps, int64_t N, int D, int K,
+                                                  int tiles, int tile0, uint32_t which, int64_t row0, const float* bias,
+                                                  const float* addend, int64_t ldc, float* out, int64_t ldo) {
+  const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, l32 = lane & 31;
+  const int total = (D + kStepFeatures - 1) / kStepFeatures;
+  float largest = 0.f;
+#pragma unroll 1
+  for (int st = 0; st < total; ++st) {
+    float a[8];
+    load8<2>(xrow, st * kStepFeatures + 8 * half, D, a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) largest = fmaxf(largest, finite_magnitude(a[e]));
+  }
+  largest = fmaxf(largest, __shfl_xor(largest, 32));
+  const int row_exp = unit_exponent(largest);
+  const int rows_left = N - row0 < kTile ? static_cast<int>(N - row0) : kTile;
+#pragma unroll 1
+  for (int tile = tile0; which != 0; ++tile, which >>= 1) {
+    if (!(which & 1u) || tile >= tiles) continue;
+    floatx16 c;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) c[v] = 0.f;
+#pragma unroll 1
+    for (int st = 0; st < total; ++st) {
+      float a[8];
+      load8<2>(xrow, st * kStepFeatures + 8 * half, D, a);
+      const u32x4* src = frags + (static_cast<int64_t>(st) * tiles + tile) * 3 * kWave + lane;
+      const u32x4 hi = src[0], mid = src[kWave], lo = src[2 * kWave];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t h = hi[e / 2], m = mid[e / 2], l = lo[e / 2];
+        const float b = e % 2 ? (high_bf16(h) + high_bf16(m)) + high_bf16(l) : (low_bf16(h) + low_bf16(m)) + low_bf16(l);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(ldexpf(a[e], -row_exp), b, c, 0, 0, 0);
+      }
+    }
+    const int col = tile * kTile + l32;
+    const int col_exp = exps ? exps[col] : 0;
+    const float b = (bias != nullptr && col < K) ? bias[col] : 0.f;
+    float* dst = out + (row0 + 4 * half) * ldo + col;
+    const float* src = addend == nullptr ? nullptr : addend + (row0 + 4 * half) * ldc + col;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int r = 8 * (v / 4) + 4 * half + (v % 4);
+      const int e = static_cast<int>(__shfl(static_cast<uint32_t>(row_exp), r)) + col_exp;
+      if (r < rows_left && col < K) {
+        float val = ldexpf(c[v], e);
+        if (bias != nullptr) val = val + b;
+        if (src != nullptr) val = val + *src;
+        *dst = val;
+      }
+      dst += v % 4 == 3 ? 5 * ldo : ldo;
+      if (src != nullptr) src += v % 4 == 3 ? 5 * ldc : ldc;
+    }
+  }
 }
 
 // A workgroup of four wavefronts (128 rows) copies the fragments of KS k-steps x NT column tiles into LDS once and all
 // read them from there; each wavefront owns 32 rows and a slab of NT column tiles.  What bounds it at [169343, 256] x
 // [256, 256]: six matrix-core products per fp32 product (67 us at the 1.9 GHz the chip holds under this load), the
 // vector instructions that split X, and HBM (58 us) -- overlapped only by other wavefronts, so their number is what
-// counts: four tiles with one k-step per chunk at four wavefronts per SIMD 144 us, two steps at three 151, the next
-// chunk fetched ahead into a second buffer at two 204, two row tiles per wavefront 287.  Narrower slabs take longer
-// chunks (two steps for three tiles, four for one and two: 45 against 57 us at 256 -> 40 with four wavefronts forced).
+// counts: four tiles with one k-step per chunk at four wavefronts per SIMD, two steps at three 5 % slower, the next
+// chunk fetched ahead into a second buffer at two 40 %, two row tiles per wavefront twice the time.  Narrower slabs take
+// longer chunks (two steps for three tiles, four for one and two), and are held to four wavefronts as well: without
+// that the compiler leaves two for three tiles (150 against 123 us at 256 -> 160) and three for two (64 against 61 at
+// 256 -> 40, both with the fragments' launch).
 template <int NT, int KS>
-__global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(const float* __restrict__ X, const u32x4* __restrict__ table,
-                                                              int64_t N, int D, int K, int tiles, int slabs,
-                                                              const float* __restrict__ bias, const float* addend,
-                                                              int64_t ldc, float* out, int64_t ldo) {
+__global__ __launch_bounds__(kBlock, 4) void tall_gemm_kernel(const float* __restrict__ X, const u32x4* __restrict__ table,
+                                                              const int32_t* __restrict__ exps, int64_t N, int D, int K,
+                                                              int tiles, int slabs, const float* __restrict__ bias,
+                                                              const float* addend, int64_t ldc, float* out, int64_t ldo) {
   HIP_DYNAMIC_SHARED(u32x4, shared_frags)  // [KS][NT][3][64]
   // One launch covers `slabs` column slabs of NT tiles each.  Workgroups are handed to the 8 XCDs (each with its own
   // L2) round-robin by index, so the workgroups of one row block -- one per slab -- take indices 8 apart: they run on
@@ -413,7 +587,7 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
   constexpr int kUnits = KS * NT * 3 * kWave;  // 16-byte units per chunk
   constexpr int kPerThread = (kUnits + kBlock - 1) / kBlock;
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int half = lane >> 5, l32 = lane & 31;
   const int64_t row0 = (row_block * (kBlock / kWave) + wave) * kTile;
   const u32x4* frags = table + 1;
@@ -424,6 +598,10 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[nt][v] = 0.f;
+  float row_max = 0.f;
+  int32_t flags[NT];  // scalar loads, long done when they are wanted
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) flags[nt] = exps != nullptr ? exps[tiles * kTile + (tile0 + nt < tiles ? tile0 + nt : tiles - 1)] : 0;
 
   // This thread's share of a chunk's fragments.  A step past the row meets zeros of X and a tile past the last column
   // feeds accumulators that are never stored: any valid fragment will do for either.
@@ -431,12 +609,14 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
   auto fetch_frags = [&](int s0, u32x4 (&mine)[kPerThread]) {
 #pragma unroll
     for (int u = 0; u < kPerThread; ++u) {
-      int c = u * kBlock + static_cast<int>(threadIdx.x);  // unit of the chunk: [step][tile][piece][lane]
-      if (c >= kUnits) c = 0;                              // not parked
-      const int sb = c / (NT * 3 * kWave), tp = c / kWave % (NT * 3);
+      // units [step][tile][piece][lane] of the chunk, 64 of one fragment piece per wavefront: all but the lane is scalar
+      int piece = u * (kBlock / kWave) + wave;
+      if (piece >= KS * NT * 3) piece = 0;  // not parked
+      const int sb = piece / (NT * 3), tp = piece % (NT * 3);
       const int st = s0 + sb < total ? s0 + sb : s0;
       const int tile = tile0 + tp / 3 < tiles ? tile0 + tp / 3 : tiles - 1;
-      mine[u] = frags[static_cast<uint32_t>(st * step_units + (tile * 3 + tp % 3) * kWave + (c & (kWave - 1)))];
+      const u32x4* src = frags + (st * step_units + (tile * 3 + tp % 3) * kWave);
+      mine[u] = src[lane];
     }
   };
   auto fetch_rows = [&](int s0, float (&a)[KS][8]) {
@@ -456,6 +636,8 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int p = 0; p < 3; ++p) b[nt][p] = shared_frags[((sb * NT + nt) * 3 + p) * kWave + lane];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) row_max = magnitude_or(row_max, a[sb][i]);
       const Split8 pieces = split3x8(a[sb]);
       // the six products of step_product<3>, in its order for every tile, issued tile after tile: consecutive
       // matrix-core instructions write different accumulators and none waits for its predecessor
@@ -488,15 +670,21 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
     __syncthreads();
     multiply(a);
   }
+  row_max = magnitude_or(row_max, __shfl_xor(row_max, 32));
+  // tiles that the pieces do not carry, a bit each
+  uint32_t again = __ballot(row_needs_fp32(row_max)) != 0 ? (1u << NT) - 1u : 0u;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) again |= flags[nt] != 0 ? 1u << nt : 0u;
   // Accumulator register v is row 8 (v / 4) + 4 half + v % 4 of the wavefront's 32.
   float* first = out + (row0 + 4 * half) * ldo + tile0 * kTile + l32;
   // Rows all inside (all but the last wavefront of the matrix): the addresses advance by additions.  A bounds test
-  // and a 64-bit product per element were a third of the kernel's vector instructions (183 against 144 us).
+  // and a 64-bit product per element were a third of the kernel's vector instructions (a fifth of the time at 256 x 256).
   if (row0 + kTile <= N) {
     const float* add = addend == nullptr ? nullptr : addend + (row0 + 4 * half) * ldc + tile0 * kTile + l32;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int col = (tile0 + nt) * kTile + l32;
+      if ((again >> nt) & 1u) continue;
       if (col >= K) continue;
       const float b = bias != nullptr ? bias[col] : 0.f;
       float* dst = first + nt * kTile;
@@ -521,23 +709,26 @@ __global__ __launch_bounds__(kBlock, NT == 4 ? 4 : 1) void tall_gemm_kernel(cons
         }
       }
     }
-    return;
-  }
+  } else {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int col = (tile0 + nt) * kTile + l32;
-    const float b = (bias != nullptr && col < K) ? bias[col] : 0.f;
+    for (int nt = 0; nt < NT; ++nt) {
+      const int col = (tile0 + nt) * kTile + l32;
+      if ((again >> nt) & 1u) continue;
+      const float b = (bias != nullptr && col < K) ? bias[col] : 0.f;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t n = row0 + 8 * (v / 4) + 4 * half + (v % 4);
-      if (n < N && col < K) {
-        float val = acc[nt][v];
-        if (bias != nullptr) val = val + b;
-        if (addend != nullptr) val = val + addend[n * ldc + col];
-        __builtin_nontemporal_store(val, out + n * ldo + col);
+      for (int v = 0; v < 16; ++v) {
+        const int64_t n = row0 + 8 * (v / 4) + 4 * half + (v % 4);
+        if (n < N && col < K) {
+          float val = acc[nt][v];
+          if (bias != nullptr) val = val + b;
+          if (addend != nullptr) val = val + addend[n * ldc + col];
+          __builtin_nontemporal_store(val, out + n * ldo + col);
+        }
       }
     }
   }
+  if (__builtin_expect(again != 0, 0))
+    tall_gemm_fp32_tiles(xrow, frags, exps, N, D, K, tiles, tile0, again, row0, bias, addend, ldc, out, ldo);
 }
 
 // ---- backward ----------------------------------------------------------------
@@ -706,6 +897,34 @@ static bool rp_shape_ok(int64_t N, int64_t D, int64_t k) {
 static bool rp_mode_ok(int mode) { return mode == EXACT_RP_BF16_SPLIT || mode == EXACT_RP_BF16_SIGNS; }
 static int rp_pieces(int mode) { return mode == EXACT_RP_BF16_SIGNS ? 1 : 3; }
 
+static int tall_gemm_refused(int64_t N, int64_t D, int64_t K, const float* addend, int64_t ldc, int64_t ldo) {
+  if (N < 0 || D <= 0 || K <= 0 || D > 4096 || K > 4096 || D % 2 != 0) return EXACT_E_SHAPE;
+  if (ldo < K || (addend && ldc < K)) return EXACT_E_SHAPE;
+  return EXACT_OK;
+}
+
+static int tall_gemm_launch(const float* X, const u32x4* table, const int32_t* exps, int64_t N, int D, int K, const float* bias,
+                            const float* addend, int64_t ldc, float* out, int64_t ldo, hipStream_t s) {
+  const int tiles = (K + kTile - 1) / kTile;
+  // slabs of equal width, at most four tiles: every slab in one launch, less than one tile per slab for padding
+  const int slabs = (tiles + kGemmSlabTiles - 1) / kGemmSlabTiles;
+  const int64_t rows = static_cast<int64_t>(kBlock / kWave) * kTile;
+  const int64_t groups = ((N + rows - 1) / rows + kGemmXcds - 1) / kGemmXcds;  // groups of 8 row blocks
+  if (groups * kGemmXcds * slabs > 0x7FFFFFFF) return EXACT_E_SHAPE;
+  const dim3 grid(static_cast<unsigned>(groups * kGemmXcds * slabs)), block(kBlock);
+#define EXACT_GEMM_GO(NT, KS)                                                                                            \
+  hipLaunchKernelGGL((tall_gemm_kernel<NT, KS>), grid, block, sizeof(u32x4) * KS * NT * 3 * kWave, s, X, table, exps, N, \
+                     D, K, tiles, slabs, bias, addend, ldc, out, ldo)
+  switch ((tiles + slabs - 1) / slabs) {
+    case 1: EXACT_GEMM_GO(1, 4); break;
+    case 2: EXACT_GEMM_GO(2, 4); break;
+    case 3: EXACT_GEMM_GO(3, 2); break;
+    default: EXACT_GEMM_GO(4, 1); break;
+  }
+#undef EXACT_GEMM_GO
+  return launch_status();
+}
+
 }  // namespace exact
 
 using namespace exact;
@@ -824,42 +1043,41 @@ int exact_tall_gemm_prepare_bf16(const float* M, int64_t ld, int transposed, int
   if (ld < (transposed ? D : K)) return EXACT_E_SHAPE;
   if (!M || !table) return EXACT_E_NULL;
   if (!al16(table)) return EXACT_E_ALIGN;
-  const TableShape ts = table_shape(static_cast<int>(D), static_cast<int>(K), 3);
-  const int64_t frags = ts.fwd_units() / 3;
-  const dim3 grid(static_cast<unsigned>((frags + kBlock - 1) / kBlock)), block(kBlock);
-  hipLaunchKernelGGL(gemm_prepare_kernel, grid, block, 0, static_cast<hipStream_t>(stream), M, ld, transposed,
-                     static_cast<int>(D), static_cast<int>(K), static_cast<u32x4*>(table));
+  gemm_prepare(M, ld, transposed, static_cast<int>(D), static_cast<int>(K), static_cast<u32x4*>(table), nullptr,
+               static_cast<hipStream_t>(stream));
   return launch_status();
 }
 
 int exact_tall_gemm_bf16_f32(const float* X, const void* table, int64_t N, int64_t D, int64_t K, const float* bias,
                              const float* addend, int64_t ldc, float* out, int64_t ldo, void* stream) {
-  if (N < 0 || D <= 0 || K <= 0 || D > 4096 || K > 4096 || D % 2 != 0) return EXACT_E_SHAPE;
-  if (ldo < K || (addend && ldc < K)) return EXACT_E_SHAPE;
+  if (const int rc = tall_gemm_refused(N, D, K, addend, ldc, ldo)) return rc;
   if (N == 0) return EXACT_OK;
   if (!X || !table || !out) return EXACT_E_NULL;
   if (!al16(table) || !al8(X)) return EXACT_E_ALIGN;
+  return tall_gemm_launch(X, static_cast<const u32x4*>(table), nullptr, N, static_cast<int>(D), static_cast<int>(K), bias, addend, ldc,
+                          out, ldo, static_cast<hipStream_t>(stream));
+}
+
+int64_t exact_tall_product_work_nbytes(int64_t D, int64_t K) {
+  const int64_t table = exact_tall_gemm_table_nbytes(D, K);
+  return table == 0 ? 0 : table + (K + kTile - 1) / kTile * (kTile + 1) * static_cast<int64_t>(sizeof(int32_t));
+}
+
+int exact_tall_product_f32(const float* X, const float* M, int64_t ld, int transposed, int64_t N, int64_t D, int64_t K,
+                           const float* bias, const float* addend, int64_t ldc, float* out, int64_t ldo, void* work,
+                           void* stream) {
+  if (const int rc = tall_gemm_refused(N, D, K, addend, ldc, ldo)) return rc;
+  if (transposed != 0 && transposed != 1) return EXACT_E_ARG;
+  if (ld < (transposed ? D : K)) return EXACT_E_SHAPE;
+  if (N == 0) return EXACT_OK;
+  if (!X || !M || !work || !out) return EXACT_E_NULL;
+  if (!al16(work) || !al8(X)) return EXACT_E_ALIGN;
+  const int d = static_cast<int>(D), k = static_cast<int>(K);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const u32x4* t = static_cast<const u32x4*>(table);
-  const int d = static_cast<int>(D), kk = static_cast<int>(K);
-  const int tiles = (kk + kTile - 1) / kTile;
-  // slabs of equal width, at most four tiles: every slab in one launch, less than one tile per slab for padding
-  const int slabs = (tiles + kGemmSlabTiles - 1) / kGemmSlabTiles;
-  const int64_t rows = static_cast<int64_t>(kBlock / kWave) * kTile;
-  const int64_t groups = ((N + rows - 1) / rows + kGemmXcds - 1) / kGemmXcds;  // groups of 8 row blocks
-  if (groups * kGemmXcds * slabs > 0x7FFFFFFF) return EXACT_E_SHAPE;
-  const dim3 grid(static_cast<unsigned>(groups * kGemmXcds * slabs)), block(kBlock);
-#define EXACT_GEMM_GO(NT, KS)                                                                                          \
-  hipLaunchKernelGGL((tall_gemm_kernel<NT, KS>), grid, block, sizeof(u32x4) * KS * NT * 3 * kWave, s, X, t, N, d, kk, \
-                     tiles, slabs, bias, addend, ldc, out, ldo)
-  switch ((tiles + slabs - 1) / slabs) {
-    case 1: EXACT_GEMM_GO(1, 4); break;
-    case 2: EXACT_GEMM_GO(2, 4); break;
-    case 3: EXACT_GEMM_GO(3, 2); break;
-    default: EXACT_GEMM_GO(4, 1); break;
-  }
-#undef EXACT_GEMM_GO
-  return launch_status();
+  u32x4* table = static_cast<u32x4*>(work);
+  int32_t* exps = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(work) + exact_tall_gemm_table_nbytes(D, K));
+  gemm_prepare(M, ld, transposed, d, k, table, exps, s);
+  return tall_gemm_launch(X, table, exps, N, d, k, bias, addend, ldc, out, ldo, s);
 }
 
 }  // extern "C"

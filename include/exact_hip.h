@@ -407,15 +407,24 @@ int exact_rp_minmax_pack_bf16_f32(const float *X, const void *table, int mode, c
  * matrices and six bf16 matrix-core products stand for each fp32 product (the
  * neglected ones are below 2^-24 of it), accumulated in fp32.  No atomics: the
  * result is reproducible.
- * exact_tall_gemm_prepare_bf16 writes the operand fragments of M into `table`
- * (exact_tall_gemm_table_nbytes(D, K) bytes, 16-byte aligned, owned by the
- * caller, valid while M is unchanged); M has row stride `ld` elements and is
- * read as M[d * ld + c], or as M[c * ld + d] when `transposed` is 1 (a weight
- * [K, D] as F.linear holds it).
- * exact_tall_gemm_bf16_f32: X contiguous [N, D], D even, 8-byte aligned (16-byte
- * loads are used when D % 4 == 0 and X is 16-byte aligned, else 8-byte ones),
- * D and K at most 4096; `bias` and `addend` may be NULL; `addend` (row stride
- * ldc) may be `out` itself (row stride ldo >= K): out += X . M. */
+ * exact_tall_product_f32 is the whole product from M itself, every fp32 value
+ * taken: infinities and NaN come out as in fp32 arithmetic, columns of M and
+ * rows of X of any size keep their digits.  X contiguous [N, D], D even, 8-byte
+ * aligned, D and K at most 4096; M has row stride `ld` elements and is read as
+ * M[d * ld + c], or as M[c * ld + d] when `transposed` is 1 (a weight [K, D] as
+ * F.linear holds it); `bias` and `addend` may be NULL; `addend` (row stride ldc)
+ * may be `out` itself (row stride ldo >= K): out += X . M.  `work`:
+ * exact_tall_product_work_nbytes(D, K) bytes, 16-byte aligned, scratch of the
+ * call, which other work on the same stream may reuse.
+ * The two halves of it: exact_tall_gemm_prepare_bf16 writes the operand
+ * fragments of M into `table` (exact_tall_gemm_table_nbytes(D, K) bytes, 16-byte
+ * aligned, owned by the caller, valid while M is unchanged) and
+ * exact_tall_gemm_bf16_f32 multiplies by it.  This table has no room for a scale
+ * per column: entries of M below 1e-30 keep fewer than 24 bits. */
+int64_t exact_tall_product_work_nbytes(int64_t D, int64_t K);
+int exact_tall_product_f32(const float *X, const float *M, int64_t ld, int transposed, int64_t N,
+                           int64_t D, int64_t K, const float *bias, const float *addend, int64_t ldc,
+                           float *out, int64_t ldo, void *work, void *stream);
 int64_t exact_tall_gemm_table_nbytes(int64_t D, int64_t K);
 int exact_tall_gemm_prepare_bf16(const float *M, int64_t ld, int transposed, int64_t D, int64_t K,
                                  void *table, void *stream);

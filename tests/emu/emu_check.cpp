@@ -554,6 +554,33 @@ static void check_gemm(int64_t N, int64_t D, int64_t K, int64_t pad, std::mt1993
   const int64_t tbytes = exact_tall_gemm_table_nbytes(D, K);
   CHECK(tbytes > 0 && tbytes % 16 == 0, "gemm table size");
   Buf<uint32_t> table(tbytes / 4);
+  const int64_t wbytes = exact_tall_product_work_nbytes(D, K);
+  CHECK(wbytes > tbytes && wbytes % 4 == 0, "product work size");
+  Buf<uint32_t> work(wbytes / 4);
+  for (int transposed = 0; transposed < 2 && D % 2 == 0; ++transposed)
+    for (int odd = 0; odd < 2; ++odd) {  // odd: a row of X and a column of M that the fp32 instruction has to take
+      Buf<float> Xo(static_cast<size_t>(N * D)), Mo(static_cast<size_t>(transposed ? K * ldt : D * ld));
+      const float xs = odd ? 0x1p-120f : 1.f, ms = odd ? 0x1p-110f : 1.f;
+      for (int64_t i = 0; i < N * D; ++i) Xo[i] = X[i] * (i / D == N / 2 ? xs : 1.f);
+      for (int64_t i = 0; i < (transposed ? K * ldt : D * ld); ++i) {
+        const int64_t c = transposed ? i / ldt : i % ld;
+        Mo[i] = (transposed ? Mt[i] : M[i]) * (c == K / 2 ? ms : 1.f);
+      }
+      for (int64_t i = 0; i < N * ldo; ++i) out[i] = -777.f;
+      CHECK(exact_tall_product_f32(Xo.p, Mo.p, transposed ? ldt : ld, transposed, N, D, K, nullptr, nullptr, ldc, out.p, ldo, work.p, nullptr) == 0,
+            "product rc");
+      for (int64_t n = 0; n < N; ++n)
+        for (int64_t c = 0; c < ldo; ++c) {
+          double want = -777.;
+          if (c < K) {
+            want = 0;
+            for (int64_t d = 0; d < D; ++d) want += static_cast<double>(X[n * D + d]) * M[d * ld + c];
+            want *= (n == N / 2 ? xs : 1.f) * static_cast<double>(c == K / 2 ? ms : 1.f);
+          }
+          CHECK(out[n * ldo + c] == static_cast<float>(want), "product transposed=%d odd=%d N=%lld D=%lld K=%lld at (%lld, %lld)", transposed, odd,
+                (long long)N, (long long)D, (long long)K, (long long)n, (long long)c);
+        }
+    }
   // variant 4: the rows start 8 bytes into a 16-byte line (and still end where the allocation ends)
   Buf<float> X8(static_cast<size_t>(N * D + 2));
   for (int64_t i = 0; i < N * D; ++i) X8[i + 2] = X[i];

@@ -41,6 +41,7 @@
 #define __device__
 #define __host__
 #define __forceinline__ inline __attribute__((always_inline))
+#define __noinline__ __attribute__((noinline))
 #define __launch_bounds__(...)
 #define __shared__ static thread_local
 #define HIP_DYNAMIC_SHARED(type, var) type* var = reinterpret_cast<type*>(hipemu::dyn_shared());
@@ -536,6 +537,7 @@ static inline uint64_t __ballot(bool p) { return hipemu::ballot(p); }
 // lanes of a wavefront move in lockstep anyway; here the lanes are fibres and must really wait)
 #define __builtin_amdgcn_wave_barrier() ((void)hipemu::ballot(true))
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
+#define __builtin_amdgcn_sched_barrier(mask) ((void)0)
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) hipemu::mfma_f32_32x32x16_bf16((a), (b), (c), (x), (y), (z))
 
 static inline float __fmaf_rn(float a, float b, float c) { return std::fmaf(a, b, c); }
