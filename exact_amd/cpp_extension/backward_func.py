@@ -60,10 +60,11 @@ def batch_statistics(matrix):
 
 def weight_gradient(grad_output, input):  # noqa: A002
     """`grad_output.t().mm(input)` (backward_func.cc:88-89): [N, out]^T . [N, in].
-    Tall device operands, fp32 or fp16, take the library's matrix-core kernel for this
-    shape -- on the bf16 instruction with operands split in three, or on the
-    fp32 instruction (config.matrix_cores) -- whose slabs meet through atomics,
-    so deterministic mode and everything else keep the framework's GEMM."""
+    Tall device operands take the library's matrix-core kernel for this shape: fp32
+    ones on the bf16 instruction with operands split in three, or on the fp32
+    instruction (config.matrix_cores), whose slabs meet through atomics; fp16 ones on
+    the fp16 instruction, whose slabs are added in a fixed order.  Deterministic mode
+    and everything else keep the framework's GEMM."""
     half = grad_output.dtype == torch.float16 and input.dtype == torch.float16 and config.matrix_cores == "bf16"
     usable = (grad_output.dim() == 2 and input.dim() == 2 and (half or (grad_output.dtype == torch.float32
               and input.dtype == torch.float32)) and _checks.on_device(grad_output) and _checks.on_device(input)
@@ -76,14 +77,22 @@ def weight_gradient(grad_output, input):  # noqa: A002
         return grad_output.t().mm(input)
     N, K = grad_output.shape
     D = input.shape[1]
+    if half:
+        L = _lib.lib()
+        out = torch.empty((K, D), dtype=torch.float16, device=grad_output.device)
+        work = torch.empty(int(L.exact_linear_dw_f16_work_nbytes(N, K, D)), dtype=torch.uint8, device=grad_output.device)
+        rc = L.exact_linear_dw_ordered_f16(_checks.ptr(grad_output), grad_output.stride(0), _checks.ptr(input), input.stride(0),
+                                           N, K, D, _checks.ptr(out), _checks.ptr(work), _checks.stream_ptr(grad_output))
+        _lib.check(rc, "weight_gradient")
+        return out
     out = torch.empty((K, D), dtype=torch.float32, device=grad_output.device)
     if config.matrix_cores not in ("bf16", "fp32"):
         raise ValueError("config.matrix_cores must be 'bf16' or 'fp32'")
-    kernel = _lib.lib().exact_linear_dw_f16 if half else _lib.lib().exact_linear_dw_bf16_f32 if config.matrix_cores == "bf16" else _lib.lib().exact_linear_dw_f32
+    kernel = _lib.lib().exact_linear_dw_bf16_f32 if config.matrix_cores == "bf16" else _lib.lib().exact_linear_dw_f32
     rc = kernel(_checks.ptr(grad_output), grad_output.stride(0), _checks.ptr(input), input.stride(0),
                 N, K, D, _checks.ptr(out), _checks.stream_ptr(grad_output))
     _lib.check(rc, "weight_gradient")
-    return out.to(torch.float16) if half else out          # fp16 operands: one rounding of the fp32 sums
+    return out
 
 
 # ---- the dense products of a layer on the bf16 matrix cores ---------------------

@@ -259,12 +259,9 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_bf16_kernel(const float* 
 // 166 -> 134.  Where a workgroup's block is one tile or fewer wavefronts share a fragment the barrier costs more than
 // the split ([20000, 40]^T x [.., 128] 25 -> 33, [2449029, 47]^T x [.., 64] 306 -> 359, [2449029, 256]^T x [.., 25]
 // 560 -> 620): those keep the form above.
-//
-// fp16 operands (autocast) are widened as they are loaded: exact, and exact again as bf16 pieces ([40000, 256]^T x
-// [.., 256]: 59 us; the framework's fp16 product takes 123 and rounds its partial sums' result once, as the caller does).
-template <int MK, int MD, int WK, typename T>
-__global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __restrict__ dY, int64_t ldy,
-                                                                const T* __restrict__ X, int64_t ldx, int64_t N,
+template <int MK, int MD, int WK>
+__global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const float* __restrict__ dY, int64_t ldy,
+                                                                const float* __restrict__ X, int64_t ldx, int64_t N,
                                                                 int Kout, int D, int64_t rows_per_slab, int blocks_d, int blocks, int64_t slabs,
                                                                 float* __restrict__ out) {
   constexpr int WD = 4 / WK;
@@ -288,7 +285,7 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __
   const int64_t n_end = (n_begin + rows_per_slab < N) ? n_begin + rows_per_slab : N;
 
   // my fragments' columns; past the last column: clamped, they only feed accumulators that are never stored
-  const T* src[FPW];
+  const float* src[FPW];
   int64_t ld[FPW];
 #pragma unroll
   for (int j = 0; j < FPW; ++j) {
@@ -306,12 +303,12 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  T raw[FPW][8];
+  float raw[FPW][8];
   auto load_step = [&](int64_t n0) {
     if (n0 + kRows <= n_end) {  // the same in the whole workgroup: the step lies inside the slab, nothing to clamp
 #pragma unroll
       for (int j = 0; j < FPW; ++j) {
-        const T* p = src[j] + (n0 + 8 * half) * ld[j];
+        const float* p = src[j] + (n0 + 8 * half) * ld[j];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           raw[j][e] = *p;
@@ -324,8 +321,8 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int64_t row = n0 + 8 * half + e;
-          const T v = src[j][(row < N ? row : N - 1) * ld[j]];
-          raw[j][e] = row < n_end ? v : static_cast<T>(0.f);
+          const float v = src[j][(row < N ? row : N - 1) * ld[j]];
+          raw[j][e] = row < n_end ? v : 0.f;
         }
     }
   };
@@ -334,10 +331,7 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __
     for (int j = 0; j < FPW; ++j) {
       const int f = wave + 4 * j;
       if (f >= F) continue;  // wave-uniform
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(raw[j][e]);
-      const Split8 s = split3x8(v);
+      const Split8 s = split3x8(raw[j]);
       u32x4* dst = shared + (buffer * F + f) * 3 * kWave + lane;
       dst[0] = s.hi;
       dst[kWave] = s.mid;
@@ -390,8 +384,193 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const T* __
     }
 }
 
-template <int MK, int MD, int WK, bool BF16, typename T>
-static void launch_dw(const T* dY, int64_t ldy, const T* X, int64_t ldx, int64_t N, int Kout, int D, float* out,
+// fp16 operands (autocast): the same walk on v_mfma_f32_32x32x16_f16, which takes them as they are -- products of two
+// fp16 numbers are exact in fp32, infinities, NaN and subnormal numbers among them.  A fragment is one 16-byte unit per
+// lane, so a step is 32 rows.  A slab's block goes to `partial` [slab][Kout][D] and dw_finish_half_kernel adds the slabs
+// in their order: two equal calls give equal bits.
+template <int MK, int MD, int WK>
+__global__ __launch_bounds__(kBlock, 2) void linear_dw_half_kernel(const half_t* __restrict__ dY, int64_t ldy,
+                                                                   const half_t* __restrict__ X, int64_t ldx, int64_t N,
+                                                                   int Kout, int D, int64_t rows_per_slab, int blocks_d, int blocks, int64_t slabs,
+                                                                   float* __restrict__ partial) {
+  constexpr int WD = 4 / WK;
+  constexpr int KT = MK * WK, DT = MD * WD, F = KT + DT;  // fragments of 16 rows: KT of dY, then DT of X
+  constexpr int FPW = (F + 3) / 4;                        // of them, per wavefront: wave, wave + 4, ..
+  constexpr int SUB = 2, kRows = 16 * SUB;                // rows per step
+  HIP_DYNAMIC_SHARED(u32x4, shared)                       // [2][SUB][F][lane]
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int half = lane >> 5;
+  const int l32 = lane & 31;
+  int block;
+  int64_t slab;
+  if (!dw_block_and_slab(blocks, slabs, block, slab)) return;  // whole workgroup, before any barrier
+  const int bk = block / blocks_d, bd = block % blocks_d;
+  const int wk = wave / WD, wd = wave % WD;
+  const int k0 = (bk * WK + wk) * (32 * MK);
+  const int d0 = (bd * WD + wd) * (32 * MD);
+  const bool active = k0 < Kout && d0 < D;  // wave-uniform; an inactive wavefront still brings its fragments
+  const int64_t n_begin = slab * rows_per_slab;
+  const int64_t n_end = (n_begin + rows_per_slab < N) ? n_begin + rows_per_slab : N;
+
+  // my fragments' columns; past the last column: clamped, they only feed accumulators that are never stored
+  const half_t* src[FPW];
+  int64_t ld[FPW];
+#pragma unroll
+  for (int j = 0; j < FPW; ++j) {
+    const int f = wave + 4 * j < F ? wave + 4 * j : F - 1;
+    const bool is_y = f < KT;
+    const int c = is_y ? (bk * KT + f) * 32 + l32 : (bd * DT + f - KT) * 32 + l32;
+    src[j] = is_y ? dY + min(c, Kout - 1) : X + min(c, D - 1);
+    ld[j] = is_y ? ldy : ldx;
+  }
+  floatx16 acc[MK][MD];
+#pragma unroll
+  for (int i = 0; i < MK; ++i)
+#pragma unroll
+    for (int j = 0; j < MD; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  half8 raw[SUB][FPW];
+  auto load_step = [&](int64_t n0) {
+    if (n0 + kRows <= n_end) {  // the same in the whole workgroup: the step lies inside the slab, nothing to clamp
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int j = 0; j < FPW; ++j) {
+          const half_t* p = src[j] + (n0 + 16 * s + 8 * half) * ld[j];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            raw[s][j][e] = *p;
+            p += ld[j];
+          }
+        }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int j = 0; j < FPW; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int64_t row = n0 + 16 * s + 8 * half + e;
+            const half_t v = src[j][(row < N ? row : N - 1) * ld[j]];
+            raw[s][j][e] = row < n_end ? v : static_cast<half_t>(0.f);
+          }
+    }
+  };
+  auto park_step = [&](int buffer) {
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+#pragma unroll
+      for (int j = 0; j < FPW; ++j) {
+        const int f = wave + 4 * j;
+        if (f < F) shared[((buffer * SUB + s) * F + f) * kWave + lane] = __builtin_bit_cast(u32x4, raw[s][j]);  // wave-uniform
+      }
+  };
+  auto multiply = [&](int buffer) {
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) {
+      const u32x4* base = shared + (buffer * SUB + s) * F * kWave + lane;
+      half8 b[MD];
+#pragma unroll
+      for (int j = 0; j < MD; ++j) b[j] = __builtin_bit_cast(half8, base[(KT + wd * MD + j) * kWave]);
+#pragma unroll
+      for (int i = 0; i < MK; ++i) {
+        const half8 a = __builtin_bit_cast(half8, base[(wk * MK + i) * kWave]);
+#pragma unroll
+        for (int j = 0; j < MD; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+
+  if (n_begin < n_end) {  // the same in the whole workgroup; the last slabs of a short batch may be empty
+    load_step(n_begin);
+    park_step(0);
+    load_step(n_begin + kRows);  // past the slab: clamped addresses, zeroed values
+    __syncthreads();
+    int buffer = 0;
+    for (int64_t n0 = n_begin; n0 < n_end; n0 += kRows) {
+      if (active) multiply(buffer);
+      buffer ^= 1;
+      if (n0 + kRows < n_end) {  // the same in the whole workgroup
+        park_step(buffer);       // last read before the barrier that ended the previous step
+        load_step(n0 + 2 * kRows);
+        __syncthreads();
+      }
+    }
+  }
+  if (!active) return;
+  float* mine = partial + slab * Kout * D;
+#pragma unroll
+  for (int i = 0; i < MK; ++i)
+#pragma unroll
+    for (int j = 0; j < MD; ++j) {
+      const int cj = d0 + 32 * j + l32;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ri = k0 + 32 * i + 8 * (v / 4) + 4 * half + (v % 4);
+        if (ri < Kout && cj < D) mine[static_cast<int64_t>(ri) * D + cj] = acc[i][j][v];
+      }
+    }
+}
+
+// out[i] = fp16(sum over the slabs): eight groups of 32 lanes take every eighth slab, then meet in LDS in their order.
+__global__ __launch_bounds__(kBlock) void dw_finish_half_kernel(const float* __restrict__ partial, int64_t total, int64_t slabs,
+                                                                half_t* __restrict__ out) {
+  __shared__ float part[kBlock];
+  const int t = threadIdx.x, g = t >> 5;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 32 + (t & 31);
+  const float* p = partial + (i < total ? i : total - 1);
+  float s = 0.f;
+  for (int64_t k = g; k < slabs; k += 64) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[(k + 8 * u < slabs ? k + 8 * u : k) * total];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += k + 8 * u < slabs ? v[u] : 0.f;
+  }
+  part[t] = s;
+  __syncthreads();
+  if (g == 0 && i < total) {
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s += part[32 * k + t];
+    out[i] = static_cast<half_t>(s);
+  }
+}
+
+// How the fp16 form cuts its work: about 512 workgroups (two per compute unit), at least 512 rows a slab, whole steps.
+struct DwHalfPlan {
+  int mk, md, wk, blocks_d, blocks;
+  int64_t rows, slabs;
+};
+static DwHalfPlan plan_dw_half(int64_t N, int K, int D) {
+  DwHalfPlan p{};
+  p.mk = K <= 32 ? 1 : 2;
+  p.md = (K <= 64 ? D <= 128 : D <= 32) ? 1 : 2;
+  p.wk = K <= 64 ? 1 : D <= 64 ? 4 : 2;
+  const int kb = 32 * p.mk * p.wk, db = 32 * p.md * (4 / p.wk);
+  p.blocks_d = (D + db - 1) / db;
+  p.blocks = (K + kb - 1) / kb * p.blocks_d;
+  const int64_t wanted = (512 + p.blocks - 1) / p.blocks;
+  p.rows = (N + wanted - 1) / wanted;
+  if (p.rows < 512) p.rows = 512;
+  p.rows = (p.rows + 31) / 32 * 32;
+  p.slabs = (N + p.rows - 1) / p.rows;
+  return p;
+}
+
+template <int MK, int MD, int WK>
+static void launch_dw_half(const DwHalfPlan& p, const half_t* dY, int64_t ldy, const half_t* X, int64_t ldx, int64_t N, int Kout, int D,
+                           float* partial, hipStream_t s) {
+  constexpr size_t lds = sizeof(u32x4) * 2 * 2 * (MK * WK + MD * (4 / WK)) * kWave;
+  const dim3 grid(static_cast<unsigned>((p.slabs + kDwXcds - 1) / kDwXcds * kDwXcds * p.blocks));
+  hipLaunchKernelGGL((linear_dw_half_kernel<MK, MD, WK>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, p.rows, p.blocks_d,
+                     p.blocks, p.slabs, partial);
+}
+
+template <int MK, int MD, int WK, bool BF16>
+static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int Kout, int D, float* out,
                       hipStream_t s) {
   constexpr int WD = 4 / WK;
   const int blocks_k = (Kout + 32 * MK * WK - 1) / (32 * MK * WK);
@@ -405,14 +584,14 @@ static void launch_dw(const T* dY, int64_t ldy, const T* X, int64_t ldx, int64_t
   slabs = (N + rows - 1) / rows;
   const dim3 grid(static_cast<unsigned>((slabs + kDwXcds - 1) / kDwXcds * kDwXcds * blocks));
   constexpr size_t lds = sizeof(u32x4) * 2 * (MK * WK + MD * WD) * 3 * kWave;
-  constexpr bool shared = sizeof(T) == 2 || (MK == 2 && MD == 2 && WK < 4) || MK == 1;  // measured, see the kernel
-  if constexpr (BF16 && shared) hipLaunchKernelGGL((linear_dw_shared_kernel<MK, MD, WK, T>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  constexpr bool shared = (MK == 2 && MD == 2 && WK < 4) || MK == 1;  // measured, see the kernel
+  if constexpr (BF16 && shared) hipLaunchKernelGGL((linear_dw_shared_kernel<MK, MD, WK>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
   else if constexpr (BF16) hipLaunchKernelGGL((linear_dw_bf16_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
   else hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
 }
 
-template <bool BF16, typename T>
-static int linear_dw_any(const T* dY, int64_t ldy, const T* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
+template <bool BF16>
+static int linear_dw_any(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                          float* out, hipStream_t s) {
   if (N < 0 || Kout < 0 || D < 0 || Kout > 65536 || D > 65536 || N > (int64_t{1} << 40)) return EXACT_E_SHAPE;
   if (ldy < Kout || ldx < D) return EXACT_E_SHAPE;
@@ -425,15 +604,15 @@ static int linear_dw_any(const T* dY, int64_t ldy, const T* X, int64_t ldx, int6
     // wavefront block: up to 64 x 64 of dW (wider blocks need more accumulator registers than two wavefronts
     // per SIMD leave); the four wavefronts side by side along the longer extent when the other fits one wavefront
     if (K <= 32) {
-      if (Dd <= 128) launch_dw<1, 1, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<1, 2, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 128) launch_dw<1, 1, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<1, 2, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
     } else if (K <= 64) {
-      if (Dd <= 128) launch_dw<2, 1, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<2, 2, 1, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 128) launch_dw<2, 1, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<2, 2, 1, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
     } else {
-      if (Dd <= 32) launch_dw<2, 1, 4, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else if (Dd <= 64) launch_dw<2, 2, 4, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
-      else launch_dw<2, 2, 2, BF16, T>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      if (Dd <= 32) launch_dw<2, 1, 4, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else if (Dd <= 64) launch_dw<2, 2, 4, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
+      else launch_dw<2, 2, 2, BF16>(dY, ldy, X, ldx, N, K, Dd, out, s);
     }
   }
   return launch_status();
@@ -447,18 +626,51 @@ extern "C" {
 
 int exact_linear_dw_f32(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                         float* out, void* stream) {
-  return linear_dw_any<false, float>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
+  return linear_dw_any<false>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
 }
 
 int exact_linear_dw_bf16_f32(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
                              float* out, void* stream) {
-  return linear_dw_any<true, float>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
+  return linear_dw_any<true>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
 }
 
-int exact_linear_dw_f16(const uint16_t* dY, int64_t ldy, const uint16_t* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
-                        float* out, void* stream) {
-  return linear_dw_any<true, half_t>(reinterpret_cast<const half_t*>(dY), ldy, reinterpret_cast<const half_t*>(X), ldx, N, Kout, D,
-                                     out, static_cast<hipStream_t>(stream));
+int64_t exact_linear_dw_f16_work_nbytes(int64_t N, int64_t Kout, int64_t D) {
+  if (N < 0 || Kout < 0 || D < 0 || Kout > 65536 || D > 65536 || N > (int64_t{1} << 40)) return 0;
+  if (N == 0 || Kout == 0 || D == 0) return 0;
+  return plan_dw_half(N, static_cast<int>(Kout), static_cast<int>(D)).slabs * Kout * D * static_cast<int64_t>(sizeof(float));
+}
+
+int exact_linear_dw_ordered_f16(const uint16_t* dY, int64_t ldy, const uint16_t* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D,
+                                uint16_t* out, void* work, void* stream) {
+  if (N < 0 || Kout < 0 || D < 0 || Kout > 65536 || D > 65536 || N > (int64_t{1} << 40)) return EXACT_E_SHAPE;
+  if (ldy < Kout || ldx < D) return EXACT_E_SHAPE;
+  if (Kout == 0 || D == 0) return EXACT_OK;
+  if (!out || (N > 0 && (!dY || !X || !work))) return EXACT_E_NULL;
+  const int K = static_cast<int>(Kout), Dd = static_cast<int>(D);
+  const int64_t total = Kout * D;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* partial = static_cast<float*>(work);
+  const half_t* y = reinterpret_cast<const half_t*>(dY);
+  const half_t* x = reinterpret_cast<const half_t*>(X);
+  int64_t slabs = 0;  // an empty batch: zeros
+  if (N > 0) {
+    const DwHalfPlan p = plan_dw_half(N, K, Dd);
+    slabs = p.slabs;
+    if (p.wk == 1) {
+      if (p.mk == 1 && p.md == 1) launch_dw_half<1, 1, 1>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+      else if (p.mk == 1) launch_dw_half<1, 2, 1>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+      else if (p.md == 1) launch_dw_half<2, 1, 1>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+      else launch_dw_half<2, 2, 1>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+    } else if (p.wk == 4) {
+      if (p.md == 1) launch_dw_half<2, 1, 4>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+      else launch_dw_half<2, 2, 4>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+    } else {
+      launch_dw_half<2, 2, 2>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
+    }
+  }
+  hipLaunchKernelGGL(dw_finish_half_kernel, dim3(static_cast<unsigned>((total + 31) / 32)), dim3(kBlock), 0, s, partial, total, slabs,
+                     reinterpret_cast<half_t*>(out));
+  return launch_status();
 }
 
 }  // extern "C"

@@ -263,9 +263,13 @@ int exact_linear_dw_f32(const float *dY, int64_t ldy, const float *X, int64_t ld
 int exact_linear_dw_bf16_f32(const float *dY, int64_t ldy, const float *X, int64_t ldx, int64_t N,
                              int64_t Kout, int64_t D, float *out, void *stream);
 
-/* The same for fp16 operands, exact products summed and returned in fp32. */
-int exact_linear_dw_f16(const uint16_t *dY, int64_t ldy, const uint16_t *X, int64_t ldx, int64_t N,
-                        int64_t Kout, int64_t D, float *out, void *stream);
+/* The same for fp16 operands and an fp16 result: exact products summed in fp32 in
+ * a fixed order (two equal calls give equal bits), rounded once; infinities and
+ * NaN as in fp32 arithmetic.  `work`: exact_linear_dw_f16_work_nbytes(N, Kout, D)
+ * bytes of scratch, 16-byte aligned. */
+int64_t exact_linear_dw_f16_work_nbytes(int64_t N, int64_t Kout, int64_t D);
+int exact_linear_dw_ordered_f16(const uint16_t *dY, int64_t ldy, const uint16_t *X, int64_t ldx, int64_t N,
+                                int64_t Kout, int64_t D, uint16_t *out, void *work, void *stream);
 
 /* Fused epilogues (no single counterpart in the reference: each replaces a
  * chain of its calls with one pass over the data, bit-identical to the chain).

@@ -538,6 +538,28 @@ static void check_dw(int64_t N, int64_t K, int64_t D, int64_t pad, std::mt19937&
   }
 }
 
+// The fp16 form: small integers, so the fp32 sums are exact; one rounding to fp16.
+static void check_dw_half(int64_t N, int64_t K, int64_t D, int64_t pad, std::mt19937& rng) {
+  std::uniform_int_distribution<int> id(-3, 3);
+  const int64_t ldy = K + pad, ldx = D + 2 * pad;
+  Buf<_Float16> dy(static_cast<size_t>(N * ldy)), x(static_cast<size_t>(N * ldx)), out(static_cast<size_t>(K * D));
+  for (int64_t i = 0; i < N * ldy; ++i) dy[i] = static_cast<_Float16>(id(rng));
+  for (int64_t i = 0; i < N * ldx; ++i) x[i] = static_cast<_Float16>(id(rng));
+  const int64_t bytes = exact_linear_dw_f16_work_nbytes(N, K, D);
+  CHECK(N == 0 ? bytes == 0 : bytes > 0 && bytes % 4 == 0, "dw half work size");
+  Buf<float> work(static_cast<size_t>(bytes / 4));
+  const int rc = exact_linear_dw_ordered_f16(reinterpret_cast<const uint16_t*>(dy.p), ldy, reinterpret_cast<const uint16_t*>(x.p), ldx, N,
+                                             K, D, reinterpret_cast<uint16_t*>(out.p), work.p, nullptr);
+  CHECK(rc == 0, "dw half rc %d", rc);
+  for (int64_t k = 0; k < K; ++k)
+    for (int64_t d = 0; d < D; ++d) {
+      double want = 0;
+      for (int64_t n = 0; n < N; ++n) want += static_cast<double>(dy[n * ldy + k]) * static_cast<double>(x[n * ldx + d]);
+      CHECK(out[k * D + d] == static_cast<_Float16>(static_cast<float>(want)), "dw half N=%lld K=%lld D=%lld at (%lld, %lld)", (long long)N,
+            (long long)K, (long long)D, (long long)k, (long long)d);
+    }
+}
+
 // exact_tall_gemm_bf16_f32 on exactly sized buffers: small integers, so the result is the integer product
 // bit for bit; the matrix direct with a row stride and transposed; bias, addend and in-place accumulation.
 static void check_gemm(int64_t N, int64_t D, int64_t K, int64_t pad, std::mt19937& rng) {
@@ -664,6 +686,8 @@ int main(int argc, char** argv) {
     check_dw(600, 130, 70, 0, rng);
     check_dw(513, 32, 200, 5, rng);
     check_dw(1100, 256, 256, 0, rng);
+    check_dw_half(1100, 256, 256, 0, rng);
+    check_dw_half(40, 1000, 300, 0, rng);
     std::printf("dw shapes ok (failures so far %d)\n", g_fail);
     return g_fail != 0;
   }
@@ -712,6 +736,10 @@ int main(int argc, char** argv) {
   const int64_t ds[][4] = {{1, 1, 1, 0}, {7, 3, 5, 1}, {100, 40, 256, 0}, {515, 256, 128, 3}, {333, 47, 25, 0}, {1201, 256, 76, 2},
                            {600, 130, 70, 0}, {513, 32, 200, 5}};
   for (auto& d : ds) check_dw(d[0], d[1], d[2], d[3], rng);
+  for (auto& d : ds) check_dw_half(d[0], d[1], d[2], d[3], rng);
+  check_dw_half(0, 5, 4, 0, rng);
+  check_dw_half(700, 33, 60, 1, rng);
+  check_dw_half(600, 64, 129, 0, rng);
   std::printf("weight gradient ok (failures so far %d)\n", g_fail);
   check_gemm_shapes(rng);
   std::printf("tall gemm ok (failures so far %d)\n", g_fail);

@@ -432,14 +432,26 @@ inline floatx16_t mfma_f32_32x32x2f32(float a, float b, floatx16_t c, int, int, 
   return c;
 }
 
-// v_mfma_f32_32x32x16_bf16: lane l holds row (A) / column (B) l % 32 and the eight
-// k-slots 8 * (l / 32) .. + 7 as bf16; accumulator layout as for 32x32x2.  The
-// products of two bf16 numbers are exact in fp32; they are added one after the
+// v_mfma_f32_32x32x16_bf16 and _f16: lane l holds row (A) / column (B) l % 32 and the eight
+// k-slots 8 * (l / 32) .. + 7 as bf16 / fp16; accumulator layout as for 32x32x2.  The
+// products of two such numbers are exact in fp32; they are added one after the
 // other in fp32 (the hardware's own order is not specified, so tests compare
 // against float64 with a tolerance, and launches that must agree bit for bit
 // with each other go through this same routine).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-inline floatx16_t mfma_f32_32x32x16_bf16(bf16x8_t a, bf16x8_t b, floatx16_t c, int, int, int) {
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+inline float widen16(uint16_t bits, __bf16) {
+  const uint32_t u = static_cast<uint32_t>(bits) << 16;
+  float f;
+  std::memcpy(&f, &u, 4);
+  return f;
+}
+inline float widen16(uint16_t bits, _Float16 h) {
+  std::memcpy(&h, &bits, 2);
+  return static_cast<float>(h);
+}
+template <typename E, typename V>
+inline floatx16_t mfma_f32_32x32x16_any(V a, V b, floatx16_t c) {
   uint64_t words[4];
   std::memcpy(&words[0], &a, 16);
   std::memcpy(&words[2], &b, 16);
@@ -454,12 +466,9 @@ inline floatx16_t mfma_f32_32x32x16_bf16(bf16x8_t a, bf16x8_t b, floatx16_t c, i
     }
     for (int l = 0; l < 64; ++l) all[q][l] = w->slot[buf][l];
   }
-  auto element = [&](int base, int l, int e) {      // bf16 element e (0..7) of lane l's operand -> float
+  auto element = [&](int base, int l, int e) {      // element e (0..7) of lane l's operand
     const uint64_t word = all[base + e / 4][l];
-    const uint32_t bits = static_cast<uint32_t>((word >> (16 * (e % 4))) & 0xFFFFu) << 16;
-    float f;
-    std::memcpy(&f, &bits, 4);
-    return f;
+    return widen16(static_cast<uint16_t>(word >> (16 * (e % 4))), E{});
   };
   const int j = lane % 32;
   for (int v = 0; v < 16; ++v) {
@@ -470,6 +479,8 @@ inline floatx16_t mfma_f32_32x32x16_bf16(bf16x8_t a, bf16x8_t b, floatx16_t c, i
   }
   return c;
 }
+inline floatx16_t mfma_f32_32x32x16_bf16(bf16x8_t a, bf16x8_t b, floatx16_t c, int, int, int) { return mfma_f32_32x32x16_any<__bf16>(a, b, c); }
+inline floatx16_t mfma_f32_32x32x16_f16(half8_t a, half8_t b, floatx16_t c, int, int, int) { return mfma_f32_32x32x16_any<_Float16>(a, b, c); }
 
 inline void syncthreads() {
   BlockState* b = g_block;
@@ -538,6 +549,7 @@ static inline uint64_t __ballot(bool p) { return hipemu::ballot(p); }
 #define __builtin_amdgcn_wave_barrier() ((void)hipemu::ballot(true))
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 #define __builtin_amdgcn_sched_barrier(mask) ((void)0)
+#define __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, x, y, z) hipemu::mfma_f32_32x32x16_f16((a), (b), (c), (x), (y), (z))
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) hipemu::mfma_f32_32x32x16_bf16((a), (b), (c), (x), (y), (z))
 
 static inline float __fmaf_rn(float a, float b, float c) { return std::fmaf(a, b, c); }

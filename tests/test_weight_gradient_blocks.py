@@ -1,22 +1,94 @@
-"""Weight gradients at every block shape of the kernel (columns below, at and past
+"""Weight gradients at every block shape of the kernels (columns below, at and past
 a tile; row counts that end inside a step and leave slabs empty) for fp32 and fp16
-operands, against float64: at most N additions of products exact to 2^-23."""
+operands.  Sparse integers, whose sums are exact whatever the order, have to give
+the float64 product bit for bit: a row lost or counted twice shows, and so does a
+piece of an operand, as the integers use every bit of it.  Dense random operands
+have to stay within what the rounding of fp32 sums can do."""
 import pytest
 import torch
 
 from exact_amd.cpp_extension import backward_func as bf
 
+SHAPES = [(1, 5), (20, 100), (32, 129), (33, 128), (47, 300), (64, 130), (65, 30), (100, 64), (129, 65), (256, 200)]
+DTYPES = [torch.float32, torch.float16]
+
+
+def _sparse_integers(N, K, D, dtype, device):
+    """dy holds 1, -1 or 2 in about eight rows a column, the last row among them, x integers of 20 (fp32) or 11 bits:
+    sums below 2^24 in fp32, below 2^16 in fp16."""
+    g = torch.Generator().manual_seed(N + K + D)
+    dy = torch.zeros(N, K)
+    rows = torch.cat([torch.randint(0, N, (6, K), generator=g), torch.full((1, K), N - 1), torch.zeros(1, K, dtype=torch.long)])
+    dy.scatter_(0, rows, torch.tensor([1.0, -1.0, 2.0])[torch.randint(0, 3, (8, K), generator=g)])
+    top = 2 ** 20 if dtype == torch.float32 else 2 ** 11
+    x = torch.randint(-top + 1, top, (N, D), generator=g).float()
+    return dy.to(device, dtype), x.to(device, dtype)
+
+
+def _check_integers(device, N, K, D, dtype):
+    dy, x = _sparse_integers(N, K, D, dtype, device)
+    want = (dy.double().t() @ x.double()).to(dtype)                      # one rounding to fp16
+    got = bf.weight_gradient(dy, x)
+    assert got.dtype == dtype and torch.equal(got, want)
+    wide_dy = torch.full((N, K + 3), float("nan"), dtype=dtype, device=device)   # row strides of their own, NaN between
+    wide_x = torch.full((N, D + 5), float("nan"), dtype=dtype, device=device)
+    wide_dy[:, 1:1 + K], wide_x[:, 3:3 + D] = dy, x
+    assert torch.equal(bf.weight_gradient(wide_dy[:, 1:1 + K], wide_x[:, 3:3 + D]), want)
+
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("K,D", [(1, 5), (20, 100), (32, 129), (33, 128), (47, 300), (64, 130), (65, 30), (100, 64), (129, 65), (256, 200)])
+@pytest.mark.parametrize("K,D", SHAPES)
 @pytest.mark.parametrize("N", [16384, 17003, 70001])
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_integers_are_exact(cuda, K, D, N, dtype):
+    _check_integers(cuda, N, K, D, dtype)
+
+
+@pytest.mark.parametrize("K,D", [(20, 40), (33, 33)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_integers_are_exact_on_the_emulated_kernels(backend, K, D, dtype):
+    _check_integers(backend, 16397, K, D, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,D", SHAPES)
+@pytest.mark.parametrize("N", [16384, 17003, 70001])
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_against_float64(cuda, K, D, N, dtype):
     g = torch.Generator(device=cuda).manual_seed(N + K + D)
     dy = torch.randn(N, K + 3, generator=g, device=cuda).to(dtype)[:, :K]      # a row stride of its own
     x = torch.randn(N, D, generator=g, device=cuda).to(dtype)
     got = bf.weight_gradient(dy, x)
-    want, total = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
-    # sums of at most 512 + 137 rows per slab in fp32, slabs met one by one; one rounding to fp16 at the end
-    bound = (6 * 649 + 137) * 2.0 ** -24 * total + (2.0 ** -11 * want.abs() + 2.0 ** -24 if dtype == torch.float16 else 0)
+    want = dy.double().t() @ x.double()
+    # A slab sums up to 700 products one after the other; with terms of random sign its rounding errors, 0.3 x 2^-24 of
+    # a running sum that grows as the square root, come to 0.3 x sqrt(700 / 2) x 2^-24 of the slab's rms, and slabs add
+    # in squares: a standard deviation of 6 x 2^-24 of the rms of the whole.  Ten of them; an operand that lost all but
+    # one bf16 piece is off by 2^-10 of the rms, two hundred times this.
+    rms = ((dy.double() ** 2).t() @ (x.double() ** 2)).sqrt()
+    bound = 60 * 2.0 ** -24 * rms + (2.0 ** -11 * want.abs() + 2.0 ** -25 if dtype == torch.float16 else 0)
     assert got.dtype == dtype and got.shape == (K, D) and ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("K,D", [(20, 40), (70, 35)])
+def test_half_operands_at_the_ends_of_their_range(backend, K, D):
+    """Infinities and NaN where fp32 sums put them, subnormal fp16 numbers kept, sums past 65504 infinite."""
+    N, inf = 16397, float("inf")
+    dy, x = _sparse_integers(N, K, D, torch.float16, backend)
+    dy[:, 3] *= 2.0 ** -24                                               # subnormal: 1, 2 units of the last place
+    dy[100, 4], dy[N - 1, 5] = 1000.0, float("nan")
+    dy[200, 6], dy[201, 6] = inf, -inf
+    x[100, 0], x[200, 1], x[201, 1] = 600.0, 2.0, 2.0
+    x[N - 1, 7] = inf                                                    # times dy[N - 1] != 0
+    want = (dy.double().t() @ x.double()).half()
+    got = bf.weight_gradient(dy, x)
+    assert torch.isinf(want).any() and torch.isnan(want).any() and (want[3].double() != 0).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(7.0, 8e4, -8e4), want.nan_to_num(7.0, 8e4, -8e4))
+
+
+@pytest.mark.parametrize("K,D", [(20, 40), (70, 35)])
+def test_half_operands_give_equal_bits_twice(backend, K, D):
+    g = torch.Generator().manual_seed(5)
+    dy, x = torch.randn(16500, K, generator=g).half().to(backend), torch.randn(16500, D, generator=g).half().to(backend)
+    first = bf.weight_gradient(dy, x)
+    for _ in range(3):
+        assert torch.equal(bf.weight_gradient(dy, x), first)
