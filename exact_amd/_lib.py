@@ -67,9 +67,10 @@ SIGNATURES = {
     "exact_stream_probe_f32": (_c_int, [_c_ptr, _c_i64, _c_int, _c_ptr, _c_ptr]),
     "exact_col_moments_f32": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
     "exact_bn_backward_reduce_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
-    "exact_bn_stats_f32": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_f32, _c_f32] + [_c_ptr] * 8),
+    "exact_bn_work_floats": (_c_i64, [_c_i64, _c_i64]),
+    "exact_bn_statistics_f32": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_f32, _c_f32] + [_c_ptr] * 8),
     "exact_bn_apply_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr]),
-    "exact_bn_backward_packed_f32": (_c_int, [_c_ptr, _c_ptr, _c_f32, _c_ptr, _c_int] + [_c_ptr] * 5 + [_c_i64, _c_i64] + [_c_ptr] * 4),
+    "exact_bn_backward_ordered_f32": (_c_int, [_c_ptr, _c_ptr, _c_f32, _c_ptr, _c_int] + [_c_ptr] * 5 + [_c_i64, _c_i64] + [_c_ptr] * 5),
     "exact_elu_bwd_f16": (_c_int, [_c_ptr, _c_ptr, _c_f32, _c_i64, _c_ptr, _c_ptr]),
     "exact_rp_fwd_f32": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr]),
     "exact_rp_bwd_f32": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr]),

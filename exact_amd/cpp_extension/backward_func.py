@@ -224,15 +224,16 @@ def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, e
     if not usable:
         return None
     N, K = matrix.shape
-    buffer = torch.empty((6, K), dtype=torch.float32, device=matrix.device)      # sums [2, K], centre, mean, invstd, mult
-    rc = _lib.lib().exact_bn_stats_f32(_checks.ptr(matrix), N, K, float(eps), float(momentum), _checks.ptr(weight),
-                                       _checks.ptr(running_mean), _checks.ptr(running_var), _checks.ptr(buffer),
-                                       _checks.ptr(buffer[3]), _checks.ptr(buffer[4]), _checks.ptr(buffer[5]),
-                                       _checks.stream_ptr(matrix))
+    L = _lib.lib()
+    mean, invstd, mult = torch.empty((3, K), dtype=torch.float32, device=matrix.device)
+    work = torch.empty(int(L.exact_bn_work_floats(N, K)), dtype=torch.float32, device=matrix.device)
+    rc = L.exact_bn_statistics_f32(_checks.ptr(matrix), N, K, float(eps), float(momentum), _checks.ptr(weight),
+                                   _checks.ptr(running_mean), _checks.ptr(running_var), _checks.ptr(work),
+                                   _checks.ptr(mean), _checks.ptr(invstd), _checks.ptr(mult), _checks.stream_ptr(matrix))
     _lib.check(rc, "batch_norm_statistics")
     if running_mean is not None:
         torch.autograd.graph.increment_version((running_mean, running_var))
-    return buffer[3], buffer[4], buffer[5]
+    return mean, invstd, mult
 
 
 def batch_norm_apply(matrix, mean, mult, bias):
@@ -266,13 +267,15 @@ def batch_norm_backward_packed(grad_out, mask, p, quantized, weight, mean, invst
     if not usable:
         return None
     N, K = grad_out.shape
+    L = _lib.lib()
     sums = torch.empty((2, K), dtype=torch.float32, device=grad_out.device)
+    work = torch.empty(int(L.exact_bn_work_floats(N, K)), dtype=torch.float32, device=grad_out.device)
     grad_input = torch.empty_like(grad_out) if output_mask[0] else None
     grad_weight = torch.empty(K, dtype=torch.float32, device=grad_out.device) if output_mask[1] else None
-    rc = _lib.lib().exact_bn_backward_packed_f32(_checks.ptr(grad_out), _checks.ptr(mask), float(p), _checks.ptr(packed), bits,
-                                                 _checks.ptr(scale), _checks.ptr(mn), _checks.ptr(mean), _checks.ptr(invstd),
-                                                 _checks.ptr(weight), N, K, _checks.ptr(sums), _checks.ptr(grad_input),
-                                                 _checks.ptr(grad_weight), _checks.stream_ptr(grad_out))
+    rc = L.exact_bn_backward_ordered_f32(_checks.ptr(grad_out), _checks.ptr(mask), float(p), _checks.ptr(packed), bits,
+                                         _checks.ptr(scale), _checks.ptr(mn), _checks.ptr(mean), _checks.ptr(invstd),
+                                         _checks.ptr(weight), N, K, _checks.ptr(work), _checks.ptr(sums), _checks.ptr(grad_input),
+                                         _checks.ptr(grad_weight), _checks.stream_ptr(grad_out))
     _lib.check(rc, "batch_norm_backward_packed")
     return grad_input, grad_weight, sums[0] if output_mask[2] else None
 

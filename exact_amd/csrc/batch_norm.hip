@@ -13,7 +13,6 @@
 namespace exact {
 
 constexpr int kBnMaxK = 8192;
-constexpr int kBnSample = 256;  // rows whose mean is the centre of the moments
 
 // One column block's geometry, the same in every kernel below.
 struct BnBlock {
@@ -29,38 +28,6 @@ __device__ __forceinline__ BnBlock bn_block(int K) {
   return b;
 }
 
-// The centre of the moments: the mean of up to 256 rows spread evenly over the matrix (also for sorted or clustered
-// rows within a fraction of a standard deviation of the column mean, so that the difference of the moments loses no
-// digits).  16 columns x 16 row groups per workgroup, 16 loads in flight per thread: the kernel is a few load
-// latencies long whatever N is.  It also clears the two sums, which the next kernel meets with atomics.
-__global__ __launch_bounds__(kBlock) void bn_center_kernel(const float* __restrict__ x, int64_t N, int K,
-                                                           float* __restrict__ center, float* __restrict__ sums) {
-  __shared__ float part[kBlock];
-  const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
-  const int k = static_cast<int>(blockIdx.x) * 16 + c;
-  const int64_t step = N / kBnSample > 0 ? N / kBnSample : 1;
-  const int count = static_cast<int>(N < kBnSample ? N : kBnSample);
-  float s = 0.f;
-  if (k < K) {
-    float v[kBnSample / 16];
-#pragma unroll
-    for (int i = 0; i < kBnSample / 16; ++i) {
-      const int row = g + 16 * i;
-      v[i] = x[(row < count ? row : 0) * step * K + k];
-    }
-#pragma unroll
-    for (int i = 0; i < kBnSample / 16; ++i) s += g + 16 * i < count ? v[i] : 0.f;
-  }
-  part[threadIdx.x] = s;
-  __syncthreads();
-  if (g == 0 && k < K) {
-    for (int i = 1; i < 16; ++i) s += part[16 * i + c];
-    center[k] = s / static_cast<float>(count);
-    sums[k] = 0.f;
-    sums[K + k] = 0.f;
-  }
-}
-
 template <int VEC>
 __device__ __forceinline__ void bn_load(const float* p, float (&v)[VEC]) {
   if constexpr (VEC == 4) {
@@ -71,91 +38,205 @@ __device__ __forceinline__ void bn_load(const float* p, float (&v)[VEC]) {
   }
 }
 
-// The partial sums of the threads that share a column meet in LDS, then one atomic add per column and sum.
-template <int VEC>
-__device__ __forceinline__ void bn_meet(const BnBlock& b, int K, const float (&s0)[VEC], const float (&s1)[VEC], float* sums) {
-  __shared__ float part[2][kBlock * VEC];
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int c = 0; c < VEC; ++c) {
-    part[0][t * VEC + c] = s0[c];
-    part[1][t * VEC + c] = s1[c];
+// Reductions over rows end in a fixed order whatever the launch does: the threads of a workgroup that share a column
+// meet in LDS, the workgroup stores two or three numbers per column, partial[workgroup][2 or 3][K], and one small kernel
+// takes the workgroups of a column in their order.  (Atomic adds into the result, half a million of them at
+// [169343, 256], cost as much and gave other last bits on every run.)
+
+// Count, mean and sum of squared deviations of two disjoint sets of values make those of their union (Chan, Golub and
+// LeVeque 1979): no difference of large sums is formed, however the rows are ordered.  The means are kept in 64 bits, so
+// that columns far from zero lose nothing either: deviations are differences of means, of which fp32 at 300 would leave
+// 3e-5 units.
+__device__ __forceinline__ void bn_join(float na, double& mean, float& dev, float nb, double mean_b, float dev_b) {
+  if (nb == 0.f) return;
+  if (na == 0.f) {
+    mean = mean_b;
+    dev = dev_b;
+    return;
   }
-  __syncthreads();
-  const int cols = b.units * VEC;
-  for (int i = t; i < 2 * cols; i += kBlock) {
-    const int which = i >= cols, c = which ? i - cols : i;
-    float s = 0.f;
-    for (int r = 0; r < b.rpp; ++r) s += part[which][r * cols + c];
-    if (s != 0.f) unsafeAtomicAdd(sums + static_cast<int64_t>(which) * K + b.first + c, s);
-  }
+  const float share = nb / (na + nb);
+  const double d = mean_b - mean;
+  const float df = static_cast<float>(d);
+  mean += d * static_cast<double>(share);
+  dev = dev + dev_b + df * df * (na * share);
 }
 
-// sums[k] = sum_n (x - center), sums[K + k] = sum_n (x - center)^2.  [50000, 512]: 36 us (2.8 TB/s); the framework's
-// statistics took 504 us there, with two workgroups; [169343, 256]: 42 us.
+// Mean and squared deviations of a workgroup's rows, per column: partial[workgroup][3][K], the mean as the sum of two
+// floats.  A thread takes eight rows at a time: their mean and their deviations from it, formed from the differences to
+// the first of them, joined to what it has.  Bound by reading x.
 template <int VEC>
-__global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restrict__ x, const float* __restrict__ center,
-                                                            int64_t N, int K, int64_t rows_per_wg, float* __restrict__ sums) {
+__global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restrict__ x, int64_t N, int K, int64_t rows_per_wg,
+                                                            float* __restrict__ partial) {
   constexpr int U = 8;  // rows in flight per thread
+  __shared__ double part_mean[kBlock * VEC];
+  __shared__ float part_dev[kBlock * VEC];
+  __shared__ float count[kBlock];
   const BnBlock b = bn_block<VEC>(K);
   const int t = threadIdx.x;
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_wg;
   const int64_t r1 = r0 + rows_per_wg < N ? r0 + rows_per_wg : N;
-  float acc[VEC], acc2[VEC], ctr[VEC];
-#pragma unroll
-  for (int c = 0; c < VEC; ++c) acc[c] = acc2[c] = ctr[c] = 0.f;
   if (t < b.rpp * b.units) {
     const int k = b.first + (t % b.units) * VEC;
+    double mean[VEC];
+    float dev[VEC], n = 0.f;
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) ctr[c] = center[k + c];
-    auto add = [&](const float (&v)[VEC]) {
-#pragma unroll
-      for (int c = 0; c < VEC; ++c) {
-        const float d = v[c] - ctr[c];
-        acc[c] += d;
-        acc2[c] = __fmaf_rn(d, d, acc2[c]);
-      }
-    };
+    for (int c = 0; c < VEC; ++c) mean[c] = 0., dev[c] = 0.f;
     int64_t r = r0 + t / b.units;
     for (; r + static_cast<int64_t>(U - 1) * b.rpp < r1; r += static_cast<int64_t>(U) * b.rpp) {
       float v[U][VEC];
 #pragma unroll
       for (int i = 0; i < U; ++i) bn_load<VEC>(x + (r + static_cast<int64_t>(i) * b.rpp) * K + k, v[i]);
 #pragma unroll
-      for (int i = 0; i < U; ++i) add(v[i]);
+      for (int c = 0; c < VEC; ++c) {
+        float e[U], m = 0.f, q = 0.f;
+#pragma unroll
+        for (int i = 1; i < U; ++i) {
+          e[i] = v[i][c] - v[0][c];
+          m = __fmaf_rn(e[i], 1.f / U, m);  // an exact eighth: the sum cannot overflow
+        }
+        e[0] = 0.f;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float d = e[i] - m;
+          q = __fmaf_rn(d, d, q);
+        }
+        bn_join(n, mean[c], dev[c], static_cast<float>(U), static_cast<double>(v[0][c]) + static_cast<double>(m), q);
+      }
+      n += static_cast<float>(U);
     }
     for (; r < r1; r += b.rpp) {
       float v[VEC];
       bn_load<VEC>(x + r * K + k, v);
-      add(v);
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) bn_join(n, mean[c], dev[c], 1.f, static_cast<double>(v[c]), 0.f);
+      n += 1.f;
     }
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+      part_mean[t * VEC + c] = mean[c];
+      part_dev[t * VEC + c] = dev[c];
+    }
+    if (t % b.units == 0) count[t / b.units] = n;
   }
-  bn_meet<VEC>(b, K, acc, acc2, sums);
+  __syncthreads();
+  const int cols = b.units * VEC;
+  int rows = b.rpp;
+  while (rows > 1) {  // the upper half of the row slots joins the lower one
+    const int keep = (rows + 1) / 2;
+    for (int i = t; i < (rows - keep) * cols; i += kBlock) {
+      const int slot = i / cols, other = i + keep * cols;
+      bn_join(count[slot], part_mean[i], part_dev[i], count[slot + keep], part_mean[other], part_dev[other]);
+    }
+    __syncthreads();
+    if (t < rows - keep) count[t] += count[t + keep];
+    __syncthreads();
+    rows = keep;
+  }
+  float* dst = partial + static_cast<int64_t>(blockIdx.x) * 3 * K + b.first;
+  for (int i = t; i < cols; i += kBlock) {
+    const float hi = static_cast<float>(part_mean[i]);
+    dst[i] = hi;
+    dst[K + i] = fabsf(hi) <= 0x1.fffffep+127f ? static_cast<float>(part_mean[i] - static_cast<double>(hi)) : 0.f;
+    dst[2 * K + i] = part_dev[i];
+  }
 }
 
-// Moments -> mean, 1 / sqrt(var + eps), weight * that, and the running statistics with torch's bookkeeping: one
-// launch where the framework's element-wise routines took fourteen.
-__global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restrict__ center, const float* __restrict__ sums,
+// The kernels that take the workgroups of a column in their order: 8 columns x 32 groups of workgroups, each group
+// every 32nd of them, then the groups.
+constexpr int kBnCols = 8, kBnGroups = kBlock / kBnCols, kBnFlight = 8;
+
+// -> mean, 1 / sqrt(var + eps), weight * that, and the running statistics with torch's bookkeeping: one launch where
+// the framework's element-wise routines took fourteen.
+__global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restrict__ partial, int64_t wgs, int64_t rows_per_wg,
                                                            int64_t N, int K, float eps, float factor,
                                                            const float* __restrict__ weight, float* __restrict__ running_mean,
                                                            float* __restrict__ running_var, float* __restrict__ mean,
                                                            float* __restrict__ invstd, float* __restrict__ mult) {
-  const int k = static_cast<int>(blockIdx.x) * kBlock + threadIdx.x;
-  if (k >= K) return;
-  const float n = static_cast<float>(N);
-  const float shift = sums[k] / n;
-  const float raw = sums[K + k] / n - shift * shift;
-  const float var = raw < 0.f ? 0.f : raw;  // a NaN stays one
-  const float m = center[k] + shift;
+  __shared__ double part_mean[kBlock];
+  __shared__ float part_dev[kBlock], count[kBlock];
+  const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
+  const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
+  const float* src = partial + (k < K ? k : K - 1);
+  double m = 0.;
+  float n = 0.f, dev = 0.f;
+  for (int64_t w = g; w < wgs; w += kBnGroups * kBnFlight) {
+    float hi[kBnFlight], lo[kBnFlight], pd[kBnFlight];
+#pragma unroll
+    for (int i = 0; i < kBnFlight; ++i) {
+      const float* p = src + (w + i * kBnGroups < wgs ? w + i * kBnGroups : w) * 3 * K;
+      hi[i] = p[0];
+      lo[i] = p[K];
+      pd[i] = p[2 * K];
+    }
+#pragma unroll
+    for (int i = 0; i < kBnFlight; ++i) {
+      const int64_t at = w + i * kBnGroups;
+      if (at >= wgs) break;
+      const int64_t left = N - at * rows_per_wg;
+      const float rows = static_cast<float>(left < rows_per_wg ? left : rows_per_wg);
+      bn_join(n, m, dev, rows, static_cast<double>(hi[i]) + static_cast<double>(lo[i]), pd[i]);
+      n += rows;
+    }
+  }
+  count[t] = n;
+  part_mean[t] = m;
+  part_dev[t] = dev;
+  __syncthreads();
+  if (g != 0 || k >= K) return;
+  for (int i = 1; i < kBnGroups; ++i) {
+    const int o = i * kBnCols + c;
+    bn_join(n, m, dev, count[o], part_mean[o], part_dev[o]);
+    n += count[o];
+  }
+  const float rows = static_cast<float>(N);
+  const float var = dev / rows;
   const float inv = 1.f / sqrtf(var + eps);
-  mean[k] = m;
+  const float m32 = static_cast<float>(m);
+  mean[k] = m32;
   invstd[k] = inv;
   mult[k] = weight ? weight[k] * inv : inv;
   if (running_mean) {
-    const float unbiased = var * (n / static_cast<float>(N > 1 ? N - 1 : 1));
-    running_mean[k] = running_mean[k] * (1.f - factor) + m * factor;
+    const float unbiased = var * (rows / static_cast<float>(N > 1 ? N - 1 : 1));
+    running_mean[k] = running_mean[k] * (1.f - factor) + m32 * factor;
     running_var[k] = running_var[k] * (1.f - factor) + unbiased * factor;
   }
+}
+
+// The same for plain sums: sums[0 .. K) and sums[K .. 2 K), and the gradient of the weight.
+__global__ __launch_bounds__(kBlock) void bn_sums_kernel(const float* __restrict__ partial, int64_t wgs, int K,
+                                                         const float* __restrict__ invstd, float* __restrict__ sums,
+                                                         float* __restrict__ grad_weight) {
+  __shared__ float part[2][kBlock];
+  const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
+  const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
+  const float* src = partial + (k < K ? k : K - 1);
+  float s0 = 0.f, s1 = 0.f;
+  for (int64_t w = g; w < wgs; w += kBnGroups * kBnFlight) {
+    float p0[kBnFlight], p1[kBnFlight];
+#pragma unroll
+    for (int i = 0; i < kBnFlight; ++i) {
+      const int64_t at = w + i * kBnGroups < wgs ? w + i * kBnGroups : w;
+      p0[i] = src[at * 2 * K];
+      p1[i] = src[at * 2 * K + K];
+    }
+#pragma unroll
+    for (int i = 0; i < kBnFlight; ++i) {
+      if (w + i * kBnGroups >= wgs) break;
+      s0 += p0[i];
+      s1 += p1[i];
+    }
+  }
+  part[0][t] = s0;
+  part[1][t] = s1;
+  __syncthreads();
+  if (g != 0 || k >= K) return;
+  for (int i = 1; i < kBnGroups; ++i) {
+    s0 += part[0][i * kBnCols + c];
+    s1 += part[1][i * kBnCols + c];
+  }
+  sums[k] = s0;
+  sums[K + k] = s1;
+  if (grad_weight) grad_weight[k] = s1 * invstd[k];
 }
 
 // y = (x - mean) * mult + shift
@@ -220,9 +301,9 @@ struct BnBackward {
   int64_t N;
   int K;
   int64_t rows_per_wg;  // a multiple of 4
+  float* partial;       // [workgroups, 2, K]
   float* sums;          // [2, K]
   float* dx;
-  float* grad_weight;  // null, or S1 * invstd
 };
 
 template <int BITS>
@@ -293,7 +374,21 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_reduce_kernel(const BnBackward 
         }
     }
   }
-  bn_meet<4>(b, a.K, s0, s1, a.sums);
+  __shared__ float part[2][kBlock * 4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    part[0][t * 4 + c] = s0[c];
+    part[1][t * 4 + c] = s1[c];
+  }
+  __syncthreads();
+  const int cols = b.units * 4;
+  float* dst = a.partial + static_cast<int64_t>(blockIdx.x) * 2 * a.K + b.first;
+  for (int i = t; i < 2 * cols; i += kBlock) {
+    const int which = i >= cols, c = which ? i - cols : i;
+    float s = 0.f;
+    for (int r = 0; r < b.rpp; ++r) s += part[which][r * cols + c];
+    dst[which * a.K + c] = s;
+  }
 }
 
 template <int BITS>
@@ -313,9 +408,7 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_apply_kernel(const BnBackward a
     m_dy[c] = a.sums[k + c] / n;
     f1[c] = inv * inv * (a.sums[a.K + k + c] / n);
     f2[c] = a.weight ? a.weight[k + c] * inv : inv;
-    if (a.grad_weight && blockIdx.x == 0 && t < b.units) a.grad_weight[k + c] = a.sums[a.K + k + c] * inv;
   }
-  if (!a.dx) return;
   for (int64_t row = r0 + 4 * (t / b.units); row < r1; row += 4 * b.rpp) {
     float g[4][4], x[4][4];
     bn_bwd_rows<BITS>(a, row, k, g, x);
@@ -330,14 +423,14 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_apply_kernel(const BnBackward a
   }
 }
 
-__global__ __launch_bounds__(kBlock) void bn_zero_kernel(float* __restrict__ out, int n) {
-  const int i = static_cast<int>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < n) out[i] = 0.f;
-}
-
-// Rows per workgroup.  A reduction ends with two atomic adds per column into the same words, which are served one
-// after the other: about 1024 long-lived workgroups, at least 16 KiB of the stream each.  An element-wise pass has no
-// such end: up to eight times as many, which evens out the last wave.
+// Rows per workgroup.  A reduction stores two or three numbers per column and workgroup and reads them again, so its
+// workgroups are few and long-lived, with at least 16 KiB of the stream each.  Statistics: 512 in fours of columns
+// ([50000, 512] 28 against 34 us with 1024), 1024 otherwise ([100003, 301] 37 against 47 with 512, whose wavefronts have
+// a quarter of the bytes in flight).  The backward's: 1024 ([169343, 256] both passes 116 against 123).  An element-wise
+// pass has no such end: 8192, which evens out the last wave.
+constexpr int kBnApplyWgs = 8192, kBnBackwardWgs = 1024;
+template <int VEC>
+constexpr int bn_moments_wgs() { return VEC == 4 ? 512 : 1024; }
 static int64_t bn_rows_per_wg(int64_t N, int K, int vec, int wgs, int multiple) {
   const int block = kBlock * vec, blocks = (K + block - 1) / block;
   const int cols = K < block ? K : block;
@@ -354,14 +447,24 @@ static dim3 bn_grid(int64_t N, int K, int vec, int64_t rows) {
 static bool on(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 template <int BITS>
-static void launch_bn_backward(BnBackward a, hipStream_t s) {
-  a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, 1024, 4);
-  hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS>), bn_grid(a.N, a.K, 4, a.rows_per_wg), dim3(kBlock), 0, s, a);
-  a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, 8192, 4);
-  if (a.dx || a.grad_weight) {
-    const dim3 grid = bn_grid(a.N, a.K, 4, a.rows_per_wg);
-    hipLaunchKernelGGL((bn_bwd_apply_kernel<BITS>), a.dx ? grid : dim3(1, grid.y), dim3(kBlock), 0, s, a);
+static void launch_bn_backward(BnBackward a, float* grad_weight, hipStream_t s) {
+  a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnBackwardWgs, 4);
+  const dim3 grid = bn_grid(a.N, a.K, 4, a.rows_per_wg);
+  hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS>), grid, dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, a.partial,
+                     static_cast<int64_t>(grid.x), a.K, a.invstd, a.sums, grad_weight);
+  if (a.dx) {
+    a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnApplyWgs, 4);
+    hipLaunchKernelGGL((bn_bwd_apply_kernel<BITS>), bn_grid(a.N, a.K, 4, a.rows_per_wg), dim3(kBlock), 0, s, a);
   }
+}
+
+template <int VEC>
+static void launch_bn_moments(const float* x, int64_t N, int K, float* partial, int64_t& rows, int64_t& wgs, hipStream_t s) {
+  rows = bn_rows_per_wg(N, K, VEC, bn_moments_wgs<VEC>(), 1);
+  const dim3 grid = bn_grid(N, K, VEC, rows);
+  wgs = grid.x;
+  hipLaunchKernelGGL((bn_moments_kernel<VEC>), grid, dim3(kBlock), 0, s, x, N, K, rows, partial);
 }
 
 }  // namespace exact
@@ -370,25 +473,32 @@ using namespace exact;
 
 extern "C" {
 
-int exact_bn_stats_f32(const float* x, int64_t N, int64_t K, float eps, float factor, const float* weight,
-                       float* running_mean, float* running_var, float* work, float* mean, float* invstd, float* mult,
-                       void* stream) {
+int64_t exact_bn_work_floats(int64_t N, int64_t K) {
+  if (N < 1 || K < 1 || K > kBnMaxK || N > (int64_t{1} << 40) / K) return 0;
+  const int k = static_cast<int>(K);
+  int64_t most = 3 * static_cast<int64_t>(bn_grid(N, k, 1, bn_rows_per_wg(N, k, 1, bn_moments_wgs<1>(), 1)).x);
+  if (K % 4 == 0) {
+    const int64_t fours = 3 * static_cast<int64_t>(bn_grid(N, k, 4, bn_rows_per_wg(N, k, 4, bn_moments_wgs<4>(), 1)).x);
+    const int64_t back = 2 * static_cast<int64_t>(bn_grid(N, k, 4, bn_rows_per_wg(N, k, 4, kBnBackwardWgs, 4)).x);
+    most = fours > most ? fours : most;
+    most = back > most ? back : most;
+  }
+  return most * K;
+}
+
+int exact_bn_statistics_f32(const float* x, int64_t N, int64_t K, float eps, float factor, const float* weight,
+                            float* running_mean, float* running_var, float* work, float* mean, float* invstd, float* mult,
+                            void* stream) {
   if (N < 1 || K < 0 || K > kBnMaxK || N > (int64_t{1} << 40) / (K > 0 ? K : 1)) return EXACT_E_SHAPE;
   if (K == 0) return EXACT_OK;
   if (!x || !work || !mean || !invstd || !mult || (running_mean == nullptr) != (running_var == nullptr)) return EXACT_E_NULL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int k = static_cast<int>(K);
-  float* center = work + 2 * K;
-  hipLaunchKernelGGL(bn_center_kernel, dim3(static_cast<unsigned>((K + 15) / 16)), dim3(kBlock), 0, s, x, N, k, center, work);
-  if (K % 4 == 0 && on(x, 16)) {
-    const int64_t rows = bn_rows_per_wg(N, k, 4, 1024, 1);
-    hipLaunchKernelGGL((bn_moments_kernel<4>), bn_grid(N, k, 4, rows), dim3(kBlock), 0, s, x, center, N, k, rows, work);
-  } else {
-    const int64_t rows = bn_rows_per_wg(N, k, 1, 1024, 1);
-    hipLaunchKernelGGL((bn_moments_kernel<1>), bn_grid(N, k, 1, rows), dim3(kBlock), 0, s, x, center, N, k, rows, work);
-  }
-  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((K + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, center, work, N, k,
-                     eps, factor, weight, running_mean, running_var, mean, invstd, mult);
+  int64_t rows = 0, wgs = 0;
+  if (K % 4 == 0 && on(x, 16)) launch_bn_moments<4>(x, N, k, work, rows, wgs, s);
+  else launch_bn_moments<1>(x, N, k, work, rows, wgs, s);
+  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((k + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, work, wgs, rows, N,
+                     k, eps, factor, weight, running_mean, running_var, mean, invstd, mult);
   return launch_status();
 }
 
@@ -400,24 +510,24 @@ int exact_bn_apply_f32(const float* x, const float* mean, const float* mult, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int k = static_cast<int>(K);
   if (K % 4 == 0 && on(x, 16) && on(y, 16)) {
-    const int64_t rows = bn_rows_per_wg(N, k, 4, 8192, 4);
+    const int64_t rows = bn_rows_per_wg(N, k, 4, kBnApplyWgs, 4);
     hipLaunchKernelGGL((bn_apply_kernel<4>), bn_grid(N, k, 4, rows), dim3(kBlock), 0, s, x, mean, mult, bias, N, k, rows, y);
   } else {
-    const int64_t rows = bn_rows_per_wg(N, k, 1, 8192, 4);
+    const int64_t rows = bn_rows_per_wg(N, k, 1, kBnApplyWgs, 4);
     hipLaunchKernelGGL((bn_apply_kernel<1>), bn_grid(N, k, 1, rows), dim3(kBlock), 0, s, x, mean, mult, bias, N, k, rows, y);
   }
   return launch_status();
 }
 
-int exact_bn_backward_packed_f32(const float* dy, const uint32_t* mask, float p, const uint8_t* packed, int bits,
+int exact_bn_backward_ordered_f32(const float* dy, const uint32_t* mask, float p, const uint8_t* packed, int bits,
                                  const uint16_t* scale_bf16, const uint16_t* min_bf16, const float* mean, const float* invstd,
-                                 const float* weight, int64_t N, int64_t K, float* sums, float* dx, float* grad_weight,
-                                 void* stream) {
+                                 const float* weight, int64_t N, int64_t K, float* work, float* sums, float* dx,
+                                 float* grad_weight, void* stream) {
   if (bits != 1 && bits != 2 && bits != 4 && bits != 8) return EXACT_E_BITS;
   if (!(p >= 0.f && p < 1.f)) return EXACT_E_ARG;
   if (N < 1 || K < 0 || K > kBnMaxK || K % 4 != 0 || N > (int64_t{1} << 40) / (K > 0 ? K : 1)) return EXACT_E_SHAPE;
   if (K == 0) return EXACT_OK;
-  if (!dy || !packed || !scale_bf16 || !min_bf16 || !mean || !invstd || !sums) return EXACT_E_NULL;
+  if (!dy || !packed || !scale_bf16 || !min_bf16 || !mean || !invstd || !work || !sums) return EXACT_E_NULL;
   if (!on(dy, 16) || !on(dx, 16) || !on(packed, 4) || !on(mask, 4)) return EXACT_E_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   BnBackward a{};
@@ -432,16 +542,14 @@ int exact_bn_backward_packed_f32(const float* dy, const uint32_t* mask, float p,
   a.weight = weight;
   a.N = N;
   a.K = static_cast<int>(K);
+  a.partial = work;
   a.sums = sums;
   a.dx = dx;
-  a.grad_weight = grad_weight;
-  hipLaunchKernelGGL(bn_zero_kernel, dim3(static_cast<unsigned>((2 * K + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, sums,
-                     static_cast<int>(2 * K));
   switch (bits) {
-    case 1: launch_bn_backward<1>(a, s); break;
-    case 2: launch_bn_backward<2>(a, s); break;
-    case 4: launch_bn_backward<4>(a, s); break;
-    default: launch_bn_backward<8>(a, s); break;
+    case 1: launch_bn_backward<1>(a, grad_weight, s); break;
+    case 2: launch_bn_backward<2>(a, grad_weight, s); break;
+    case 4: launch_bn_backward<4>(a, grad_weight, s); break;
+    default: launch_bn_backward<8>(a, grad_weight, s); break;
   }
   return launch_status();
 }

@@ -219,10 +219,14 @@ int exact_col_moments_f32(const float *x, const float *center, int64_t N, int64_
  * as called by qbatch_norm.forward, ops.py:213):
  *   mean[k], invstd[k] = 1 / sqrt(biased variance + eps), mult[k] = weight[k] * invstd[k] (weight NULL: 1),
  * and, unless both are NULL, running = running * (1 - factor) + batch * factor (variance unbiased there).
- * `work` holds 3 K floats.  fp32 atomics: the summation order is not fixed. */
-int exact_bn_stats_f32(const float *x, int64_t N, int64_t K, float eps, float factor, const float *weight,
-                       float *running_mean, float *running_var, float *work, float *mean, float *invstd, float *mult,
-                       void *stream);
+ * Sums are taken in a fixed order (two equal calls give equal bits), means and
+ * squared deviations of parts of the rows joined pairwise: no common centre, so
+ * the order of the rows does not matter to the accuracy.  `work`:
+ * exact_bn_work_floats(N, K) floats of scratch. */
+int64_t exact_bn_work_floats(int64_t N, int64_t K);
+int exact_bn_statistics_f32(const float *x, int64_t N, int64_t K, float eps, float factor, const float *weight,
+                            float *running_mean, float *running_var, float *work, float *mean, float *invstd, float *mult,
+                            void *stream);
 
 /* y[n, k] = (x[n, k] - mean[k]) * mult[k] + bias[k] (bias NULL: 0), K <= 8192. */
 int exact_bn_apply_f32(const float *x, const float *mean, const float *mult, const float *bias, int64_t N, int64_t K,
@@ -234,11 +238,11 @@ int exact_bn_apply_f32(const float *x, const float *mean, const float *mult, con
  *   sums[k] = sum_n g, sums[K + k] = sum_n g (x - mean[k])      (sums[0..K) is the gradient of the bias)
  *   dx = (g - sums[k] / N - (x - mean[k]) invstd[k]^2 sums[K + k] / N) invstd[k] weight[k]     unless dx is NULL
  *   grad_weight[k] = sums[K + k] invstd[k]                                                     unless NULL
- * dy and dx start on 16 bytes, packed on 4.  fp32 atomics: the summation order is not fixed. */
-int exact_bn_backward_packed_f32(const float *dy, const uint32_t *mask, float p, const uint8_t *packed, int bits,
+ * dy and dx start on 16 bytes, packed on 4.  Sums in a fixed order; `work`: exact_bn_work_floats(N, K) floats. */
+int exact_bn_backward_ordered_f32(const float *dy, const uint32_t *mask, float p, const uint8_t *packed, int bits,
                                  const uint16_t *scale_bf16, const uint16_t *min_bf16, const float *mean,
-                                 const float *invstd, const float *weight, int64_t N, int64_t K, float *sums, float *dx,
-                                 float *grad_weight, void *stream);
+                                  const float *invstd, const float *weight, int64_t N, int64_t K, float *work, float *sums,
+                                  float *dx, float *grad_weight, void *stream);
 
 /* FOR BENCHMARKS ONLY -- not part of the operator interface; no product code calls it and a binding of the
  * reference's operators has no use for it.  Measurement aid with no counterpart in the reference: the memory

@@ -1,5 +1,5 @@
 """The batch norm on wide matrices and on the packed copy of its input
-(exact_bn_stats_f32, exact_bn_apply_f32, exact_bn_backward_packed_f32) against
+(exact_bn_statistics_f32, exact_bn_apply_f32, exact_bn_backward_ordered_f32) against
 the same formulas in float64 on the dequantised input."""
 import pytest
 import torch
@@ -70,3 +70,74 @@ def test_what_the_kernels_do_not_take_goes_to_the_separate_routines(backend):
     kept = ops.CompressedActivation(copy, None, x.shape, x.shape)
     config.simulate = True
     assert ops._batch_norm_backward_packed(dy, None, 0.0, kept, None, mean, invstd, want) is None
+
+
+def _rows(kind, N, K, g):
+    """Row orders that a sampled centre, or sums that run through the rows, get wrong."""
+    x = torch.randn(N, K, generator=g)
+    i = torch.arange(N)[:, None].float()
+    if kind == "periodic":                                   # every 512th row far off, with the period of N / 256 and of any power of two
+        x[::512] += 100.0
+    elif kind == "sorted":
+        x = (x * 0.01 + torch.linspace(-50.0, 50.0, N)[:, None]).sort(0).values
+    elif kind == "first rows":
+        x[:N // 64] += 1000.0
+    elif kind == "far from zero":
+        x = x * 0.01 + 300.0
+    elif kind == "alternating":
+        x = x * 1e-3 + torch.where(i % 2 == 0, 5.0, -5.0)
+    return x.contiguous()
+
+
+def _check_statistics(backend, kind, N, K):
+    g = torch.Generator().manual_seed(N + K)
+    x = _rows(kind, N, K, g)
+    mean, invstd, _ = bf.batch_norm_statistics(x.to(backend), None, None, None, 0.1, 0.0)
+    var64, mean64 = torch.var_mean(x.double(), dim=0, unbiased=False)
+    var = 1.0 / invstd.cpu().double() ** 2
+    # a few roundings per join, and the rounding of a mean far from zero, squared, is all that the variance can carry
+    assert ((var - var64).abs() <= 2e-6 * var64 + (4 * 2.0 ** -24 * mean64.abs()) ** 2).all()
+    assert ((mean.cpu() - mean64).abs() <= 4 * 2.0 ** -24 * (mean64.abs() + var64.sqrt())).all()
+
+
+KINDS = ["plain", "periodic", "sorted", "first rows", "far from zero", "alternating"]
+
+
+# rows enough for the eight-row loop of every workgroup, in fours and (3 columns) one by one
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("N,K", [(65536, 8), (30011, 3), (131072, 4)])
+def test_statistics_whatever_the_order_of_the_rows(backend, kind, N, K):
+    _check_statistics(backend, kind, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("N,K", [(131072, 256), (262144, 512), (70001, 301), (169343, 1028), (1000000, 16)])
+def test_statistics_whatever_the_order_of_the_rows_at_scale(cuda, kind, N, K):
+    _check_statistics(cuda, kind, N, K)
+
+
+def test_statistics_of_equal_rows_and_of_values_at_the_end_of_the_range(backend):
+    x = torch.full((5000, 12), 0.1).to(backend)
+    mean, invstd, _ = bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5)
+    assert torch.equal(mean, x[0]) and ((invstd - 1e-5 ** -0.5).abs() < 1e-3).all()
+    x[:, 3], x[7, 5], x[9, 6] = 3e38, float("nan"), float("inf")
+    mean, invstd, _ = bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5)
+    assert abs(mean[3].item() / 3e38 - 1) < 1e-6 and invstd[3].item() > 0
+    assert invstd[5].isnan() and mean[5].isnan() and invstd[6].isnan() and not torch.isfinite(mean[6])
+    assert torch.equal(mean[:3], x[0, :3])
+
+
+@pytest.mark.parametrize("N,K", [(9001, 36), (4099, 7)])
+def test_equal_calls_give_equal_bits(backend, N, K):
+    g = torch.Generator().manual_seed(N)
+    x, dy = (torch.randn(N, K, generator=g) + 3).to(backend), torch.randn(N, K, generator=g).to(backend)
+    first = bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5)
+    packed, scale, mn = extq.minmax_pack(x, 2)
+    back = bf.batch_norm_backward_packed(dy, None, 0.0, (packed, 2, scale, mn), None, first[0], first[1], [True] * 3)
+    for _ in range(3):
+        again = bf.batch_norm_statistics(x, None, None, None, 0.1, 1e-5)
+        assert all(torch.equal(a, b) for a, b in zip(again, first))
+        if back is not None:
+            more = bf.batch_norm_backward_packed(dy, None, 0.0, (packed, 2, scale, mn), None, first[0], first[1], [True] * 3)
+            assert all(torch.equal(a, b) for a, b in zip(more, back))
