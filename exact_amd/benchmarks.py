@@ -226,7 +226,6 @@ def kernel_extras(x, log):
         bias = torch.randn(G, device=x.device)
         flops = 2.0 * N * G * G
         gemm_bytes = 8 * N * G + 4 * G * G
-        config.tall_gemm_min_depth = 1
         w40 = torch.randn(40, G, device=x.device) / G ** 0.5
         for cores in ("bf16", "fp32"):
             config.matrix_cores = cores

@@ -99,11 +99,11 @@ _EXTRA_FIELDS = {
     # matrix-core kernel (config.matrix_cores == "bf16") from this many rows on;
     # shorter operands keep the framework's GEMM, which is as fast there.
     "tall_gemm_min_rows": 16384,
-    # ... and, for results of more than 64 columns, a reduction over at least this
-    # many features and at most this many rows: no limit by default (82 against
-    # 129 us at [169343, 128] x [128, 256], 2.0 against 2.5 ms at [2449029, 256] x
-    # [256, 256], 0.67 against 0.86 at [2449029, 46] x [46, 256]).
-    "tall_gemm_min_depth": 1,
+    # ... of which results of more than 64 columns have to reduce over at least
+    # this many features and to have at most this many rows.  A depth of 0 sets no
+    # such limit and takes the sizes at which the kernel was measured to be the
+    # faster routine.
+    "tall_gemm_min_depth": 0,
     "tall_gemm_max_rows_wide": 2 ** 31 - 1,
 }
 

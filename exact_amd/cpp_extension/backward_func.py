@@ -96,13 +96,26 @@ def weight_gradient(grad_output, input):  # noqa: A002
 
 
 # ---- the dense products of a layer on the bf16 matrix cores ---------------------
+def _worth_a_tall_product(N, D, K):
+    """Whether exact_tall_product_f32 is the faster routine.  Its workgroups take 128
+    rows by up to 128 columns and walk the whole depth: where they are too few to
+    hide the loads of a step, the framework's GEMM, which can split the depth, wins
+    by up to three times.  Measured, kernel / framework: at 128 workgroups (16,384
+    rows) 0.87 - 0.97 up to 128 features, 1.0 at 180, 1.2 - 1.4 at 256, 1.4 - 3.1
+    from 602 on; at 256 of them the same up to 180, 1.2 - 1.3 beyond; at 313 (40,000
+    rows) 0.6 - 0.9 up to 602 and 1.0 - 1.24 beyond, with 32 columns or fewer 0.9 at
+    256 and 1.4 from 602 on; from 626 on 0.5 - 0.9 nearly everywhere."""
+    groups = -(-N // 128) * -(-K // 128)
+    return groups >= 512 or D <= 160 or (groups >= 280 and D <= (800 if K > 32 else 400))
+
+
 def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     """x[N, D] . M (+ bias[K]) (+ addend[N, K]) -> [N, K], where M = `matrix`
     ([D, K]) or, with transposed=True, the transpose of `matrix` ([K, D]: a weight
     as F.linear holds it).  `into` names the result tensor; it may be `addend`
-    itself (accumulate in place).  Tall fp32 device operands with an even number of
-    features (config.tall_gemm_min_rows, tall_gemm_min_depth and
-    tall_gemm_max_rows_wide) take the library's kernel (six bf16 matrix-core
+    itself (accumulate in place).  Tall fp32 device operands (config.tall_gemm_min_rows)
+    with an even number of features, where the sizes suit it (_worth_a_tall_product, or
+    config.tall_gemm_min_depth and tall_gemm_max_rows_wide), take the library's kernel (six bf16 matrix-core
     products per fp32 product, fp32 accuracy, reproducible, infinities and the ends
     of the range as in fp32; config.matrix_cores == "bf16"); everything else the
     framework's GEMM."""
@@ -112,6 +125,7 @@ def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
               and x.shape[1] == M.shape[0] and x.shape[0] >= config.tall_gemm_min_rows and x.shape[1] % 2 == 0
               and 0 < x.shape[1] <= 4096 and 0 < M.shape[1] <= 4096
               and (M.shape[1] <= 64 or (x.shape[1] >= config.tall_gemm_min_depth and x.shape[0] <= config.tall_gemm_max_rows_wide))
+              and (config.tall_gemm_min_depth != 0 or _worth_a_tall_product(*x.shape, M.shape[1]))
               and x.is_contiguous() and x.data_ptr() % 8 == 0
               and matrix.stride(1) == 1 and matrix.stride(0) >= matrix.shape[1]
               and (bias is None or (bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == M.shape[1]

@@ -44,3 +44,21 @@ def test_projection_back_to_any_width(backend, D, k):
     got = ops.rp2input(x, (261, D), r)
     want, bound = x.double() @ r.double().t(), (7 * k + 2) * 2.0 ** -24 * (x.abs().double() @ r.abs().double().t()) + 1e-30
     assert got.shape == (261, D) and ((got.double() - want).abs() <= bound).all()
+
+
+def test_few_workgroups_and_a_deep_sum_stay_with_the_framework(backend):
+    """The sizes rule: 200 rows make two workgroups, which take 160 features and no more; a depth set by hand is obeyed."""
+    config.tall_gemm_min_rows = 1
+    x = torch.randn(200, 162).to(backend)
+
+    def taken(d, k):
+        w = torch.randn(k, d).to(backend)
+        bf.tall_matmul(x[:, :d].contiguous(), w, transposed=True)
+        return hasattr(w, "_exact_gemm_table")
+    assert taken(160, 40) and not taken(162, 40)
+    config.tall_gemm_min_depth = 1
+    assert taken(162, 40) and taken(162, 100)
+    worth = bf._worth_a_tall_product
+    assert worth(16384, 128, 256) and not worth(16384, 256, 256) and worth(16384, 4096, 600)
+    assert worth(40000, 602, 40) and not worth(40000, 602, 16) and not worth(40000, 1024, 40) and worth(40000, 1024, 256)
+    assert worth(169343, 256, 256) and worth(2449029, 100, 256)
