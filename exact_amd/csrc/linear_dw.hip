@@ -255,10 +255,6 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_bf16_kernel(const float* 
 // split (44 vector instructions per fragment) competes with the matrix cores.  Here the four wavefronts divide the
 // fragments of a step between them, split each once and hand the pieces round through LDS, in two buffers so that one
 // barrier per step suffices; the rows of the step after next are on their way while a step is multiplied.
-// [169343, 256]^T x [169343, 256]: 247 -> 161 us, [169343, 256]^T x [.., 128] 140 -> 95, [232965, 47]^T x [.., 300]
-// 166 -> 134.  Where a workgroup's block is one tile or fewer wavefronts share a fragment the barrier costs more than
-// the split ([20000, 40]^T x [.., 128] 25 -> 33, [2449029, 47]^T x [.., 64] 306 -> 359, [2449029, 256]^T x [.., 25]
-// 560 -> 620): those keep the form above.
 template <int MK, int MD, int WK>
 __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const float* __restrict__ dY, int64_t ldy,
                                                                 const float* __restrict__ X, int64_t ldx, int64_t N,
@@ -584,10 +580,25 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   slabs = (N + rows - 1) / rows;
   const dim3 grid(static_cast<unsigned>((slabs + kDwXcds - 1) / kDwXcds * kDwXcds * blocks));
   constexpr size_t lds = sizeof(u32x4) * 2 * (MK * WK + MD * WD) * 3 * kWave;
-  constexpr bool shared = (MK == 2 && MD == 2 && WK < 4) || MK == 1;  // measured, see the kernel
-  if constexpr (BF16 && shared) hipLaunchKernelGGL((linear_dw_shared_kernel<MK, MD, WK>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
-  else if constexpr (BF16) hipLaunchKernelGGL((linear_dw_bf16_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
-  else hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  // Which form, measured as shared / own over 16,384 to 1,000,000 rows (us at 100,000 in brackets):
+  //   more than 64 x more than 64    0.72 - 0.98 (157 / 196 at 256 x 300), 1.03 at 16,384 x 100 x 100: shared
+  //   33 - 64 x more than 128        1.03 - 1.11 at 16,384 rows, 0.86 - 1.04 at 100,000 (72 / 82 at 64 x 300), 0.79 - 0.89
+  //                                  at 1,000,000: shared from 65,536 rows on
+  //   up to 32 x more than 128       1.14 - 1.38, 0.97 - 1.31 (95 / 77 at 32 x 602), 0.83 - 0.96: shared from 500,000 on
+  //   fewer columns of either        1.02 - 1.5 nearly everywhere (31 / 23 at 8 x 32): own
+  constexpr bool can_share = MD == 2 && WK <= 2;
+  const bool shared = can_share && (WK == 2 || N >= (MK == 2 ? 65536 : 500000));
+  if constexpr (!BF16) {
+    hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  } else {
+    if constexpr (can_share) {
+      if (shared) {
+        hipLaunchKernelGGL((linear_dw_shared_kernel<MK, MD, WK>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((linear_dw_bf16_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+  }
 }
 
 template <bool BF16>
