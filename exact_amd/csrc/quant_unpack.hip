@@ -178,6 +178,25 @@ struct UnpackFlatArgs {
 // every compute unit four workgroups of such threads.
 constexpr int kFlatPieces = 4;
 
+// the first nv (1 .. 7) of eight fp16 values, at any element boundary: up to three stores
+__device__ __forceinline__ void store_half_tail(half_t* p, int nv, const float (&r)[8]) {
+  typedef half_t half2_any __attribute__((ext_vector_type(2), aligned(2)));
+  typedef half_t half4_any __attribute__((ext_vector_type(4), aligned(2)));
+  half_t h[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) h[i] = to_half(r[i]);
+  int at = 0;
+  if (nv & 4) {
+    *reinterpret_cast<half4_any*>(p) = half4_any{h[0], h[1], h[2], h[3]};
+    at = 4;
+  }
+  if (nv & 2) {
+    *reinterpret_cast<half2_any*>(p + at) = at ? half2_any{h[4], h[5]} : half2_any{h[0], h[1]};
+    at += 2;
+  }
+  if (nv & 1) p[at] = at == 0 ? h[0] : at == 2 ? h[2] : at == 4 ? h[4] : h[6];
+}
+
 template <int BITS, int PARAM, int PIECES>
 __global__ __launch_bounds__(kBlock) void unpack_flat_kernel(const UnpackFlatArgs a) {
   constexpr bool F16 = PARAM == kParamF16;
@@ -244,9 +263,7 @@ __global__ __launch_bounds__(kBlock) void unpack_flat_kernel(const UnpackFlatArg
         for (int i = 0; i < 8; ++i) q[i] = to_half(r[i]);
         *reinterpret_cast<half8_any*>(p) = q;
       } else {
-#pragma unroll
-        for (int i = 0; i < PIECE - 1; ++i)
-          if (i < nv) p[i] = to_half(r[i]);
+        store_half_tail(p, nv, r);
       }
     } else {
       float* p = static_cast<float*>(a.out) + flat;
