@@ -600,22 +600,32 @@ __global__ __launch_bounds__(kFlatThreads) void pack_flat_kernel(const PackFlatA
     }
   }
   __syncthreads();
-  for (int first = 0; first < rows_here; first += T >> 3) {
-    const int r = first + (t >> 3);
+  // 2^lanes_log2 lanes a row: 8, fewer where a row has fewer octs (with 8 throughout, rows of one oct took a third
+  // longer than the whole of pack_kernel's pass)
+  const int lanes_log2 = a.opr > 4 ? 3 : a.opr > 2 ? 2 : a.opr > 1 ? 1 : 0;
+  const int lane = t & ((1 << lanes_log2) - 1);
+  for (int first = 0; first < rows_here; first += T >> lanes_log2) {
+    const int r = first + (t >> lanes_log2);
     const bool ok = r < rows_here;
     int lo = 0x7FFFFFFF, hi = static_cast<int>(0x80000000u);
-    for (int c = t & 7; c < a.opr; c += 8) {
+    for (int c = lane; c < a.opr; c += 1 << lanes_log2) {
       const uint2 m = oct_lds[(ok ? r : 0) * a.opr + c];
       lo = min(lo, static_cast<int>(m.x));
       hi = max(hi, static_cast<int>(m.y));
     }
-    lo = min(lo, dpp_lanes<0xB1>(lo));
-    hi = max(hi, dpp_lanes<0xB1>(hi));
-    lo = min(lo, dpp_lanes<0x4E>(lo));
-    hi = max(hi, dpp_lanes<0x4E>(hi));
-    lo = min(lo, dpp_lanes<0x141>(lo));
-    hi = max(hi, dpp_lanes<0x141>(hi));
-    if (ok && (t & 7) == 0) {
+    if (lanes_log2 > 0) {  // the same for the whole launch
+      lo = min(lo, dpp_lanes<0xB1>(lo));
+      hi = max(hi, dpp_lanes<0xB1>(hi));
+    }
+    if (lanes_log2 > 1) {
+      lo = min(lo, dpp_lanes<0x4E>(lo));
+      hi = max(hi, dpp_lanes<0x4E>(hi));
+    }
+    if (lanes_log2 > 2) {
+      lo = min(lo, dpp_lanes<0x141>(lo));
+      hi = max(hi, dpp_lanes<0x141>(hi));
+    }
+    if (ok && lane == 0) {
       const float mnv = key_value(lo);
       float sc;
       // ops.py:39, two roundings (see pack_kernel)
