@@ -32,7 +32,7 @@ def spmm_csr(rowptr, col, value, mat, reduce):
         raise NotImplementedError(f"reduce='{reduce}': use spmm_max_fw / spmm_min_fw for max and min")
     reproducible = config.deterministic_spmm or torch.are_deterministic_algorithms_enabled()
     half = isinstance(mat, torch.Tensor) and mat.dtype == torch.float16
-    if half and (reproducible or not _checks.on_device(mat)):
+    if half and (reproducible or not _gathers_half(mat)):
         # fp16 activations (autocast): accumulate in fp32, round the result once
         return spmm_csr(rowptr, col, value, mat.float(), reduce).to(torch.float16)
     _check_index(rowptr, "rowptr")
@@ -70,6 +70,19 @@ def spmm_csr(rowptr, col, value, mat, reduce):
                     col.numel(), REDUCE[reduce], ptr(out), K, _checks.stream_ptr(mat))
     _lib.check(rc, f"spmm_{reduce}")
     return out.to(torch.float16) if half else out          # one rounding of the fp32 sum
+
+
+def _gathers_half(mat):
+    """Whether an fp16 operand is gathered as it is rather than widened first.  A
+    lane has to take two elements or more: 0.41 - 0.8 of the widened form's time from
+    100 columns on, while one element a lane (64 columns or fewer, an odd number, rows
+    off a 4-byte boundary) takes 1.05 - 1.4 times as long, half the bytes a gather
+    costing as much as the whole (300,000 nodes, 15 entries a row: 64 columns 297
+    against 231 us, 128 columns 251 against 487)."""
+    if not _checks.on_device(mat) or mat.dim() != 2 or mat.shape[1] <= 64 or mat.shape[1] % 2:
+        return False
+    whole = mat.stride(1) != 1 or mat.stride(0) < mat.shape[1]      # copied to rows of its own by _aligned_rows
+    return whole or (mat.stride(0) % 2 == 0 and mat.data_ptr() % 4 == 0)
 
 
 def _aligned_rows(mat, nnz):
