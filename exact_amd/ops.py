@@ -312,6 +312,13 @@ def _batch_norm_backward_packed(grad_output, mask, p, kept, weight, mean, invstd
     return ext_backward_func.batch_norm_backward_packed(grad_output, mask, p, (packed, bits, scale, mn), weight, mean, invstd, wanted)
 
 
+def _large_enough_for_own_statistics(input):  # noqa: A002
+    """Where the forward is bound by the device: below, it is one call into the
+    framework against two into the library with an allocation each (38 - 45 against
+    52 us up to 4096 rows, equal at [5000, 300], 62 against 52 at [20000, 128])."""
+    return input.shape[0] >= 8192 or input.numel() >= 2 ** 23
+
+
 class qbatch_norm(Function):
     """Training-mode batch norm that keeps its input compressed (reference ops.py:206-254)."""
 
@@ -320,7 +327,7 @@ class qbatch_norm(Function):
                 training, exponential_average_factor, eps, scheme):
         kept = CompressedActivation.compress(input, scheme, project=False)
         stats = (ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps)
-                 if training else None)
+                 if training and _large_enough_for_own_statistics(input) else None)
         if stats is not None:
             save_mean, save_invstd, mult = stats
             output = ext_backward_func.batch_norm_apply(input, save_mean, mult, bias)

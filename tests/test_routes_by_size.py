@@ -3,7 +3,7 @@ below it the framework's routine (or the widened operand) runs as it did."""
 import pytest
 import torch
 
-from exact_amd import _lib
+from exact_amd import _lib, ops
 from exact_amd.cpp_extension import spmm
 
 
@@ -36,3 +36,15 @@ def test_half_operands_of_the_sparse_product(calls, K, shift, direct):
     assert ("exact_spmm_csr_strided_f16" in seen) == direct and ("exact_spmm_csr_strided_f32" in seen) == (not direct)
     want = torch.zeros(n, K, dtype=torch.double).index_add_(0, row, mat.cpu().double()[col])
     assert got.dtype == torch.float16 and ((got.cpu().double() - want).abs() <= 2.0 ** -11 * want.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("N,K,own", [(1024, 16, False), (8000, 8, False), (8192, 8, True)])
+def test_statistics_of_a_batch_norm_layer(calls, N, K, own):
+    seen, device = calls
+    x = (torch.randn(N, K) + 2).to(device).requires_grad_()
+    rm, rv, w, b = (t.to(device) for t in (torch.zeros(K), torch.ones(K), torch.ones(K), torch.zeros(K)))
+    y = ops.qbatch_norm.apply(x, rm, rv, w, b, True, 0.1, 1e-5, None)
+    assert ("exact_bn_statistics_f32" in seen) == own
+    want = (x.detach().double() - x.detach().double().mean(0)) / (x.detach().double().var(0, unbiased=False) + 1e-5).sqrt()
+    assert (y.detach().double() - want).abs().max() < 1e-4
+    y.backward(torch.ones_like(y))
