@@ -221,19 +221,22 @@ def native_batch_norm_backward(grad_out, input, weight, running_mean, running_va
     return grad_input, grad_weight, grad_bias
 
 
-def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, eps):
+def _column_vector(t, matrix):
+    """Whether a kernel may read `t` as one fp32 number per column of `matrix` (None: absent)."""
+    return t is None or (t.dtype == torch.float32 and t.device == matrix.device and t.is_contiguous() and t.dim() == 1
+                         and t.numel() == matrix.shape[1])
+
+
+def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, eps, bias=None):
     """The statistics half of native_batch_norm in training mode -> (mean,
     1 / sqrt(var + eps), weight * that), with running_mean / running_var updated
-    in place; None where the library's kernels do not apply (the caller then
-    takes the framework's routines).  From 1024 rows on: below, the framework's
-    reduction is no slower."""
-    def vector_ok(t):
-        return (t is None or (t.dtype == torch.float32 and t.device == matrix.device and t.is_contiguous()
-                              and t.numel() == matrix.shape[1]))
-
+    in place; None where the library's kernels do not apply, `bias` for
+    batch_norm_apply among what they need (the caller then takes the framework's
+    routines, which refuse what is malformed).  From 1024 rows on: below, the
+    framework's reduction is no slower."""
     usable = (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
               and 0 < matrix.shape[1] <= 8192 and 1024 <= matrix.shape[0] < 2 ** 31
-              and vector_ok(weight) and vector_ok(running_mean) and vector_ok(running_var)
+              and all(_column_vector(t, matrix) for t in (weight, bias, running_mean, running_var))
               and (running_mean is None) == (running_var is None) and momentum is not None and _atomics_allowed())
     if not usable:
         return None
@@ -252,9 +255,10 @@ def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, e
 
 def batch_norm_apply(matrix, mean, mult, bias):
     """(matrix - mean) * mult + bias per column, for the statistics above."""
+    if not (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
+            and mean is not None and mult is not None and all(_column_vector(t, matrix) for t in (mean, mult, bias))):
+        raise RuntimeError("batch_norm_apply: an fp32 matrix and one fp32 number per column on its device are needed")
     out = torch.empty_like(matrix)
-    if bias is not None:
-        bias = bias.detach().to(torch.float32).contiguous()
     rc = _lib.lib().exact_bn_apply_f32(_checks.ptr(matrix), _checks.ptr(mean), _checks.ptr(mult), _checks.ptr(bias), *matrix.shape,
                                        _checks.ptr(out), _checks.stream_ptr(matrix))
     _lib.check(rc, "batch_norm_apply")
@@ -276,7 +280,9 @@ def batch_norm_backward_packed(grad_out, mask, p, quantized, weight, mean, invst
               and scale.dtype == torch.bfloat16 and mn.dtype == torch.bfloat16
               and scale.numel() == mn.numel() == grad_out.shape[0] and scale.is_contiguous() and mn.is_contiguous()
               and all(t.device == grad_out.device for t in (packed, scale, mn, *vectors))
-              and all(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == grad_out.shape[1] for t in vectors)
+              and all(_column_vector(t, grad_out) for t in vectors)
+              and (mask is None or (mask.dtype == torch.int32 and mask.device == grad_out.device and mask.is_contiguous()
+                                    and mask.numel() * 32 >= grad_out.numel()))
               and _atomics_allowed())
     if not usable:
         return None

@@ -326,7 +326,7 @@ class qbatch_norm(Function):
     def forward(ctx, input, running_mean, running_var, weight, bias,  # noqa: A002
                 training, exponential_average_factor, eps, scheme):
         kept = CompressedActivation.compress(input, scheme, project=False)
-        stats = (ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps)
+        stats = (ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps, bias)
                  if training and _large_enough_for_own_statistics(input) else None)
         if stats is not None:
             save_mean, save_invstd, mult = stats

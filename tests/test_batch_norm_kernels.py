@@ -141,3 +141,29 @@ def test_equal_calls_give_equal_bits(backend, N, K):
         if back is not None:
             more = bf.batch_norm_backward_packed(dy, None, 0.0, (packed, 2, scale, mn), None, first[0], first[1], [True] * 3)
             assert all(torch.equal(a, b) for a, b in zip(more, back))
+
+
+def test_malformed_column_vectors_are_refused(backend, monkeypatch):
+    """A bias or weight of another length, type or device: the layer leaves it to the framework's routine, and the
+    kernels' own entry refuses it; none reads past it."""
+    x = torch.randn(9000, 12).to(backend).requires_grad_()
+    rm, rv, w = (t.to(backend) for t in (torch.zeros(12), torch.ones(12), torch.ones(12)))
+
+    def framework(*args):
+        raise RuntimeError("left to the framework")
+    monkeypatch.setattr(bf, "native_batch_norm", framework)
+    for bad in (torch.zeros(11).to(backend), torch.zeros(1).to(backend), torch.zeros(13).to(backend), torch.zeros(12).half().to(backend)):
+        with pytest.raises(RuntimeError, match="left to the framework"):
+            ops.qbatch_norm.apply(x, rm, rv, w, bad, True, 0.1, 1e-5, None)
+        with pytest.raises(RuntimeError, match="left to the framework"):
+            ops.qbatch_norm.apply(x, rm, rv, bad, w, True, 0.1, 1e-5, None)
+    mean, _, mult = bf.batch_norm_statistics(x.detach(), w, None, None, 0.1, 1e-5)
+    for bad in (torch.zeros(11).to(backend), torch.zeros(12, dtype=torch.double).to(backend), torch.zeros(24).to(backend)[::2]):
+        with pytest.raises(RuntimeError):
+            bf.batch_norm_apply(x.detach(), mean, mult, bad)
+        assert bf.batch_norm_statistics(x.detach(), w, None, None, 0.1, 1e-5, bad) is None
+    if backend.type == "cuda":
+        with pytest.raises(RuntimeError):
+            bf.batch_norm_apply(x.detach(), mean, mult, torch.zeros(12))
+    with pytest.raises(RuntimeError):
+        bf.batch_norm_apply(x.detach()[:, :6], mean[:6], mult[:6], None)
