@@ -25,6 +25,13 @@ def plain_values(*tensors):
     return all(type(t) in (torch.Tensor, torch.nn.Parameter) and unpack(t).tangent is None for t in tensors if t is not None)
 
 
+def recorded(*tensors):
+    """True where operations on these tensors are being recorded for a derivative (a
+    backward under create_graph): kernels that autograd knows nothing of would end
+    the record without a word."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
 def check_device_tensor(t, name, dim=None, dtypes=(torch.float32,)):
     if not isinstance(t, torch.Tensor):
         _fail(f"{name} must be a tensor!")

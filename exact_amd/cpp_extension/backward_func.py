@@ -65,7 +65,8 @@ def weight_gradient(grad_output, input):  # noqa: A002
     instruction (config.matrix_cores), whose slabs meet through atomics; fp16 ones on
     the fp16 instruction, whose slabs are added in a fixed order.  Deterministic mode
     and everything else keep the framework's GEMM."""
-    half = grad_output.dtype == torch.float16 and input.dtype == torch.float16 and config.matrix_cores == "bf16"
+    half = (grad_output.dtype == torch.float16 and input.dtype == torch.float16 and config.matrix_cores == "bf16"
+            and not _checks.recorded(grad_output, input))
     usable = (grad_output.dim() == 2 and input.dim() == 2 and (half or (grad_output.dtype == torch.float32
               and input.dtype == torch.float32)) and _checks.on_device(grad_output) and _checks.on_device(input)
               and grad_output.shape[0] == input.shape[0] and grad_output.shape[0] >= 16384
@@ -283,6 +284,7 @@ def batch_norm_backward_packed(grad_out, mask, p, quantized, weight, mean, invst
               and all(_column_vector(t, grad_out) for t in vectors)
               and (mask is None or (mask.dtype == torch.int32 and mask.device == grad_out.device and mask.is_contiguous()
                                     and mask.numel() * 32 >= grad_out.numel()))
+              and not _checks.recorded(grad_out, weight)
               and _atomics_allowed())
     if not usable:
         return None
