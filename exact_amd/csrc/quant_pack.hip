@@ -22,6 +22,8 @@
 
 #include <cmath>
 
+#include <type_traits>
+
 #include "exact_common.hpp"
 
 namespace exact {
@@ -600,49 +602,54 @@ __global__ __launch_bounds__(kFlatThreads) void pack_flat_kernel(const PackFlatA
     }
   }
   __syncthreads();
-  // 2^lanes_log2 lanes a row: 8, fewer where a row has fewer octs (with 8 throughout, rows of one oct took a third
-  // longer than the whole of pack_kernel's pass)
-  const int lanes_log2 = a.opr > 4 ? 3 : a.opr > 2 ? 2 : a.opr > 1 ? 1 : 0;
-  const int lane = t & ((1 << lanes_log2) - 1);
-  for (int first = 0; first < rows_here; first += T >> lanes_log2) {
-    const int r = first + (t >> lanes_log2);
-    const bool ok = r < rows_here;
-    int lo = 0x7FFFFFFF, hi = static_cast<int>(0x80000000u);
-    for (int c = lane; c < a.opr; c += 1 << lanes_log2) {
-      const uint2 m = oct_lds[(ok ? r : 0) * a.opr + c];
-      lo = min(lo, static_cast<int>(m.x));
-      hi = max(hi, static_cast<int>(m.y));
-    }
-    if (lanes_log2 > 0) {  // the same for the whole launch
-      lo = min(lo, dpp_lanes<0xB1>(lo));
-      hi = max(hi, dpp_lanes<0xB1>(hi));
-    }
-    if (lanes_log2 > 1) {
-      lo = min(lo, dpp_lanes<0x4E>(lo));
-      hi = max(hi, dpp_lanes<0x4E>(hi));
-    }
-    if (lanes_log2 > 2) {
-      lo = min(lo, dpp_lanes<0x141>(lo));
-      hi = max(hi, dpp_lanes<0x141>(hi));
-    }
-    if (ok && lane == 0) {
-      const float mnv = key_value(lo);
-      float sc;
-      // ops.py:39, two roundings (see pack_kernel)
-      if constexpr (HALF) {
-        const float recip = round_to_half(1.0f / round_to_half(key_value(hi) - mnv));
-        sc = round_to_half(recip * B);
-      } else {
-        const float recip = 1.0f / (key_value(hi) - mnv);
-        sc = recip * B;
+  // 8 lanes a row, fewer where a row has fewer octs (with 8 throughout, rows of one oct took a third longer than the
+  // whole of pack_kernel's pass)
+  auto row_statistics = [&](auto log2) {
+    constexpr int LOG2 = decltype(log2)::value, L = 1 << LOG2;
+    for (int first = 0; first < rows_here; first += T >> LOG2) {
+      const int r = first + (t >> LOG2);
+      const bool ok = r < rows_here;
+      int lo = 0x7FFFFFFF, hi = static_cast<int>(0x80000000u);
+      for (int c = t & (L - 1); c < a.opr; c += L) {
+        const uint2 m = oct_lds[(ok ? r : 0) * a.opr + c];
+        lo = min(lo, static_cast<int>(m.x));
+        hi = max(hi, static_cast<int>(m.y));
       }
-      row_lds[r] = make_float2(mnv, sc);
-      if (a.scale_f32) (a.scale_f32 + row_base)[r] = sc;
-      if (a.min_f32) (a.min_f32 + row_base)[r] = mnv;
-      if (a.scale_16) (a.scale_16 + row_base)[r] = HALF ? half_bits(sc) : f32_to_bf16_rne(sc);
-      if (a.min_16) (a.min_16 + row_base)[r] = HALF ? half_bits(mnv) : f32_to_bf16_rne(mnv);
+      if constexpr (LOG2 > 0) {
+        lo = min(lo, dpp_lanes<0xB1>(lo));
+        hi = max(hi, dpp_lanes<0xB1>(hi));
+      }
+      if constexpr (LOG2 > 1) {
+        lo = min(lo, dpp_lanes<0x4E>(lo));
+        hi = max(hi, dpp_lanes<0x4E>(hi));
+      }
+      if constexpr (LOG2 > 2) {
+        lo = min(lo, dpp_lanes<0x141>(lo));
+        hi = max(hi, dpp_lanes<0x141>(hi));
+      }
+      if (ok && (t & (L - 1)) == 0) {
+        const float mnv = key_value(lo);
+        float sc;
+        // ops.py:39, two roundings (see pack_kernel)
+        if constexpr (HALF) {
+          const float recip = round_to_half(1.0f / round_to_half(key_value(hi) - mnv));
+          sc = round_to_half(recip * B);
+        } else {
+          const float recip = 1.0f / (key_value(hi) - mnv);
+          sc = recip * B;
+        }
+        row_lds[r] = make_float2(mnv, sc);
+        if (a.scale_f32) (a.scale_f32 + row_base)[r] = sc;
+        if (a.min_f32) (a.min_f32 + row_base)[r] = mnv;
+        if (a.scale_16) (a.scale_16 + row_base)[r] = HALF ? half_bits(sc) : f32_to_bf16_rne(sc);
+        if (a.min_16) (a.min_16 + row_base)[r] = HALF ? half_bits(mnv) : f32_to_bf16_rne(mnv);
+      }
     }
-  }
+  };
+  if (a.opr > 4) row_statistics(std::integral_constant<int, 3>{});  // the same for the whole launch
+  else if (a.opr > 2) row_statistics(std::integral_constant<int, 2>{});
+  else if (a.opr > 1) row_statistics(std::integral_constant<int, 1>{});
+  else row_statistics(std::integral_constant<int, 0>{});
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < OPT; ++k) {

@@ -263,7 +263,14 @@ __global__ __launch_bounds__(kBlock) void unpack_flat_kernel(const UnpackFlatArg
         for (int i = 0; i < 8; ++i) q[i] = to_half(r[i]);
         *reinterpret_cast<half8_any*>(p) = q;
       } else {
-        store_half_tail(p, nv, r);
+        // wide where the rows start on 4 bytes; off them a wide store is taken apart and the single ones are as fast
+        if (a.G % 2 == 0) {
+          store_half_tail(p, nv, r);
+        } else {
+#pragma unroll
+          for (int i = 0; i < PIECE - 1; ++i)
+            if (i < nv) p[i] = to_half(r[i]);
+        }
       }
     } else {
       float* p = static_cast<float*>(a.out) + flat;
