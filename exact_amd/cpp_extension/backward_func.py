@@ -2,11 +2,19 @@
 (backward_func.cc:83-107).  The reference only re-exports ATen routines plus
 the two-GEMM linear backward, which are reachable from Python as they are;
 its one kernel of its own, the ELU derivative, is a kernel of the library."""
+import functools
+
 import torch
 
 from .. import _lib
 from ..conf import config
 from . import _checks
+
+
+@functools.lru_cache(maxsize=512)
+def _scratch_size(entry, *sizes):
+    """What a size entry of the library answers: a function of the sizes alone."""
+    return int(getattr(_lib.lib(), entry)(*sizes))
 
 
 def _atomics_allowed():
@@ -81,7 +89,7 @@ def weight_gradient(grad_output, input):  # noqa: A002
     if half:
         L = _lib.lib()
         out = torch.empty((K, D), dtype=torch.float16, device=grad_output.device)
-        work = torch.empty(int(L.exact_linear_dw_f16_work_nbytes(N, K, D)), dtype=torch.uint8, device=grad_output.device)
+        work = torch.empty(_scratch_size("exact_linear_dw_f16_work_nbytes", N, K, D), dtype=torch.uint8, device=grad_output.device)
         rc = L.exact_linear_dw_ordered_f16(_checks.ptr(grad_output), grad_output.stride(0), _checks.ptr(input), input.stride(0),
                                            N, K, D, _checks.ptr(out), _checks.ptr(work), _checks.stream_ptr(grad_output))
         _lib.check(rc, "weight_gradient")
@@ -156,7 +164,7 @@ def tall_matmul(x, matrix, transposed=False, bias=None, addend=None, into=None):
     # not remembered: a weight changes through `.data` without raising its version, a captured graph has to read the
     # weight of its replay, and another stream would have to wait for the one that made the copy.
     L = _lib.lib()
-    work = torch.empty(int(L.exact_tall_product_work_nbytes(D, K)), dtype=torch.uint8, device=x.device)
+    work = torch.empty(_scratch_size("exact_tall_product_work_nbytes", D, K), dtype=torch.uint8, device=x.device)
     rc = L.exact_tall_product_f32(_checks.ptr(x), _checks.ptr(matrix), matrix.stride(0), int(bool(transposed)), N, D, K,
                                   _checks.ptr(bias) if bias is not None else None,
                                   _checks.ptr(addend) if addend is not None else None,
@@ -244,7 +252,7 @@ def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, e
     N, K = matrix.shape
     L = _lib.lib()
     mean, invstd, mult = torch.empty((3, K), dtype=torch.float32, device=matrix.device)
-    work = torch.empty(int(L.exact_bn_work_floats(N, K)), dtype=torch.float32, device=matrix.device)
+    work = torch.empty(_scratch_size("exact_bn_work_floats", N, K), dtype=torch.float32, device=matrix.device)
     rc = L.exact_bn_statistics_f32(_checks.ptr(matrix), N, K, float(eps), float(momentum), _checks.ptr(weight),
                                    _checks.ptr(running_mean), _checks.ptr(running_var), _checks.ptr(work),
                                    _checks.ptr(mean), _checks.ptr(invstd), _checks.ptr(mult), _checks.stream_ptr(matrix))
@@ -291,7 +299,7 @@ def batch_norm_backward_packed(grad_out, mask, p, quantized, weight, mean, invst
     N, K = grad_out.shape
     L = _lib.lib()
     sums = torch.empty((2, K), dtype=torch.float32, device=grad_out.device)
-    work = torch.empty(int(L.exact_bn_work_floats(N, K)), dtype=torch.float32, device=grad_out.device)
+    work = torch.empty(_scratch_size("exact_bn_work_floats", N, K), dtype=torch.float32, device=grad_out.device)
     grad_input = torch.empty_like(grad_out) if output_mask[0] else None
     grad_weight = torch.empty(K, dtype=torch.float32, device=grad_out.device) if output_mask[1] else None
     rc = L.exact_bn_backward_ordered_f32(_checks.ptr(grad_out), _checks.ptr(mask), float(p), _checks.ptr(packed), bits,
