@@ -44,26 +44,9 @@ def column_sums(matrix):
 
 
 def batch_statistics(matrix):
-    """(biased variance, mean) of every column of a 2-D tensor, what
-    torch.var_mean(matrix, dim=0, unbiased=False) returns.  Tall fp32 device
-    matrices of at most 256 columns take the library's one-pass kernel (moments
-    centred on the mean of 256 rows spread evenly over the matrix -- also for
-    sorted or clustered rows a centre within a fraction of a standard deviation
-    of the column mean, so that the difference of the two moments loses no
-    digits); everything else the framework's reduction."""
-    usable = (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
-              and 0 < matrix.shape[1] <= 256 and matrix.shape[0] >= 4096
-              and _atomics_allowed())
-    if not usable:
-        return torch.var_mean(matrix, dim=0, unbiased=False)
-    N, K = matrix.shape
-    center = matrix[::N // 256][:256].mean(0)
-    sums = torch.empty((2, K), dtype=torch.float32, device=matrix.device)
-    rc = _lib.lib().exact_col_moments_f32(_checks.ptr(matrix), _checks.ptr(center), N, K, _checks.ptr(sums[0]),
-                                          _checks.ptr(sums[1]), _checks.stream_ptr(matrix))
-    _lib.check(rc, "batch_statistics")
-    shift = sums[0] / N
-    return (sums[1] / N - shift * shift).clamp_(min=0.0), center + shift
+    """(biased variance, mean) of every column of a 2-D tensor by the framework's
+    reduction: for the matrices that batch_norm_statistics does not take."""
+    return torch.var_mean(matrix, dim=0, unbiased=False)
 
 
 def weight_gradient(grad_output, input):  # noqa: A002
