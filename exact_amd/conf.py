@@ -89,9 +89,10 @@ _EXTRA_FIELDS = {
     # also switched on by torch.use_deterministic_algorithms(True).  The default
     # kernel balances hub rows across wavefronts and adds their parts atomically.
     "deterministic_spmm": False,
-    # Column sums, weight gradients, batch statistics and the batch-norm
-    # backward reductions combine partial results with fp32 atomics (no fixed
-    # summation order: the last bits vary from run to run).  True sends all four
+    # Column sums, fp32 weight gradients and the batch-norm backward on a
+    # dequantised input combine partial results with fp32 atomics (no fixed
+    # summation order: the last bits vary from run to run).  True sends these,
+    # and the fp16 weight gradients and batch-norm kernels whose order is fixed,
     # to the framework's own, reproducible routines, as
     # torch.use_deterministic_algorithms(True) does.
     "deterministic_reductions": False,

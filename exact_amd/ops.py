@@ -717,8 +717,10 @@ class qbn_relu_dropout(Function):
     in two passes over the input instead of six: the batch norm's compressed
     copy of its input (ops.py:213), the batch statistics, and then ONE pass that
     normalises, applies ReLU and dropout with one joint mask and quantises the
-    result for the following layer.  Backward: the joint mask, then
-    native_batch_norm_backward on the dequantised input as in ops.py:228-254.
+    result for the following layer.  Backward (ops.py:228-254): two passes that read
+    the gradient, the joint mask and the packed input
+    (batch_norm_backward_packed); where those do not apply, dropout_bwd and then
+    native_batch_norm_backward on the dequantised input.
     -> (output, packed, scale bf16, min bf16)."""
 
     @staticmethod

@@ -428,7 +428,8 @@ int exact_rp_minmax_pack_bf16_f32(const float *X, const void *table, int mode, c
  * fragments of M into `table` (exact_tall_gemm_table_nbytes(D, K) bytes, 16-byte
  * aligned, owned by the caller, valid while M is unchanged) and
  * exact_tall_gemm_bf16_f32 multiplies by it.  This table has no room for a scale
- * per column: entries of M below 1e-30 keep fewer than 24 bits. */
+ * per column: M has to be finite, and entries of it below 1e-30 keep fewer than
+ * 24 bits. */
 int64_t exact_tall_product_work_nbytes(int64_t D, int64_t K);
 int exact_tall_product_f32(const float *X, const float *M, int64_t ld, int transposed, int64_t N,
                            int64_t D, int64_t K, const float *bias, const float *addend, int64_t ldc,

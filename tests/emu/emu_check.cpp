@@ -7,6 +7,7 @@
 // `large` adds grids of thousands of workgroups (20011 x 256, a 20000-node
 // graph; minutes); `full` adds the benchmark shapes (169343 x 256 and a
 // 169343-node graph; hours under the sanitizer).
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -167,6 +168,39 @@ static void check_spmm(int64_t M, int64_t ncols, int64_t K, double avg, int64_t 
                              : exact_spmm_csr_rowwise_f32(rp32.p, col32.p, valued ? val.p : nullptr, 4, X.p, M, ncols, K, nnz, reduce, out.p, nullptr);
         CHECK(rc2 == 0 && std::memcmp(out.p, want.p, M * K * 4) == 0, "rowwise spmm differs M=%ld K=%ld reduce=%d valued=%d wide=%d", (long)M, (long)K, reduce, valued, wide);
       }
+}
+
+// fp16 operand, rows padded to ldx, the result's to ldo: fp32 sums of the widened values
+static void check_spmm_half(int64_t M, int64_t ncols, int64_t K, int64_t pad, double avg, int64_t hub, std::mt19937& rng) {
+  const Csr g = powerlaw(M, ncols, avg, hub, rng);
+  const int64_t nnz = (int64_t)g.col.size(), ldx = K + pad, ldo = K + 2 * pad;
+  std::normal_distribution<float> nd(0.f, 1.f);
+  Buf<_Float16> X(ncols * ldx);
+  Buf<float> wide(ncols * K), out(M * ldo), want(M * K), val(nnz);
+  Buf<int64_t> rp64(M + 1), col64(nnz);
+  Buf<int32_t> rp32(M + 1), col32(nnz);
+  for (int64_t i = 0; i < ncols * ldx; ++i) X[i] = (_Float16)nd(rng);
+  for (int64_t r = 0; r < ncols; ++r)
+    for (int64_t k = 0; k < K; ++k) wide[r * K + k] = (float)X[r * ldx + k];
+  for (int64_t i = 0; i <= M; ++i) { rp64[i] = g.rowptr[i]; rp32[i] = (int32_t)g.rowptr[i]; }
+  for (int64_t i = 0; i < nnz; ++i) { col64[i] = g.col[i]; col32[i] = (int32_t)g.col[i]; val[i] = g.val[i]; }
+  for (int reduce = 0; reduce < 2; ++reduce)
+    for (int idx = 4; idx <= 8; idx += 4) {
+      oracle_spmm_csr(rp64.p, col64.p, val.p, wide.p, M, K, reduce, want.p);
+      for (int64_t i = 0; i < M * ldo; ++i) out[i] = -777.f;
+      const int rc = exact_spmm_csr_strided_f16(idx == 8 ? (const void*)rp64.p : rp32.p, idx == 8 ? (const void*)col64.p : col32.p, val.p, idx,
+                                                (const uint16_t*)X.p, ldx, M, ncols, K, nnz, reduce, out.p, ldo, nullptr);
+      CHECK(rc == 0, "spmm f16 rc=%d", rc);
+      double worst = 0, scale = 1e-30;
+      int64_t spilt = 0;
+      for (int64_t i = 0; i < M * K; ++i) scale = std::max(scale, (double)std::fabs(want[i]));
+      for (int64_t r = 0; r < M; ++r)
+        for (int64_t k = 0; k < ldo; ++k)
+          if (k < K) worst = std::max(worst, (double)std::fabs(out[r * ldo + k] - want[r * K + k]));
+          else spilt += out[r * ldo + k] != -777.f;
+      CHECK(worst <= 1e-5 * scale && spilt == 0, "spmm f16 M=%ld K=%ld pad=%ld reduce=%d idx=%d: %g of %g, %ld", (long)M, (long)K, (long)pad, reduce,
+            idx, worst, scale, (long)spilt);
+    }
 }
 
 // mode 0: the fp32 instruction; EXACT_RP_BF16_SPLIT on a Gaussian matrix; EXACT_RP_BF16_SIGNS on a +-c matrix
@@ -538,6 +572,72 @@ static void check_dw(int64_t N, int64_t K, int64_t D, int64_t pad, std::mt19937&
   }
 }
 
+// Batch norm: statistics, normalisation and the backward from the packed input, against double sums; `shift` floats off
+// a 16-byte boundary the statistics take their one-column form.
+static void check_batch_norm(int64_t N, int64_t K, int bits, bool masked, int64_t shift, std::mt19937& rng) {
+  std::normal_distribution<float> nd(3.f, 2.f);
+  std::uniform_real_distribution<float> ud(0.f, 1.f);
+  const int64_t n = N * K;
+  Buf<float> store(n + shift), y(n), w(K), b(K), rm(K), rv(K), mean(K), inv(K), mult(K);
+  float* x = store.p + shift;
+  for (int64_t i = 0; i < n; ++i) x[i] = nd(rng);
+  for (int64_t k = 0; k < K; ++k) { w[k] = 0.5f + ud(rng); b[k] = ud(rng); rm[k] = ud(rng); rv[k] = ud(rng); }
+  std::vector<double> m64(K, 0.0), v64(K, 0.0), rm64(rm.p, rm.p + K), rv64(rv.p, rv.p + K);
+  for (int64_t i = 0; i < n; ++i) m64[i % K] += x[i] / (double)N;
+  for (int64_t i = 0; i < n; ++i) v64[i % K] += (x[i] - m64[i % K]) * (x[i] - m64[i % K]) / N;
+  const int64_t floats = exact_bn_work_floats(N, K);
+  CHECK(floats > 0, "bn work size");
+  Buf<float> work(floats);
+  CHECK(exact_bn_statistics_f32(x, N, K, 1e-5f, 0.25f, w.p, rm.p, rv.p, work.p, mean.p, inv.p, mult.p, nullptr) == 0, "bn statistics rc");
+  CHECK(exact_bn_apply_f32(x, mean.p, mult.p, b.p, N, K, y.p, nullptr) == 0, "bn apply rc");
+  double worst = 0;
+  for (int64_t k = 0; k < K; ++k) {
+    const double want = 1 / std::sqrt(v64[k] + 1e-5), unbiased = v64[k] * N / (N > 1 ? N - 1 : 1);
+    worst = std::max({worst, std::fabs(mean[k] - m64[k]), std::fabs(inv[k] / want - 1), std::fabs(mult[k] / (want * w[k]) - 1),
+                      std::fabs(rm[k] - (0.75 * rm64[k] + 0.25 * m64[k])), std::fabs(rv[k] - (0.75 * rv64[k] + 0.25 * unbiased)) / (1 + unbiased)});
+  }
+  for (int64_t i = 0; i < n; ++i) worst = std::max(worst, std::fabs(y[i] - ((x[i] - (double)mean[i % K]) * mult[i % K] + b[i % K])) / 100);
+  CHECK(worst < 3e-6, "bn N=%ld K=%ld: %g", (long)N, (long)K, worst);
+  if (K % 4 != 0) return;
+  const int64_t nb = exact_packed_nbytes(N, K, bits);
+  Buf<uint8_t> packed(nb);
+  Buf<uint16_t> sc(N), mn(N);
+  Buf<float> sc32(N), mn32(N), hat(n), dy(n), dx(n), sums(2 * K), gw(K);
+  Buf<uint32_t> mask((n + 31) / 32);
+  for (int64_t i = 0; i < n; ++i) dy[i] = nd(rng) - 3.f;
+  for (int64_t i = 0; i < (n + 31) / 32; ++i) mask[i] = rng();
+  Buf<float> base(n);
+  std::memcpy(base.p, x, n * 4);
+  CHECK(exact_minmax_pack_f32(base.p, nullptr, 1, 2, N, K, bits, packed.p, sc32.p, mn32.p, sc.p, mn.p, nullptr) == 0, "bn pack rc");
+  for (int64_t i = 0; i < N; ++i) {
+    const uint32_t a = (uint32_t)sc[i] << 16, c = (uint32_t)mn[i] << 16;
+    std::memcpy(&sc32[i], &a, 4);
+    std::memcpy(&mn32[i], &c, 4);
+  }
+  oracle_unpack(packed.p, bits, sc32.p, mn32.p, N, K, hat.p);
+  const float p = masked ? 0.25f : 0.f;
+  const int rc = exact_bn_backward_ordered_f32(dy.p, masked ? mask.p : nullptr, p, packed.p, bits, sc.p, mn.p, mean.p, inv.p, w.p, N, K, work.p,
+                                               sums.p, dx.p, gw.p, nullptr);
+  CHECK(rc == 0, "bn backward rc %d", rc);
+  std::vector<double> s0(K, 0.0), s1(K, 0.0), size(K, 1e-30);
+  auto grad = [&](int64_t i) { return masked ? ((mask[i >> 5] >> (i & 31)) & 1u ? dy[i] / (1.0 - p) : 0.0) : (double)dy[i]; };
+  for (int64_t i = 0; i < n; ++i) {
+    s0[i % K] += grad(i);
+    s1[i % K] += grad(i) * (hat[i] - (double)mean[i % K]);
+    size[i % K] += std::fabs(grad(i)) * (1 + std::fabs(hat[i] - (double)mean[i % K]));
+  }
+  worst = 0;
+  for (int64_t k = 0; k < K; ++k)
+    worst = std::max({worst, std::fabs(sums[k] - s0[k]) / size[k], std::fabs(sums[K + k] - s1[k]) / size[k],
+                      std::fabs(gw[k] - s1[k] * inv[k]) / (size[k] * inv[k])});
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t k = i % K;
+    const double want = (grad(i) - s0[k] / N - (hat[i] - (double)mean[k]) * inv[k] * inv[k] * s1[k] / N) * inv[k] * w[k];
+    worst = std::max(worst, std::fabs(dx[i] - want) / 100);
+  }
+  CHECK(worst < 2e-6, "bn backward N=%ld K=%ld bits=%d: %g", (long)N, (long)K, bits, worst);
+}
+
 // The fp16 form: small integers, so the fp32 sums are exact; one rounding to fp16.
 static void check_dw_half(int64_t N, int64_t K, int64_t D, int64_t pad, std::mt19937& rng) {
   std::uniform_int_distribution<int> id(-3, 3);
@@ -677,6 +777,13 @@ int main(int argc, char** argv) {
     std::printf("gemm shapes ok (failures so far %d)\n", g_fail);
     return g_fail != 0;
   }
+  if (mode == "bn") {  // the batch-norm kernels only
+    for (int bits : {1, 2, 4, 8}) check_batch_norm(1027, 100, bits, bits != 2, 0, rng);
+    check_batch_norm(9001, 8, 2, true, 0, rng);
+    check_batch_norm(5003, 7, 2, true, 1, rng);
+    std::printf("batch norm ok (failures so far %d)\n", g_fail);
+    return g_fail != 0;
+  }
   if (mode == "dw") {  // the weight-gradient kernels only
     check_dw(1, 1, 1, 0, rng);
     check_dw(7, 3, 5, 2, rng);
@@ -707,6 +814,13 @@ int main(int argc, char** argv) {
   check_spmm(90, 90, 47, 4, 80, rng);
   check_spmm(130, 130, 6, 30, 120, rng);
   check_spmm(4, 9, 8, 0, 0, rng);
+  check_spmm_half(300, 300, 256, 0, 8, 200, rng);
+  check_spmm_half(200, 200, 40, 1, 5, 0, rng);
+  check_spmm_half(100, 100, 602, 2, 10, 90, rng);
+  check_spmm_half(90, 90, 47, 0, 4, 80, rng);
+  check_spmm_half(130, 130, 132, 4, 30, 120, rng);
+  check_spmm_half(70, 40, 1, 0, 3, 0, rng);
+  check_spmm_half(4, 9, 8, 0, 0, 0, rng);
   std::printf("spmm shapes ok (failures so far %d)\n", g_fail);
   for (auto& s : kRpShapes) check_rp(s[0], s[1], s[2], rng);
   std::printf("rp shapes ok (failures so far %d)\n", g_fail);
@@ -731,6 +845,10 @@ int main(int argc, char** argv) {
   const int64_t cs[][2] = {{1, 1}, {3, 5}, {7, 47}, {1000, 41}, {4099, 47}, {513, 256}, {33, 602}, {5, 8192}, {20000, 3}};
   for (auto& c : cs) check_colsum(c[0], c[1], rng);
   std::printf("column sums ok (failures so far %d)\n", g_fail);
+  const int64_t bs[][3] = {{1, 4, 0}, {7, 3, 0}, {1027, 100, 0}, {1500, 257, 0}, {400, 1028, 0}, {300, 1100, 1}, {9001, 8, 0}, {5003, 12, 3}, {65, 4, 0}};
+  for (auto& b : bs)
+    for (int bits : {1, 2, 4, 8}) check_batch_norm(b[0], b[1], bits, bits != 2, b[2], rng);
+  std::printf("batch norm ok (failures so far %d)\n", g_fail);
   for (int64_t n : {100, 4096, 3 * 4096 + 77, 20 * 4096}) check_probe(n, rng);
   std::printf("traffic probe ok (failures so far %d)\n", g_fail);
   const int64_t ds[][4] = {{1, 1, 1, 0}, {7, 3, 5, 1}, {100, 40, 256, 0}, {515, 256, 128, 3}, {333, 47, 25, 0}, {1201, 256, 76, 2},

@@ -1,4 +1,4 @@
-"""exact_tall_gemm_bf16_f32 at the edges of its column slabs, k-steps and row
+"""exact_tall_product_f32 at the edges of its column slabs, k-steps and row
 blocks, with every epilogue, and exact_rp_bwd_bf16_f32 at row widths that are no
 multiple of four: against float64.  An element is the sum of six bf16 products
 per feature in fp32, in whatever order the accumulator takes them: at most
