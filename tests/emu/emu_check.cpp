@@ -632,8 +632,9 @@ static void check_batch_norm(int64_t N, int64_t K, int bits, bool masked, int64_
                       std::fabs(gw[k] - s1[k] * inv[k]) / (size[k] * inv[k])});
   for (int64_t i = 0; i < n; ++i) {
     const int64_t k = i % K;
-    const double want = (grad(i) - s0[k] / N - (hat[i] - (double)mean[k]) * inv[k] * inv[k] * s1[k] / N) * inv[k] * w[k];
-    worst = std::max(worst, std::fabs(dx[i] - want) / 100);
+    const double pull = (hat[i] - (double)mean[k]) * inv[k] * inv[k] * s1[k] / N, want = (grad(i) - s0[k] / N - pull) * inv[k] * w[k];
+    const double size_i = (1 + std::fabs(grad(i)) + std::fabs(s0[k] / N) + std::fabs(pull)) * inv[k] * w[k];  // of the terms: one row leaves var 0
+    worst = std::max(worst, std::fabs(dx[i] - want) / size_i);
   }
   CHECK(worst < 2e-6, "bn backward N=%ld K=%ld bits=%d: %g", (long)N, (long)K, bits, worst);
 }
@@ -779,6 +780,9 @@ int main(int argc, char** argv) {
   }
   if (mode == "bn") {  // the batch-norm kernels only
     for (int bits : {1, 2, 4, 8}) check_batch_norm(1027, 100, bits, bits != 2, 0, rng);
+    check_batch_norm(1, 4, 2, false, 0, rng);
+    check_batch_norm(400, 1028, 8, true, 0, rng);
+    check_batch_norm(300, 1100, 1, true, 1, rng);
     check_batch_norm(9001, 8, 2, true, 0, rng);
     check_batch_norm(5003, 7, 2, true, 1, rng);
     std::printf("batch norm ok (failures so far %d)\n", g_fail);
