@@ -36,6 +36,8 @@
 // (col, h) holding R[32 tile + col][16 step + 8 h + i].  SIGNS: one piece (the
 // signs as +-1 in bf16); SPLIT: three (hi, mid, lo).  Padding entries are 0.
 
+#include <type_traits>
+
 #include "bf16_split.hpp"
 #include "rp_common.hpp"
 
@@ -133,66 +135,157 @@ __global__ __launch_bounds__(kBlock) void rp_prepare_kernel(const float* __restr
 }
 
 // ---- forward -----------------------------------------------------------------
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One wavefront per 32 rows, one wavefront per workgroup: no workgroup barrier
-// anywhere.  The wavefront walks the D features in k-steps of 16, the loads of
-// KS steps issued together (two 16-byte loads per lane and step, the steps'
-// table fragments beside them), and accumulates in step order.  (A workgroup of
-// four wavefronts that split the features and met in LDS was measured against
-// this form: equal at 256 -> 32, 15 % slower at 256 -> 64.)
-// `frags` holds `tiles` column tiles per k-step; the wavefront multiplies by the NT tiles from `tile0` on.
-template <int VEC, int NT, int BP, int KS>
+// anywhere.  The wavefront walks the D features in chunks of 64 (four k-steps).  The instruction wants a lane to hold
+// eight features of one row, but loads in that arrangement touch 64 pieces of 16 bytes in 32 rows and ran at 3 TB/s
+// (190 us at 602 -> 76 columns of 232,965 rows).  So 16 lanes read 256 consecutive bytes of a row, the chunk passes
+// through a tile in LDS that belongs to the wavefront (its accesses complete in order), and the lanes read their
+// features from there; the next chunk's loads fly while this one is multiplied.  Before -> after, with the quantiser:
+// 602 -> 76 of 232,965 rows 190 -> 153 us, 301 -> 38 of 100,000 52 -> 35, 100 -> 25 of 2.4 M 268 -> 223, 256 -> 64 of
+// 2.4 M 591 -> 525, 256 -> 32 of 169,343 38.6 -> 36.4.  At 602 -> 76 the loads and the hand-over alone take 120 us (a
+// kernel that only reads in 256-byte runs 98), the split and the products the rest.  Four wavefronts that share the
+// fragments through LDS: 148 us there, but 28 instead of 22 at 20,000 rows, whose workgroups then miss half the chip;
+// two chunks in flight: 166.
+// `frags` holds NT column tiles per k-step.  A feature past the row is zero.
+constexpr int kChunkSteps = 4, kChunk = kChunkSteps * kStepFeatures;
+constexpr int kChunkPitch = kChunk + 4;  // floats: 16-byte aligned rows; 16 lanes on 16 rows meet 64 different banks
+constexpr int kChunkFloats = kTile * kChunkPitch;
+
+// How many of the four columns from `col` on a load that has to stay inside a row of D >= 4 columns starts too early.
+__device__ __forceinline__ int early_by(int col, int D) { return col > D - 4 ? col - (D - 4) : 0; }
+// What such a load brought -> the four columns, zeros past the row.
+__device__ __forceinline__ f32x4 shifted_by(f32x4 v, int early) {
+  f32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x = 0.f;
+#pragma unroll
+    for (int j = 3; j >= e; --j) x = early == j - e ? v[j] : x;
+    r[e] = x;
+  }
+  return r;
+}
+
+template <int NT, int BP>
 __device__ __forceinline__ void rp_fwd_rows(const float* __restrict__ X, const u32x4* __restrict__ frags, int64_t N,
-                                            int D, int64_t row0, floatx16 (&acc)[NT], int tiles = NT, int tile0 = 0) {
+                                            int D, int64_t row0, float* chunk, floatx16 (&acc)[NT]) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int half = lane >> 5;
-  const int64_t my_row = (row0 + (lane & 31) < N) ? row0 + (lane & 31) : N - 1;
-  const float* xrow = X + my_row * D;
+  const int half = lane >> 5, l32 = lane & 31, q = lane & 15;
   const int total = (D + kStepFeatures - 1) / kStepFeatures;
+  const int last = N - row0 < kTile ? static_cast<int>(N - row0) - 1 : kTile - 1;
+  const float* xtile = X + row0 * D;
 
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[nt][v] = 0.f;
 
-  for (int s0 = 0; s0 < total; s0 += KS) {
-    float a[KS][8];
-    if ((s0 + KS) * kStepFeatures <= D) {  // wave-uniform: the KS steps lie inside the row, nothing to mask
+  if (D < 4) {  // less than a piece a row
+    float a[8];
+    load8<1>(xtile + static_cast<int64_t>(min(l32, last)) * D, 8 * half, D, a);
+    const Split8 pieces = split3x8(a);
 #pragma unroll
-      for (int sb = 0; sb < KS; ++sb) load8_inside(xrow + (s0 + sb) * kStepFeatures + 8 * half, a[sb]);
-    } else {
+    for (int nt = 0; nt < NT; ++nt) {
+      u32x4 b[BP];
 #pragma unroll
-      for (int sb = 0; sb < KS; ++sb) load8<VEC>(xrow, (s0 + sb) * kStepFeatures + 8 * half, D, a[sb]);  // zeros past the row
+      for (int p = 0; p < BP; ++p) b[p] = frags[(nt * BP + p) * kWave + lane];
+      acc[nt] = step_product<BP>(pieces, b, acc[nt]);
     }
-#pragma unroll
-    for (int sb = 0; sb < KS; ++sb) {
-      const int st = (s0 + sb < total) ? s0 + sb : s0;  // a step past the row meets zeros: any valid fragment will do
-      const Split8 pieces = split3x8(a[sb]);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const u32x4* src = frags + (static_cast<int64_t>(st) * tiles + tile0 + nt) * BP * kWave + lane;
-        u32x4 b[BP];
-#pragma unroll
-        for (int p = 0; p < BP; ++p) b[p] = src[p * kWave];
-        acc[nt] = step_product<BP>(pieces, b, acc[nt]);
-      }
-    }
+    return;
   }
+  uint32_t at[8];  // bytes from the tile's first row to feature 4 q of rows lane / 16 + 4 i; D <= 2^20
+#pragma unroll
+  for (int i = 0; i < 8; ++i) at[i] = 4u * (static_cast<uint32_t>(min((lane >> 4) + 4 * i, last)) * static_cast<uint32_t>(D) + 4u * q);
+  f32x4 ahead[8];
+  auto load_inside = [&](int s0) {
+    const char* base = reinterpret_cast<const char*>(xtile + s0 * kStepFeatures);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ahead[i] = *reinterpret_cast<const f32x4_any*>(base + at[i]);
+  };
+  auto load_tail = [&](int s0) {  // from the tile's start: less than four columns may be left, and then a piece starts before the chunk
+    const char* base = reinterpret_cast<const char*>(xtile);
+    const uint32_t shift = 4u * (s0 * kStepFeatures - early_by(s0 * kStepFeatures + 4 * q, D));  // at[] + shift is no less than 0 (mod 2^32)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ahead[i] = *reinterpret_cast<const f32x4_any*>(base + (at[i] + shift));
+  };
+  float* const park = chunk + (lane >> 4) * kChunkPitch + 4 * q;
+  const float* const mine = chunk + l32 * kChunkPitch + 8 * half;
+  // The chunk in `ahead`, from step s0 on.  NEXT: what follows -- 0 nothing, 1 a chunk inside the row, 2 the row's tail.
+  auto multiply_chunk = [&](int s0, auto next) {
+    constexpr int NEXT = decltype(next)::value;
+    auto load_next = [&]() {
+      if constexpr (NEXT == 1) load_inside(s0 + kChunkSteps);
+      if constexpr (NEXT == 2) load_tail(s0 + kChunkSteps);
+    };
+    if (NEXT == 0 && (s0 + kChunkSteps) * kStepFeatures > D) {  // the row's tail, as load_tail brought it
+      const int early = early_by(s0 * kStepFeatures + 4 * q, D);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ahead[i] = shifted_by(ahead[i], early);
+    }
+    wave_sync_lds();  // the previous chunk has been read
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(park + 4 * i * kChunkPitch) = ahead[i];
+    // Loads return in order.  The fragments of a sign matrix are few enough to be asked for before the next rows; those
+    // of a split one are not, and the rows wait for them instead.
+    u32x4 b[BP == 1 ? kChunkSteps : 1][NT * BP];
+    auto load_frags = [&](int st, u32x4 (&f)[NT * BP]) {
+      const u32x4* src = frags + static_cast<int64_t>(min(st, total - 1)) * NT * BP * kWave + lane;  // a step past the row meets zeros
+#pragma unroll
+      for (int p = 0; p < NT * BP; ++p) f[p] = src[p * kWave];
+    };
+    if constexpr (BP == 1) {
+#pragma unroll
+      for (int sb = 0; sb < kChunkSteps; ++sb) load_frags(s0 + sb, b[sb]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_next();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wave_sync_lds();
+#pragma unroll
+    for (int sb = 0; sb < kChunkSteps; ++sb) {
+      if (NEXT == 0 && s0 + sb >= total) break;  // wave-uniform
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(mine + sb * kStepFeatures);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(mine + sb * kStepFeatures + 4);
+      const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (BP != 1) load_frags(s0 + sb, b[0]);
+      const Split8 pieces = split3x8(a);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = step_product<BP>(pieces, b[BP == 1 ? sb : 0] + nt * BP, acc[nt]);
+    }
+    if constexpr (BP != 1) load_next();
+  };
+  if (kChunk <= D) load_inside(0);
+  else load_tail(0);
+  int s0 = 0;
+#pragma unroll 1
+  for (; (s0 + 2 * kChunkSteps) * kStepFeatures <= D; s0 += kChunkSteps) multiply_chunk(s0, std::integral_constant<int, 1>{});
+  if (s0 + kChunkSteps < total) {
+    multiply_chunk(s0, std::integral_constant<int, 2>{});
+    s0 += kChunkSteps;
+  }
+  multiply_chunk(s0, std::integral_constant<int, 0>{});
 }
 
-// k-steps in flight: four with one column tile (more wavefronts per SIMD do better than more loads per
-// wavefront), eight with several (measured at 256 -> 32 and 256 -> 64)
+// Wavefronts a SIMD that the registers have to leave room for (LDS holds three with three tiles, four with fewer).
 template <int NT>
-constexpr int fwd_steps_in_flight() { return NT == 1 ? 4 : 8; }
+constexpr int fwd_waves() { return NT == 1 ? 4 : NT < 4 ? 3 : 2; }
 
-template <int VEC, int NT, int BP>
-__global__ __launch_bounds__(kWave) void rp_fwd_bf16_kernel(const float* __restrict__ X,
+template <int NT, int BP>
+__global__ __launch_bounds__(kWave, fwd_waves<NT>()) void rp_fwd_bf16_kernel(const float* __restrict__ X,
                                                             const u32x4* __restrict__ table, int64_t N, int D,
                                                             int k, float* __restrict__ out) {
+  HIP_DYNAMIC_SHARED(float, chunk)  // [32][kChunkPitch]
   const int lane = threadIdx.x & (kWave - 1);
   const int half = lane >> 5, l32 = lane & 31;
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kTile;
   floatx16 acc[NT];
-  rp_fwd_rows<VEC, NT, BP, fwd_steps_in_flight<NT>()>(X, table + 1, N, D, row0, acc);
+  rp_fwd_rows<NT, BP>(X, table + 1, N, D, row0, chunk, acc);
   const float c = BP == 1 ? __uint_as_float(table[0][0]) : 1.f;
   // accumulator register v of lane l is C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32]: a store instruction writes two
   // rows of 32 consecutive columns
@@ -204,12 +297,6 @@ __global__ __launch_bounds__(kWave) void rp_fwd_bf16_kernel(const float* __restr
       const int col = nt * kTile + l32;
       if (n < N && col < k) __builtin_nontemporal_store(BP == 1 ? acc[nt][v] * c : acc[nt][v], out + n * k + col);
     }
-}
-
-__device__ __forceinline__ void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Projection and quantisation in one launch.  The wavefront turns its finished
@@ -230,18 +317,21 @@ constexpr int kStagePitch = 16;  // octs per row in the hand-over array: k <= 12
 template <int NT>
 constexpr int fwd_tile_pitch() { return NT * kTile + 4; }  // floats per tile row: 16-byte aligned rows, rows 4 apart on other banks
 
-template <int VEC, int NT, int BP, bool NOISE_IN>
-__global__ __launch_bounds__(kWave) void rp_fwd_pack_bf16_kernel(const RpPackArgs a, const u32x4* __restrict__ table) {
-  HIP_DYNAMIC_SHARED(float, tile)  // [32][pitch] floats, then uint64 [32][kStagePitch]
+template <int NT, int BP, bool NOISE_IN>
+__global__ __launch_bounds__(kWave, fwd_waves<NT>()) void rp_fwd_pack_bf16_kernel(const RpPackArgs a, const u32x4* __restrict__ table) {
+  // One after the other in the same bytes: the chunks of X, the tile of sums [32][pitch], the codes uint64 [32][kStagePitch].
+  // Each is whole in registers before the next is written, and LDS is what bounds the wavefronts in flight.
+  HIP_DYNAMIC_SHARED(float, tile)
   constexpr int PITCH = fwd_tile_pitch<NT>();
   // passes of the 64 lanes over the tile's (row, oct) pairs: 32 rows x (1, 2 or 4 | 8 | 16) lanes per row
   constexpr int PASSES = NT == 1 ? 2 : (NT == 2 ? 4 : 8);
-  uint64_t* stage = reinterpret_cast<uint64_t*>(tile + kTile * PITCH);
+  uint64_t* stage = reinterpret_cast<uint64_t*>(tile);
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kTile;
   {
     floatx16 acc[NT];
-    rp_fwd_rows<VEC, NT, BP, fwd_steps_in_flight<NT>()>(a.X, table + 1, a.N, a.D, row0, acc);
+    rp_fwd_rows<NT, BP>(a.X, table + 1, a.N, a.D, row0, tile, acc);
+    wave_sync_lds();  // the last chunk has been read
     const float c = BP == 1 ? __uint_as_float(table[0][0]) : 1.f;
     const int half = lane >> 5, l32 = lane & 31;
 #pragma unroll
@@ -325,6 +415,7 @@ __global__ __launch_bounds__(kWave) void rp_fwd_pack_bf16_kernel(const RpPackArg
     word[1] = ((low_bytes4(q[4], q[5], q[6], q[7]) & keep) << shift) & static_cast<uint32_t>(valid >> 32);
     parked[pass] = static_cast<uint64_t>(word[0]) | (static_cast<uint64_t>(word[1]) << 32);
   }
+  wave_sync_lds();  // the sums have been read
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
     const int t = pass * kWave + lane;
@@ -843,29 +934,33 @@ __global__ __launch_bounds__(kBlock) void rp_bwd_bf16_kernel(const float* __rest
 
 // ---- launches ----------------------------------------------------------------
 template <int NT>
-constexpr size_t fwd_pack_lds_bytes() { return sizeof(float) * kTile * fwd_tile_pitch<NT>() + sizeof(uint64_t) * kTile * kStagePitch; }
+constexpr size_t fwd_pack_lds_bytes() {
+  constexpr size_t chunk = sizeof(float) * kChunkFloats, sums = sizeof(float) * kTile * fwd_tile_pitch<NT>();
+  static_assert(sizeof(uint64_t) * kTile * kStagePitch <= chunk, "the codes fit where a chunk was");
+  return chunk > sums ? chunk : sums;
+}
 
-template <int VEC, int BP>
+template <int BP>
 static int rp_fwd_bf16_launch(const float* X, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((N + kTile - 1) / kTile)), block(kWave);
   switch ((k + kTile - 1) / kTile) {
-    case 1: hipLaunchKernelGGL((rp_fwd_bf16_kernel<VEC, 1, BP>), grid, block, 0, s, X, table, N, D, k, out); break;
-    case 2: hipLaunchKernelGGL((rp_fwd_bf16_kernel<VEC, 2, BP>), grid, block, 0, s, X, table, N, D, k, out); break;
-    case 3: hipLaunchKernelGGL((rp_fwd_bf16_kernel<VEC, 3, BP>), grid, block, 0, s, X, table, N, D, k, out); break;
-    case 4: hipLaunchKernelGGL((rp_fwd_bf16_kernel<VEC, 4, BP>), grid, block, 0, s, X, table, N, D, k, out); break;
+    case 1: hipLaunchKernelGGL((rp_fwd_bf16_kernel<1, BP>), grid, block, sizeof(float) * kChunkFloats, s, X, table, N, D, k, out); break;
+    case 2: hipLaunchKernelGGL((rp_fwd_bf16_kernel<2, BP>), grid, block, sizeof(float) * kChunkFloats, s, X, table, N, D, k, out); break;
+    case 3: hipLaunchKernelGGL((rp_fwd_bf16_kernel<3, BP>), grid, block, sizeof(float) * kChunkFloats, s, X, table, N, D, k, out); break;
+    case 4: hipLaunchKernelGGL((rp_fwd_bf16_kernel<4, BP>), grid, block, sizeof(float) * kChunkFloats, s, X, table, N, D, k, out); break;
     default: return EXACT_E_SHAPE;
   }
   return launch_status();
 }
 
-template <int VEC, int BP, bool NOISE_IN>
+template <int BP, bool NOISE_IN>
 static int rp_fwd_pack_bf16_launch(const RpPackArgs& a, const u32x4* table, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((a.N + kTile - 1) / kTile)), block(kWave);
   switch ((a.k + kTile - 1) / kTile) {
-    case 1: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<VEC, 1, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<1>(), s, a, table); break;
-    case 2: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<VEC, 2, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<2>(), s, a, table); break;
-    case 3: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<VEC, 3, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<3>(), s, a, table); break;
-    case 4: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<VEC, 4, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<4>(), s, a, table); break;
+    case 1: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<1, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<1>(), s, a, table); break;
+    case 2: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<2, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<2>(), s, a, table); break;
+    case 3: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<3, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<3>(), s, a, table); break;
+    case 4: hipLaunchKernelGGL((rp_fwd_pack_bf16_kernel<4, BP, NOISE_IN>), grid, block, fwd_pack_lds_bytes<4>(), s, a, table); break;
     default: return EXACT_E_SHAPE;
   }
   return launch_status();
@@ -974,12 +1069,7 @@ int exact_rp_fwd_bf16_f32(const float* X, const void* table, int64_t N, int64_t 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const u32x4* t = static_cast<const u32x4*>(table);
   const int d = static_cast<int>(D), kk = static_cast<int>(k);
-#define EXACT_RP_GO(V) \
-  (mode == EXACT_RP_BF16_SIGNS ? rp_fwd_bf16_launch<V, 1>(X, t, N, d, kk, out, s) : rp_fwd_bf16_launch<V, 3>(X, t, N, d, kk, out, s))
-  if (D % 4 == 0 && al16(X)) return EXACT_RP_GO(4);
-  if (D % 2 == 0 && al8(X)) return EXACT_RP_GO(2);
-  return EXACT_RP_GO(1);
-#undef EXACT_RP_GO
+  return mode == EXACT_RP_BF16_SIGNS ? rp_fwd_bf16_launch<1>(X, t, N, d, kk, out, s) : rp_fwd_bf16_launch<3>(X, t, N, d, kk, out, s);
 }
 
 int exact_rp_minmax_pack_bf16_f32(const float* X, const void* table, int mode, const float* noise, uint64_t seed,
@@ -1016,12 +1106,8 @@ int exact_rp_minmax_pack_bf16_f32(const float* X, const void* table, int mode, c
   a.min_f32 = min_f32;
   a.scale_bf16 = scale_bf16;
   a.min_bf16 = min_bf16;
-#define EXACT_RP_GO(V, NOISE) \
-  (mode == EXACT_RP_BF16_SIGNS ? rp_fwd_pack_bf16_launch<V, 1, NOISE>(a, t, s) : rp_fwd_pack_bf16_launch<V, 3, NOISE>(a, t, s))
-  if (D % 4 == 0 && al16(X)) return noise ? EXACT_RP_GO(4, true) : EXACT_RP_GO(4, false);
-  if (D % 2 == 0 && al8(X)) return noise ? EXACT_RP_GO(2, true) : EXACT_RP_GO(2, false);
-  return noise ? EXACT_RP_GO(1, true) : EXACT_RP_GO(1, false);
-#undef EXACT_RP_GO
+  if (mode == EXACT_RP_BF16_SIGNS) return noise ? rp_fwd_pack_bf16_launch<1, true>(a, t, s) : rp_fwd_pack_bf16_launch<1, false>(a, t, s);
+  return noise ? rp_fwd_pack_bf16_launch<3, true>(a, t, s) : rp_fwd_pack_bf16_launch<3, false>(a, t, s);
 }
 
 int exact_rp_bwd_bf16_f32(const float* Xr, const void* table, int64_t N, int64_t D, int64_t k, int mode, float* out,

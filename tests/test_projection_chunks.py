@@ -1,0 +1,36 @@
+"""The projection kernels at the edges of their 64-feature chunks, 16-feature
+steps, 4-feature pieces, column tiles and row tiles, on any matrix and on a sign
+matrix, with and without the quantiser.  A sum of D fp32 products of which each
+is three or six bf16 products in fp32 is wrong by at most 2^-24 of the absolute
+terms per addition, 6 D of them, and one rounding per term for what is left out."""
+import pytest
+import torch
+
+from exact_amd import ops
+from exact_amd.conf import config
+from exact_amd.cpp_extension import quantization as extq
+
+
+@pytest.mark.parametrize("signs", [False, True])
+@pytest.mark.parametrize("k", [7, 40, 76, 128])                        # one to four column tiles
+@pytest.mark.parametrize("N,D", [(1, 1), (33, 3), (31, 4), (32, 5), (65, 63), (40, 64), (33, 65), (32, 66), (1, 67), (64, 127),
+                                 (33, 128), (31, 129), (70, 130), (2, 131), (33, 133), (32, 197), (5, 258)])
+def test_projection(backend, N, D, k, signs):
+    g = torch.Generator().manual_seed(1000 * N + D + k)
+    x = torch.randn(N, D, generator=g).to(backend)
+    matrix = (2.0 * torch.randint(2, (D, k), generator=g) - 1) / k ** 0.5 if signs else torch.randn(D, k, generator=g)
+    matrix = matrix.to(backend)
+    if signs:
+        matrix._exact_sign_matrix = True
+
+    def source(*_):
+        return matrix
+    config.rp_matrix_source = source
+    reduced, used = ops.input2rp(x, k)
+    want = x.double() @ matrix.double()
+    bound = (7 * D + 2) * 2.0 ** -24 * (x.double().abs() @ matrix.double().abs()) + 1e-30
+    assert reduced.shape == (N, k) and ((reduced.double() - want).abs() <= bound).all()
+    # the fused launch quantises exactly these sums
+    config.noise_source = lambda shape, device: torch.full(shape, 0.25).to(device)
+    for one, two in zip(extq.rp_minmax_pack(x, used, 2), extq.minmax_pack(reduced, 2)):
+        assert torch.equal(one, two)
