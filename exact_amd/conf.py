@@ -50,7 +50,8 @@ _EXTRA_FIELDS = {
     # reproduce that memory behaviour.  Results do not depend on it.
     "keep_unused_spmm_operand": False,
     # ReLU -> dropout -> (quantise for the next layer) as one pass where the
-    # model offers the pair as one module (QReLUDropout).  Results are
+    # model offers the pair as one module (QReLUDropout) or the layers stand in
+    # a QMLP.  Results are
     # bit-identical to the separate layers; False runs them separately.
     "fuse_epilogue": True,
     # A QBatchNorm1d ahead of that pair joins the same pass (normalise -> ReLU ->

@@ -1,0 +1,75 @@
+"""QMLP runs (batch norm ->) ReLU -> dropout ahead of a linear layer in one pass:
+against the same layers called one by one."""
+import pytest
+import torch
+
+import exact_amd as exact
+from exact_amd import layers
+from exact_amd.conf import config
+from gpu_util import SeededNoise
+
+
+def _step(backend, net, x, gy, one_pass, before=None):
+    config.fuse_epilogue = one_pass
+    noise = SeededNoise(5)
+    config.noise_source = noise.noise_source
+    net = net().to(backend).train()
+    if before is not None:
+        before(net)
+    x = x.to(backend).requires_grad_()
+    y = net(x)
+    y.backward(gy.to(backend))
+    return [y.detach(), x.grad] + [p.grad for p in net.parameters()] + list(net.buffers())
+
+
+def _net(widths, norm, **kw):
+    torch.manual_seed(11)
+    return layers.QMLP(widths, norm, **kw)
+
+
+@pytest.mark.parametrize("norm", ["batch", None])
+@pytest.mark.parametrize("N,widths", [(2, [8, 8, 4]), (33, [16, 24, 40, 8]), (1100, [12, 64, 10]), (50, [20, 30, 16])])   # 30: no multiple of 8
+def test_one_pass_equals_the_layers(backend, N, widths, norm):
+    g = torch.Generator().manual_seed(N)
+    x, gy = torch.randn(N, widths[0], generator=g), torch.randn(N, widths[-1], generator=g)
+    make = lambda: _net(widths, norm, bias=norm is None, dropout=0.5)       # noqa: E731
+    for one, many in zip(_step(backend, make, x, gy, True), _step(backend, make, x, gy, False)):
+        # without a norm bit for bit; with one, its statistics are sums in another order: 1e-5 of the largest value, and
+        # a kept copy may round the other way where a value lies within that of a boundary (one level of 3 in a row)
+        if norm is None:
+            assert torch.equal(one, many)
+        else:
+            assert ((one - many).abs() <= 1e-4 * many.abs().max()).float().mean() > 0.98
+
+
+def test_what_hooks_and_other_layers_see_stays(backend, monkeypatch):
+    calls = []
+    real = layers.bn_relu_dropout
+    monkeypatch.setattr(layers, "bn_relu_dropout", lambda *a: calls.append(1) or real(*a))
+    g = torch.Generator().manual_seed(1)
+    x, gy = torch.randn(40, 16, generator=g), torch.randn(40, 8, generator=g)
+    make = lambda: _net([16, 16, 8], "batch", dropout=0.25)                 # noqa: E731
+    _step(backend, make, x, gy, True)
+    assert calls == [1]
+    seen = []
+
+    def hook(net):
+        net[2].register_forward_hook(lambda m, i, o: seen.append(o.shape))
+
+    def backward_hook(net):
+        net[3].register_full_backward_hook(lambda m, gi, go: seen.append(go[0].shape))
+
+    def frozen(net):
+        net[1].eval()
+
+    class Own(layers.QReLU):
+        pass
+
+    def own(net):
+        net[2] = Own()
+    for change, sights in ((hook, 1), (backward_hook, 2), (frozen, 2), (own, 2)):
+        _step(backend, make, x, gy, True, change)
+        assert calls == [1] and len(seen) == sights
+    config.kept_frac = 0.5                                                  # the next layer projects: no copy to make ahead
+    _step(backend, make, x, gy, True)
+    assert calls == [1]
