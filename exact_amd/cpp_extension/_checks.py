@@ -54,7 +54,9 @@ def suffix(t):
 
 
 def stream_ptr(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The handle of the current stream of t's device, as torch.cuda.current_stream(t.device).cuda_stream
+    gives it; without the Stream object in between, 0.2 instead of 4 us."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t):

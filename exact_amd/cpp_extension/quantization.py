@@ -8,6 +8,8 @@ and one call into libexact_hip.so on the current stream.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from .. import _lib
@@ -17,6 +19,7 @@ from . import _checks
 from ._checks import FLOAT_OR_HALF, check_device_tensor, ptr, suffix
 
 
+@functools.lru_cache(maxsize=1024)
 def packed_nbytes(N: int, G: int, bits: int) -> int:
     return int(_lib.lib().exact_packed_nbytes(N, G, bits))
 
