@@ -45,6 +45,7 @@ namespace exact {
 
 constexpr int kStepFeatures = 16;  // K of one MFMA
 constexpr int kRpXcds = 8;         // accelerator complex dies of an MI355X, each with its own L2
+constexpr int kRpCus = 256;        // compute units
 
 // Eight consecutive floats of a row starting at column `col`, zeros from column
 // `limit` on; VEC = the widest aligned access (limit % VEC == 0, col % VEC == 0).
@@ -932,6 +933,133 @@ __global__ __launch_bounds__(kBlock) void rp_bwd_bf16_kernel(const float* __rest
   }
 }
 
+// The same product with the reference's signs where rows of the result do not start on whole lines.  Above, a wavefront
+// writes pieces of 512 bytes of 32 rows: with rows of 2408 bytes each piece has two partial lines, and writing alone takes
+// 155 us at [232965, 602] where one run takes 104; and every slab loads and splits the rows of Xr anew.  Here a workgroup
+// takes 32 whole rows at a time -- one run of memory that starts on a line -- and goes on to the next 32: its four
+// wavefronts own TW column tiles each, whose fragments (KS steps at most) stay in registers throughout; the rows of Xr
+// come in one run, a tile ahead; and eight rows of the result at a time pass through LDS as they lie in memory (two
+// buffers, one barrier each).
+template <int TW, int KS>
+constexpr int bwd_rows_per_cu() {  // workgroups a compute unit, by registers
+  constexpr int regs = 16 * TW + 4 * TW * KS + 2 * KS + 36;
+  return regs <= 64 ? 8 : regs <= 80 ? 6 : regs <= 96 ? 5 : regs <= 128 ? 4 : regs <= 168 ? 3 : 2;
+}
+template <int TW, int KS>
+__global__ __launch_bounds__(kBlock, (bwd_rows_per_cu<TW, KS>())) void rp_bwd_rows_kernel(const float* __restrict__ Xr,
+                                                                                        const u32x4* __restrict__ table, int64_t N,
+                                                                                        int D, int k, float* __restrict__ out) {
+  HIP_DYNAMIC_SHARED(float, lds)  // [32][kPitch] of Xr, then two images of eight rows
+  constexpr int kPitch = KS * kStepFeatures + 4;  // 16-byte units: an odd number of them, 16 rows meet 64 different banks
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int half = lane >> 5, l32 = lane & 31;
+  const int64_t tiles_n = (N + kTile - 1) / kTile;
+  const TableShape ts = table_shape(D, k, 1);
+  float* image = lds + kTile * kPitch;
+  // fragments [step][tile][lane]; a tile past the last column is never stored, a step past k meets zeros: any will do
+  u32x4 b[KS][TW];
+#pragma unroll
+  for (int st = 0; st < KS; ++st)
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      b[st][j] = table[1 + ts.fwd_units() + (static_cast<int64_t>(min(st, ts.steps_k - 1)) * ts.tiles_d + min(wave * TW + j, ts.tiles_d - 1)) * kWave + lane];
+  const float c = __uint_as_float(table[0][0]);
+  for (int e = t; e < kTile * kPitch; e += kBlock) lds[e] = 0.f;  // features past k stay zeros
+
+  constexpr int kPerThread = kTile * KS * kStepFeatures / kBlock;  // of the at most 32 KS 16 features of a tile
+  const int drow = kBlock / k, dcol = kBlock - drow * k;
+  float x[kPerThread];
+  auto load_tile = [&](int64_t tile) {  // one run; zeros past the last row
+    const float* src = Xr + tile * kTile * k;
+    const int count = static_cast<int>(min<int64_t>(N - tile * kTile, kTile)) * k;
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      const int e = i * kBlock + t;
+      const float v = src[min(e, count - 1)];
+      x[i] = e < count ? v : 0.f;
+    }
+  };
+  auto park_tile = [&]() {
+    int row = t / k, col = t - row * k;
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      if (row < kTile) lds[row * kPitch + col] = x[i];
+      row += drow;
+      col += dcol;
+      if (col >= k) {
+        col -= k;
+        ++row;
+      }
+    }
+  };
+  // One tile; FULL: all its 32 rows are there.  A wait for loads waits for the stores issued ahead of them too, and where
+  // some stores may or may not have been issued the compiler has to wait for all: a full tile stores the same number
+  // from every lane, lanes past the end the last piece again (860 -> 654 us at 64 -> 256 of 2.4 M rows).
+  auto one_tile = [&](int64_t tile, int64_t next, auto whole) {
+    constexpr bool FULL = decltype(whole)::value;
+    park_tile();  // the tile before was last read ahead of the barrier of its first eight rows
+    __syncthreads();
+    load_tile(next);
+    floatx16 acc[TW];
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[j][v] = 0.f;
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+      const float* src = lds + l32 * kPitch + st * kStepFeatures + 8 * half;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
+      const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const Split8 pieces = split3x8(a);
+#pragma unroll
+      for (int j = 0; j < TW; ++j) acc[j] = step_product<1>(pieces, &b[st][j], acc[j]);
+    }
+    // Addresses of the epilogue, made anew for every tile: kept across tiles they take more registers than there are
+    // (480 us at 602 columns, of which 84 registers spilled).
+    int lane_at = 4 * half * D + wave * TW * kTile + l32, quad_at = 4 * t;
+    EXACT_VALUE_BARRIER(lane_at);
+    EXACT_VALUE_BARRIER(quad_at);
+    const int left = D - wave * TW * kTile - l32;  // columns from this lane's first on
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {  // rows 8 g .. 8 g + 7
+      float* eight = image + (g & 1) * 8 * D;  // last read before the barrier of the eight rows in between
+#pragma unroll
+      for (int j = 0; j < TW; ++j) {
+        if (j * kTile < left) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) eight[lane_at + r * D + j * kTile] = acc[j][4 * g + r] * c;
+        }
+      }
+      __syncthreads();
+      float* dst = out + (tile * kTile + 8 * g) * D;
+      constexpr int kQuads = (8 * 4 * kTile * TW / 4 + kBlock - 1) / kBlock;  // of a thread at most
+      f32x4 v[kQuads];
+#pragma unroll
+      for (int i = 0; i < kQuads; ++i) v[i] = *reinterpret_cast<const f32x4*>(eight + min(quad_at + 4 * i * kBlock, 8 * D - 4));
+      if constexpr (FULL) {
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) *reinterpret_cast<f32x4_any*>(dst + min(quad_at + 4 * i * kBlock, 8 * D - 4)) = v[i];
+      } else {
+        const int count = min(max(static_cast<int>(N - tile * kTile) - 8 * g, 0), 8) * D;  // floats
+#pragma unroll
+        for (int i = 0; i < kQuads; ++i) {
+          const int e = quad_at + 4 * i * kBlock;
+          if (e < count) {
+            for (int q = 0; q < min(count - e, 4); ++q) dst[e + q] = v[i][q];
+          }
+        }
+      }
+    }
+  };
+  int64_t tile = blockIdx.x;  // the grid is no larger than the tiles
+  load_tile(tile);
+  __syncthreads();
+  const int64_t whole = N / kTile, step = gridDim.x;
+  for (; tile < whole; tile += step) one_tile(tile, tile + step < tiles_n ? tile + step : tiles_n - 1, std::true_type{});
+  if (tile < tiles_n) one_tile(tile, tile, std::false_type{});
+}
+
 // ---- launches ----------------------------------------------------------------
 template <int NT>
 constexpr size_t fwd_pack_lds_bytes() {
@@ -966,6 +1094,38 @@ static int rp_fwd_pack_bf16_launch(const RpPackArgs& a, const u32x4* table, hipS
   return launch_status();
 }
 
+template <int TW, int KS>
+static void rp_bwd_rows_launch(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
+  const int64_t tiles = (N + kTile - 1) / kTile;
+  const int64_t most = static_cast<int64_t>(kRpCus) * bwd_rows_per_cu<TW, KS>();
+  const size_t lds = sizeof(float) * (kTile * (KS * kStepFeatures + 4) + 2 * 8 * static_cast<size_t>(D));
+  hipLaunchKernelGGL((rp_bwd_rows_kernel<TW, KS>), dim3(static_cast<unsigned>(tiles < most ? tiles : most)), dim3(kBlock), lds, s, Xr, table, N,
+                     D, k, out);
+}
+// Whether rp_bwd_rows_kernel took the product.
+static bool rp_bwd_rows(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
+  const int steps = (k + kStepFeatures - 1) / kStepFeatures, tw = ((D + kTile - 1) / kTile + 3) / 4;
+  // Measured over cold operands, this form / the other: 602 -> 232,965 rows of 76 128 / 196 us, of 61 130 / 199, 640 of 100,000
+  // 62 / 89, 480 of 60,000 30 / 37, 301 of 100,000 31 / 39, 130 of 200,000 30 / 37; up to 256 columns of whole lines (256 of
+  // 2.4 M rows 654 / 604) and up to 128 of any (100 of 2.4 M 245 / 231) the other is as fast or faster, and so it is
+  // where the tiles do not reach every compute unit (602 of 3,000 rows 10.2 / 9.1).
+  if (tw > 5 || steps > 5 || N < kRpCus * kTile || !(D > 256 || (D > 128 && D % 32 != 0))) return false;
+#define EXACT_RP_ROWS(TW)                                                                  \
+  case TW:                                                                                 \
+    if (steps <= 2) rp_bwd_rows_launch<TW, 2>(Xr, table, N, D, k, out, s);                 \
+    else if (steps <= 4) rp_bwd_rows_launch<TW, 4>(Xr, table, N, D, k, out, s);            \
+    else rp_bwd_rows_launch<TW, 5>(Xr, table, N, D, k, out, s);                            \
+    break
+  switch (tw) {
+    EXACT_RP_ROWS(2);
+    EXACT_RP_ROWS(3);
+    EXACT_RP_ROWS(4);
+    EXACT_RP_ROWS(5);
+  }
+#undef EXACT_RP_ROWS
+  return true;
+}
+
 template <int VEC, int BP, int KS>
 static int rp_bwd_bf16_launch(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
   const int steps = (k + kStepFeatures - 1) / kStepFeatures;
@@ -985,6 +1145,7 @@ static int rp_bwd_bf16_launch(const float* Xr, const u32x4* table, int64_t N, in
 
 template <int VEC, int BP>
 static int rp_bwd_bf16_steps(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
+  if (BP == 1 && rp_bwd_rows(Xr, table, N, D, k, out, s)) return launch_status();
   const int steps = (k + kStepFeatures - 1) / kStepFeatures;
   if (steps <= 2) return rp_bwd_bf16_launch<VEC, BP, 2>(Xr, table, N, D, k, out, s);
   if (steps <= 4) return rp_bwd_bf16_launch<VEC, BP, 4>(Xr, table, N, D, k, out, s);

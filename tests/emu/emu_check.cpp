@@ -753,7 +753,7 @@ static const int64_t kRpShapes[][3] = {{1, 256, 32}, {31, 256, 32}, {200, 256, 3
                                        {64, 128, 64}, {77, 50, 15}, {130, 7, 4}, {100, 256, 126}, {33, 256, 128}, {70, 96, 96},
                                        {133, 97, 13}, {260, 1024, 32}, {2000, 256, 32}, {1700, 100, 25},
                                        {1100, 602, 76}, {900, 64, 128}, {1537, 50, 15},
-    {33, 65, 9}, {32, 66, 40}, {1, 130, 100}, {31, 129, 7}, {2, 131, 128}, {3, 3, 5}};
+    {8195, 131, 5}, {33, 65, 9}, {32, 66, 40}, {1, 130, 100}, {31, 129, 7}, {2, 131, 128}, {3, 3, 5}};
 
 int main(int argc, char** argv) {
   std::setvbuf(stdout, nullptr, _IOLBF, 0);

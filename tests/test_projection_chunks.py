@@ -34,3 +34,16 @@ def test_projection(backend, N, D, k, signs):
     config.noise_source = lambda shape, device: torch.full(shape, 0.25).to(device)
     for one, two in zip(extq.rp_minmax_pack(x, used, 2), extq.minmax_pack(reduced, 2)):
         assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("N,D,k", [(8192, 130, 5), (8200, 131, 33), (8223, 290, 64), (8193, 385, 20), (8200, 639, 80),
+                                   (16500, 602, 76)])                    # the last: a second tile for some workgroups
+def test_back_by_whole_rows(backend, N, D, k):
+    """rp2input of a sign matrix where a workgroup owns whole rows: tiles of 32 rows, steps of 16 features, pieces of four columns."""
+    g = torch.Generator().manual_seed(N + D + k)
+    matrix = ((2.0 * torch.randint(2, (D, k), generator=g) - 1) / k ** 0.5).to(backend)
+    matrix._exact_sign_matrix = True
+    x = torch.randn(N, k, generator=g).to(backend)
+    got, want = ops.rp2input(x, (N, D), matrix), x.double() @ matrix.double().t()
+    bound = (4 * k + 2) * 2.0 ** -24 * (x.double().abs() @ matrix.double().t().abs()) + 1e-30
+    assert got.shape == (N, D) and ((got.double() - want).abs() <= bound).all()
