@@ -94,16 +94,21 @@ __host__ __device__ inline TableShape table_shape(int D, int k, int pieces) {
 }
 
 // one thread per (direction, step, tile, lane): eight entries of R -> one fragment per piece
+// With `matrix`, R holds 0 and 1 and what is prepared is the matrix of -c and c, which is written there as well.
 template <int BP>
 __global__ __launch_bounds__(kBlock) void rp_prepare_kernel(const float* __restrict__ R, int D, int k,
-                                                            u32x4* __restrict__ table) {
+                                                            u32x4* __restrict__ table, float* __restrict__ matrix, float c) {
   const TableShape ts = table_shape(D, k, BP);
   const int64_t fwd_frags = static_cast<int64_t>(ts.steps_d) * ts.tiles_k * kWave;
   const int64_t bwd_frags = static_cast<int64_t>(ts.steps_k) * ts.tiles_d * kWave;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (idx == 0) {
-    u32x4 head = {__float_as_uint(fabsf(R[0])), 0u, 0u, 0u};
+    u32x4 head = {__float_as_uint(matrix != nullptr ? c : fabsf(R[0])), 0u, 0u, 0u};
     table[0] = head;
+  }
+  if (matrix != nullptr) {
+    // every fragment is eight entries: the forward ones alone are at least an eighth of the entries
+    for (int64_t i = idx; i < static_cast<int64_t>(D) * k; i += static_cast<int64_t>(gridDim.x) * kBlock) matrix[i] = R[i] > 0.f ? c : -c;
   }
   if (idx >= fwd_frags + bwd_frags) return;
   const bool fwd = idx < fwd_frags;
@@ -124,6 +129,9 @@ __global__ __launch_bounds__(kBlock) void rp_prepare_kernel(const float* __restr
   u32x4* dst = table + 1 + (fwd ? 0 : ts.fwd_units()) + (static_cast<int64_t>(step) * tiles + tile) * BP * kWave + l;
   if constexpr (BP == 1) {
     u32x4 w;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (matrix != nullptr) r[i] = r[i] > 0.f ? 1.f : -1.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[i] = sign_bf16(r[2 * i], inside[2 * i]) | (sign_bf16(r[2 * i + 1], inside[2 * i + 1]) << 16);
     dst[0] = w;
@@ -1205,19 +1213,32 @@ int64_t exact_rp_table_nbytes(int64_t D, int64_t k, int mode) {
   return 16 * (1 + ts.fwd_units() + ts.bwd_units());
 }
 
-int exact_rp_prepare_bf16(const float* R, int64_t D, int64_t k, int mode, void* table, void* stream) {
-  if (!rp_shape_ok(0, D, k)) return EXACT_E_SHAPE;
-  if (!rp_mode_ok(mode)) return EXACT_E_ARG;
-  if (!R || !table) return EXACT_E_NULL;
-  if (!al16(table)) return EXACT_E_ALIGN;
+static int rp_prepare(const float* R, int64_t D, int64_t k, int mode, void* table, float* matrix, float c, void* stream) {
   const TableShape ts = table_shape(static_cast<int>(D), static_cast<int>(k), rp_pieces(mode));
   const int64_t frags = (ts.fwd_units() + ts.bwd_units()) / ts.pieces;
   const dim3 grid(static_cast<unsigned>((frags + kBlock - 1) / kBlock)), block(kBlock);
   hipStream_t s = static_cast<hipStream_t>(stream);
   u32x4* t = static_cast<u32x4*>(table);
-  if (mode == EXACT_RP_BF16_SIGNS) hipLaunchKernelGGL((rp_prepare_kernel<1>), grid, block, 0, s, R, static_cast<int>(D), static_cast<int>(k), t);
-  else hipLaunchKernelGGL((rp_prepare_kernel<3>), grid, block, 0, s, R, static_cast<int>(D), static_cast<int>(k), t);
+  const int d = static_cast<int>(D), kk = static_cast<int>(k);
+  if (mode == EXACT_RP_BF16_SIGNS) hipLaunchKernelGGL((rp_prepare_kernel<1>), grid, block, 0, s, R, d, kk, t, matrix, c);
+  else hipLaunchKernelGGL((rp_prepare_kernel<3>), grid, block, 0, s, R, d, kk, t, matrix, c);
   return launch_status();
+}
+
+int exact_rp_prepare_bf16(const float* R, int64_t D, int64_t k, int mode, void* table, void* stream) {
+  if (!rp_shape_ok(0, D, k)) return EXACT_E_SHAPE;
+  if (!rp_mode_ok(mode)) return EXACT_E_ARG;
+  if (!R || !table) return EXACT_E_NULL;
+  if (!al16(table)) return EXACT_E_ALIGN;
+  return rp_prepare(R, D, k, mode, table, nullptr, 0.f, stream);
+}
+
+int exact_rp_draw_signs_f32(const float* bernoulli, int64_t D, int64_t k, float c, float* R, void* table, void* stream) {
+  if (!rp_shape_ok(0, D, k)) return EXACT_E_SHAPE;
+  if (!(c > 0.f)) return EXACT_E_ARG;
+  if (!bernoulli || !R || !table) return EXACT_E_NULL;
+  if (!al16(table)) return EXACT_E_ALIGN;
+  return rp_prepare(bernoulli, D, k, EXACT_RP_BF16_SIGNS, table, R, c, stream);
 }
 
 int exact_rp_fwd_bf16_f32(const float* X, const void* table, int64_t N, int64_t D, int64_t k, int mode, float* out,

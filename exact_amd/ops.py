@@ -131,6 +131,9 @@ def _projection_matrix(D, k, device, dtype):
         return torch.randn((D, k), device=device, dtype=dtype) / k ** 0.5
     # reference ops.py:112-114: Rademacher entries +-1/sqrt(k)
     signs = torch.randint(2, size=(D, k), device=device, dtype=dtype)
+    if (dtype == torch.float32 and 0 < k <= RP_KERNEL_MAX_COLUMNS and config.matrix_cores == "bf16" and _checks.on_device(signs)
+            and _checks.plain_values(signs)):
+        return ext_quantization.sign_matrix(signs)
     matrix = (2.0 * signs - 1) / k ** 0.5
     matrix._exact_sign_matrix = True     # every entry is +-c with one c: the projection kernels may work on the signs alone
     return matrix

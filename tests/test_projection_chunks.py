@@ -47,3 +47,15 @@ def test_back_by_whole_rows(backend, N, D, k):
     got, want = ops.rp2input(x, (N, D), matrix), x.double() @ matrix.double().t()
     bound = (4 * k + 2) * 2.0 ** -24 * (x.double().abs() @ matrix.double().t().abs()) + 1e-30
     assert got.shape == (N, D) and ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("D,k", [(1, 1), (5, 3), (64, 8), (100, 25), (602, 76), (33, 128)])
+def test_drawn_matrix(backend, D, k):
+    """The matrix and its fragments in one launch: the values of the reference's expression, the fragments of the matrix."""
+    draws = torch.randint(2, (D, k), generator=torch.Generator().manual_seed(D), dtype=torch.float32).to(backend)
+    got, want = extq.sign_matrix(draws), (2.0 * draws - 1) / k ** 0.5
+    assert torch.equal(got, want) and got._exact_sign_matrix
+    want._exact_sign_matrix = True
+    assert torch.equal(extq.rp_table(got, extq.RP_BF16_SIGNS), extq.rp_table(want, extq.RP_BF16_SIGNS))
+    got += 0.0                                                            # written to: the kept table is not used any more
+    assert torch.equal(extq.rp_table(got, extq.RP_BF16_SIGNS), extq.rp_table(want, extq.RP_BF16_SIGNS))
