@@ -39,6 +39,7 @@ SIGNATURES = {
     "exact_spmm_csr_strided_f16": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_i64, _c_ptr]),
     "exact_spmm_csr_rowwise_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr]),
     "exact_spmm_csr_minmax_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr, _c_ptr]),
+    "exact_gather_values_f32": (_c_int, [_c_ptr, _c_int, _c_ptr, _c_int, _c_i64, _c_i64, _c_ptr, _c_ptr]),
     "exact_sddmm_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr]),
     "exact_leaky_relu_fwd_f32": (_c_int, [_c_ptr, _c_i64, _c_f32, _c_ptr, _c_ptr, _c_ptr]),
     "exact_leaky_relu_bwd_f32": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_f32, _c_ptr, _c_ptr]),

@@ -164,6 +164,37 @@ def _slot_hit(entry, value, has_value):
     return version == value._version and held._version == value._version
 
 
+# The row indices alone, for graphs whose values are new every step (they require grad, or are the fp16 copies of an
+# autocast region).  Kept only for the very tensors they came from as they were then (versions), and for the stream that
+# made them: csr2csc -> (row, versions, stream, row[csr2csc]).
+_ROW_CSC = WeakIdKeyDictionary()
+
+
+def _transposed_rows(row, csr2csc):
+    if row.is_inference() or csr2csc.is_inference() or not csr2csc.is_cuda or torch.cuda.is_current_stream_capturing():
+        return row.index_select(0, csr2csc)
+    state = (row._version, csr2csc._version, _checks.stream_ptr(csr2csc))
+    held = _ROW_CSC.get(csr2csc)
+    if held is None or held[0] is not row or held[1] != state:
+        held = _ROW_CSC[csr2csc] = (row, state, row.index_select(0, csr2csc))
+    return held[2]
+
+
+def _transposed_values(value, csr2csc):
+    """value[csr2csc] in fp32."""
+    value = value.detach()
+    usable = (value.dtype in (torch.float32, torch.float16) and value.dim() == 1 and csr2csc.dim() == 1
+              and csr2csc.dtype in (torch.int32, torch.int64) and value.is_contiguous() and csr2csc.is_contiguous()
+              and _checks.on_device(value) and value.device == csr2csc.device and value.numel() > 0)
+    if not usable:
+        return value.index_select(0, csr2csc)
+    out = torch.empty(csr2csc.shape, dtype=torch.float32, device=value.device)
+    rc = _lib.lib().exact_gather_values_f32(ptr(value), int(value.dtype == torch.float16), ptr(csr2csc), csr2csc.element_size(),
+                                            csr2csc.numel(), value.numel(), ptr(out), _checks.stream_ptr(value))
+    _lib.check(rc, "spmm backward")
+    return out
+
+
 def _csc_operands(kind, row, value, rowcount, csr2csc, has_value, dtype):
     # fp16 values are per-call copies made by autocast, values that require grad are new every step
     cacheable = not (has_value and (value.dtype != torch.float32 or value.requires_grad))
@@ -172,12 +203,15 @@ def _csc_operands(kind, row, value, rowcount, csr2csc, has_value, dtype):
         slot = None                                         # the same permutation handed in with other rows
     if slot is not None and kind in slot and _slot_hit(slot[kind], value, has_value):
         return slot["row_csc"], slot[kind][2]
-    row_csc = slot["row_csc"] if slot is not None else row.index_select(0, csr2csc)
+    if slot is not None:
+        row_csc = slot["row_csc"]
+    else:
+        row_csc = row.index_select(0, csr2csc) if cacheable else _transposed_rows(row, csr2csc)
     if kind == "sum":
-        w = value.detach().index_select(0, csr2csc) if has_value else None
+        w = _transposed_values(value, csr2csc) if has_value else None
     else:
         cnt = rowcount.to(torch.float32).index_select(0, row_csc).clamp_(min=1)   # fp32 whatever `dtype` is
-        w = value.detach().index_select(0, csr2csc).div(cnt) if has_value else cnt.pow_(-1)
+        w = _transposed_values(value, csr2csc).div(cnt) if has_value else cnt.pow_(-1)
     if cacheable:
         if slot is None:
             slot = _CSC_CACHE[csr2csc] = {"row": (row.data_ptr(), row.numel()), "row_csc": row_csc, "keep": row}
@@ -187,6 +221,7 @@ def _csc_operands(kind, row, value, rowcount, csr2csc, has_value, dtype):
 
 def clear_csc_cache():
     _CSC_CACHE.clear()
+    _ROW_CSC.clear()
 
 
 def _same_index_dtype(*ts):
@@ -212,7 +247,7 @@ def spmm_value_bw(row, rowptr, col, mat, grad, reduce):
     mat, grad = mat.contiguous(), grad.contiguous()
     if mat.shape[1] != grad.shape[1]:
         raise RuntimeError("Input mismatch")
-    out = torch.zeros(row.numel(), dtype=grad.dtype, device=grad.device)
+    out = (torch.empty if mat.shape[1] else torch.zeros)(row.numel(), dtype=grad.dtype, device=grad.device)
     rc = _lib.lib().exact_sddmm_f32(ptr(row), ptr(rowptr), ptr(col), row.element_size(), ptr(mat), ptr(grad),
                                     row.numel(), mat.shape[1], REDUCE[reduce], ptr(out), _checks.stream_ptr(grad))
     _lib.check(rc, "spmm_value_bw")

@@ -165,6 +165,11 @@ int exact_spmm_csr_minmax_f32(const void *rowptr, const void *col, const float *
                               int64_t K, int64_t nnz, int is_max, float *out,
                               void *arg_out, void *stream);
 
+/* out[i] = values[index[i]], widened to fp32 (half = 1: fp16 values): the edge values in the order of the transposed
+ * graph, value.index_select(0, csr2csc) of spmm.cc:73-75.  An index outside [0, n_values) gives NaN. */
+int exact_gather_values_f32(const void *values, int half, const void *index, int idx_bytes, int64_t n,
+                            int64_t n_values, float *out, void *stream);
+
 /* Gradient with respect to the edge values: out[e] = sum_k mat[col[e], k] *
  * grad[row[e], k], divided by max(length of row[e], 1) for EXACT_REDUCE_MEAN.
  * row is the COO row index of every entry.  Replaces spmm_value_bw_cuda
