@@ -62,6 +62,8 @@ SIGNATURES = {
     "exact_elu_bwd_f32": (_c_int, [_c_ptr, _c_ptr, _c_f32, _c_i64, _c_ptr, _c_ptr]),
     "exact_linear_dw_f32": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr]),
     "exact_linear_dw_bf16_f32": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr]),
+    "exact_linear_dw_short_work_nbytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "exact_linear_dw_short_f32": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
     "exact_linear_dw_f16_work_nbytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "exact_linear_dw_ordered_f16": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
     "exact_colsum_f32": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr]),

@@ -25,6 +25,8 @@
 // MFMA 32x32x2 f32 accumulator layout (wave64): register v of lane l is
 // C[8 * (v / 4) + 4 * (l / 32) + v % 4][l % 32].
 
+#include <cmath>
+
 #include "bf16_split.hpp"
 
 namespace exact {
@@ -50,8 +52,9 @@ __device__ __forceinline__ bool dw_block_and_slab(int blocks, int64_t slabs, int
   return slab < slabs;
 }
 
-// WK x (4 / WK) wavefronts per workgroup along Kout x D.
-template <int MK, int MD, int WK>
+// WK x (4 / WK) wavefronts per workgroup along Kout x D.  ORDERED: `out` is scratch [slab][Kout][D] and
+// dw_finish_kernel adds the slabs in their order; else they meet in `out` through atomics.
+template <int MK, int MD, int WK, bool ORDERED>
 __global__ __launch_bounds__(kBlock) void linear_dw_kernel(const float* __restrict__ dY, int64_t ldy,
                                                            const float* __restrict__ X, int64_t ldx, int64_t N,
                                                            int Kout, int D, int64_t rows_per_slab, int blocks_d, int blocks, int64_t slabs,
@@ -134,7 +137,10 @@ __global__ __launch_bounds__(kBlock) void linear_dw_kernel(const float* __restri
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int ri = k0 + 32 * i + 8 * (v / 4) + 4 * half + (v % 4);
-        if (ri < Kout && cj < D) unsafeAtomicAdd(out + static_cast<int64_t>(ri) * D + cj, acc[i][j][v]);
+        if (ri < Kout && cj < D) {
+          if constexpr (ORDERED) out[(slab * Kout + ri) * D + cj] = acc[i][j][v];
+          else unsafeAtomicAdd(out + static_cast<int64_t>(ri) * D + cj, acc[i][j][v]);
+        }
       }
     }
 }
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_shared_kernel(const float
 
 // fp16 operands (autocast): the same walk on v_mfma_f32_32x32x16_f16, which takes them as they are -- products of two
 // fp16 numbers are exact in fp32, infinities, NaN and subnormal numbers among them.  A fragment is one 16-byte unit per
-// lane, so a step is 32 rows.  A slab's block goes to `partial` [slab][Kout][D] and dw_finish_half_kernel adds the slabs
+// lane, so a step is 32 rows.  A slab's block goes to `partial` [slab][Kout][D] and dw_finish_kernel adds the slabs
 // in their order: two equal calls give equal bits.
 template <int MK, int MD, int WK>
 __global__ __launch_bounds__(kBlock, 2) void linear_dw_half_kernel(const half_t* __restrict__ dY, int64_t ldy,
@@ -513,9 +519,11 @@ __global__ __launch_bounds__(kBlock, 2) void linear_dw_half_kernel(const half_t*
     }
 }
 
-// out[i] = fp16(sum over the slabs): eight groups of 32 lanes take every eighth slab, then meet in LDS in their order.
-__global__ __launch_bounds__(kBlock) void dw_finish_half_kernel(const float* __restrict__ partial, int64_t total, int64_t slabs,
-                                                                half_t* __restrict__ out) {
+// out[i] = the sum over the slabs, rounded to T: eight groups of 32 lanes take every eighth slab, then meet in LDS in
+// their order.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void dw_finish_kernel(const float* __restrict__ partial, int64_t total, int64_t slabs,
+                                                           T* __restrict__ out) {
   __shared__ float part[kBlock];
   const int t = threadIdx.x, g = t >> 5;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 32 + (t & 31);
@@ -533,23 +541,28 @@ __global__ __launch_bounds__(kBlock) void dw_finish_half_kernel(const float* __r
   if (g == 0 && i < total) {
 #pragma unroll
     for (int k = 1; k < 8; ++k) s += part[32 * k + t];
-    out[i] = static_cast<half_t>(s);
+    out[i] = static_cast<T>(s);
   }
 }
 
-// How the fp16 form cuts its work: about 512 workgroups (two per compute unit), at least 512 rows a slab, whole steps.
-struct DwHalfPlan {
+// How the forms with a fixed order cut their work.
+struct DwOrderedPlan {
   int mk, md, wk, blocks_d, blocks;
   int64_t rows, slabs;
 };
-static DwHalfPlan plan_dw_half(int64_t N, int K, int D) {
-  DwHalfPlan p{};
+static DwOrderedPlan plan_dw_blocks(int K, int D) {
+  DwOrderedPlan p{};
   p.mk = K <= 32 ? 1 : 2;
   p.md = (K <= 64 ? D <= 128 : D <= 32) ? 1 : 2;
   p.wk = K <= 64 ? 1 : D <= 64 ? 4 : 2;
   const int kb = 32 * p.mk * p.wk, db = 32 * p.md * (4 / p.wk);
   p.blocks_d = (D + db - 1) / db;
   p.blocks = (K + kb - 1) / kb * p.blocks_d;
+  return p;
+}
+// fp16: about 512 workgroups (two per compute unit), at least 512 rows a slab, whole steps.
+static DwOrderedPlan plan_dw_half(int64_t N, int K, int D) {
+  DwOrderedPlan p = plan_dw_blocks(K, D);
   const int64_t wanted = (512 + p.blocks - 1) / p.blocks;
   p.rows = (N + wanted - 1) / wanted;
   if (p.rows < 512) p.rows = 512;
@@ -557,14 +570,38 @@ static DwHalfPlan plan_dw_half(int64_t N, int K, int D) {
   p.slabs = (N + p.rows - 1) / p.rows;
   return p;
 }
+// Rows of a slab for which the two things that grow with its length and with its number are together least: a
+// wavefront's walk, `row_us` a row, and the slabs' results, `value_us` each.  Whole steps of 16, between `least` and 512.
+static int64_t dw_slab_rows(int64_t N, int K, int D, double row_us, double value_us, int64_t least) {
+  int64_t rows = static_cast<int64_t>(std::sqrt(static_cast<double>(N) * K * D * value_us / row_us));
+  rows = rows < least ? least : rows > 512 ? 512 : rows;
+  return (rows + 15) / 16 * 16;
+}
+// fp32, short batches: a row takes 0.11 us, a result 8 bytes of traffic.  Against the framework's GEMM, which does not
+// split the rows: 4,096 rows 128 x 128 15.7 / 24.5 us, 64 x 64 10.3 / 32, 256 x 256 22.9 / 25.3; 16,000 rows 23.8 / 84,
+// 13.0 / 113, 46.7 / 86, 256 x 602 97 / 93.
+static DwOrderedPlan plan_dw_short(int64_t N, int K, int D) {
+  DwOrderedPlan p = plan_dw_blocks(K, D);
+  p.rows = dw_slab_rows(N, K, D, 0.11, 2e-6, 64);
+  p.slabs = (N + p.rows - 1) / p.rows;
+  return p;
+}
 
 template <int MK, int MD, int WK>
-static void launch_dw_half(const DwHalfPlan& p, const half_t* dY, int64_t ldy, const half_t* X, int64_t ldx, int64_t N, int Kout, int D,
+static void launch_dw_half(const DwOrderedPlan& p, const half_t* dY, int64_t ldy, const half_t* X, int64_t ldx, int64_t N, int Kout, int D,
                            float* partial, hipStream_t s) {
   constexpr size_t lds = sizeof(u32x4) * 2 * 2 * (MK * WK + MD * (4 / WK)) * kWave;
   const dim3 grid(static_cast<unsigned>((p.slabs + kDwXcds - 1) / kDwXcds * kDwXcds * p.blocks));
   hipLaunchKernelGGL((linear_dw_half_kernel<MK, MD, WK>), grid, dim3(kBlock), lds, s, dY, ldy, X, ldx, N, Kout, D, p.rows, p.blocks_d,
                      p.blocks, p.slabs, partial);
+}
+
+template <int MK, int MD, int WK>
+static void launch_dw_short(const DwOrderedPlan& p, const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int Kout, int D,
+                            float* partial, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>((p.slabs + kDwXcds - 1) / kDwXcds * kDwXcds * p.blocks));
+  hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK, true>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, p.rows, p.blocks_d, p.blocks,
+                     p.slabs, partial);
 }
 
 template <int MK, int MD, int WK, bool BF16>
@@ -574,10 +611,14 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   const int blocks_k = (Kout + 32 * MK * WK - 1) / (32 * MK * WK);
   const int blocks_d = (D + 32 * MD * WD - 1) / (32 * MD * WD);
   const int blocks = blocks_k * blocks_d;
-  // about 1024 workgroups in all, at least 512 rows per slab, whole batches per slab
+  // About 1024 workgroups in all, whole batches per slab, and slabs no shorter than their results are worth.  The bf16
+  // forms walk a row in 0.068 us and 100,000 results a microsecond meet in memory.  512 rows throughout -> this: 16,384 rows
+  // 128 x 128 37.6 -> 23.4 us, 64 x 64 23.9 -> 12.9, 256 x 40 35.8 -> 19.3; 40,000 rows 41.9 -> 34.6, 25.0 -> 19.9, 44.4 ->
+  // 31.5; the same from 110,000 rows or 256 x 256 on.
   int64_t slabs = (1024 + blocks - 1) / blocks;
   int64_t rows = (N + slabs - 1) / slabs;
-  if (rows < 512) rows = 512;
+  const int64_t least = BF16 ? dw_slab_rows(N, Kout, D, 0.068, 1e-5, 128) : 512;
+  if (rows < least) rows = least;
   rows = (rows + 15) / 16 * 16;  // whole batches (8 rows) resp. steps (16 rows)
   slabs = (N + rows - 1) / rows;
   const dim3 grid(static_cast<unsigned>((slabs + kDwXcds - 1) / kDwXcds * kDwXcds * blocks));
@@ -591,7 +632,7 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   constexpr bool can_share = MD == 2 && WK <= 2;
   const bool shared = can_share && (WK == 2 || N >= (MK == 2 ? 65536 : 500000));
   if constexpr (!BF16) {
-    hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
+    hipLaunchKernelGGL((linear_dw_kernel<MK, MD, WK, false>), grid, dim3(kBlock), 0, s, dY, ldy, X, ldx, N, Kout, D, rows, blocks_d, blocks, slabs, out);
   } else {
     if constexpr (can_share) {
       if (shared) {
@@ -647,6 +688,42 @@ int exact_linear_dw_bf16_f32(const float* dY, int64_t ldy, const float* X, int64
   return linear_dw_any<true>(dY, ldy, X, ldx, N, Kout, D, out, static_cast<hipStream_t>(stream));
 }
 
+static bool dw_short_shape_ok(int64_t N, int64_t Kout, int64_t D) { return N >= 0 && Kout >= 0 && D >= 0 && Kout <= 65536 && D <= 65536 && N <= (int64_t{1} << 40); }
+
+int64_t exact_linear_dw_short_work_nbytes(int64_t N, int64_t Kout, int64_t D) {
+  if (!dw_short_shape_ok(N, Kout, D) || N == 0 || Kout == 0 || D == 0) return 0;
+  return plan_dw_short(N, static_cast<int>(Kout), static_cast<int>(D)).slabs * Kout * D * static_cast<int64_t>(sizeof(float));
+}
+
+int exact_linear_dw_short_f32(const float* dY, int64_t ldy, const float* X, int64_t ldx, int64_t N, int64_t Kout, int64_t D, float* out,
+                              void* work, void* stream) {
+  if (!dw_short_shape_ok(N, Kout, D) || ldy < Kout || ldx < D) return EXACT_E_SHAPE;
+  if (Kout == 0 || D == 0) return EXACT_OK;
+  if (!out || (N > 0 && (!dY || !X || !work))) return EXACT_E_NULL;
+  const int K = static_cast<int>(Kout), Dd = static_cast<int>(D);
+  const int64_t total = Kout * D;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* partial = static_cast<float*>(work);
+  int64_t slabs = 0;  // an empty batch: zeros
+  if (N > 0) {
+    const DwOrderedPlan p = plan_dw_short(N, K, Dd);
+    slabs = p.slabs;
+    if (p.wk == 1) {
+      if (p.mk == 1 && p.md == 1) launch_dw_short<1, 1, 1>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+      else if (p.mk == 1) launch_dw_short<1, 2, 1>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+      else if (p.md == 1) launch_dw_short<2, 1, 1>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+      else launch_dw_short<2, 2, 1>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+    } else if (p.wk == 4) {
+      if (p.md == 1) launch_dw_short<2, 1, 4>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+      else launch_dw_short<2, 2, 4>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+    } else {
+      launch_dw_short<2, 2, 2>(p, dY, ldy, X, ldx, N, K, Dd, partial, s);
+    }
+  }
+  hipLaunchKernelGGL((dw_finish_kernel<float>), dim3(static_cast<unsigned>((total + 31) / 32)), dim3(kBlock), 0, s, partial, total, slabs, out);
+  return launch_status();
+}
+
 int64_t exact_linear_dw_f16_work_nbytes(int64_t N, int64_t Kout, int64_t D) {
   if (N < 0 || Kout < 0 || D < 0 || Kout > 65536 || D > 65536 || N > (int64_t{1} << 40)) return 0;
   if (N == 0 || Kout == 0 || D == 0) return 0;
@@ -667,7 +744,7 @@ int exact_linear_dw_ordered_f16(const uint16_t* dY, int64_t ldy, const uint16_t*
   const half_t* x = reinterpret_cast<const half_t*>(X);
   int64_t slabs = 0;  // an empty batch: zeros
   if (N > 0) {
-    const DwHalfPlan p = plan_dw_half(N, K, Dd);
+    const DwOrderedPlan p = plan_dw_half(N, K, Dd);
     slabs = p.slabs;
     if (p.wk == 1) {
       if (p.mk == 1 && p.md == 1) launch_dw_half<1, 1, 1>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
@@ -681,7 +758,7 @@ int exact_linear_dw_ordered_f16(const uint16_t* dY, int64_t ldy, const uint16_t*
       launch_dw_half<2, 2, 2>(p, y, ldy, x, ldx, N, K, Dd, partial, s);
     }
   }
-  hipLaunchKernelGGL(dw_finish_half_kernel, dim3(static_cast<unsigned>((total + 31) / 32)), dim3(kBlock), 0, s, partial, total, slabs,
+  hipLaunchKernelGGL((dw_finish_kernel<half_t>), dim3(static_cast<unsigned>((total + 31) / 32)), dim3(kBlock), 0, s, partial, total, slabs,
                      reinterpret_cast<half_t*>(out));
   return launch_status();
 }

@@ -272,6 +272,12 @@ int exact_linear_dw_f32(const float *dY, int64_t ldy, const float *X, int64_t ld
 int exact_linear_dw_bf16_f32(const float *dY, int64_t ldy, const float *X, int64_t ldx, int64_t N,
                              int64_t Kout, int64_t D, float *out, void *stream);
 
+/* exact_linear_dw_f32 for short batches: shorter slabs, added in a fixed order (two equal calls give equal bits);
+ * infinities and NaN as in fp32 arithmetic.  `work`: exact_linear_dw_short_work_nbytes(N, Kout, D) bytes of scratch. */
+int64_t exact_linear_dw_short_work_nbytes(int64_t N, int64_t Kout, int64_t D);
+int exact_linear_dw_short_f32(const float *dY, int64_t ldy, const float *X, int64_t ldx, int64_t N, int64_t Kout,
+                              int64_t D, float *out, void *work, void *stream);
+
 /* The same for fp16 operands and an fp16 result: exact products summed in fp32 in
  * a fixed order (two equal calls give equal bits), rounded once; infinities and
  * NaN as in fp32 arithmetic.  `work`: exact_linear_dw_f16_work_nbytes(N, Kout, D)

@@ -92,3 +92,44 @@ def test_half_operands_give_equal_bits_twice(backend, K, D):
     first = bf.weight_gradient(dy, x)
     for _ in range(3):
         assert torch.equal(bf.weight_gradient(dy, x), first)
+
+
+# one, several and partial blocks; N: the shortest, whole slabs of 64, a last slab of one row
+@pytest.mark.parametrize("K,D", [(1, 1), (33, 128), (32, 130), (64, 70), (40, 256), (130, 32), (96, 64), (65, 100), (256, 256)])
+@pytest.mark.parametrize("N", [4096, 4161, 5000])
+def test_short_batches(backend, N, K, D):
+    """At most N / 2 + 16 additions in a chain (two rows a product, at most 80 slabs in eight chains), each wrong by at most
+    2^-24 of the absolute terms; in a fixed order, infinities where fp32 has them."""
+    if N > 4096 and K * D > 20000 and backend.type == "cpu":
+        pytest.skip("slow on the emulator")
+    g = torch.Generator().manual_seed(N + 7 * K + D)
+    dy = torch.randn(N, K + 2, generator=g)[:, :K].to(backend)
+    x = torch.randn(N, D, generator=g).to(backend)
+    calls = []
+    real = bf._scratch_size
+    bf._scratch_size = lambda *a: calls.append(a[0]) or real(*a)
+    try:
+        got = bf.weight_gradient(dy, x)
+        again = bf.weight_gradient(dy, x)
+        dy[3, 0], x[N - 1, D - 1] = float("inf"), float("-inf")
+        ends = bf.weight_gradient(dy, x)
+    finally:
+        bf._scratch_size = real
+    assert calls == ["exact_linear_dw_short_work_nbytes"] * 3 and torch.equal(got, again)
+    dy[3, 0] = x[N - 1, D - 1] = 0.0
+    # (both tensors had a finite value there before: compare what those rows do not reach)
+    want, bound = dy.double().t() @ x.double(), (N // 2 + 20) * 2.0 ** -24 * (dy.double().abs().t() @ x.double().abs())
+    keep = torch.ones(K, D, dtype=torch.bool, device=got.device)
+    keep[0, :] = False
+    keep[:, D - 1] = False
+    assert ((got.double() - want).abs() <= bound)[keep].all()
+    if K > 1 and D > 1:
+        assert torch.isinf(ends[0, : D - 1]).all() and torch.isinf(ends[1:, D - 1]).all()
+        assert torch.equal(ends[1:, : D - 1], got[1:, : D - 1])
+
+
+def test_short_batches_under_a_recorded_backward(backend):
+    dy, x = torch.randn(4096, 3).to(backend).requires_grad_(), torch.randn(4096, 5).to(backend)
+    out = bf.weight_gradient(dy, x)
+    back, = torch.autograd.grad(out.sum(), dy)
+    assert torch.allclose(back, x.sum(1, keepdim=True).expand(-1, 3), atol=1e-4)
