@@ -8,6 +8,8 @@
 // four rows, 512 with two, 1024 with one: every width up to 8192 is served, not only the widths of at most 256
 // columns that one row of scalar units covers.
 
+#include <cmath>
+
 #include "exact_common.hpp"
 
 namespace exact {
@@ -287,12 +289,12 @@ __global__ __launch_bounds__(kBlock) void bn_apply_kernel(const float* __restric
 // each read dy, one mask bit and `bits` code bits per element: neither the masked gradient nor the dequantised
 // input is ever written to memory.  A thread takes four consecutive rows of its four columns per step: with 1 and 2
 // bits their codes are one 32-bit word, and four 16-byte loads of dy are in flight.  At [169343, 256] INT2 with a
-// mask the two passes take 62 + 90 us (and the sums between them 12) where mask 58 + dequantise 36 + reduce 68 + apply
-// 100 were; at [50000, 512] without one 26 + 54 for dequantise 22 + reduce 699 + apply 59.
+// mask the passes and the sums between them take 119 us where mask 58 + dequantise 36 + reduce 68 + apply
+// 100 were; at [50000, 512] without one 87 for dequantise 22 + reduce 699 + apply 59.
 struct BnBackward {
   const float* dy;
   const uint32_t* mask;  // null: g = dy
-  float p1m;
+  float p1m, inv_p1m;
   const uint8_t* packed;
   const uint16_t* scale;
   const uint16_t* mn;
@@ -307,7 +309,10 @@ struct BnBackward {
   float* dx;
 };
 
-template <int BITS>
+// MASK: 0 none, 1 behind a mask with 1 - p a power of two (the gradient times its reciprocal is the quotient, exactly),
+// 2 behind any other.  Nothing here branches by element: with a branch around each quotient and each masked gradient
+// the two passes were bound by the vector instructions (160 -> 119 us with 1 - p = 1 / 2, 130 with 0.7, at [169343, 256] INT2).
+template <int BITS, int MASK>
 __device__ __forceinline__ void bn_bwd_rows(const BnBackward& a, int64_t row, int k, float (&g)[4][4], float (&x)[4][4]) {
   constexpr int WPT = 8 / BITS;
   constexpr int WORDS = WPT >= 4 ? 1 : 4 / WPT;
@@ -319,8 +324,7 @@ __device__ __forceinline__ void bn_bwd_rows(const BnBackward& a, int64_t row, in
   for (int r = 0; r < 4; ++r) {
     const int64_t n = row + r < a.N ? row + r : a.N - 1;  // rows past the end repeat the last one, with g = 0
     d[r] = nt_load4(a.dy + n * a.K + k);
-    mk[r] = 0xFu;
-    if (a.mask) {
+    if constexpr (MASK != 0) {
       const int64_t e = n * a.K + k;  // K % 4 == 0: the four bits lie in one word
       mk[r] = a.mask[e >> 5] >> (e & 31);
     }
@@ -332,28 +336,50 @@ __device__ __forceinline__ void bn_bwd_rows(const BnBackward& a, int64_t row, in
     const int64_t n = row + i * WPT < a.N ? row + i * WPT : a.N - 1;
     w[i] = *reinterpret_cast<const uint32_t*>(a.packed + (n / WPT) * a.K + k);
   }
+  float scale[4], mn[4];
+  bool fast = true;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float scale = bf16_to_f32(sc16[r]), mn = bf16_to_f32(mn16[r]);
-    const float as = fabsf(scale);
-    const bool fast = as >= 0x1p-64f && as <= 0x1p64f;  // exact_quotient's range
-    const float rcp = 1.f / scale;
+    scale[r] = bf16_to_f32(sc16[r]);
+    mn[r] = bf16_to_f32(mn16[r]);
+    const float as = fabsf(scale[r]);
+    fast = fast && as >= 0x1p-64f && as <= 0x1p64f;  // exact_quotient's range
+  }
+  auto code = [&](int r, int c) {
     // row is a multiple of 4, so the shift is known but for which half of an INT1 group the rows are
     const int shift = WPT == 8 ? static_cast<int>((row & 7) + r) : (r % WPT) * BITS;
-    const uint32_t word = w[r / (4 / WORDS)] >> shift;
+    return static_cast<float>(((w[r / (4 / WORDS)] >> shift) >> (8 * c)) & FIELD);
+  };
+  if (fast) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float rcp = 1.f / scale[r];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[r][c] = exact_quotient(code(r, c), scale[r], rcp) + mn[r];
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[r][c] = code(r, c) / scale[r] + mn[r];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if constexpr (MASK != 0) mk[r] = row + r < a.N ? mk[r] : 0u;
     const bool live = row + r < a.N;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const float q = static_cast<float>((word >> (8 * c)) & FIELD);
-      x[r][c] = (fast ? exact_quotient(q, scale, rcp) : q / scale) + mn;
-      const float dv = d[r][c];
-      const float gv = a.mask ? (((mk[r] >> c) & 1u) ? dv / a.p1m : 0.f) : dv;
-      g[r][c] = live ? gv : 0.f;
+      if constexpr (MASK == 0) {
+        g[r][c] = live ? d[r][c] : 0.f;
+      } else {
+        const float dv = ((mk[r] >> c) & 1u) ? d[r][c] : 0.f;
+        g[r][c] = MASK == 1 ? dv * a.inv_p1m : dv / a.p1m;
+      }
     }
   }
 }
 
-template <int BITS>
+template <int BITS, int MASK>
 __global__ __launch_bounds__(kBlock) void bn_bwd_reduce_kernel(const BnBackward a) {
   const BnBlock b = bn_block<4>(a.K);
   const int t = threadIdx.x;
@@ -365,7 +391,7 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_reduce_kernel(const BnBackward 
     const f32x4 m = *reinterpret_cast<const f32x4_any*>(a.mean + k);
     for (int64_t row = r0 + 4 * (t / b.units); row < r1; row += 4 * b.rpp) {
       float g[4][4], x[4][4];
-      bn_bwd_rows<BITS>(a, row, k, g, x);
+      bn_bwd_rows<BITS, MASK>(a, row, k, g, x);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -392,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_reduce_kernel(const BnBackward 
   }
 }
 
-template <int BITS>
+template <int BITS, int MASK>
 __global__ __launch_bounds__(kBlock) void bn_bwd_apply_kernel(const BnBackward a) {
   const BnBlock b = bn_block<4>(a.K);
   const int t = threadIdx.x;
@@ -412,7 +438,7 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_apply_kernel(const BnBackward a
   }
   for (int64_t row = r0 + 4 * (t / b.units); row < r1; row += 4 * b.rpp) {
     float g[4][4], x[4][4];
-    bn_bwd_rows<BITS>(a, row, k, g, x);
+    bn_bwd_rows<BITS, MASK>(a, row, k, g, x);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (row + r >= a.N) break;
@@ -447,17 +473,25 @@ static dim3 bn_grid(int64_t N, int K, int vec, int64_t rows) {
 }
 static bool on(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-template <int BITS>
+template <int BITS, int MASK>
 static void launch_bn_backward(BnBackward a, float* grad_weight, hipStream_t s) {
   a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnBackwardWgs, 4);
   const dim3 grid = bn_grid(a.N, a.K, 4, a.rows_per_wg);
-  hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS>), grid, dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS, MASK>), grid, dim3(kBlock), 0, s, a);
   hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, a.partial,
                      static_cast<int64_t>(grid.x), a.K, a.invstd, a.sums, grad_weight);
   if (a.dx) {
     a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnApplyWgs, 4);
-    hipLaunchKernelGGL((bn_bwd_apply_kernel<BITS>), bn_grid(a.N, a.K, 4, a.rows_per_wg), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((bn_bwd_apply_kernel<BITS, MASK>), bn_grid(a.N, a.K, 4, a.rows_per_wg), dim3(kBlock), 0, s, a);
   }
+}
+
+template <int BITS>
+static void launch_bn_backward(const BnBackward& a, float* grad_weight, hipStream_t s) {
+  int e;
+  if (!a.mask) launch_bn_backward<BITS, 0>(a, grad_weight, s);
+  else if (std::frexp(a.p1m, &e) == 0.5f) launch_bn_backward<BITS, 1>(a, grad_weight, s);
+  else launch_bn_backward<BITS, 2>(a, grad_weight, s);
 }
 
 template <int VEC>
@@ -535,6 +569,7 @@ int exact_bn_backward_ordered_f32(const float* dy, const uint32_t* mask, float p
   a.dy = dy;
   a.mask = mask;
   a.p1m = static_cast<float>(1.0 - static_cast<double>(p));  // as the dropout backward divides
+  a.inv_p1m = 1.f / a.p1m;
   a.packed = packed;
   a.scale = scale_bf16;
   a.mn = min_bf16;

@@ -167,3 +167,27 @@ def test_malformed_column_vectors_are_refused(backend, monkeypatch):
             bf.batch_norm_apply(x.detach(), mean, mult, torch.zeros(12))
     with pytest.raises(RuntimeError):
         bf.batch_norm_apply(x.detach()[:, :6], mean[:6], mult[:6], None)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.5, 0.75, 0.3])                   # 1 - p: three powers of two and another number
+@pytest.mark.parametrize("bits", [1, 2, 8])
+def test_masked_backward_at_the_ends_of_the_range(backend, p, bits):
+    """Behind a mask with a subnormal and a huge gradient and rows whose scale has no reciprocal within range (constant ones,
+    spreads of 1e-30 and 1e25): the gradients that the separate routines give, to the rounding of the two sums."""
+    N, K = 1030, 36
+    g = torch.Generator().manual_seed(bits)
+    x = torch.randn(N, K, generator=g)
+    x[3], x[4], x[5] = 2.0, 1e-30 * x[4], 1e25 * x[5]
+    x, dy = x.to(backend), torch.randn(N, K, generator=g).to(backend)
+    dy[7, 3], dy[8, 5] = 1e-40, 1e30
+    mask = extq.relu_dropout_fwd(torch.ones(N, K).to(backend), p)[1]
+    packed, scale, mn = extq.minmax_pack(x, bits)
+    mean, invstd = torch.zeros(K).to(backend), torch.ones(K).to(backend)
+    got = bf.batch_norm_backward_packed(dy, mask, p, (packed, bits, scale, mn), None, mean, invstd, [True, True, True])
+    masked, x_hat = extq.dropout_bwd(dy, mask, p).double(), extq.unpack_bf16param(packed, bits, scale, mn, N, K).double()
+    s0, s1 = masked.sum(0), (masked * x_hat).sum(0)
+    terms = masked.abs() + masked.abs().sum(0) / N + x_hat.abs() * (masked * x_hat).abs().sum(0) / N
+    within = terms < 1e37                                                # the row of 1e25 times its own sum leaves fp32
+    assert ((got[0].double() - (masked - s0 / N - x_hat * s1 / N)).abs() <= 1e-5 * terms + 1e-30)[within].all()
+    assert within.all(1).sum() >= N - 1
+    assert ((got[2].double() - s0).abs() <= 1e-5 * masked.abs().sum(0)).all()
