@@ -614,10 +614,11 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   // About 1024 workgroups in all, whole batches per slab, and slabs no shorter than their results are worth.  The bf16
   // forms walk a row in 0.068 us and 100,000 results a microsecond meet in memory.  512 rows throughout -> this: 16,384 rows
   // 128 x 128 37.6 -> 23.4 us, 64 x 64 23.9 -> 12.9, 256 x 40 35.8 -> 19.3; 40,000 rows 41.9 -> 34.6, 25.0 -> 19.9, 44.4 ->
-  // 31.5; the same from 110,000 rows or 256 x 256 on.
+  // 31.5; the same from 110,000 rows or 256 x 256 on.  From 200,000 on the many slabs of a small product meet at too few
+  // addresses (300,000 rows 128 x 16 53 -> 59): 512 there.
   int64_t slabs = (1024 + blocks - 1) / blocks;
   int64_t rows = (N + slabs - 1) / slabs;
-  const int64_t least = BF16 ? dw_slab_rows(N, Kout, D, 0.068, 1e-5, 128) : 512;
+  const int64_t least = BF16 && N < 200000 ? dw_slab_rows(N, Kout, D, 0.068, 1e-5, 128) : 512;
   if (rows < least) rows = least;
   rows = (rows + 15) / 16 * 16;  // whole batches (8 rows) resp. steps (16 rows)
   slabs = (N + rows - 1) / rows;
