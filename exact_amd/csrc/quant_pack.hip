@@ -377,14 +377,13 @@ __global__ __launch_bounds__(kBlock) void pack_kernel(const PackArgs a) {
       const Philox4 r = philox4x32_10(static_cast<uint32_t>(j), n_lo, a.off_lo, a.off_hi, a.seed_lo, a.seed_hi);
       philox_uniform8(r, u);
     }
+    float half[8];
+    if constexpr (HALF) scaled_difference_half(v[k], mnv, sc, half);
     uint32_t q[8];  // the code in the low byte
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       // quantization_cuda_kernel.cu:89, one rounding per operation
-      float tq = v[k][i] - mnv;
-      if constexpr (HALF) tq = round_to_half(tq);
-      tq = tq * sc;
-      if constexpr (HALF) tq = round_to_half(tq);
+      float tq = HALF ? half[i] : (v[k][i] - mnv) * sc;
       tq = tq + u[i];
       if constexpr (FUSED) {
         // scale and min come from this row: tq < 2^bits + 2
@@ -665,15 +664,11 @@ __global__ __launch_bounds__(kFlatThreads) void pack_flat_kernel(const PackFlatA
                                         a.off_lo, a.off_hi, a.seed_lo, a.seed_hi);
         philox_uniform8(r, u);
       }
+      float half[8];
+      if constexpr (HALF) scaled_difference_half(v[k], par.x, par.y, half);
       uint32_t q[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float tq = v[k][i] - par.x;
-        if constexpr (HALF) tq = round_to_half(tq);
-        tq = tq * par.y;
-        if constexpr (HALF) tq = round_to_half(tq);
-        q[i] = code_in_low_byte(tq + u[i]);
-      }
+      for (int i = 0; i < 8; ++i) q[i] = code_in_low_byte((HALF ? half[i] : (v[k][i] - par.x) * par.y) + u[i]);
       const uint2 codes = make_uint2(low_bytes4(q[0], q[1], q[2], q[3]), low_bytes4(q[4], q[5], q[6], q[7]));
       if constexpr (WPT == 1)  // one row per byte: nothing to combine
         store_bytes8(a.packed + row_base * a.G + (row_of[k] * a.G + 8 * oct_of[k]), min(8, a.G - 8 * oct_of[k]), codes.x, codes.y);

@@ -179,12 +179,9 @@ struct UnpackFlatArgs {
 constexpr int kFlatPieces = 4;
 
 // the first nv (1 .. 7) of eight fp16 values, at any element boundary: up to three stores
-__device__ __forceinline__ void store_half_tail(half_t* p, int nv, const float (&r)[8]) {
+__device__ __forceinline__ void store_half_tail(half_t* p, int nv, half8 h) {
   typedef half_t half2_any __attribute__((ext_vector_type(2), aligned(2)));
   typedef half_t half4_any __attribute__((ext_vector_type(4), aligned(2)));
-  half_t h[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) h[i] = to_half(r[i]);
   int at = 0;
   if (nv & 4) {
     *reinterpret_cast<half4_any*>(p) = half4_any{h[0], h[1], h[2], h[3]};
@@ -248,28 +245,37 @@ __global__ __launch_bounds__(kBlock) void unpack_flat_kernel(const UnpackFlatArg
     const int shift = static_cast<int>((row_base + row_of[k]) & (WPT - 1)) * BITS;
     float r[PIECE];
 #pragma unroll
-    for (int i = 0; i < PIECE; ++i) {
-      const float code = static_cast<float>((((w[k][i / 4] >> shift) & FIELD) >> (8 * (i & 3))) & 0xFFu);
-      const float quo = __builtin_expect(fast_div, 1) ? exact_quotient(code, sc[k], rcp) : code / sc[k];
-      r[i] = (F16 ? round_to_half(quo) : quo) + mnv[k];
+    for (int i = 0; i < PIECE; ++i) r[i] = static_cast<float>((((w[k][i / 4] >> shift) & FIELD) >> (8 * (i & 3))) & 0xFFu);
+    if (__builtin_expect(fast_div, 1)) {  // a branch for the piece, not one for every element
+#pragma unroll
+      for (int i = 0; i < PIECE; ++i) r[i] = exact_quotient(r[i], sc[k], rcp);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECE; ++i) r[i] = r[i] / sc[k];
+    }
+    half8 sum;  // of fp16 numbers: one rounding of the exact sum is what rounding it to fp32 first gives (scaled_difference_half)
+    if constexpr (F16) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum[i] = to_half(r[i]);
+      sum = sum + to_half(mnv[k]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECE; ++i) r[i] = r[i] + mnv[k];
     }
     const int nv = min(PIECE, a.G - col_of[k]);
     const int64_t flat = (row_base + row_of[k]) * a.G + col_of[k];
     if constexpr (F16) {
       half_t* p = static_cast<half_t*>(a.out) + flat;
       if (nv == PIECE) {
-        half8 q;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) q[i] = to_half(r[i]);
-        *reinterpret_cast<half8_any*>(p) = q;
+        *reinterpret_cast<half8_any*>(p) = sum;
       } else {
         // wide where the rows start on 4 bytes; off them a wide store is taken apart and the single ones are as fast
         if (a.G % 2 == 0) {
-          store_half_tail(p, nv, r);
+          store_half_tail(p, nv, sum);
         } else {
 #pragma unroll
           for (int i = 0; i < PIECE - 1; ++i)
-            if (i < nv) p[i] = to_half(r[i]);
+            if (i < nv) p[i] = sum[i];
         }
       }
     } else {

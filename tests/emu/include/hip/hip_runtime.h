@@ -542,6 +542,9 @@ static inline uint64_t __ballot(bool p) { return hipemu::ballot(p); }
 #define __builtin_amdgcn_update_dpp(old, v, ctrl, rm, bm, bc) hipemu::update_dpp_any((v), (ctrl), (rm), (bm), (bc))
 #define __builtin_amdgcn_bitop3_b32(a, b, c, table) hipemu::bitop3((a), (b), (c), (table))
 #define __builtin_amdgcn_perm(hi, lo, sel) hipemu::byte_perm((hi), (lo), (sel))
+// v_cvt_pkrtz_f16_f32 of numbers that are fp16 numbers (all that the kernels give it): no rounding to get wrong
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+#define __builtin_amdgcn_cvt_pkrtz(a, b) (half2_t{static_cast<_Float16>(a), static_cast<_Float16>(b)})
 #define __builtin_amdgcn_fmed3f(a, b, c) hipemu::fmed3((a), (b), (c))
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) hipemu::mfma_f32_32x32x2f32((a), (b), (c), (x), (y), (z))
 // every active lane of the wavefront arrives before any goes on (a scheduling barrier on the hardware, where the
