@@ -66,7 +66,7 @@ __device__ __forceinline__ void bn_join(float na, double& mean, float& dev, floa
 // Mean and squared deviations of a workgroup's rows, per column: partial[workgroup][3][K], the mean as the sum of two
 // floats.  A thread takes eight rows at a time: their mean and their deviations from it, formed from the differences to
 // the first of them, joined to what it has.  Bound by reading x: [50000, 512] 20 us of 102 MB and [169343, 256] 33 us,
-// and 12 us each for the small kernel behind (50 and 46 us when sums about a sampled centre met through atomics).
+// and 9 us each for the small kernel behind (50 and 46 us when sums about a sampled centre met through atomics).
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restrict__ x, int64_t N, int K, int64_t rows_per_wg,
                                                             float* __restrict__ partial) {
@@ -144,19 +144,22 @@ __global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restr
   }
 }
 
-// The kernels that take the workgroups of a column in their order: 8 columns x 32 groups of workgroups, each group
-// every 32nd of them, then the groups.
-constexpr int kBnCols = 8, kBnGroups = kBlock / kBnCols, kBnFlight = 8;
+// The kernels that take the workgroups of a column: 8 columns x 128 groups, each group every 128th of the workgroups in
+// their order, then the groups pair by pair.  Bound by latency: a column has at most 1024 workgroups, so all its numbers
+// are loaded at once, and seven steps join 128 groups.  (32 groups loaded up to four times and were joined one behind
+// the other: at [169343, 256] statistics 41.7 us, now 38.7, the backward's sums 45.5, now 37.4; [9000, 256] 18.5 -> 15.4
+// and 13.9 -> 10.1.  At [8200, 8000], 1000 of these workgroups, the sums take 56.1 where they took 54.6.)
+constexpr int kBnCols = 8, kBnGroups = 128, kBnFlight = 8, kBnEndBlock = kBnCols * kBnGroups;
 
 // -> mean, 1 / sqrt(var + eps), weight * that, and the running statistics with torch's bookkeeping: one launch where
 // the framework's element-wise routines took fourteen.
-__global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restrict__ partial, int64_t wgs, int64_t rows_per_wg,
+__global__ __launch_bounds__(kBnEndBlock) void bn_finish_kernel(const float* __restrict__ partial, int64_t wgs, int64_t rows_per_wg,
                                                            int64_t N, int K, float eps, float factor,
                                                            const float* __restrict__ weight, float* __restrict__ running_mean,
                                                            float* __restrict__ running_var, float* __restrict__ mean,
                                                            float* __restrict__ invstd, float* __restrict__ mult) {
-  __shared__ double part_mean[kBlock];
-  __shared__ float part_dev[kBlock], count[kBlock];
+  __shared__ double part_mean[kBnEndBlock];
+  __shared__ float part_dev[kBnEndBlock], count[kBnEndBlock];
   const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
   const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
   const float* src = partial + (k < K ? k : K - 1);
@@ -181,16 +184,20 @@ __global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restri
       n += rows;
     }
   }
-  count[t] = n;
-  part_mean[t] = m;
-  part_dev[t] = dev;
-  __syncthreads();
-  if (g != 0 || k >= K) return;
-  for (int i = 1; i < kBnGroups; ++i) {
-    const int o = i * kBnCols + c;
-    bn_join(n, m, dev, count[o], part_mean[o], part_dev[o]);
-    n += count[o];
+  for (int half = kBnGroups / 2; half > 0; half /= 2) {
+    if (g >= half && g < 2 * half) {
+      count[t] = n;
+      part_mean[t] = m;
+      part_dev[t] = dev;
+    }
+    __syncthreads();
+    if (g < half) {
+      const int o = t + half * kBnCols;
+      bn_join(n, m, dev, count[o], part_mean[o], part_dev[o]);
+      n += count[o];
+    }
   }
+  if (g != 0 || k >= K) return;
   const float rows = static_cast<float>(N);
   const float var = dev / rows;
   const float inv = 1.f / sqrtf(var + eps);
@@ -206,10 +213,10 @@ __global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restri
 }
 
 // The same for plain sums: sums[0 .. K) and sums[K .. 2 K), and the gradient of the weight.
-__global__ __launch_bounds__(kBlock) void bn_sums_kernel(const float* __restrict__ partial, int64_t wgs, int K,
+__global__ __launch_bounds__(kBnEndBlock) void bn_sums_kernel(const float* __restrict__ partial, int64_t wgs, int K,
                                                          const float* __restrict__ invstd, float* __restrict__ sums,
                                                          float* __restrict__ grad_weight) {
-  __shared__ float part[2][kBlock];
+  __shared__ float part[2][kBnEndBlock];
   const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
   const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
   const float* src = partial + (k < K ? k : K - 1);
@@ -229,14 +236,18 @@ __global__ __launch_bounds__(kBlock) void bn_sums_kernel(const float* __restrict
       s1 += p1[i];
     }
   }
-  part[0][t] = s0;
-  part[1][t] = s1;
-  __syncthreads();
-  if (g != 0 || k >= K) return;
-  for (int i = 1; i < kBnGroups; ++i) {
-    s0 += part[0][i * kBnCols + c];
-    s1 += part[1][i * kBnCols + c];
+  for (int half = kBnGroups / 2; half > 0; half /= 2) {
+    if (g >= half && g < 2 * half) {
+      part[0][t] = s0;
+      part[1][t] = s1;
+    }
+    __syncthreads();
+    if (g < half) {
+      s0 += part[0][t + half * kBnCols];
+      s1 += part[1][t + half * kBnCols];
+    }
   }
+  if (g != 0 || k >= K) return;
   sums[k] = s0;
   sums[K + k] = s1;
   if (grad_weight) grad_weight[k] = s1 * invstd[k];
@@ -289,7 +300,7 @@ __global__ __launch_bounds__(kBlock) void bn_apply_kernel(const float* __restric
 // each read dy, one mask bit and `bits` code bits per element: neither the masked gradient nor the dequantised
 // input is ever written to memory.  A thread takes four consecutive rows of its four columns per step: with 1 and 2
 // bits their codes are one 32-bit word, and four 16-byte loads of dy are in flight.  At [169343, 256] INT2 with a
-// mask the passes and the sums between them take 119 us where mask 58 + dequantise 36 + reduce 68 + apply
+// mask the passes and the sums between them take 111 us where mask 58 + dequantise 36 + reduce 68 + apply
 // 100 were; at [50000, 512] without one 87 for dequantise 22 + reduce 699 + apply 59.
 struct BnBackward {
   const float* dy;
@@ -311,7 +322,7 @@ struct BnBackward {
 
 // MASK: 0 none, 1 behind a mask with 1 - p a power of two (the gradient times its reciprocal is the quotient, exactly),
 // 2 behind any other.  Nothing here branches by element: with a branch around each quotient and each masked gradient
-// the two passes were bound by the vector instructions (160 -> 119 us with 1 - p = 1 / 2, 130 with 0.7, at [169343, 256] INT2).
+// the two passes were bound by the vector instructions (160 -> 119 us with 1 - p = 1 / 2, 130 with 0.7, both with 8 more of the sums between, at [169343, 256] INT2).
 template <int BITS, int MASK>
 __device__ __forceinline__ void bn_bwd_rows(const BnBackward& a, int64_t row, int k, float (&g)[4][4], float (&x)[4][4]) {
   constexpr int WPT = 8 / BITS;
@@ -478,7 +489,7 @@ static void launch_bn_backward(BnBackward a, float* grad_weight, hipStream_t s) 
   a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnBackwardWgs, 4);
   const dim3 grid = bn_grid(a.N, a.K, 4, a.rows_per_wg);
   hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS, MASK>), grid, dim3(kBlock), 0, s, a);
-  hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, a.partial,
+  hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBnEndBlock), 0, s, a.partial,
                      static_cast<int64_t>(grid.x), a.K, a.invstd, a.sums, grad_weight);
   if (a.dx) {
     a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnApplyWgs, 4);
@@ -532,7 +543,7 @@ int exact_bn_statistics_f32(const float* x, int64_t N, int64_t K, float eps, flo
   int64_t rows = 0, wgs = 0;
   if (K % 4 == 0 && on(x, 16)) launch_bn_moments<4>(x, N, k, work, rows, wgs, s);
   else launch_bn_moments<1>(x, N, k, work, rows, wgs, s);
-  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((k + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, work, wgs, rows, N,
+  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((k + kBnCols - 1) / kBnCols)), dim3(kBnEndBlock), 0, s, work, wgs, rows, N,
                      k, eps, factor, weight, running_mean, running_var, mean, invstd, mult);
   return launch_status();
 }

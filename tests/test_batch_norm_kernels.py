@@ -191,3 +191,19 @@ def test_masked_backward_at_the_ends_of_the_range(backend, p, bits):
     assert ((got[0].double() - (masked - s0 / N - x_hat * s1 / N)).abs() <= 1e-5 * terms + 1e-30)[within].all()
     assert within.all(1).sum() >= N - 1
     assert ((got[2].double() - s0).abs() <= 1e-5 * masked.abs().sum(0)).all()
+
+
+# 512 rows a workgroup: few workgroups, all but one of the 128 groups, one each, one more, and five in one group
+@pytest.mark.parametrize("wgs", [17, 127, 128, 129, 513])
+def test_the_workgroups_of_a_column_whatever_their_number(backend, wgs):
+    """Statistics and the sums of the backward where the last workgroup holds one row and the others unequal values."""
+    N, K = (wgs - 1) * 512 + 1, 8
+    _check_statistics(backend, "sorted", N, K)
+    g = torch.Generator().manual_seed(wgs)
+    dy, x = torch.randn(N, K, generator=g).to(backend), torch.randn(N, K, generator=g).to(backend)
+    packed, scale, mn = extq.minmax_pack(x, 2)
+    mean, invstd = torch.zeros(K).to(backend), torch.ones(K).to(backend)
+    sums = bf.batch_norm_backward_packed(dy, None, 0.0, (packed, 2, scale, mn), None, mean, invstd, [False, True, True])
+    x_hat = extq.unpack_bf16param(packed, 2, scale, mn, N, K).double()
+    for got, terms in ((sums[1], dy.double() * x_hat), (sums[2], dy.double())):
+        assert ((got.double() - terms.sum(0)).abs() <= 1e-6 * terms.abs().sum(0)).all()
