@@ -63,7 +63,8 @@ _EXTRA_FIELDS = {
     # reference's chain qlinear -> qspmm keeps.  False: the chain.
     "gcn_single_node": True,
     # In that node the sparse product runs on the narrower side of the linear
-    # map: (A X) W^T when in < out, and, where no input gradient is wanted,
+    # map: (A X) W^T when in < out (or in = out and there is a bias, which that
+    # GEMM takes along), and, where no input gradient is wanted,
     # dW = dY^T (A X_hat) instead of (A^T dY)^T X_hat.  Same numbers up to the
     # order of fp32 sums; nothing kept changes.
     "gcn_aggregate_narrow": True,

@@ -587,6 +587,34 @@ def test_gcn_node_runs_the_sparse_product_on_the_narrow_side(backend):
         ext_spmm.spmm_csr = real
 
 
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("tall", [False, True])                                # the framework's GEMM and the tall one
+def test_gcn_layer_of_equal_widths(backend, tall, bias):
+    """in = out: the sparse product ahead of the linear map where that takes the bias along, behind it elsewhere; the
+    output and all gradients are those of the chain (fp32 sums of `width` and about 9 terms, in another order)."""
+    n, width = 500, 64
+    if tall:
+        config.tall_gemm_min_rows = config.tall_gemm_min_depth = 1
+    adj = gcn_norm(SparseTensor.from_scipy(er_graph(n, 8, 4)).set_value(None), add_self_loops=True).to(backend).fill_cache_()
+    conv = exact.QGCNConv(width, width, normalize=False, bias=bias).to(backend).train()
+    config.activation_compression_bits = [8]
+    g = torch.Generator().manual_seed(7)
+    x, dy = torch.randn(n, width, generator=g).to(backend), torch.randn(n, width, generator=g).to(backend)
+    got = []
+    for single in (True, False):
+        config.gcn_single_node = single
+        conv.zero_grad()
+        xd = x.clone().requires_grad_()
+        torch.manual_seed(9)
+        y = conv(xd, adj)
+        y.backward(dy)
+        got.append([y.detach(), xd.grad, conv.weight.grad] + ([conv.bias.grad] if bias else []))
+    for name, a, b in zip(("y", "dx", "dW", "db"), *got):
+        # dW goes through a copy of 8 bits, rounded at random: a code is worth 12 / 255, its error sums over n rows as sqrt(n)
+        allowed = 6 * 12 / 255 * n ** 0.5 * 2 if name == "dW" else 1e-5 * b.abs().max().item()
+        assert (a - b).abs().max().item() <= allowed, name
+
+
 def test_qmodule_conversion_and_state_dict(backend):
     net = GCN(16, 32, 4, 3, dropout=0.3, batch_norm=True)
     ref_keys = list(net.state_dict().keys())
