@@ -222,6 +222,13 @@ static void check_rp_mode(int mode, int64_t N, int64_t D, int64_t k, std::mt1993
   CHECK(tbytes > 0 && tbytes % 16 == 0, "rp table size");
   Buf<uint32_t> table(tbytes / 4);
   if (mode != 0) CHECK(exact_rp_prepare_bf16(R.p, D, k, mode, table.p, nullptr) == 0, "rp prepare rc");
+  if (mode == EXACT_RP_BF16_SIGNS) {  // the same matrix and table from its draws, in one launch
+    Buf<float> draws(D * k), R2(D * k);
+    Buf<uint32_t> table2(tbytes / 4);
+    for (int64_t i = 0; i < D * k; ++i) draws[i] = R[i] > 0.f ? 1.f : 0.f;
+    CHECK(exact_rp_draw_signs_f32(draws.p, D, k, c, R2.p, table2.p, nullptr) == 0, "rp draw rc");
+    CHECK(std::memcmp(R2.p, R.p, D * k * 4) == 0 && std::memcmp(table2.p, table.p, tbytes) == 0, "rp draw differs D=%ld k=%ld", (long)D, (long)k);
+  }
   oracle_rp_fwd(X.p, R.p, N, D, k, wxr.p);
   CHECK(rp_fwd_any(mode, X.p, R.p, table.p, N, D, k, xr.p) == 0, "rp fwd rc");
   double worst = 0, scale = 1e-30;
@@ -298,6 +305,24 @@ static void check_extra(int64_t M, int64_t ncols, int64_t K, double avg, std::mt
           }
         CHECK(bad == 0, "minmax differs M=%ld K=%ld max=%d valued=%d wide=%d: %ld cells", (long)M, (long)K, is_max, valued, wide, (long)bad);
       }
+  // values in another order: the entries back to front, and two indices that name none
+  Buf<_Float16> val16(nnz);
+  for (int64_t i = 0; i < nnz; ++i) val16[i] = (_Float16)val[i];
+  for (int wide = 0; wide < 2; ++wide)
+    for (int half = 0; half < 2; ++half) {
+      Buf<int64_t> at64(nnz);
+      Buf<int32_t> at32(nnz);
+      for (int64_t i = 0; i < nnz; ++i) { at64[i] = nnz - 1 - i; at32[i] = (int32_t)(nnz - 1 - i); }
+      if (nnz > 2) { at64[0] = at32[0] = -1; at64[1] = nnz; at32[1] = (int32_t)nnz; }
+      const void* index = wide ? (const void*)at64.p : (const void*)at32.p;
+      CHECK(exact_gather_values_f32(half ? (const void*)val16.p : (const void*)val.p, half, index, wide ? 8 : 4, nnz, nnz, ev.p, nullptr) == 0, "gather rc");
+      int64_t bad = 0;
+      for (int64_t i = 0; i < nnz; ++i) {
+        const bool none = at64[i] < 0 || at64[i] >= nnz;
+        bad += none ? ev[i] == ev[i] : ev[i] != (half ? (float)val16[nnz - 1 - i] : val[nnz - 1 - i]);
+      }
+      CHECK(bad == 0, "gather differs nnz=%ld half=%d wide=%d: %ld", (long)nnz, half, wide, (long)bad);
+    }
   for (int reduce = 0; reduce < 2; ++reduce)
     for (int wide = 0; wide < 2; ++wide) {
       const int rc = wide ? exact_sddmm_f32(row64.p, rp64.p, col64.p, 8, X.p, grad.p, nnz, K, reduce, ev.p, nullptr)
@@ -558,8 +583,12 @@ static void check_dw(int64_t N, int64_t K, int64_t D, int64_t pad, std::mt19937&
   Buf<float> dy(static_cast<size_t>(N * ldy)), x(static_cast<size_t>(N * ldx)), out(static_cast<size_t>(K * D));
   for (int64_t i = 0; i < N * ldy; ++i) dy[i] = static_cast<float>(id(rng));
   for (int64_t i = 0; i < N * ldx; ++i) x[i] = static_cast<float>(id(rng));
-  for (int bf16 = 0; bf16 < 2; ++bf16) {  // the fp32 and the bf16 matrix-core kernel
-    const int rc = bf16 ? exact_linear_dw_bf16_f32(dy.p, ldy, x.p, ldx, N, K, D, out.p, nullptr)
+  const int64_t scratch = exact_linear_dw_short_work_nbytes(N, K, D);
+  Buf<char> work(static_cast<size_t>(scratch));
+  for (int bf16 = 0; bf16 < 3; ++bf16) {  // the fp32 and the bf16 matrix-core kernel, and the fp32 one with its results in scratch
+    if (bf16 == 2 && scratch <= 0) continue;
+    const int rc = bf16 == 2 ? exact_linear_dw_short_f32(dy.p, ldy, x.p, ldx, N, K, D, out.p, work.p, nullptr)
+                   : bf16 ? exact_linear_dw_bf16_f32(dy.p, ldy, x.p, ldx, N, K, D, out.p, nullptr)
                         : exact_linear_dw_f32(dy.p, ldy, x.p, ldx, N, K, D, out.p, nullptr);
     CHECK(rc == 0, "dw rc %d", rc);
     for (int64_t k = 0; k < K; ++k)
@@ -785,6 +814,7 @@ int main(int argc, char** argv) {
     check_batch_norm(400, 1028, 8, true, 0, rng);
     check_batch_norm(300, 1100, 1, true, 1, rng);
     check_batch_norm(9001, 8, 2, true, 0, rng);
+    check_batch_norm(66049, 8, 2, true, 0, rng);  // 130 workgroups to a column: two in one of the 128 groups
     check_batch_norm(5003, 7, 2, true, 1, rng);
     std::printf("batch norm ok (failures so far %d)\n", g_fail);
     return g_fail != 0;
@@ -798,6 +828,7 @@ int main(int argc, char** argv) {
     check_dw(600, 130, 70, 0, rng);
     check_dw(513, 32, 200, 5, rng);
     check_dw(1100, 256, 256, 0, rng);
+    check_dw(4133, 40, 70, 1, rng);
     check_dw_half(1100, 256, 256, 0, rng);
     check_dw_half(40, 1000, 300, 0, rng);
     std::printf("dw shapes ok (failures so far %d)\n", g_fail);
