@@ -612,13 +612,15 @@ static void launch_dw(const float* dY, int64_t ldy, const float* X, int64_t ldx,
   const int blocks_d = (D + 32 * MD * WD - 1) / (32 * MD * WD);
   const int blocks = blocks_k * blocks_d;
   // About 1024 workgroups in all, whole batches per slab, and slabs no shorter than their results are worth.  The bf16
-  // forms walk a row in 0.068 us and 100,000 results a microsecond meet in memory.  512 rows throughout -> this: 16,384 rows
-  // 128 x 128 37.6 -> 23.4 us, 64 x 64 23.9 -> 12.9, 256 x 40 35.8 -> 19.3; 40,000 rows 41.9 -> 34.6, 25.0 -> 19.9, 44.4 ->
-  // 31.5; the same from 110,000 rows or 256 x 256 on.  From 200,000 on the many slabs of a small product meet at too few
-  // addresses (300,000 rows 128 x 16 53 -> 59): 512 there.
+  // forms walk a row in 0.068 us and 100,000 results a microsecond meet in memory; 64 slabs at most are made shorter than 512
+  // rows for that, since every slab is one more rounding of the growing sum.  (70,001 rows 20 x 100 in 487 slabs: the worst of
+  // 2000 results off by 40 - 71 times 2^-24 of their rms, 28 - 40 in 137 slabs of 512.)  512 rows throughout -> this: 16,384
+  // rows 128 x 128 37.4 -> 24.5 us, worst 28.7 -> 24.7 such units on average, 64 x 64 23.8 -> 15.3, 256 x 40 36.7 -> 25.8;
+  // 24,000 rows 128 x 128 38.1 -> 32.0, 30.3 -> 27.6 units; the same from 32,768 rows on.
   int64_t slabs = (1024 + blocks - 1) / blocks;
   int64_t rows = (N + slabs - 1) / slabs;
-  const int64_t least = BF16 && N < 200000 ? dw_slab_rows(N, Kout, D, 0.068, 1e-5, 128) : 512;
+  int64_t least = BF16 ? dw_slab_rows(N, Kout, D, 0.068, 1e-5, 128) : 512;
+  if (least < 512 && least * 64 < N) least = N < 512 * 64 ? (N + 63) / 64 : 512;
   if (rows < least) rows = least;
   rows = (rows + 15) / 16 * 16;  // whole batches (8 rows) resp. steps (16 rows)
   slabs = (N + rows - 1) / rows;
