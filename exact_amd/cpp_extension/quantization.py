@@ -233,9 +233,9 @@ def sign_matrix(bernoulli):
     D, k = bernoulli.shape
     matrix = torch.empty_like(bernoulli)
     table = torch.empty(_rp_table_nbytes(D, k, RP_BF16_SIGNS), dtype=torch.uint8, device=bernoulli.device)
-    # torch divides by a number by multiplying with its fp32 reciprocal, 1 / fp32(sqrt(k)) rounded once; a quotient of
-    # two fp32 numbers formed in fp64 and rounded is that same number
-    c = _fp32(1.0 / _fp32(k ** 0.5))
+    # torch divides a device tensor by a number by multiplying with 1 / number, formed in fp64 and rounded to fp32 once.
+    # (1 / fp32(sqrt(k)) is the neighbouring number for 31 of the 128 widths, k = 6, 7, 17, 18, .. 122, 127.)
+    c = _fp32(1.0 / k ** 0.5)
     rc = _lib.lib().exact_rp_draw_signs_f32(ptr(bernoulli), D, k, c, ptr(matrix), ptr(table), _checks.stream_ptr(bernoulli))
     _lib.check(rc, "sign_matrix")
     matrix._exact_sign_matrix = True

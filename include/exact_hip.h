@@ -409,7 +409,7 @@ int exact_rp_minmax_pack_f32(const float *X, const float *R, const float *noise,
 int64_t exact_rp_table_nbytes(int64_t D, int64_t k, int mode);
 int exact_rp_prepare_bf16(const float *R, int64_t D, int64_t k, int mode, void *table, void *stream);
 /* Draws to matrix and table in one launch: bernoulli[D, k] of 0 and 1 (fp32) -> R = c where it is 1, -c where it is 0
- * (ops.py:112-114, (2 b - 1) / sqrt(k) with c = 1 / sqrt(k) in fp32), and the SIGNS table of R.  Not in place. */
+ * (ops.py:112-114, (2 b - 1) / sqrt(k) with c = 1 / sqrt(k) rounded to fp32 once), and the SIGNS table of R.  Not in place. */
 int exact_rp_draw_signs_f32(const float *bernoulli, int64_t D, int64_t k, float c, float *R, void *table,
                             void *stream);
 int exact_rp_fwd_bf16_f32(const float *X, const void *table, int64_t N, int64_t D, int64_t k, int mode,

@@ -59,3 +59,14 @@ def test_drawn_matrix(backend, D, k):
     assert torch.equal(extq.rp_table(got, extq.RP_BF16_SIGNS), extq.rp_table(want, extq.RP_BF16_SIGNS))
     got += 0.0                                                            # written to: the kept table is not used any more
     assert torch.equal(extq.rp_table(got, extq.RP_BF16_SIGNS), extq.rp_table(want, extq.RP_BF16_SIGNS))
+
+
+def test_drawn_matrix_of_every_width(backend):
+    """Bit for bit the framework's (2 b - 1) / sqrt(k) on the device, which multiplies by 1 / sqrt(k) formed in fp64 and
+    rounded once; rounding sqrt(k) to fp32 first gives the neighbouring number for 31 of the 128 widths."""
+    for k in range(1, extq.RP_PACK_MAX_COLUMNS + 1):
+        draws = torch.randint(2, (3, k), dtype=torch.float32).to(backend)
+        got = extq.sign_matrix(draws)
+        assert torch.equal(got, (2.0 * draws - 1) * torch.tensor(1.0 / k ** 0.5, device=backend)), k
+        if backend.type == "cuda":
+            assert torch.equal(got, (2.0 * draws - 1) / k ** 0.5), k
