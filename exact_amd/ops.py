@@ -802,9 +802,10 @@ def take_compressed(tensor, project=True):
 def consumer_bits(input, for_consumer):  # noqa: A002
     """Bit width of the compressed copy the fused pass can make of its result for
     the next layer, or None where it cannot (needs 2-D fp32 rows of a multiple
-    of 8 <= 1024 columns, compression on, no projection, no autocast)."""
-    if (for_consumer and config.compress_activation and config.kept_frac == 1.0 and input.dim() == 2
-            and input.dtype == torch.float32 and not torch.is_autocast_enabled()
+    of 8 <= 1024 columns, compression on, no projection, no autocast, and a result
+    with a version, by which a copy is known to be of its values)."""
+    if (for_consumer and not torch.is_inference_mode_enabled() and config.compress_activation and config.kept_frac == 1.0
+            and input.dim() == 2 and input.dtype == torch.float32 and not torch.is_autocast_enabled()
             and not config.simulate and ext_quantization.fusable_width(input.shape[1])):
         return config.activation_compression_bits[0]
     return None

@@ -73,3 +73,18 @@ def test_what_hooks_and_other_layers_see_stays(backend, monkeypatch):
     config.kept_frac = 0.5                                                  # the next layer projects: no copy to make ahead
     _step(backend, make, x, gy, True)
     assert calls == [1]
+
+
+@pytest.mark.parametrize("norm", ["batch", None])
+def test_training_mode_under_inference_mode(backend, norm):
+    """A training-mode block whose results carry no version: nothing is handed over ahead, outputs and running statistics
+    are those of the layers one by one.  (8200 rows: sizes that take the one pass elsewhere.)"""
+    x = torch.randn(8200, 8, generator=torch.Generator().manual_seed(2)).to(backend)
+    got = []
+    for one_pass in (True, False):
+        config.fuse_epilogue = one_pass
+        config.noise_source = SeededNoise(5).noise_source
+        net = _net([8, 16, 8], norm, bias=norm is None, dropout=0.5).to(backend).train()
+        with torch.inference_mode():
+            got.append([net(x), *net.buffers()])
+    assert all(torch.equal(one, many) for one, many in zip(*got))
