@@ -786,9 +786,10 @@ def hand_over_compressed(tensor, quantized):
     _HANDED_OVER[tensor] = (tensor._version, quantized)
 
 
-def take_compressed(tensor, project=True):
+def take_compressed(tensor, project=True, scheme=None):
     """The compressed copy a fused producer made of exactly this tensor for a
-    consumer that would call quantize_activation(tensor) itself, or None."""
+    consumer that would call quantize_activation(tensor, scheme) itself, or None.
+    Taking one is a quantisation by that consumer as far as `scheme` goes."""
     entry = _HANDED_OVER.pop(tensor, None) if isinstance(tensor, torch.Tensor) else None
     if entry is None:
         return None
@@ -796,6 +797,8 @@ def take_compressed(tensor, project=True):
     usable = (config.compress_activation and version == tensor._version and not torch.is_autocast_enabled()
               and quantized[1] == config.activation_compression_bits[0]
               and not (project and config.kept_frac < 1.0))
+    if usable and scheme:
+        scheme.note_use()
     return quantized if usable else None
 
 

@@ -4,8 +4,9 @@ import pytest
 import torch
 
 import exact_amd as exact
-from exact_amd import layers
+from exact_amd import layers, ops
 from exact_amd.conf import config
+from exact_amd.qsheme import QScheme
 from gpu_util import SeededNoise
 
 
@@ -88,3 +89,29 @@ def test_training_mode_under_inference_mode(backend, norm):
         with torch.inference_mode():
             got.append([net(x), *net.buffers()])
     assert all(torch.equal(one, many) for one, many in zip(*got))
+
+
+@pytest.mark.parametrize("norm", ["batch", None])
+def test_the_consumers_scheme_is_noted(backend, norm):
+    """A copy made ahead counts as a quantisation by the layer that takes it, as where that layer makes its own."""
+    x = torch.randn(8200, 8, generator=torch.Generator().manual_seed(2)).to(backend)
+    for one_pass in (True, False):
+        config.fuse_epilogue = one_pass
+        net = _net([8, 16, 8], norm, dropout=0.5).to(backend).train()
+        QScheme.prev_layer = None
+        net(x)
+        assert net[-1].scheme is not None and QScheme.prev_layer is net[-1].scheme
+
+
+@pytest.mark.parametrize("conv", [exact.QGCNConv, exact.QSAGEConv])
+def test_the_scheme_of_a_convolution_is_noted(backend, monkeypatch, conv):
+    adj = exact.SparseTensor(torch.arange(34).to(backend), torch.arange(33).to(backend), None, (33, 33)).fill_cache_()
+    layer = (conv(8, 8, normalize=False) if conv is exact.QGCNConv else conv(8, 8)).to(backend).train()
+    scheme = layer.lin_scheme if conv is exact.QGCNConv else layer.scheme
+    handed = ops.relu_dropout(torch.randn(33, 8).to(backend), 0.5, for_consumer=True)
+    noted = []
+    monkeypatch.setattr(QScheme, "note_use", lambda self: noted.append(self))
+    layer(handed, adj)
+    with_copy = list(noted)
+    layer(handed.clone(), adj)
+    assert scheme in with_copy and noted == with_copy * 2
