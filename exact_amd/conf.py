@@ -51,13 +51,15 @@ _EXTRA_FIELDS = {
     "keep_unused_spmm_operand": False,
     # ReLU -> dropout -> (quantise for the next layer) as one pass where the
     # model offers the pair as one module (QReLUDropout) or the layers stand in
-    # a QMLP.  Results are
-    # bit-identical to the separate layers; False runs them separately.
+    # a QMLP.  Results are bit-identical to the separate layers; False runs them
+    # separately.
     "fuse_epilogue": True,
     # A QBatchNorm1d ahead of that pair joins the same pass (normalise -> ReLU ->
-    # dropout -> quantise).  The batch statistics then come from torch.var_mean
-    # instead of native_batch_norm, so results agree with the separate layers to
-    # rounding (about 1e-6 relative), not bit for bit.  Needs fuse_epilogue.
+    # dropout -> quantise).  Bit-identical to the separate layers from 8192 rows on,
+    # where both take the library's statistics; with fewer rows, or in the
+    # deterministic modes, the statistics of QReLUDropout's pass are not those of
+    # native_batch_norm and results agree to rounding (about 1e-6 relative), while a
+    # QMLP runs its layers separately.  Needs fuse_epilogue.
     "fold_batch_norm": True,
     # QGCNConv as one autograd node (aggregate(x W^T) + b) that keeps what the
     # reference's chain qlinear -> qspmm keeps.  False: the chain.

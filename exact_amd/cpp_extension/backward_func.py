@@ -246,6 +246,14 @@ def _column_vector(t, matrix):
                          and t.numel() == matrix.shape[1])
 
 
+def takes_batch_norm_statistics(matrix, weight, running_mean, running_var, bias=None):
+    """Whether batch_norm_statistics takes these operands."""
+    return (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
+            and 0 < matrix.shape[1] <= 8192 and 1024 <= matrix.shape[0] < 2 ** 31
+            and all(_column_vector(t, matrix) for t in (weight, bias, running_mean, running_var))
+            and (running_mean is None) == (running_var is None) and _atomics_allowed())
+
+
 def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, eps, bias=None):
     """The statistics half of native_batch_norm in training mode -> (mean,
     1 / sqrt(var + eps), weight * that), with running_mean / running_var updated
@@ -253,11 +261,7 @@ def batch_norm_statistics(matrix, weight, running_mean, running_var, momentum, e
     batch_norm_apply among what they need (the caller then takes the framework's
     routines, which refuse what is malformed).  From 1024 rows on: below, the
     framework's reduction is no slower."""
-    usable = (matrix.dim() == 2 and matrix.dtype == torch.float32 and _checks.on_device(matrix) and matrix.is_contiguous()
-              and 0 < matrix.shape[1] <= 8192 and 1024 <= matrix.shape[0] < 2 ** 31
-              and all(_column_vector(t, matrix) for t in (weight, bias, running_mean, running_var))
-              and (running_mean is None) == (running_var is None) and momentum is not None and _atomics_allowed())
-    if not usable:
+    if momentum is None or not takes_batch_norm_statistics(matrix, weight, running_mean, running_var, bias):
         return None
     N, K = matrix.shape
     L = _lib.lib()

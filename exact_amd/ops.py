@@ -315,7 +315,7 @@ def _batch_norm_backward_packed(grad_output, mask, p, kept, weight, mean, invstd
     return ext_backward_func.batch_norm_backward_packed(grad_output, mask, p, (packed, bits, scale, mn), weight, mean, invstd, wanted)
 
 
-def _large_enough_for_own_statistics(input):  # noqa: A002
+def large_enough_for_own_statistics(input):  # noqa: A002
     """Where the forward is bound by the device: below, it is one call into the
     framework against two into the library with an allocation each (38 - 45 against
     52 us up to 4096 rows, equal at [5000, 300], 62 against 52 at [20000, 128])."""
@@ -330,7 +330,7 @@ class qbatch_norm(Function):
                 training, exponential_average_factor, eps, scheme):
         kept = CompressedActivation.compress(input, scheme, project=False)
         stats = (ext_backward_func.batch_norm_statistics(input, weight, running_mean, running_var, exponential_average_factor, eps, bias)
-                 if training and _large_enough_for_own_statistics(input) else None)
+                 if training and large_enough_for_own_statistics(input) else None)
         if stats is not None:
             save_mean, save_invstd, mult = stats
             output = ext_backward_func.batch_norm_apply(input, save_mean, mult, bias)

@@ -28,19 +28,18 @@ def _net(widths, norm, **kw):
     return layers.QMLP(widths, norm, **kw)
 
 
+# below and from 8192 rows on (where the one pass begins), widths of whole octs and not (30, 36), a block behind a block
 @pytest.mark.parametrize("norm", ["batch", None])
-@pytest.mark.parametrize("N,widths", [(2, [8, 8, 4]), (33, [16, 24, 40, 8]), (1100, [12, 64, 10]), (50, [20, 30, 16])])   # 30: no multiple of 8
-def test_one_pass_equals_the_layers(backend, N, widths, norm):
+@pytest.mark.parametrize("p", [0.0, 0.3, 0.5])
+@pytest.mark.parametrize("N,widths", [(2, [8, 8, 4]), (33, [16, 24, 40, 8]), (1100, [12, 64, 10]), (50, [20, 30, 16]),
+                                      (8191, [4, 16, 4]), (8192, [4, 16, 24, 4]), (8193, [4, 40, 4]), (8200, [4, 36, 4])])
+def test_one_pass_equals_the_layers(backend, N, widths, p, norm):
+    """Bit for bit: results, gradients, running statistics.  (The sums of a bias gradient meet through atomics from 4096 rows on.)"""
     g = torch.Generator().manual_seed(N)
     x, gy = torch.randn(N, widths[0], generator=g), torch.randn(N, widths[-1], generator=g)
-    make = lambda: _net(widths, norm, bias=norm is None, dropout=0.5)       # noqa: E731
+    make = lambda: _net(widths, norm, bias=norm is None and N < 4096, dropout=p)    # noqa: E731
     for one, many in zip(_step(backend, make, x, gy, True), _step(backend, make, x, gy, False)):
-        # without a norm bit for bit; with one, its statistics are sums in another order: 1e-5 of the largest value, and
-        # a kept copy may round the other way where a value lies within that of a boundary (one level of 3 in a row)
-        if norm is None:
-            assert torch.equal(one, many)
-        else:
-            assert ((one - many).abs() <= 1e-4 * many.abs().max()).float().mean() > 0.98
+        assert torch.isfinite(one).all() and torch.equal(one, many)
 
 
 def test_what_hooks_and_other_layers_see_stays(backend, monkeypatch):
@@ -48,8 +47,13 @@ def test_what_hooks_and_other_layers_see_stays(backend, monkeypatch):
     real = layers.bn_relu_dropout
     monkeypatch.setattr(layers, "bn_relu_dropout", lambda *a: calls.append(1) or real(*a))
     g = torch.Generator().manual_seed(1)
-    x, gy = torch.randn(40, 16, generator=g), torch.randn(40, 8, generator=g)
-    make = lambda: _net([16, 16, 8], "batch", dropout=0.25)                 # noqa: E731
+    x, gy = torch.randn(8192, 4, generator=g), torch.randn(8192, 4, generator=g)
+    make = lambda: _net([4, 16, 4], "batch", dropout=0.25)                  # noqa: E731
+    _step(backend, make, x[1:], gy[1:], True)                               # too short: the framework's statistics
+    config.deterministic_reductions = True                                  # the framework's statistics as well
+    _step(backend, make, x, gy, True)
+    config.deterministic_reductions = False
+    assert calls == []
     _step(backend, make, x, gy, True)
     assert calls == [1]
     seen = []
