@@ -59,10 +59,10 @@ def _short_weight_gradient(grad_output, input):  # noqa: A002
             and 4096 <= grad_output.shape[0] < 16384 and grad_output.shape[0] == input.shape[0]
             and 0 < grad_output.shape[1] * input.shape[1] <= 65536
             and _checks.on_device(grad_output) and _checks.on_device(input) and grad_output.device == input.device
+            and not _checks.recorded(grad_output, input) and _checks.plain_values(grad_output, input)
             and grad_output.stride(1) == 1 and input.stride(1) == 1
             and grad_output.stride(0) >= grad_output.shape[1] and input.stride(0) >= input.shape[1]
-            and _atomics_allowed() and not _checks.recorded(grad_output, input) and _checks.plain_values(grad_output, input)
-            and not torch.compiler.is_compiling())
+            and _atomics_allowed() and not torch.compiler.is_compiling())
 
 
 def weight_gradient(grad_output, input):  # noqa: A002

@@ -70,3 +70,10 @@ def test_drawn_matrix_of_every_width(backend):
         assert torch.equal(got, (2.0 * draws - 1) * torch.tensor(1.0 / k ** 0.5, device=backend)), k
         if backend.type == "cuda":
             assert torch.equal(got, (2.0 * draws - 1) / k ** 0.5), k
+
+
+def test_drawn_matrices_under_vmap(backend):
+    """A draw inside a function transform has no memory of its own: the framework's expression."""
+    torch.manual_seed(3)
+    got = torch.vmap(lambda x: ops._projection_matrix(12, 5, x.device, x.dtype), randomness="different")(torch.zeros(2, 3, device=backend))
+    assert got.shape == (2, 12, 5) and torch.equal(got.abs(), torch.full_like(got, 1.0 / 5 ** 0.5))

@@ -7,6 +7,8 @@ have to stay within what the rounding of fp32 sums can do."""
 import pytest
 import torch
 
+from exact_amd import layers
+from exact_amd.conf import config
 from exact_amd.cpp_extension import backward_func as bf
 
 SHAPES = [(1, 5), (20, 100), (32, 129), (33, 128), (47, 300), (64, 130), (65, 30), (100, 64), (129, 65), (256, 200)]
@@ -133,3 +135,21 @@ def test_short_batches_under_a_recorded_backward(backend):
     out = bf.weight_gradient(dy, x)
     back, = torch.autograd.grad(out.sum(), dy)
     assert torch.allclose(back, x.sum(1, keepdim=True).expand(-1, 3), atol=1e-4)
+
+
+@pytest.mark.parametrize("N", [4096, 5000])
+def test_short_batches_whose_values_do_not_lie_in_plain_memory(backend, N):
+    """Function transforms, batched backward passes, sparse layouts and negated views: the framework's product, as
+    outside the range of the kernel."""
+    g = torch.Generator().manual_seed(N)
+    dy, x = torch.randn(3, N, 4, generator=g).to(backend), torch.randn(N, 5, generator=g).to(backend)
+    want = torch.stack([one.t().mm(x) for one in dy])
+    close = lambda got: torch.allclose(got, want, rtol=1e-4, atol=1e-3)     # noqa: E731  (sums of N products in two orders)
+    assert close(torch.vmap(bf.weight_gradient, (0, None))(dy, x))
+    assert close(torch.stack([torch.func.functionalize(bf.weight_gradient)(one, x) for one in dy]))
+    assert close(torch.stack([bf.weight_gradient(one, x.to_sparse_csr()) for one in dy]))
+    assert close(torch.stack([-bf.weight_gradient(torch._neg_view(one), x) for one in dy]))
+    layer = layers.QLinear(5, 4, bias=False).to(backend).train()
+    config.compress_activation = False
+    got, = torch.autograd.grad(layer(x), layer.weight, dy, is_grads_batched=True)
+    assert close(got)
