@@ -546,8 +546,8 @@ class qgcn(Function):
 
       forward   in < out: (A X) W^T + b, the bias folded into the GEMM; also
                 where in = out and there is a bias, which costs a pass of its
-                own otherwise ([169343, 256]: 25 us); else A (X W^T) + b as in
-                the reference.
+                own otherwise ([169343, 256]: 25 us), unless the graph has more
+                rows than x; else A (X W^T) + b as in the reference.
       backward  G = A^T dY serves both dX = G W and dW = G^T X_hat.  Where dX is
                 not wanted (the first layer) and the kept copy is narrower
                 than `out`, dW = dY^T (A X_hat) instead: the sparse product
@@ -561,7 +561,10 @@ class qgcn(Function):
     def forward(ctx, x, weight, bias, graph, reduce, kept):
         row, rowptr, col, value, rowcount, colptr, csr2csc = graph
         cout, cin = weight.shape
-        if config.gcn_aggregate_narrow and (cin < cout or (cin == cout and bias is not None)):
+        # of equal widths: where that GEMM takes the bias as it is, has no more rows to go through, and x is what its memory holds
+        with_bias = (cin == cout and bias is not None and bias.dtype == x.dtype and rowptr.numel() - 1 <= x.shape[0]
+                     and _checks.plain_values(x))
+        if config.gcn_aggregate_narrow and (cin < cout or with_bias):
             aggregated = spmm.spmm_csr(rowptr, col, value, x, reduce)
             out = ext_backward_func.tall_matmul(aggregated, weight, transposed=True, bias=bias)
             del aggregated

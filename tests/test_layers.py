@@ -605,14 +605,35 @@ def test_gcn_layer_of_equal_widths(backend, tall, bias):
         config.gcn_single_node = single
         conv.zero_grad()
         xd = x.clone().requires_grad_()
-        torch.manual_seed(9)
+        config.noise_source = SeededNoise(9).noise_source                      # the same copy of x on both routes
         y = conv(xd, adj)
         y.backward(dy)
         got.append([y.detach(), xd.grad, conv.weight.grad] + ([conv.bias.grad] if bias else []))
     for name, a, b in zip(("y", "dx", "dW", "db"), *got):
-        # dW goes through a copy of 8 bits, rounded at random: a code is worth 12 / 255, its error sums over n rows as sqrt(n)
-        allowed = 6 * 12 / 255 * n ** 0.5 * 2 if name == "dW" else 1e-5 * b.abs().max().item()
-        assert (a - b).abs().max().item() <= allowed, name
+        assert (a - b).abs().max().item() <= 1e-5 * b.abs().max().item(), name
+
+
+@pytest.mark.parametrize("change", ["double", "half", "rows", "negated"])
+def test_gcn_layer_of_equal_widths_keeps_its_order(backend, monkeypatch, change):
+    """A bias of another type, which the linear map cannot take along, a graph with more rows than the operand, and an
+    operand whose memory holds its negative: the linear map first, as in the reference."""
+    order = []
+    from exact_amd.cpp_extension import spmm as ext_spmm
+    real = ext_spmm.spmm_csr
+    monkeypatch.setattr(ext_spmm, "spmm_csr", lambda rowptr, col, value, mat, reduce: (order.append(mat), real(rowptr, col, value, mat, reduce))[1])
+    n, rows = 33, 40 if change == "rows" else 33
+    index = torch.arange(rows) % n
+    adj = SparseTensor(torch.arange(rows + 1).to(backend), index.to(backend), None, (rows, n)).fill_cache_()
+    conv = exact.QGCNConv(8, 8, normalize=False).to(backend).train()
+    conv.bias = torch.nn.Parameter(torch.arange(8.0, dtype={"double": torch.float64, "half": torch.float16}.get(change)).to(backend))
+    x = torch.randn(n, 8).to(backend)
+    given = torch._neg_view(x) if change == "negated" else x
+    y = conv(given, adj)
+    y.sum().backward()
+    want = given @ conv.weight.detach().t()
+    assert len(order) == 2 and torch.allclose(order[0], want, atol=1e-5)      # forward: behind the linear map (backward: dY)
+    assert y.dtype == torch.float32 and torch.allclose(y, want[index.to(backend)] + torch.arange(8.0, device=backend), atol=1e-5)
+    assert torch.equal(conv.bias.grad, torch.full_like(conv.bias, rows))
 
 
 def test_qmodule_conversion_and_state_dict(backend):
