@@ -185,7 +185,8 @@ def _transposed_values(value, csr2csc):
     value = value.detach()
     usable = (value.dtype in (torch.float32, torch.float16) and value.dim() == 1 and csr2csc.dim() == 1
               and csr2csc.dtype in (torch.int32, torch.int64) and value.is_contiguous() and csr2csc.is_contiguous()
-              and _checks.on_device(value) and value.device == csr2csc.device and value.numel() > 0)
+              and _checks.on_device(value) and value.device == csr2csc.device and value.numel() > 0
+              and _checks.plain_values(value, csr2csc))
     if not usable:
         return value.index_select(0, csr2csc)
     out = torch.empty(csr2csc.shape, dtype=torch.float32, device=value.device)

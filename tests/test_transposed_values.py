@@ -24,6 +24,13 @@ def test_strided_values_take_the_frameworks_gather(backend):
     assert torch.equal(spmm._transposed_values(value, torch.tensor([2, 0, 3]).to(backend)).cpu(), torch.tensor([6.0, 0.0, 9.0]))
 
 
+def test_values_that_do_not_lie_in_plain_memory_take_the_frameworks_gather(backend):
+    value, order = torch.arange(3.0).to(backend), torch.tensor([2, 0, 1]).to(backend)
+    want = value[order]
+    assert torch.equal(spmm._transposed_values(torch._neg_view(value), order), -want)
+    assert torch.equal(torch.vmap(spmm._transposed_values, (0, None))(torch.stack([value, 2 * value]), order), torch.stack([want, 2 * want]))
+
+
 def test_rows_follow_their_tensors(backend):
     row, order = torch.tensor([0, 0, 1, 2]).to(backend), torch.tensor([1, 3, 0, 2]).to(backend)
     first = spmm._transposed_rows(row, order)
