@@ -1,5 +1,7 @@
 """QMLP runs (batch norm ->) ReLU -> dropout ahead of a linear layer in one pass:
 against the same layers called one by one."""
+import warnings
+
 import pytest
 import torch
 
@@ -119,3 +121,23 @@ def test_the_scheme_of_a_convolution_is_noted(backend, monkeypatch, conv):
     with_copy = list(noted)
     layer(handed.clone(), adj)
     assert scheme in with_copy and noted == with_copy * 2
+
+
+@pytest.mark.parametrize("norm", ["batch", None])
+def test_a_trace_asks_for_no_sizes(backend, norm):
+    """A recorded or compiled block is its layers for every number of rows: nothing in it depends on those it was
+    recorded with, and there is no warning that something might."""
+    net = _net([8, 16, 8], norm, dropout=0.5).to(backend).eval()
+    x = torch.randn(8200, 8).to(backend)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error", torch.jit.TracerWarning)
+        traced = torch.jit.trace(net, x)
+    assert torch.equal(traced(x[:7]), net(x[:7]))
+    compilations = {}
+    for block in (net, torch.nn.Sequential(*net)):                          # as often as the layers one by one
+        torch.compiler.reset()
+        made = compilations[block] = []
+        compiled = torch.compile(block, backend=lambda graph, inputs: made.append(1) or graph.forward, fullgraph=True, dynamic=True)
+        for rows in (8200, 7, 8195):
+            assert torch.equal(compiled(x[:rows]), net(x[:rows]))
+    assert len(compilations[net]) == len(made)
