@@ -195,6 +195,10 @@ def linear_backward(grad_output, input, weight, bias, need_input_grad=True):  # 
 
 
 def native_batch_norm(input, weight, bias, running_mean, running_var, training, momentum, eps):  # noqa: A002
+    # The check of torch.batch_norm, which the native routine leaves to it: it would read and write past a short vector.
+    for name, t in (("running_mean", running_mean), ("running_var", running_var), ("weight", weight), ("bias", bias)):
+        if t is not None and input.dim() >= 2 and t.numel() != input.shape[1]:
+            raise RuntimeError(f"{name} should contain {input.shape[1]} elements not {t.numel()}")
     return torch.ops.aten.native_batch_norm(input, weight, bias, running_mean, running_var, training, momentum, eps)
 
 

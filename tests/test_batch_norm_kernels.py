@@ -4,7 +4,7 @@ the same formulas in float64 on the dequantised input."""
 import pytest
 import torch
 
-from exact_amd import ops
+from exact_amd import layers, ops
 from exact_amd.conf import config
 from exact_amd.cpp_extension import backward_func as bf
 from exact_amd.cpp_extension import quantization as extq
@@ -167,6 +167,24 @@ def test_malformed_column_vectors_are_refused(backend, monkeypatch):
             bf.batch_norm_apply(x.detach(), mean, mult, torch.zeros(12))
     with pytest.raises(RuntimeError):
         bf.batch_norm_apply(x.detach()[:, :6], mean[:6], mult[:6], None)
+
+
+@pytest.mark.parametrize("which", ["weight", "bias", "running"])
+def test_vectors_of_another_length_are_refused(backend, which):
+    """3-D input whose second dimension is not the layer's, or vectors replaced: an error as from torch.nn.BatchNorm1d,
+    whose check the native routine leaves out (it would read, and for running statistics write, past their end)."""
+    x = torch.randn(6, 40, 16).to(backend)
+    layer = layers.QBatchNorm1d(16, affine=which != "running", track_running_stats=which == "running").to(backend).train()
+    with pytest.raises(RuntimeError, match="should contain 40 elements not 16"):
+        layer(x)
+    good = layers.QBatchNorm1d(40).to(backend).train()
+    y = good(x)
+    assert torch.allclose(y, torch.nn.BatchNorm1d(40).to(backend)(x), atol=1e-5)
+    vectors = dict(weight=None, bias=None, running_mean=None, running_var=None)
+    for name in (("running_mean", "running_var") if which == "running" else (which,)):
+        short = dict(vectors, **{name: torch.ones(39).to(backend)})
+        with pytest.raises(RuntimeError, match=name + " should contain 40 elements not 39"):
+            bf.native_batch_norm(x, short["weight"], short["bias"], short["running_mean"], short["running_var"], True, 0.1, 1e-5)
 
 
 @pytest.mark.parametrize("p", [0.0, 0.5, 0.75, 0.3])                   # 1 - p: three powers of two and another number
