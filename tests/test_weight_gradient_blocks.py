@@ -100,8 +100,10 @@ def test_half_operands_give_equal_bits_twice(backend, K, D):
 @pytest.mark.parametrize("K,D", [(1, 1), (33, 128), (32, 130), (64, 70), (40, 256), (130, 32), (96, 64), (65, 100), (256, 256)])
 @pytest.mark.parametrize("N", [4096, 4161, 5000])
 def test_short_batches(backend, N, K, D):
-    """At most N / 2 + 16 additions in a chain (two rows a product, at most 80 slabs in eight chains), each wrong by at most
-    2^-24 of the absolute terms; in a fixed order, infinities where fp32 has them."""
+    """In a fixed order, infinities where fp32 has them, and off by what the rounding of the sums does: a slab adds some 64 to
+    80 rows one after the other (a standard deviation of 0.3 x sqrt(80 / 2) x 2^-24 of its rms), about ten slabs follow each
+    other in eight chains (0.3 x sqrt(10 / 2) of the whole) and the chains are added (0.3 x sqrt(8 / 2)): 2.2 x 2^-24 of the
+    rms of the whole, and ten of them are allowed.  An operand cut to 16 bits is off by 2^-17 of the rms, 128 x 2^-24."""
     if N > 4096 and K * D > 20000 and backend.type == "cpu":
         pytest.skip("slow on the emulator")
     g = torch.Generator().manual_seed(N + 7 * K + D)
@@ -120,7 +122,7 @@ def test_short_batches(backend, N, K, D):
     assert calls == ["exact_linear_dw_short_work_nbytes"] * 3 and torch.equal(got, again)
     dy[3, 0] = x[N - 1, D - 1] = 0.0
     # (both tensors had a finite value there before: compare what those rows do not reach)
-    want, bound = dy.double().t() @ x.double(), (N // 2 + 20) * 2.0 ** -24 * (dy.double().abs().t() @ x.double().abs())
+    want, bound = dy.double().t() @ x.double(), 22 * 2.0 ** -24 * ((dy.double() ** 2).t() @ (x.double() ** 2)).sqrt()
     keep = torch.ones(K, D, dtype=torch.bool, device=got.device)
     keep[0, :] = False
     keep[:, D - 1] = False
@@ -128,6 +130,12 @@ def test_short_batches(backend, N, K, D):
     if K > 1 and D > 1:
         assert torch.isinf(ends[0, : D - 1]).all() and torch.isinf(ends[1:, D - 1]).all()
         assert torch.equal(ends[1:, : D - 1], got[1:, : D - 1])
+
+
+@pytest.mark.parametrize("K,D", [(1, 5), (20, 40), (33, 128), (65, 100), (130, 32)])
+@pytest.mark.parametrize("N", [4096, 4161])
+def test_integers_are_exact_in_short_batches(backend, N, K, D):
+    _check_integers(backend, N, K, D, torch.float32)
 
 
 def test_short_batches_under_a_recorded_backward(backend):
