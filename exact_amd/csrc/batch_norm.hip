@@ -50,23 +50,20 @@ __device__ __forceinline__ void bn_load(const float* p, float (&v)[VEC]) {
 // that columns far from zero lose nothing either: deviations are differences of means, of which fp32 at 300 would leave
 // 3e-5 units.
 __device__ __forceinline__ void bn_join(float na, double& mean, float& dev, float nb, double mean_b, float dev_b) {
-  if (nb == 0.f) return;
-  if (na == 0.f) {
-    mean = mean_b;
-    dev = dev_b;
-    return;
-  }
   const float share = nb / (na + nb);
   const double d = mean_b - mean;
   const float df = static_cast<float>(d);
-  mean += d * static_cast<double>(share);
-  dev = dev + dev_b + df * df * (na * share);
+  const double both_mean = mean + d * static_cast<double>(share);
+  const float both_dev = dev + dev_b + df * df * (na * share);
+  // selects, no branches: a chain of joins has its divisions ahead of it
+  mean = nb == 0.f ? mean : na == 0.f ? mean_b : both_mean;
+  dev = nb == 0.f ? dev : na == 0.f ? dev_b : both_dev;
 }
 
 // Mean and squared deviations of a workgroup's rows, per column: partial[workgroup][3][K], the mean as the sum of two
 // floats.  A thread takes eight rows at a time: their mean and their deviations from it, formed from the differences to
-// the first of them, joined to what it has.  Bound by reading x: [50000, 512] 20 us of 102 MB and [169343, 256] 33 us,
-// and 9 us each for the small kernel behind (50 and 46 us when sums about a sampled centre met through atomics).
+// the first of them, joined to what it has.  Bound by reading x: with the small kernel behind, [50000, 512] takes 33 us
+// and [169343, 256] 43 over operands that rotate.
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restrict__ x, int64_t N, int K, int64_t rows_per_wg,
                                                             float* __restrict__ partial) {
@@ -144,60 +141,58 @@ __global__ __launch_bounds__(kBlock) void bn_moments_kernel(const float* __restr
   }
 }
 
-// The kernels that take the workgroups of a column: 8 columns x 128 groups, each group every 128th of the workgroups in
-// their order, then the groups pair by pair.  Bound by latency: a column has at most 1024 workgroups, so all its numbers
-// are loaded at once, and seven steps join 128 groups.  (32 groups loaded up to four times and were joined one behind
-// the other: at [169343, 256] statistics 41.7 us, now 38.7, the backward's sums 45.5, now 37.4; [9000, 256] 18.5 -> 15.4
-// and 13.9 -> 10.1.  At [8200, 8000], 1000 of these workgroups, the sums take 56.1 where they took 54.6.)
-constexpr int kBnCols = 8, kBnGroups = 128, kBnFlight = 8, kBnEndBlock = kBnCols * kBnGroups;
+// The kernels that take the workgroups of a column in their order: 8 columns x 32 groups of workgroups, each group
+// every 32nd of them, then the groups.  Bound by latency: a group's numbers are loaded at once (eight at a time with a
+// branch around each before) and its divisions are formed ahead of the chain that needs them.  Both on one card:
+// statistics at [169343, 256] 44.1 -> 42.7 us, [50000, 512] 33.7 -> 32.6, [9000, 256] 19.8 -> 18.3, [8200, 8000] 58.9 ->
+// 59.5; the backward at [9000, 256] 23.8 -> 19.0.  (128 groups joined pair by pair end 2 to 4 us sooner: 40.7, 30.6, 16.8
+// and 55.7.  But their statistics have other last bits, and behind a quantiser those are other codes.)
+constexpr int kBnCols = 8, kBnGroups = kBlock / kBnCols, kBnFinishFlight = 16, kBnSumsFlight = 32;
 
 // -> mean, 1 / sqrt(var + eps), weight * that, and the running statistics with torch's bookkeeping: one launch where
 // the framework's element-wise routines took fourteen.
-__global__ __launch_bounds__(kBnEndBlock) void bn_finish_kernel(const float* __restrict__ partial, int64_t wgs, int64_t rows_per_wg,
+__global__ __launch_bounds__(kBlock) void bn_finish_kernel(const float* __restrict__ partial, int64_t wgs, int64_t rows_per_wg,
                                                            int64_t N, int K, float eps, float factor,
                                                            const float* __restrict__ weight, float* __restrict__ running_mean,
                                                            float* __restrict__ running_var, float* __restrict__ mean,
                                                            float* __restrict__ invstd, float* __restrict__ mult) {
-  __shared__ double part_mean[kBnEndBlock];
-  __shared__ float part_dev[kBnEndBlock], count[kBnEndBlock];
+  __shared__ double part_mean[kBlock];
+  __shared__ float part_dev[kBlock], count[kBlock];
   const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
   const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
   const float* src = partial + (k < K ? k : K - 1);
   double m = 0.;
   float n = 0.f, dev = 0.f;
-  for (int64_t w = g; w < wgs; w += kBnGroups * kBnFlight) {
-    float hi[kBnFlight], lo[kBnFlight], pd[kBnFlight];
+  for (int64_t w = g; w < wgs; w += kBnGroups * kBnFinishFlight) {
+    float hi[kBnFinishFlight], lo[kBnFinishFlight], pd[kBnFinishFlight];
 #pragma unroll
-    for (int i = 0; i < kBnFlight; ++i) {
+    for (int i = 0; i < kBnFinishFlight; ++i) {
       const float* p = src + (w + i * kBnGroups < wgs ? w + i * kBnGroups : w) * 3 * K;
       hi[i] = p[0];
       lo[i] = p[K];
       pd[i] = p[2 * K];
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < kBnFlight; ++i) {
+    for (int i = 0; i < kBnFinishFlight; ++i) {
       const int64_t at = w + i * kBnGroups;
-      if (at >= wgs) break;
       const int64_t left = N - at * rows_per_wg;
-      const float rows = static_cast<float>(left < rows_per_wg ? left : rows_per_wg);
+      const float rows = at >= wgs ? 0.f : static_cast<float>(left < rows_per_wg ? left : rows_per_wg);
       bn_join(n, m, dev, rows, static_cast<double>(hi[i]) + static_cast<double>(lo[i]), pd[i]);
       n += rows;
     }
   }
-  for (int half = kBnGroups / 2; half > 0; half /= 2) {
-    if (g >= half && g < 2 * half) {
-      count[t] = n;
-      part_mean[t] = m;
-      part_dev[t] = dev;
-    }
-    __syncthreads();
-    if (g < half) {
-      const int o = t + half * kBnCols;
-      bn_join(n, m, dev, count[o], part_mean[o], part_dev[o]);
-      n += count[o];
-    }
-  }
+  count[t] = n;
+  part_mean[t] = m;
+  part_dev[t] = dev;
+  __syncthreads();
   if (g != 0 || k >= K) return;
+#pragma unroll
+  for (int i = 1; i < kBnGroups; ++i) {
+    const int o = i * kBnCols + c;
+    bn_join(n, m, dev, count[o], part_mean[o], part_dev[o]);
+    n += count[o];
+  }
   const float rows = static_cast<float>(N);
   const float var = dev / rows;
   const float inv = 1.f / sqrtf(var + eps);
@@ -213,41 +208,39 @@ __global__ __launch_bounds__(kBnEndBlock) void bn_finish_kernel(const float* __r
 }
 
 // The same for plain sums: sums[0 .. K) and sums[K .. 2 K), and the gradient of the weight.
-__global__ __launch_bounds__(kBnEndBlock) void bn_sums_kernel(const float* __restrict__ partial, int64_t wgs, int K,
+__global__ __launch_bounds__(kBlock) void bn_sums_kernel(const float* __restrict__ partial, int64_t wgs, int K,
                                                          const float* __restrict__ invstd, float* __restrict__ sums,
                                                          float* __restrict__ grad_weight) {
-  __shared__ float part[2][kBnEndBlock];
+  __shared__ float part[2][kBlock];
   const int t = threadIdx.x, c = t % kBnCols, g = t / kBnCols;
   const int k = static_cast<int>(blockIdx.x) * kBnCols + c;
   const float* src = partial + (k < K ? k : K - 1);
   float s0 = 0.f, s1 = 0.f;
-  for (int64_t w = g; w < wgs; w += kBnGroups * kBnFlight) {
-    float p0[kBnFlight], p1[kBnFlight];
+  for (int64_t w = g; w < wgs; w += kBnGroups * kBnSumsFlight) {
+    float p0[kBnSumsFlight], p1[kBnSumsFlight];
 #pragma unroll
-    for (int i = 0; i < kBnFlight; ++i) {
+    for (int i = 0; i < kBnSumsFlight; ++i) {
       const int64_t at = w + i * kBnGroups < wgs ? w + i * kBnGroups : w;
       p0[i] = src[at * 2 * K];
       p1[i] = src[at * 2 * K + K];
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < kBnFlight; ++i) {
-      if (w + i * kBnGroups >= wgs) break;
-      s0 += p0[i];
-      s1 += p1[i];
+    for (int i = 0; i < kBnSumsFlight; ++i) {
+      const bool there = w + i * kBnGroups < wgs;
+      s0 = there ? s0 + p0[i] : s0;
+      s1 = there ? s1 + p1[i] : s1;
     }
   }
-  for (int half = kBnGroups / 2; half > 0; half /= 2) {
-    if (g >= half && g < 2 * half) {
-      part[0][t] = s0;
-      part[1][t] = s1;
-    }
-    __syncthreads();
-    if (g < half) {
-      s0 += part[0][t + half * kBnCols];
-      s1 += part[1][t + half * kBnCols];
-    }
-  }
+  part[0][t] = s0;
+  part[1][t] = s1;
+  __syncthreads();
   if (g != 0 || k >= K) return;
+#pragma unroll
+  for (int i = 1; i < kBnGroups; ++i) {
+    s0 += part[0][i * kBnCols + c];
+    s1 += part[1][i * kBnCols + c];
+  }
   sums[k] = s0;
   sums[K + k] = s1;
   if (grad_weight) grad_weight[k] = s1 * invstd[k];
@@ -300,8 +293,8 @@ __global__ __launch_bounds__(kBlock) void bn_apply_kernel(const float* __restric
 // each read dy, one mask bit and `bits` code bits per element: neither the masked gradient nor the dequantised
 // input is ever written to memory.  A thread takes four consecutive rows of its four columns per step: with 1 and 2
 // bits their codes are one 32-bit word, and four 16-byte loads of dy are in flight.  At [169343, 256] INT2 with a
-// mask the passes and the sums between them take 111 us where mask 58 + dequantise 36 + reduce 68 + apply
-// 100 were; at [50000, 512] without one 87 for dequantise 22 + reduce 699 + apply 59.
+// mask the passes and the sums between them take 115 us where mask 58 + dequantise 36 + reduce 68 + apply
+// 100 were; at [50000, 512] without one 83 for dequantise 22 + reduce 699 + apply 59.
 struct BnBackward {
   const float* dy;
   const uint32_t* mask;  // null: g = dy
@@ -322,7 +315,8 @@ struct BnBackward {
 
 // MASK: 0 none, 1 behind a mask with 1 - p a power of two (the gradient times its reciprocal is the quotient, exactly),
 // 2 behind any other.  Nothing here branches by element: with a branch around each quotient and each masked gradient
-// the two passes were bound by the vector instructions (160 -> 119 us with 1 - p = 1 / 2, 130 with 0.7, both with 8 more of the sums between, at [169343, 256] INT2).
+// the two passes were bound by the vector instructions (with the sums between them, at [169343, 256] INT2: 160 -> 115 us
+// with 1 - p = 1 / 2, 160 -> 126 with 0.7, 116 -> 110 without a mask).
 template <int BITS, int MASK>
 __device__ __forceinline__ void bn_bwd_rows(const BnBackward& a, int64_t row, int k, float (&g)[4][4], float (&x)[4][4]) {
   constexpr int WPT = 8 / BITS;
@@ -464,7 +458,8 @@ __global__ __launch_bounds__(kBlock) void bn_bwd_apply_kernel(const BnBackward a
 // Rows per workgroup.  A reduction stores two or three numbers per column and workgroup and reads them again, so its
 // workgroups are few and long-lived, with at least 16 KiB of the stream each.  Statistics: 512 in fours of columns
 // ([50000, 512] 28 against 34 us with 1024), 1024 otherwise ([100003, 301] 37 against 47 with 512, whose wavefronts have
-// a quarter of the bytes in flight).  The backward's: 1024 ([169343, 256] both passes 116 against 123).  An element-wise
+// a quarter of the bytes in flight).  The backward's: 1024 ([169343, 256] with a mask 114 us, 116 with 512, 118 with 2048;
+// [50000, 512] 85.6, 85.8 and 89.4).  An element-wise
 // pass has no such end: 8192, which evens out the last wave.
 constexpr int kBnApplyWgs = 8192, kBnBackwardWgs = 1024;
 template <int VEC>
@@ -489,7 +484,7 @@ static void launch_bn_backward(BnBackward a, float* grad_weight, hipStream_t s) 
   a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnBackwardWgs, 4);
   const dim3 grid = bn_grid(a.N, a.K, 4, a.rows_per_wg);
   hipLaunchKernelGGL((bn_bwd_reduce_kernel<BITS, MASK>), grid, dim3(kBlock), 0, s, a);
-  hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBnEndBlock), 0, s, a.partial,
+  hipLaunchKernelGGL(bn_sums_kernel, dim3(static_cast<unsigned>((a.K + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, a.partial,
                      static_cast<int64_t>(grid.x), a.K, a.invstd, a.sums, grad_weight);
   if (a.dx) {
     a.rows_per_wg = bn_rows_per_wg(a.N, a.K, 4, kBnApplyWgs, 4);
@@ -543,7 +538,7 @@ int exact_bn_statistics_f32(const float* x, int64_t N, int64_t K, float eps, flo
   int64_t rows = 0, wgs = 0;
   if (K % 4 == 0 && on(x, 16)) launch_bn_moments<4>(x, N, k, work, rows, wgs, s);
   else launch_bn_moments<1>(x, N, k, work, rows, wgs, s);
-  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((k + kBnCols - 1) / kBnCols)), dim3(kBnEndBlock), 0, s, work, wgs, rows, N,
+  hipLaunchKernelGGL(bn_finish_kernel, dim3(static_cast<unsigned>((k + kBnCols - 1) / kBnCols)), dim3(kBlock), 0, s, work, wgs, rows, N,
                      k, eps, factor, weight, running_mean, running_var, mean, invstd, mult);
   return launch_status();
 }

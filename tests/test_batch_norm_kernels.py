@@ -1,11 +1,13 @@
 """The batch norm on wide matrices and on the packed copy of its input
 (exact_bn_statistics_f32, exact_bn_apply_f32, exact_bn_backward_ordered_f32) against
 the same formulas in float64 on the dequantised input."""
+import numpy as np
 import pytest
 import torch
 
-from exact_amd import layers, ops
+from exact_amd import _lib, layers, ops
 from exact_amd.conf import config
+from exact_amd.cpp_extension import _checks
 from exact_amd.cpp_extension import backward_func as bf
 from exact_amd.cpp_extension import quantization as extq
 
@@ -225,3 +227,70 @@ def test_the_workgroups_of_a_column_whatever_their_number(backend, wgs):
     x_hat = extq.unpack_bf16param(packed, 2, scale, mn, N, K).double()
     for got, terms in ((sums[1], dy.double() * x_hat), (sums[2], dy.double())):
         assert ((got.double() - terms.sum(0)).abs() <= 1e-6 * terms.abs().sum(0)).all()
+
+
+def _in_groups_of_32(parts, start, add):
+    """The order of the kernels that end a reduction: group g takes the workgroups g, g + 32, .. one after the other, then
+    the groups follow each other."""
+    def chain(items):
+        total = start
+        for one in items:
+            total = add(total, one)
+        return total
+    groups = [chain(parts[g::32]) for g in range(min(32, len(parts)))]
+    total = groups[0]
+    for one in groups[1:]:
+        total = add(total, one)
+    return total
+
+
+def _rows_per_workgroup(N, K, vec, workgroups, multiple):
+    block = 256 * vec
+    cols = min(K, block)
+    rows = max(-(-N * -(-K // block) // workgroups), -(-4096 // cols))
+    turn = 256 // (cols // vec) * multiple
+    return -(-rows // turn) * turn
+
+
+# workgroups fewer than the groups, a few to a group, more than the 16 and 32 that are loaded at once
+@pytest.mark.parametrize("N,K", [(1100, 4), (2049, 256), (9000, 256), (2500, 257), pytest.param(50001, 101, marks=pytest.mark.gpu),
+                                 pytest.param(169343, 256, marks=pytest.mark.gpu)])
+def test_the_sums_of_workgroups_keep_their_order(backend, N, K):
+    """Bit for bit: behind a quantiser, statistics that differ in a last bit are other codes."""
+    if backend.type == "cpu" and N > 9000:
+        pytest.skip("slow on the emulator")
+    g = torch.Generator().manual_seed(N)
+    x, dy = (torch.randn(N, K, generator=g).to(backend) for _ in range(2))
+    L, ptr = _lib.lib(), _checks.ptr
+    work = torch.full((bf._scratch_size("exact_bn_work_floats", N, K),), float("nan"), device=backend)
+    mean, invstd, mult = torch.empty((3, K), device=backend)
+    _lib.check(L.exact_bn_statistics_f32(ptr(x), N, K, 1e-5, 0.1, None, None, None, ptr(work), ptr(mean), ptr(invstd), ptr(mult),
+                                         _checks.stream_ptr(x)), "statistics")
+    rows = _rows_per_workgroup(N, K, 4, 512, 1) if K % 4 == 0 else _rows_per_workgroup(N, K, 1, 1024, 1)
+    workgroups = -(-N // rows)
+    parts = work[:workgroups * 3 * K].view(workgroups, 3, K).cpu().numpy()
+    assert not np.isnan(parts).any()
+    f32 = np.float32
+
+    def join(a, b):
+        (na, ma, da), (nb, mb, db) = a, b
+        if na == 0:
+            return b
+        share, d = f32(nb / f32(na + nb)), mb - ma
+        df = d.astype(f32)
+        return f32(na + nb), ma + d * np.float64(share), da + db + df * df * f32(na * share)
+    sets = [(f32(min(rows, N - w * rows)), p[0].astype(np.float64) + p[1].astype(np.float64), p[2]) for w, p in enumerate(parts)]
+    _, m, dev = _in_groups_of_32(sets, (f32(0), None, None), join)
+    assert np.array_equal(mean.cpu().numpy(), m.astype(f32))
+    assert np.array_equal(invstd.cpu().numpy(), f32(1) / np.sqrt(dev / f32(N) + f32(1e-5)))
+    if K % 4:
+        return
+    packed, scale, mn = extq.minmax_pack(x, 2)
+    work.fill_(float("nan"))
+    sums = torch.empty((2, K), device=backend)
+    _lib.check(L.exact_bn_backward_ordered_f32(ptr(dy), None, 0.0, ptr(packed), 2, ptr(scale), ptr(mn), ptr(mean), ptr(invstd), None, N, K,
+                                               ptr(work), ptr(sums), None, None, _checks.stream_ptr(x)), "backward")
+    workgroups = -(-N // _rows_per_workgroup(N, K, 4, 1024, 4))
+    parts = work[:workgroups * 2 * K].view(workgroups, 2, K).cpu().numpy()
+    assert not np.isnan(parts).any()
+    assert np.array_equal(sums.cpu().numpy(), _in_groups_of_32(list(parts), np.zeros((2, K), f32), lambda a, b: a + b))
