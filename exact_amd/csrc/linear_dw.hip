@@ -577,9 +577,12 @@ static int64_t dw_slab_rows(int64_t N, int K, int D, double row_us, double value
   rows = rows < least ? least : rows > 512 ? 512 : rows;
   return (rows + 15) / 16 * 16;
 }
-// fp32, short batches: a row takes 0.11 us, a result 8 bytes of traffic.  Against the framework's GEMM, which does not
-// split the rows: 4,096 rows 128 x 128 15.7 / 24.5 us, 64 x 64 10.3 / 32, 256 x 256 22.9 / 25.3; 16,000 rows 23.8 / 84,
-// 13.0 / 113, 46.7 / 86, 256 x 602 97 / 93.
+// fp32, short batches: each further row of a slab costs 0.06 (64 x 64 results) to 0.13 us (256 x 256), taken as 0.11, and
+// a result 8 bytes of traffic; the launches, the first loads and the finish are another 6 to 12 us.  Both kernels, 16 / 32
+// / 64 / 128 / 256 / 512 rows a slab: 4,096 rows 64 x 64 9.8 / 9.2 / 10.3 / 14.3 / 22.5 / 39 us, 256 x 256 38 / 22 / 21 /
+// 28 / 45 / 81; 16,000 rows 17.6 / 14.6 / 13.5 / 17.4 / 27 / 46 and 149 / 90 / 59 / 46 / 49 / 82.  Against the framework's
+// GEMM: 4,096 rows 64 x 64 10.2 / 32.7, 128 x 128 17.7 / 25.2, 256 x 256 25.7 / 25.4; 16,383 rows 14.1 / 120, 25.2 / 98,
+// 46.8 / 105.
 static DwOrderedPlan plan_dw_short(int64_t N, int K, int D) {
   DwOrderedPlan p = plan_dw_blocks(K, D);
   p.rows = dw_slab_rows(N, K, D, 0.11, 2e-6, 64);

@@ -155,9 +155,9 @@ __device__ __forceinline__ void wave_sync_lds() {
 // eight features of one row, but loads in that arrangement touch 64 pieces of 16 bytes in 32 rows and ran at 3 TB/s
 // (190 us at 602 -> 76 columns of 232,965 rows).  So 16 lanes read 256 consecutive bytes of a row, the chunk passes
 // through a tile in LDS that belongs to the wavefront (its accesses complete in order), and the lanes read their
-// features from there; the next chunk's loads fly while this one is multiplied.  Before -> after, with the quantiser:
-// 602 -> 76 of 232,965 rows 190 -> 153 us, 301 -> 38 of 100,000 52 -> 35, 100 -> 25 of 2.4 M 268 -> 223, 256 -> 64 of
-// 2.4 M 591 -> 525, 256 -> 32 of 169,343 38.6 -> 36.4.  At 602 -> 76 the loads and the hand-over alone take 120 us (a
+// features from there; the next chunk's loads fly while this one is multiplied.  Before -> after, with the quantiser, both on
+// one card: 602 -> 76 of 232,965 rows 185 -> 156 us, 301 -> 38 of 100,000 54 -> 37, 100 -> 25 of 2.4 M 269 -> 224, 256 -> 64
+// of 2.4 M 581 -> 515, 256 -> 32 of 169,343 39.6 -> 37.6, 602 -> 76 of 20,000 34 -> 24.  At 602 -> 76 the loads and the hand-over alone take 120 us (a
 // kernel that only reads in 256-byte runs 98), the split and the products the rest.  Four wavefronts that share the
 // fragments through LDS: 148 us there, but 28 instead of 22 at 20,000 rows, whose workgroups then miss half the chip;
 // two chunks in flight: 166.
@@ -1113,8 +1113,10 @@ static void rp_bwd_rows_launch(const float* Xr, const u32x4* table, int64_t N, i
 // Whether rp_bwd_rows_kernel took the product.
 static bool rp_bwd_rows(const float* Xr, const u32x4* table, int64_t N, int D, int k, float* out, hipStream_t s) {
   const int steps = (k + kStepFeatures - 1) / kStepFeatures, tw = ((D + kTile - 1) / kTile + 3) / 4;
-  // Measured over cold operands, this form / the other: 602 -> 232,965 rows of 76 128 / 196 us, of 61 130 / 199, 640 of 100,000
-  // 62 / 89, 480 of 60,000 30 / 37, 301 of 100,000 31 / 39, 130 of 200,000 30 / 37; up to 256 columns of whole lines (256 of
+  // Measured over cold operands, this form / the other: 602 columns of 232,965 rows from 76 133 / 196 us, from 61 131 / 200, 640
+  // of 200,000 from 80 123 / 159, 480 of 60,000 30 / 37, 301 of 100,000 28 / 34, 130 of 200,000 30 / 37; more than 5 steps (k > 80)
+  // or 5 tiles a wavefront (D > 640) have no instance of this form, and the other takes 256 us for 602 columns of 200,000 rows from
+  // 121, 166 for 500 from 100, 148 for 400 from 100 and 181 for 700 from 70 (2.3 - 3.4 TB/s); up to 256 columns of whole lines (256 of
   // 2.4 M rows 654 / 604) and up to 128 of any (100 of 2.4 M 245 / 231) the other is as fast or faster, and so it is
   // where the tiles do not reach every compute unit (602 of 3,000 rows 10.2 / 9.1).
   if (tw > 5 || steps > 5 || N < kRpCus * kTile || !(D > 256 || (D > 128 && D % 32 != 0))) return false;
