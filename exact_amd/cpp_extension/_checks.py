@@ -18,11 +18,11 @@ def on_device(t):
 def plain_values(*tensors):
     """True where a kernel may stand in for differentiable operations on these
     tensors (None is skipped) without anyone missing them: no tensor subclass, no
-    forward-mode tangent, no trace being recorded, no dispatch mode listening; and
-    where memory holds their values as they are: no wrapper of a function transform
-    (vmap, a batched backward, functionalisation), no sparse layout, no negation
-    still to be made."""
-    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+    forward-mode tangent, no trace or compilation in progress, no dispatch mode
+    listening; and where memory holds their values as they are: no wrapper of a
+    function transform (vmap, a batched backward, functionalisation), no sparse
+    layout, no negation still to be made."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
         return False
     unpack = torch.autograd.forward_ad.unpack_dual
     wrapped, batched = torch._C._functorch.is_functorch_wrapped_tensor, torch._C._functorch.is_legacy_batchedtensor

@@ -66,7 +66,7 @@ def _short_weight_gradient(grad_output, input):  # noqa: A002
             and not _checks.recorded(grad_output, input) and _checks.plain_values(grad_output, input)
             and grad_output.stride(1) == 1 and input.stride(1) == 1
             and grad_output.stride(0) >= grad_output.shape[1] and input.stride(0) >= input.shape[1]
-            and _atomics_allowed() and not torch.compiler.is_compiling())
+            and _atomics_allowed())
 
 
 def weight_gradient(grad_output, input):  # noqa: A002

@@ -77,3 +77,10 @@ def test_drawn_matrices_under_vmap(backend):
     torch.manual_seed(3)
     got = torch.vmap(lambda x: ops._projection_matrix(12, 5, x.device, x.dtype), randomness="different")(torch.zeros(2, 3, device=backend))
     assert got.shape == (2, 12, 5) and torch.equal(got.abs(), torch.full_like(got, 1.0 / 5 ** 0.5))
+
+
+def test_drawn_matrices_inside_a_compiled_region(backend):
+    """The framework's expression, without a break in the graph."""
+    compiled = torch.compile(lambda x: ops._projection_matrix(12, 5, x.device, x.dtype) * 1, backend="eager", fullgraph=True)
+    got = compiled(torch.zeros(2, 3, device=backend))
+    assert got.shape == (12, 5) and torch.equal(got.abs(), torch.full_like(got, 1.0 / 5 ** 0.5))

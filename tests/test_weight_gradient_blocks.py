@@ -161,3 +161,11 @@ def test_short_batches_whose_values_do_not_lie_in_plain_memory(backend, N):
     config.compress_activation = False
     got, = torch.autograd.grad(layer(x), layer.weight, dy, is_grads_batched=True)
     assert close(got)
+
+
+def test_short_batches_inside_a_compiled_region(backend):
+    """The framework's product, without a break in the graph."""
+    g = torch.Generator().manual_seed(2)
+    dy, x = torch.randn(4200, 6, generator=g).to(backend), torch.randn(4200, 9, generator=g).to(backend)
+    compiled = torch.compile(bf.weight_gradient, backend="eager", fullgraph=True)
+    assert torch.equal(compiled(dy, x), dy.t().mm(x))
